@@ -100,6 +100,35 @@ def test_softmax_many_short_rows(ops, shape):
     assert_softmax_close(host(ops.softmax(dev(xh))), xh, -1, str(shape) + " half")
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,n", [(1030, n) for n in (3, 4, 7, 8, 9, 31, 33, 64, 65, 96, 127, 129, 255, 257, 385, 513, 769, 1023, 1025)] +
+                         [(1030, 1537), (1025, 2049), (5, 513), (5, 4095), (5, 4097), (3, 8191), (3, 8192), (513, 8193), (1025, 8207),
+                          (513, 16385), (512, 32767), (512, 32768)])
+def test_softmax_rows_whose_last_vector_is_moved_back(ops, rows, n, dtype):
+    """Lanes of a row hold 16-byte vectors that start on any element; a row that is no whole number
+    of them has its last one moved back, and what it shares with the one before counts once: row
+    lengths around the lanes x vectors the kernels are built for, with the tensor itself off 16
+    bytes as well; special rows; in place; and the replacement of NaN."""
+    rng = np.random.default_rng(rows + n)
+    x = (rng.standard_normal((rows, n)) * 3).astype(dtype)
+    x[0, n - 1], x[1, 0], x[2, :] = np.nan, np.inf, -np.inf
+    buf = torch.empty(rows * n + 1, dtype=torch.float16 if dtype == np.float16 else torch.float32, device="cuda")
+    view = buf[1:].view(rows, n)
+    view.copy_(dev(x))
+    exp = oracle.softmax(x, -1)
+    got = host(ops.softmax(view))
+    assert_softmax_close(got, x, -1, "%d x %d" % (rows, n))
+    nan = np.isnan(exp)
+    fixed = host(ops.softmax(view, nan_where=True, nan_value=0.25))
+    assert np.array_equal(fixed[~nan], got[~nan]) and np.all(fixed[nan] == dtype(0.25))
+    out = torch.full((rows * n + 2,), 7.0, dtype=buf.dtype, device="cuda")
+    ops.softmax(view, out=out[1:-1].view(rows, n))
+    o = host(out)
+    assert o[0] == 7.0 and o[-1] == 7.0 and np.array_equal(o[1:-1].reshape(rows, n), got, equal_nan=True)
+    ops.softmax(view, out=view)  # in place
+    assert np.array_equal(host(view), got, equal_nan=True)
+
+
 @pytest.mark.parametrize("shape,axis", [((5, 7, 9), 0), ((5, 7, 9), 1), ((5, 7, 9), 2), ((2, 3, 4, 5), 0), ((2, 3, 4, 5), 1),
                                         ((2, 3, 4, 5), -2), ((300,), 0), ((4, 2500, 3), 1), ((3, 70, 130), 1), ((2, 5, 64), 1),
                                         ((2, 1000, 64), 1), ((1, 4096, 300), 1), ((2, 200, 7, 5), 1), ((3, 129, 2), 1),

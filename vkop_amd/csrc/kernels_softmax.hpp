@@ -1,8 +1,9 @@
 // Throughput kernels for the plain softmax operator.
 //
 // Contiguous rows (the reduced axis is the last one):
+//   softmax_group_kernel    rows of up to a wave's registers: 8 to 64 lanes a row.
 //   softmax_row_kernel      one workgroup holds a whole row in registers: one
-//                           read, one write (rows up to NT * V vectors).
+//                           read, one write.
 //   softmax_stats_kernel +  long rows, or too few rows to fill the chip: a row
 //   softmax_scale_kernel    is split into chunks, one workgroup each.  The first
 //                           kernel leaves (maximum, sum of exp(x - maximum)) per
@@ -10,8 +11,7 @@
 //                           writes exp(x - M) / S for its chunk.  The second
 //                           read of the input comes from the Infinity Cache for
 //                           tensors that fit it.
-//   softmax_wave_kernel     rows of up to 512 elements: one wave per row, four rows a
-//                           workgroup, no LDS.
+//   softmax_thread_kernel   rows of fewer elements than a vector.
 // Strided lines (another axis, long lines):
 //   softmax_strided_tile_kernel  a tile of up to 64 neighbouring lines per workgroup of 16 waves,
 //                           rows dealt to the waves, three passes over the tile; with few
@@ -50,191 +50,212 @@ struct ChunkStat {
     uint32_t nmin;  // ... and how many elements equal it (0: none set apart)
 };
 
-// ---- a whole row per workgroup ------------------------------------------------------
-// A workgroup takes the rows blockIdx.x, blockIdx.x + gridDim.x, ... (the launch caps the grid:
-// half a million workgroups of one short row each are handed out at about 2 ns apiece, which
-// bounded [16,32,1024,1024] in both precisions); the next row's loads are issued before the
-// current row's arithmetic.
-constexpr uint32_t kSoftmaxRowGridMax = 16384;
-template <typename T, int NT, int V, bool ALIGNED>
-__global__ __launch_bounds__(NT) void softmax_row_kernel(const T *in, T *out, uint32_t rows, uint32_t n, int nan_where,
-                                                         float nan_value) {
-    constexpr int VEC = Vec128<T>::N;
-    constexpr int NW = NT / kWave;
-    __shared__ float fscratch[NW];
-    __shared__ double dscratch[NW];
-    const uint32_t tid = threadIdx.x;
-    auto load_row = [&](Vec128<T> (&q)[V], uint32_t row) __attribute__((always_inline)) {
-        const T *rowp = in + static_cast<size_t>(row) * n;
-#pragma unroll
-        for (int i = 0; i < V; i++) {
-            const uint32_t e0 = (static_cast<uint32_t>(i) * NT + tid) * VEC;
-            q[i].v = make_uint4(0, 0, 0, 0);
-            if constexpr (ALIGNED) {
-                q[i].load(rowp + (e0 < n ? e0 : 0u));
-            } else {
-#pragma unroll
-                for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < n ? e0 + c : 0u));
-            }
-        }
+// ---- short rows, many of them: G lanes a row, 128-bit loads ---------------------------------
+// Rows of VEC to 64 * V * VEC elements, at any alignment.  G lanes of a wave share a row (64 / G
+// rows a wave), lane l of them holds vectors l, l + G, ..., V of them; maximum and sum cross the G
+// lanes without LDS or a barrier.  A row that is no whole number of vectors has its last vector
+// moved back to end with the row: the elements it shares with the vector before are loaded twice,
+// left out of the sum once, and stored twice with the same bits (the launch makes every slot but a
+// lane's last a full vector: (V - 1) * G * VEC < n).
+// What bounds it is the memory system, once the arithmetic is out of its way: loads and stores are
+// non-temporal, a thread keeps few vectors, and a wave takes its rows and ends -- a loop over rows
+// with the next one's loads in flight, the form before, copies at 4.8 to 5.7 TB/s where waves that
+// end copy at 6.2 to 6.6.  [524288,1024] f16 422 -> 343 us (6.3 TB/s), f32 827 -> 728; [302592,197]
+// f16 83 -> 48 us (element by element before), f32 133 -> 102; [65536,64] f32 13.7 -> 7.2 us.
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
+}
+template <int G> __device__ __forceinline__ float group_max(float v) {
+    static_assert(G >= 8 && G <= kWave, "lanes a row");
+    auto step = [](float a, auto tag) { return fmaxf(a, __uint_as_float(dpp_u32<decltype(tag)::value>(__float_as_uint(a)))); };
+    v = step(v, std::integral_constant<int, 0xB1>{});   // lane ^ 1
+    v = step(v, std::integral_constant<int, 0x4E>{});   // lane ^ 2
+    v = step(v, std::integral_constant<int, 0x141>{});  // the other four of eight
+    if constexpr (G >= 16) v = step(v, std::integral_constant<int, 0x140>{});  // the other eight of sixteen
+    if constexpr (G >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    if constexpr (G >= 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    }
+    return v;
+}
+template <int G> __device__ __forceinline__ double group_sum(double v) {
+    auto join = [](uint32_t lo, uint32_t hi) { return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo)); };
+    auto step = [&](double a, auto tag) {
+        constexpr int ctrl = decltype(tag)::value;
+        const uint64_t u = static_cast<uint64_t>(__double_as_longlong(a));
+        return a + join(dpp_u32<ctrl>(static_cast<uint32_t>(u)), dpp_u32<ctrl>(static_cast<uint32_t>(u >> 32)));
     };
-    Vec128<T> q[V], qn[V];
-    load_row(q, blockIdx.x);
-    for (uint32_t row = blockIdx.x; row < rows; row += gridDim.x) {
-        const uint32_t next = row + gridDim.x;
-        if (next < rows) load_row(qn, next);  // (the same in every thread)
-        float m = -INFINITY;
+    v = step(v, std::integral_constant<int, 0xB1>{});
+    v = step(v, std::integral_constant<int, 0x4E>{});
+    v = step(v, std::integral_constant<int, 0x141>{});
+    if constexpr (G >= 16) v = step(v, std::integral_constant<int, 0x140>{});
+    if constexpr (G >= 32) {
+        const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
+        const auto lo = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(u), static_cast<uint32_t>(u), false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(static_cast<uint32_t>(u >> 32), static_cast<uint32_t>(u >> 32), false, false);
+        v = join(lo[0], hi[0]) + join(lo[1], hi[1]);
+    }
+    if constexpr (G >= 64) {
+        const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
+        const auto lo = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(u), static_cast<uint32_t>(u), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(static_cast<uint32_t>(u >> 32), static_cast<uint32_t>(u >> 32), false, false);
+        v = join(lo[0], hi[0]) + join(lo[1], hi[1]);
+    }
+    return v;
+}
+// 1 / s for a row's sum (1 <= s < 2^32, or NaN): the hardware reciprocal (about 2^-22) and two Newton steps,
+// within a unit of double; a division proper is twice the instructions, and a wave of short rows
+// pays it once per handful of elements.
+__device__ __forceinline__ double reciprocal_of_sum(double s) {
+    double y = __builtin_amdgcn_rcp(s);
+    y = fma(fma(-s, y, 1.0), y, y);
+    return fma(fma(-s, y, 1.0), y, y);
+}
+// What a lane of a row does with its V vectors, in the group kernel and in the row kernel: `stride`
+// vectors lie between two of them, `at` is the first one's number in the row.  Only the last may
+// reach the row's end.
+template <typename T, int V> struct RowPiece {
+    static constexpr int VEC = Vec128<T>::N;
+    Vec128<T> q[V];
+    float e[V][VEC];
+    uint32_t first[V];  // where in the row each vector was loaded from
+    uint32_t dup;       // leading elements of the last vector that another vector holds too (VEC: all of them)
+    __device__ __forceinline__ void load(const T *rowp, uint32_t n, uint32_t at, uint32_t stride) {
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const uint32_t e0 = (static_cast<uint32_t>(i) * NT + tid) * VEC;
-#pragma unroll
-            for (int c = 0; c < VEC; c++)
-                if (e0 + c < n) m = fmaxf(m, q[i].get(c));
+            const uint32_t e0 = (static_cast<uint32_t>(i) * stride + at) * VEC;
+            first[i] = i == V - 1 ? min(e0, n - VEC) : e0;
+            q[i].v = load16_stream(rowp + first[i]);
         }
-        m = block_max<NT>(m, fscratch);
-        // the terms replace the inputs in the registers (a term is a float; for half
-        // tensors it is kept in a float array instead)
-        float e[V][VEC];
+        const uint32_t e_last = (static_cast<uint32_t>(V - 1) * stride + at) * VEC;
+        dup = e_last > n - VEC ? min(e_last - (n - VEC), static_cast<uint32_t>(VEC)) : 0u;
+    }
+    __device__ __forceinline__ float largest() const {  // (drops NaN)
+        float m = -INFINITY;
+        if constexpr (sizeof(T) == 2) {
+            uint32_t pk = 0xFC00FC00u;
+#pragma unroll
+            for (int i = 0; i < V; i++)
+                pk = max_half2(max_half2(pk, max_half2(q[i].v.x, q[i].v.y)), max_half2(q[i].v.z, q[i].v.w));
+            m = fmaxf(__half2float(__ushort_as_half(static_cast<uint16_t>(pk & 0xFFFFu))),
+                      __half2float(__ushort_as_half(static_cast<uint16_t>(pk >> 16))));
+        } else {
+#pragma unroll
+            for (int i = 0; i < V; i++)
+                m = max3(max3(m, q[i].get(0), q[i].get(1)), q[i].get(2), q[i].get(3));
+        }
+        return m;
+    }
+    // the terms, and their sum over this lane's elements
+    __device__ __forceinline__ double terms(float m) {
         TermSum<T> acc = 0;
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const uint32_t e0 = (static_cast<uint32_t>(i) * NT + tid) * VEC;
 #pragma unroll
             for (int c = 0; c < VEC; c++) {
-                e[i][c] = e0 + c < n ? softmax_term_as<T>(q[i].get(c), m) : 0.f;
-                acc += static_cast<TermSum<T>>(e[i][c]);
+                e[i][c] = softmax_term_as<T>(q[i].get(c), m);
+                acc += static_cast<TermSum<T>>(i < V - 1 || static_cast<uint32_t>(c) >= dup ? e[i][c] : 0.f);
             }
         }
-        const double rinv = 1.0 / block_sum<NT>(static_cast<double>(acc), dscratch);
-        T *orow = out + static_cast<size_t>(row) * n;
+        return static_cast<double>(acc);
+    }
+    __device__ __forceinline__ void store(T *orow, double rinv, bool live, int nan_where, float nan_value) {
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const uint32_t e0 = (static_cast<uint32_t>(i) * NT + tid) * VEC;
             Vec128<T> r;
             r.v = make_uint4(0, 0, 0, 0);
 #pragma unroll
             for (int c = 0; c < VEC; c++) {
-                float p = round_to_storage<T>(scale_term<T>(e[i][c], rinv));
-                if (nan_where && p != p) p = nan_value;
-                if constexpr (ALIGNED) r.set(c, p);
-                else if (e0 + c < n) store_elem(orow, e0 + c, p);
+                e[i][c] = scale_term<T>(e[i][c], rinv);
+                r.set(c, e[i][c]);
             }
-            if constexpr (ALIGNED)
-                if (e0 < n) *reinterpret_cast<uint4 *>(orow + e0) = r.v;
-        }
+            if (nan_where) {  // (the same in every thread)
 #pragma unroll
-        for (int i = 0; i < V; i++) q[i] = qn[i];
+                for (int c = 0; c < VEC; c++)
+                    if (e[i][c] != e[i][c]) r.set(c, nan_value);
+            }
+            if (live && (i < V - 1 || dup < static_cast<uint32_t>(VEC))) store16_stream(orow + first[i], r.v);
+        }
     }
+};
+
+constexpr int kSoftmaxGroupThreads = 256;
+template <typename T, int G, int V>
+__global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(const T *in, T *out, uint32_t rows, uint32_t n,
+                                                                            int nan_where, float nan_value) {
+    const uint32_t row = blockIdx.x * (kSoftmaxGroupThreads / G) + threadIdx.x / G;
+    const bool live = row < rows;
+    const size_t row0 = static_cast<size_t>(live ? row : rows - 1u) * n;  // (lanes past the last row shadow it and store nothing)
+    RowPiece<T, V> p;
+    p.load(in + row0, n, threadIdx.x % G, G);
+    const float m = group_max<G>(p.largest());
+    const double rinv = reciprocal_of_sum(group_sum<G>(p.terms(m)));
+    p.store(out + row0, rinv, live, nan_where, nan_value);
 }
 
-// ---- rows of a few hundred to two thousand elements, many of them: a wave per row, 128-bit loads ----
-// Rows of up to 64 * V vectors that start on 16 bytes (n a multiple of the vector width): lane l
-// holds vectors l, l + 64, ...; maximum and sum cross the lanes without LDS or a barrier (a
-// workgroup per row pays four barriers a row for two waves' work), four rows a workgroup, each
-// wave on to its next row (grid-stride) with that row's loads issued before this row's arithmetic.
-constexpr int kSoftmaxVecRows = 4;  // rows (waves) per workgroup
+// ---- a row per workgroup ----------------------------------------------------------------------
+// Rows that a workgroup holds in registers, V vectors a thread; the workgroup has as many waves as
+// the row needs (blockDim.x: at most 1024), so that a row just past a power of two does not leave
+// half of it idle.  One read, one write, two barriers.  [9872,8296] f32 241 -> 114 us, f16 88 -> 61;
+// [2000,20001] f32 225 -> 60 us, f16 133 -> 39 (element by element before); [256,8192] f32 8.4 -> 5.5.
+constexpr int kSoftmaxRowWavesMax = 16;
 template <typename T, int V>
-__global__ __launch_bounds__(kSoftmaxVecRows *kWave) void softmax_wave_vec_kernel(const T *__restrict__ in, T *__restrict__ out,
-                                                                                  uint32_t rows, uint32_t n, int nan_where,
-                                                                                  float nan_value) {
-    constexpr int VEC = Vec128<T>::N;
-    const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const uint32_t step = gridDim.x * kSoftmaxVecRows;
-    auto load_row = [&](Vec128<T> (&q)[V], uint32_t row) __attribute__((always_inline)) {
-        const T *rowp = in + static_cast<size_t>(row) * n;
-#pragma unroll
-        for (int i = 0; i < V; i++) {
-            const uint32_t e0 = (static_cast<uint32_t>(i) * kWave + lane) * VEC;
-            q[i].load(rowp + (e0 < n ? e0 : 0u));
-        }
-    };
-    uint32_t row = blockIdx.x * kSoftmaxVecRows + wave;
-    if (row >= rows) return;  // (a whole wave)
-    Vec128<T> q[V], qn[V];
-    load_row(q, row);
-    for (; row < rows; row += step) {
-        if (row + step < rows) load_row(qn, row + step);  // (wave-uniform)
-        float m = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < V; i++) {
-            const bool live = (static_cast<uint32_t>(i) * kWave + lane) * VEC < n;
-#pragma unroll
-            for (int c = 0; c < VEC; c++)
-                if (live) m = fmaxf(m, q[i].get(c));
-        }
-        m = wave_max_f32_uniform(m);
-        float e[V][VEC];
-        TermSum<T> acc = 0;
-#pragma unroll
-        for (int i = 0; i < V; i++) {
-            const bool live = (static_cast<uint32_t>(i) * kWave + lane) * VEC < n;
-#pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                e[i][c] = live ? softmax_term_as<T>(q[i].get(c), m) : 0.f;
-                acc += static_cast<TermSum<T>>(e[i][c]);
-            }
-        }
-        const double rinv = 1.0 / wave_sum_f64_uniform(static_cast<double>(acc));
-        T *orow = out + static_cast<size_t>(row) * n;
-#pragma unroll
-        for (int i = 0; i < V; i++) {
-            const uint32_t e0 = (static_cast<uint32_t>(i) * kWave + lane) * VEC;
-            Vec128<T> r;
-            r.v = make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                float p = round_to_storage<T>(scale_term<T>(e[i][c], rinv));
-                if (nan_where && p != p) p = nan_value;
-                r.set(c, p);
-            }
-            if (e0 < n) *reinterpret_cast<uint4 *>(orow + e0) = r.v;
-        }
-#pragma unroll
-        for (int i = 0; i < V; i++) q[i] = qn[i];
+__global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel(const T *in, T *out, uint32_t n, int nan_where,
+                                                                                float nan_value) {
+    __shared__ float fscratch[kSoftmaxRowWavesMax];
+    __shared__ double dscratch[kSoftmaxRowWavesMax];
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave, waves = blockDim.x / kWave;
+    const size_t row0 = static_cast<size_t>(blockIdx.x) * n;
+    RowPiece<T, V> p;
+    p.load(in + row0, n, tid, blockDim.x);
+    float m = group_max<kWave>(p.largest());
+    if (waves > 1) {
+        if (lane == 0) fscratch[wave] = m;
+        __syncthreads();
+        const uint32_t w = lane & (kSoftmaxRowWavesMax - 1);
+        m = group_max<kSoftmaxRowWavesMax>(w < waves ? fscratch[w] : -INFINITY);
     }
+    double s = group_sum<kWave>(p.terms(m));
+    if (waves > 1) {
+        if (lane == 0) dscratch[wave] = s;
+        __syncthreads();
+        const uint32_t w = lane & (kSoftmaxRowWavesMax - 1);
+        s = group_sum<kSoftmaxRowWavesMax>(w < waves ? dscratch[w] : 0.0);
+    }
+    p.store(out + row0, reciprocal_of_sum(s), true, nan_where, nan_value);
 }
 
-// ---- short rows: one wave per row ---------------------------------------------------------
-// Rows of up to 64 * E elements (E <= 8): lane l holds elements l, l + 64, ...; every
-// load and store instruction of a wave covers 64 neighbouring elements whatever the row's
-// alignment; maximum and sum cross the lanes without LDS or a barrier.  Four rows a
-// workgroup.  (A workgroup of 256 threads per row leaves three quarters of them idle on a
-// 64-element row and takes two barriers: [65536,64] took 68 us.)
-constexpr int kSoftmaxWaveRows = 4;  // rows (waves) per workgroup
-template <typename T, int E>
-__global__ __launch_bounds__(kSoftmaxWaveRows *kWave) void softmax_wave_kernel(const T *__restrict__ in, T *__restrict__ out,
-                                                                                uint32_t rows, uint32_t n, int nan_where,
-                                                                                float nan_value) {
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t row = blockIdx.x * kSoftmaxWaveRows + threadIdx.x / kWave;
-    if (row >= rows) return;  // (the whole wave)
+// ---- rows shorter than a vector: a thread each ------------------------------------------------
+template <typename T>
+__global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_thread_kernel(const T *in, T *out, uint32_t rows, uint32_t n,
+                                                                             int nan_where, float nan_value) {
+    constexpr uint32_t VEC = Vec128<T>::N;
+    const uint32_t row = blockIdx.x * kSoftmaxGroupThreads + threadIdx.x;
+    if (row >= rows) return;
     const T *rowp = in + static_cast<size_t>(row) * n;
-    T *orow = out + static_cast<size_t>(row) * n;
-    float x[E];
+    float x[VEC - 1], m = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < E; j++) {
-        const uint32_t e = static_cast<uint32_t>(j) * kWave + lane;
-        x[j] = load_elem(rowp, e < n ? e : 0u);
+    for (uint32_t j = 0; j < VEC - 1; j++) {
+        x[j] = load_elem(rowp, j < n ? j : 0u);
+        if (j < n) m = fmaxf(m, x[j]);
     }
-    float m = -INFINITY;
-#pragma unroll
-    for (int j = 0; j < E; j++)
-        if (static_cast<uint32_t>(j) * kWave + lane < n) m = fmaxf(m, x[j]);  // (drops NaN)
-    m = wave_max_f32_uniform(m);
-    float t[E];
     TermSum<T> acc = 0;
 #pragma unroll
-    for (int j = 0; j < E; j++) {
-        t[j] = static_cast<uint32_t>(j) * kWave + lane < n ? softmax_term_as<T>(x[j], m) : 0.f;
-        acc += static_cast<TermSum<T>>(t[j]);
+    for (uint32_t j = 0; j < VEC - 1; j++) {
+        x[j] = j < n ? softmax_term_as<T>(x[j], m) : 0.f;
+        acc += static_cast<TermSum<T>>(x[j]);
     }
-    const double rinv = 1.0 / wave_sum_f64_uniform(static_cast<double>(acc));
+    const double rinv = reciprocal_of_sum(static_cast<double>(acc));
+    T *orow = out + static_cast<size_t>(row) * n;
 #pragma unroll
-    for (int j = 0; j < E; j++) {
-        const uint32_t e = static_cast<uint32_t>(j) * kWave + lane;
-        float p = round_to_storage<T>(scale_term<T>(t[j], rinv));
+    for (uint32_t j = 0; j < VEC - 1; j++) {
+        float p = round_to_storage<T>(scale_term<T>(x[j], rinv));
         if (nan_where && p != p) p = nan_value;
-        if (e < n) store_elem(orow, e, p);
+        if (j < n) store_elem(orow, j, p);
     }
 }
 

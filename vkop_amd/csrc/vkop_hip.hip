@@ -160,8 +160,8 @@ const RowShape kShapesF32[] = {{256, 1}, {256, 2}, {256, 4}, {256, 8}, {512, 8},
 const RowShape kShapesF16[] = {{128, 1}, {256, 1}, {256, 2}, {256, 4}, {512, 4}, {1024, 4}};
 
 struct SoftmaxPlan {
-    enum Kind { kGeneralLines, kGeneralStrided, kRow, kWaveRow, kChunked, kStridedRegs, kStridedTile } kind = kGeneralLines;
-    RowShape shape{0, 0};
+    enum Kind { kGeneralLines, kGeneralStrided, kThread, kGroup, kRow, kChunked, kStridedRegs, kStridedTile } kind = kGeneralLines;
+    RowShape shape{0, 0};  // kChunked; kGroup: lanes a row and vectors a lane; kRow: threads and vectors a thread
     uint32_t g = 1, per = 0;
     uint32_t ti_shift = 0;  // kStridedTile: log2 of the lines a tile
     size_t workspace = 0;
@@ -221,20 +221,30 @@ SoftmaxPlan plan_softmax(const View &v, int dtype) {
         }
         return p;
     }
-    if (n <= 8u * vkop::kWave) {  // short rows: a wave each
-        p.kind = SoftmaxPlan::kWaveRow;
+    if (n < vec) {
+        p.kind = SoftmaxPlan::kThread;
         return p;
     }
-    const uint32_t biggest = static_cast<uint32_t>(shapes[5].nt) * shapes[5].v * vec;
-    // a whole row per workgroup when rows are short or there are enough of them
-    if (n <= 8192 || (n <= biggest && rows >= 512)) {
-        for (int i = 0; i < 6; i++) {
-            if (static_cast<uint32_t>(shapes[i].nt) * shapes[i].v * vec >= n) {
-                p.kind = SoftmaxPlan::kRow;
-                p.shape = shapes[i];
-                return p;
-            }
-        }
+    // Rows that 8 to 64 lanes of a wave hold: the fewest lanes that need at most VT vectors each (16 to
+    // 24 elements a lane: the cross-lane steps and the reciprocal are paid once for that many).
+    const uint32_t nvec = (n + vec - 1) / vec, vt = dtype == VKOP_HIP_F32 ? 4u : 3u;
+    if (nvec <= vt * vkop::kWave && (n <= 512 || rows >= 1024)) {
+        uint32_t g = 8;
+        while ((nvec + g - 1) / g > vt) g *= 2;
+        p.kind = SoftmaxPlan::kGroup;
+        p.shape = RowShape{static_cast<int>(g), static_cast<int>((nvec + g - 1) / g)};
+        return p;
+    }
+    // A row per workgroup where that fills the chip or the row is short: with many rows four (f16:
+    // two) vectors a thread, else as few as the 1024 threads of a workgroup allow.
+    const uint32_t vmax = dtype == VKOP_HIP_F32 ? 8u : 4u;
+    if (nvec <= vmax * 1024u && (n <= 8192 || rows >= 512)) {
+        uint32_t v = rows >= 1024 ? vmax / 2 : 1u;
+        while ((nvec + v - 1) / v > 1024u) v++;
+        const uint32_t nt = ((nvec + v - 1) / v + vkop::kWave - 1) / vkop::kWave * vkop::kWave;
+        p.kind = SoftmaxPlan::kRow;
+        p.shape = RowShape{static_cast<int>(nt), static_cast<int>((nvec + nt - 1) / nt)};
+        return p;
     }
     // chunked: the largest chunk that still leaves >= 1024 workgroups, else the smallest
     int pick = -1;
@@ -268,44 +278,35 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
     const bool aligned = reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
                          v.g.n % vec == 0;
     switch (p.kind) {
+    case SoftmaxPlan::kThread: {
+        const uint32_t blocks = (lines + vkop::kSoftmaxGroupThreads - 1) / vkop::kSoftmaxGroupThreads;
+        vkop::softmax_thread_kernel<T><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value);
+        return launched("softmax_thread_kernel");
+    }
+    case SoftmaxPlan::kGroup: {
+        const uint32_t per_block = static_cast<uint32_t>(vkop::kSoftmaxGroupThreads / p.shape.nt);
+        const uint32_t blocks = (lines + per_block - 1) / per_block;
+#define VKOP_GROUP(G, V)                                                                                                     \
+    if (p.shape.nt == G && p.shape.v == V) {                                                                                 \
+        vkop::softmax_group_kernel<T, G, V><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value); \
+        return launched("softmax_group_kernel");                                                                             \
+    }
+#define VKOP_GROUPS(G) VKOP_GROUP(G, 1) VKOP_GROUP(G, 2) VKOP_GROUP(G, 3) if constexpr (sizeof(T) == 4) { VKOP_GROUP(G, 4) }
+        VKOP_GROUPS(8) VKOP_GROUPS(16) VKOP_GROUPS(32) VKOP_GROUPS(64)
+#undef VKOP_GROUPS
+#undef VKOP_GROUP
+        return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_group_kernel for %d lanes x %d", p.shape.nt, p.shape.v);
+    }
     case SoftmaxPlan::kRow: {
-        bool done = false;
-        const uint32_t row_grid = std::min(lines, vkop::kSoftmaxRowGridMax);
-        // thousands of rows that a wave holds in a few 128-bit loads a lane: a wave per row, no barrier
-        const uint32_t vectors = (v.g.n + vec - 1) / vec;
-        if (aligned && lines >= 4096 && vectors <= 4 * vkop::kWave) {
-            const uint32_t wgs = std::min((lines + vkop::kSoftmaxVecRows - 1) / vkop::kSoftmaxVecRows, 8192u);
-#define VKOP_VEC_ROW(V)                                                                                                          \
-    vkop::softmax_wave_vec_kernel<T, V><<<wgs, vkop::kSoftmaxVecRows * vkop::kWave, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value)
-            if (vectors <= vkop::kWave) VKOP_VEC_ROW(1);
-            else if (vectors <= 2 * vkop::kWave) VKOP_VEC_ROW(2);
-            else VKOP_VEC_ROW(4);
-#undef VKOP_VEC_ROW
-            return launched("softmax_wave_vec_kernel");
-        }
-#define VKOP_ROW(NT, V)                                                                                        \
-    if (!done && p.shape.nt == NT && p.shape.v == V) {                                                         \
-        if (aligned) vkop::softmax_row_kernel<T, NT, V, true><<<row_grid, NT, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value); \
-        else vkop::softmax_row_kernel<T, NT, V, false><<<row_grid, NT, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value);        \
-        done = true;                                                                                           \
+#define VKOP_ROW(V)                                                                                                  \
+    if (p.shape.v == V) {                                                                                            \
+        vkop::softmax_row_kernel<T, V><<<lines, p.shape.nt, 0, st>>>(in, out, v.g.n, nan_where, nan_value);          \
+        return launched("softmax_row_kernel");                                                                       \
     }
-        VKOP_FOR_EACH_ROW_SHAPE(VKOP_ROW, T)
+        VKOP_ROW(1) VKOP_ROW(2) VKOP_ROW(3) VKOP_ROW(4)
+        if constexpr (sizeof(T) == 4) { VKOP_ROW(5) VKOP_ROW(6) VKOP_ROW(7) VKOP_ROW(8) }
 #undef VKOP_ROW
-        if (!done) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_row_kernel for %d x %d", p.shape.nt, p.shape.v);
-        return launched("softmax_row_kernel");
-    }
-    case SoftmaxPlan::kWaveRow: {
-        const uint32_t blocks = (lines + vkop::kSoftmaxWaveRows - 1) / vkop::kSoftmaxWaveRows;
-        const uint32_t per_lane = (v.g.n + vkop::kWave - 1) / vkop::kWave;
-#define VKOP_WAVE_ROW(E)                                                                                    \
-    vkop::softmax_wave_kernel<T, E><<<blocks, vkop::kSoftmaxWaveRows * vkop::kWave, 0, st>>>(in, out, lines, v.g.n, \
-                                                                                              nan_where, nan_value)
-        if (per_lane <= 1) VKOP_WAVE_ROW(1);
-        else if (per_lane <= 2) VKOP_WAVE_ROW(2);
-        else if (per_lane <= 4) VKOP_WAVE_ROW(4);
-        else VKOP_WAVE_ROW(8);
-#undef VKOP_WAVE_ROW
-        return launched("softmax_wave_kernel");
+        return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_row_kernel for %d x %d", p.shape.nt, p.shape.v);
     }
     case SoftmaxPlan::kChunked: {
         if (ws == nullptr || ws_bytes < p.workspace)
