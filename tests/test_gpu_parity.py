@@ -103,7 +103,8 @@ def test_softmax_many_short_rows(ops, shape):
 @pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
 @pytest.mark.parametrize("rows,n", [(1030, n) for n in (3, 4, 7, 8, 9, 31, 33, 64, 65, 96, 127, 129, 255, 257, 385, 513, 769, 1023, 1025)] +
                          [(1030, 1537), (1025, 2049), (5, 513), (5, 4095), (5, 4097), (3, 8191), (3, 8192), (513, 8193), (1025, 8207),
-                          (513, 16385), (512, 32767), (512, 32768)])
+                          (513, 16385), (512, 32767), (512, 32768),
+                          (3, 8193), (3, 8195), (3, 16391), (67, 16384), (3, 40001), (5, 131079), (3, 600001), (3, 8400001)])
 def test_softmax_rows_whose_last_vector_is_moved_back(ops, rows, n, dtype):
     """Lanes of a row hold 16-byte vectors that start on any element; a row that is no whole number
     of them has its last one moved back, and what it shares with the one before counts once: row

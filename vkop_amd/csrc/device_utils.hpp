@@ -47,6 +47,10 @@ template <typename T> __device__ __forceinline__ uint4 load16_stream(const T *p)
     const auto v = __builtin_nontemporal_load(reinterpret_cast<const vec16_any *>(p));
     return make_uint4(v.x, v.y, v.z, v.w);
 }
+template <typename T> __device__ __forceinline__ uint4 load16_any(const T *p) {
+    const auto v = *reinterpret_cast<const vec16_any *>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
 template <typename T> __device__ __forceinline__ void store16_stream(T *p, const uint4 &u) {
     vec16_any v;
     v.x = u.x, v.y = u.y, v.z = u.z, v.w = u.w;
@@ -58,6 +62,11 @@ template <typename T> __device__ __forceinline__ void store16_stream(T *p, const
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float min3(float a, float b, float c) {
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
 // Larger halves of two pairs, NaN dropped.

@@ -557,6 +557,7 @@ template <> struct Vec128<float> {
     static constexpr int N = 4;
     uint4 v;
     __device__ __forceinline__ void load(const float *p) { v = *reinterpret_cast<const uint4 *>(p); }
+    __device__ __forceinline__ void load_any(const float *p) { v = load16_any(p); }  // (any element: no 16-byte start asked for)
     __device__ __forceinline__ float get(int c) const {
         return __uint_as_float(c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w);
     }
@@ -572,6 +573,7 @@ template <> struct Vec128<uint16_t> {
     static constexpr int N = 8;
     uint4 v;
     __device__ __forceinline__ void load(const uint16_t *p) { v = *reinterpret_cast<const uint4 *>(p); }
+    __device__ __forceinline__ void load_any(const uint16_t *p) { v = load16_any(p); }
     __device__ __forceinline__ float get(int c) const {
         const uint32_t w = (c >> 1) == 0 ? v.x : (c >> 1) == 1 ? v.y : (c >> 1) == 2 ? v.z : v.w;
         return __half2float(__ushort_as_half(static_cast<uint16_t>((c & 1) ? (w >> 16) : (w & 0xFFFFu))));

@@ -260,92 +260,88 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_thread_kernel(co
 }
 
 // ---- chunked rows: statistics ---------------------------------------------------------
-// Launch: rows * G workgroups; per = elements per chunk (multiple of the vector
-// width, <= NT * V * vector width).
-template <typename T, int NT, int V, bool ALIGNED>
+// Launch: rows * G workgroups; per = NT * V * VEC elements a chunk, whose vectors start on any
+// element (n >= VEC).  A row that is no whole number of vectors has its last one moved back to end
+// with the row; the leading elements it repeats -- of the chunk before, possibly -- count for the
+// chunk's maximum and minimum, which does no harm, and for nothing else.
+// The loads are ordinary ones: the scale kernel reads the same bytes again and finds them in the
+// Infinity Cache.
+template <typename T, int NT, int V>
 __global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__ in, ChunkStat *__restrict__ stats,
-                                                           uint32_t n, uint32_t G, uint32_t per) {
-    constexpr int VEC = Vec128<T>::N;
+                                                           uint32_t n, uint32_t G) {
+    constexpr uint32_t VEC = Vec128<T>::N;
     constexpr int NW = NT / kWave;
     __shared__ float fscratch[NW];
-    __shared__ double dscratch[NW];
     __shared__ float fscratch2[NW];
+    __shared__ double dscratch[NW];
     __shared__ uint32_t uscratch[NW];
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     const uint32_t row = blockIdx.x / G, chunk = blockIdx.x - row * G;
-    const uint32_t c0 = min(chunk * per, n), c1 = min(c0 + per, n);
+    const uint32_t e_first = chunk * (NT * V * VEC) + tid * VEC;
     const T *rowp = in + static_cast<size_t>(row) * n;
     Vec128<T> q[V];
 #pragma unroll
-    for (int i = 0; i < V; i++) {
-        const uint32_t e0 = c0 + (static_cast<uint32_t>(i) * NT + tid) * VEC;
-        q[i].v = make_uint4(0, 0, 0, 0);
-        if constexpr (ALIGNED) {
-            q[i].load(rowp + (e0 < c1 ? e0 : 0u));
-        } else {
-#pragma unroll
-            for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < c1 ? e0 + c : 0u));
-        }
-    }
-    // The copies of the chunk's smallest value are set apart and counted: a value that fills most
-    // of a row (padding, a floor, zeros) is usually its smallest, every copy of it has the same
-    // term, and that term's error would go into the sum thousands of times over -- the row's sum
-    // is DEFINED with exp_accurate(fl(x - M)) for each, which only the kernel that knows M can
-    // count (4 ulp on rows of one value and a few peaks otherwise).  Maximum and minimum in one
-    // pass and one reduction.
+    for (int i = 0; i < V; i++) q[i].load_any(rowp + min(e_first + static_cast<uint32_t>(i) * NT * VEC, n - VEC));
+    // Maximum and minimum in one pass and one reduction.
     float m = -INFINITY, mn = INFINITY;
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        const uint32_t e0 = c0 + (static_cast<uint32_t>(i) * NT + tid) * VEC;
 #pragma unroll
-        for (int c = 0; c < VEC; c++) {
-            if (e0 + c < c1) {
-                m = fmaxf(m, q[i].get(c));   // (drops NaN)
-                mn = fminf(mn, q[i].get(c));
-            }
+        for (int c = 0; c < static_cast<int>(VEC); c += 2) {
+            m = max3(m, q[i].get(c), q[i].get(c + 1));  // (drops NaN)
+            mn = min3(mn, q[i].get(c), q[i].get(c + 1));
         }
     }
-    m = wave_max(m);
-    mn = -wave_max(-mn);
+    const float own_min = mn;
+    m = group_max<kWave>(m);
+    mn = -group_max<kWave>(-mn);
     if constexpr (NW > 1) {
-        if ((tid & (kWave - 1)) == 0) {
-            fscratch[tid / kWave] = m;
-            fscratch2[tid / kWave] = mn;
+        if (lane == 0) {
+            fscratch[wave] = m;
+            fscratch2[wave] = mn;
         }
         __syncthreads();
-#pragma unroll
-        for (int w = 0; w < NW; w++) {
-            m = fmaxf(m, fscratch[w]);
-            mn = fminf(mn, fscratch2[w]);
-        }
+        m = group_max<kSoftmaxRowWavesMax>(fscratch[lane % NW]);
+        mn = -group_max<kSoftmaxRowWavesMax>(-fscratch2[lane % NW]);
     }
     // reference of the chunk's sum: its maximum, or 0 when that is not finite
     // (then every term is 0, inf or NaN, and NaN / inf must reach the sum)
     const float ref = (m > -INFINITY && m < INFINITY) ? m : 0.f;
-    const bool apart = mn > -INFINITY && mn < INFINITY;  // (copies of -inf count for nothing either way)
+    // The copies of the chunk's smallest value are set apart and counted: a value that fills most
+    // of a row (padding, a floor, zeros) is usually its smallest, every copy of it has the same
+    // term, and that term's error would go into the sum thousands of times over -- the row's sum
+    // is DEFINED with exp_accurate(fl(x - M)) for each, which only the kernel that knows M can
+    // count (4 ulp on rows of one value and a few peaks otherwise).  A value that frequent is the
+    // smallest of most lanes' elements; a wave with fewer than 16 such lanes leaves its copies in
+    // the sum and saves two instructions an element.
+    const bool apart = mn > -INFINITY && mn < INFINITY && __popcll(__ballot(own_min == mn)) >= 16;  // (copies of -inf count for nothing either way)
     double acc = 0.0;
     uint32_t copies = 0;
+    auto sum = [&](auto full_tag) {
 #pragma unroll
-    for (int i = 0; i < V; i++) {
-        const uint32_t e0 = c0 + (static_cast<uint32_t>(i) * NT + tid) * VEC;
+        for (int i = 0; i < V; i++) {
+            const uint32_t e0 = e_first + static_cast<uint32_t>(i) * NT * VEC;
+            const uint32_t dup = decltype(full_tag)::value || e0 <= n - VEC ? 0u : min(e0 - (n - VEC), VEC);
 #pragma unroll
-        for (int c = 0; c < VEC; c++) {
-            if (e0 + c < c1) {
+            for (int c = 0; c < static_cast<int>(VEC); c++) {
                 const float x = q[i].get(c);
-                copies += (x == mn) ? 1u : 0u;
-                acc += static_cast<double>(fast_term_unbiased(x, ref));
+                const double t = static_cast<double>(fast_term_unbiased(x, ref));
+                const bool counts = decltype(full_tag)::value || static_cast<uint32_t>(c) >= dup;
+                acc += counts ? t : 0.0;
+                if (apart) copies += (counts && x == mn) ? 1u : 0u;  // (wave-uniform)
             }
         }
-    }
+    };
+    if ((chunk + 1u) * (NT * V * VEC) <= n) sum(std::true_type{});
+    else sum(std::false_type{});
     // (every copy added the same float: taking them out again is exact to the sum's own rounding)
     if (apart) acc -= static_cast<double>(copies) * static_cast<double>(fast_term_unbiased(mn, ref));
-    else copies = 0;
-    acc = wave_sum(acc);
+    acc = group_sum<kWave>(acc);
     copies = wave_sum(copies);
     if constexpr (NW > 1) {
-        if ((tid & (kWave - 1)) == 0) {
-            dscratch[tid / kWave] = acc;
-            uscratch[tid / kWave] = copies;
+        if (lane == 0) {
+            dscratch[wave] = acc;
+            uscratch[wave] = copies;
         }
         __syncthreads();
         acc = dscratch[0];
@@ -360,54 +356,82 @@ __global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__
 }
 
 // ---- chunked rows: exp(x - M) / S -----------------------------------------------------
-template <typename T, int NT, int V, bool ALIGNED>
-__global__ __launch_bounds__(NT) void softmax_scale_kernel(const T *in, T *out, const ChunkStat *__restrict__ stats,
-                                                           uint32_t n, uint32_t G, uint32_t per, int nan_where,
-                                                           float nan_value) {
-    constexpr int VEC = Vec128<T>::N;
-    constexpr int NW = NT / kWave;
-    __shared__ float fscratch[NW];
-    __shared__ double dscratch[NW];
+// Launch: rows * GS workgroups of 256, V vectors a thread, GS = ceil(n / (256 * V * VEC)); G: the
+// chunks a row of the statistics kernel.  In-place calls are fine: see the moved vector.
+// [64,128256] f32, both kernels: 24.9 -> 22.3 us (2 reads and 1 write of 33 MB: 4.4 TB/s);
+// [63,132402] (rows off 16 bytes) f32 35.9 -> 24.3, f16 34.8 -> 17.3; [32,50257] f16 10.1 -> 8.0.
+constexpr int kSoftmaxScaleThreads = 256;
+template <typename T, int V>
+__global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(const T *in, T *out, const ChunkStat *__restrict__ stats,
+                                                                            uint32_t n, uint32_t G, uint32_t GS, int nan_where,
+                                                                            float nan_value) {
+    constexpr uint32_t VEC = Vec128<T>::N, NT = kSoftmaxScaleThreads;
+    __shared__ LineStats row_stats;
+    __shared__ float wave_m[NT / kWave];
+    __shared__ double wave_s[NT / kWave];
+    static_assert(NT / kWave == 4, "the two combinations below");
     const uint32_t tid = threadIdx.x;
-    const uint32_t row = blockIdx.x / G, chunk = blockIdx.x - row * G;
-    const uint32_t c0 = min(chunk * per, n), c1 = min(c0 + per, n);
+    const uint32_t row = blockIdx.x / GS, chunk = blockIdx.x - row * GS;
+    const uint32_t e_first = chunk * (NT * V * VEC) + tid * VEC;
     const size_t row0 = static_cast<size_t>(row) * n;
     const T *rowp = in + row0;
     Vec128<T> q[V];
 #pragma unroll
-    for (int i = 0; i < V; i++) {
-        const uint32_t e0 = c0 + (static_cast<uint32_t>(i) * NT + tid) * VEC;
-        q[i].v = make_uint4(0, 0, 0, 0);
-        if constexpr (ALIGNED) {
-            q[i].load(rowp + (e0 < c1 ? e0 : 0u));
-        } else {
-#pragma unroll
-            for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < c1 ? e0 + c : 0u));
-        }
-    }
-    // the row's maximum and sum from its G chunk results (G <= NT)
-    ChunkStat st{0.0, -INFINITY, 0.f, 0.f, 0u};
-    if (tid < G) st = stats[static_cast<size_t>(row) * G + tid];
-    const float M = block_max<NT>(st.m, fscratch);
+    for (int i = 0; i < V; i++) q[i].v = load16_stream(rowp + min(e_first + static_cast<uint32_t>(i) * NT * VEC, n - VEC));
+    // A row of up to 64 chunks is combined by the first wave, a chunk a lane, under everyone's loads;
+    // with more chunks each wave takes its share of them (two barriers more, a quarter of the exponentials).
+    const ChunkStat *cs = stats + static_cast<size_t>(row) * G;
+    const uint32_t takers = G <= static_cast<uint32_t>(kWave) ? static_cast<uint32_t>(kWave) : NT;
+    float M = -INFINITY;
     double part = 0.0;
-    if (tid < G && st.s != 0.0) part = st.s * sum_rescale(st.s, st.ref, M);
-    if (tid < G && st.nmin != 0u) part += static_cast<double>(st.nmin) * static_cast<double>(softmax_term_as<T>(st.vmin, M));
-    const LineStats ls{M, 0.f, 1.0 / block_sum<NT>(part, dscratch)};
+    if (tid < takers) {
+        for (uint32_t g = tid; g < G; g += takers) M = fmaxf(M, cs[g].m);
+        M = group_max<kWave>(M);
+    }
+    if (takers == NT) {
+        if ((tid & (kWave - 1)) == 0) wave_m[tid / kWave] = M;
+        __syncthreads();
+        M = fmaxf(fmaxf(wave_m[0], wave_m[1]), fmaxf(wave_m[2], wave_m[3]));
+    }
+    if (tid < takers) {
+        for (uint32_t g = tid; g < G; g += takers) {
+            const ChunkStat st = cs[g];
+            if (st.s != 0.0) part += st.s * sum_rescale(st.s, st.ref, M);
+            if (st.nmin != 0u) part += static_cast<double>(st.nmin) * static_cast<double>(softmax_term_as<T>(st.vmin, M));
+        }
+        part = group_sum<kWave>(part);
+    }
+    if (takers == NT) {
+        if ((tid & (kWave - 1)) == 0) wave_s[tid / kWave] = part;
+        __syncthreads();
+        part = (wave_s[0] + wave_s[1]) + (wave_s[2] + wave_s[3]);
+    }
+    if (tid == 0) row_stats = LineStats{M, 0.f, 1.0 / part};
+    __syncthreads();
+    const LineStats ls = row_stats;
     T *orow = out + row0;
 #pragma unroll
     for (int i = 0; i < V; i++) {
-        const uint32_t e0 = c0 + (static_cast<uint32_t>(i) * NT + tid) * VEC;
+        const uint32_t e0 = e_first + static_cast<uint32_t>(i) * NT * VEC;
+        float p[VEC];
         Vec128<T> r;
         r.v = make_uint4(0, 0, 0, 0);
 #pragma unroll
-        for (int c = 0; c < VEC; c++) {
-            float p = round_to_storage<T>(softmax_prob_as<T>(q[i].get(c), ls));
-            if (nan_where && p != p) p = nan_value;
-            if constexpr (ALIGNED) r.set(c, p);
-            else if (e0 + c < c1) store_elem(orow, e0 + c, p);
+        for (int c = 0; c < static_cast<int>(VEC); c++) {
+            p[c] = softmax_prob_as<T>(q[i].get(c), ls);
+            if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
+            r.set(c, p[c]);
         }
-        if constexpr (ALIGNED)
-            if (e0 < c1) *reinterpret_cast<uint4 *>(orow + e0) = r.v;
+        if (e0 <= n - VEC) {
+            store16_stream(orow + e0, r.v);
+        } else if (e0 < n) {
+            // (the moved vector: its own elements alone -- those it repeats may be another workgroup's,
+            // which in an in-place call has replaced them by now)
+            const uint32_t dup = e0 - (n - VEC);
+#pragma unroll
+            for (int c = 1; c < static_cast<int>(VEC); c++)
+                if (static_cast<uint32_t>(c) >= dup) store_elem(orow, n - VEC + static_cast<uint32_t>(c), p[c]);
+        }
     }
 }
 

@@ -151,13 +151,10 @@ constexpr size_t kAlign = 256;
 inline size_t align_up(size_t b) { return (b + kAlign - 1) / kAlign * kAlign; }
 
 // ---------------------------------------------------------------- softmax ----
-// Launch shapes shared by the row kernels: threads per workgroup and 128-bit
-// loads per thread, smallest first.
+// Threads per workgroup and 128-bit loads per thread.
 struct RowShape {
     int nt, v;
 };
-const RowShape kShapesF32[] = {{256, 1}, {256, 2}, {256, 4}, {256, 8}, {512, 8}, {1024, 8}};
-const RowShape kShapesF16[] = {{128, 1}, {256, 1}, {256, 2}, {256, 4}, {512, 4}, {1024, 4}};
 
 struct SoftmaxPlan {
     enum Kind { kGeneralLines, kGeneralStrided, kThread, kGroup, kRow, kChunked, kStridedRegs, kStridedTile } kind = kGeneralLines;
@@ -193,7 +190,6 @@ void launch_strided_reg(const T *in, T *out, const View &v, int nan_where, float
 SoftmaxPlan plan_softmax(const View &v, int dtype) {
     SoftmaxPlan p;
     const uint32_t vec = dtype == VKOP_HIP_F32 ? 4u : 8u;
-    const RowShape *shapes = dtype == VKOP_HIP_F32 ? kShapesF32 : kShapesF16;
     const uint32_t n = v.g.n, rows = v.g.outer;
     if (v.g.inner != 1) {
         if (n <= static_cast<uint32_t>(vkop::kStridedMaxN)) p.kind = SoftmaxPlan::kStridedRegs;
@@ -246,37 +242,28 @@ SoftmaxPlan plan_softmax(const View &v, int dtype) {
         p.shape = RowShape{static_cast<int>(nt), static_cast<int>((nvec + nt - 1) / nt)};
         return p;
     }
-    // chunked: the largest chunk that still leaves >= 1024 workgroups, else the smallest
-    int pick = -1;
-    for (int i = 0; i < 6; i++) {
-        const uint32_t span = static_cast<uint32_t>(shapes[i].nt) * shapes[i].v * vec;
-        const uint32_t g = (n + span - 1) / span;
-        if (g > static_cast<uint32_t>(shapes[i].nt) || static_cast<uint64_t>(rows) * g >= (1ull << 31)) continue;
-        if (pick < 0) pick = i;
-        if (static_cast<uint64_t>(rows) * g >= 1024) pick = i;
-    }
-    if (pick < 0) return p;  // (rows of more than 2^25 elements: the general kernel)
+    // chunked: the largest chunk that still leaves 512 workgroups, else the smallest; beyond
+    // 1024 chunks a row, workgroups of 1024 threads ([8,262144] f32 with 512 / 1024: 10.0 / 10.5 us;
+    // [4,1048576] 14.4 / 15.4: every workgroup of the scale kernel combines all chunks of its row)
+    if (n > (1u << 25)) return p;  // (the general kernel)
+    const uint32_t loads_max = 32u / vec;
+    uint32_t nt = 256, loads = loads_max;
+    auto chunks = [&] { return (n + nt * loads * vec - 1) / (nt * loads * vec); };
+    while (loads > 1 && static_cast<uint64_t>(rows) * chunks() < 512) loads /= 2;
+    if (chunks() > 1024) nt = 1024, loads = loads_max;
+    p.per = nt * loads * vec;
+    p.g = chunks();
     p.kind = SoftmaxPlan::kChunked;
-    p.shape = shapes[pick];
-    p.per = static_cast<uint32_t>(p.shape.nt) * p.shape.v * vec;
-    p.g = (n + p.per - 1) / p.per;
+    p.shape = RowShape{static_cast<int>(nt), static_cast<int>(loads)};
     p.workspace = kTicketBytes + align_up(static_cast<size_t>(rows) * p.g * sizeof(vkop::ChunkStat));
     return p;
 }
-
-#define VKOP_FOR_EACH_ROW_SHAPE(X, T) \
-    X(256, 1) X(256, 2) X(256, 4) X(512, 4) X(1024, 4)                          \
-    if constexpr (sizeof(T) == 4) { X(256, 8) X(512, 8) X(1024, 8) }          \
-    if constexpr (sizeof(T) == 2) { X(128, 1) }
 
 template <typename T>
 int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, float nan_value, void *ws,
                  size_t ws_bytes, hipStream_t st) {
     const SoftmaxPlan p = plan_softmax(v, dtype);
     const uint32_t lines = v.g.outer * v.g.inner;
-    const uint32_t vec = 16 / sizeof(T);
-    const bool aligned = reinterpret_cast<uintptr_t>(in) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0 &&
-                         v.g.n % vec == 0;
     switch (p.kind) {
     case SoftmaxPlan::kThread: {
         const uint32_t blocks = (lines + vkop::kSoftmaxGroupThreads - 1) / vkop::kSoftmaxGroupThreads;
@@ -314,22 +301,29 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
         auto *stats = reinterpret_cast<vkop::ChunkStat *>(static_cast<unsigned char *>(ws) + kTicketBytes);
         const uint32_t blocks = v.g.outer * p.g;
         bool done = false;
-#define VKOP_CHUNKED(NT, V)                                                                                    \
-    if (!done && p.shape.nt == NT && p.shape.v == V) {                                                         \
-        if (aligned) {                                                                                         \
-            vkop::softmax_stats_kernel<T, NT, V, true><<<blocks, NT, 0, st>>>(in, stats, v.g.n, p.g, p.per);   \
-            vkop::softmax_scale_kernel<T, NT, V, true>                                                         \
-                <<<blocks, NT, 0, st>>>(in, out, stats, v.g.n, p.g, p.per, nan_where, nan_value);              \
-        } else {                                                                                               \
-            vkop::softmax_stats_kernel<T, NT, V, false><<<blocks, NT, 0, st>>>(in, stats, v.g.n, p.g, p.per);  \
-            vkop::softmax_scale_kernel<T, NT, V, false>                                                        \
-                <<<blocks, NT, 0, st>>>(in, out, stats, v.g.n, p.g, p.per, nan_where, nan_value);              \
-        }                                                                                                      \
-        done = true;                                                                                           \
+#define VKOP_STATS(NT, V)                                                                              \
+    if (!done && p.shape.nt == NT && p.shape.v == V) {                                                 \
+        vkop::softmax_stats_kernel<T, NT, V><<<blocks, NT, 0, st>>>(in, stats, v.g.n, p.g);            \
+        done = true;                                                                                   \
     }
-        VKOP_FOR_EACH_ROW_SHAPE(VKOP_CHUNKED, T)
-#undef VKOP_CHUNKED
-        if (!done) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no chunked softmax for %d x %d", p.shape.nt, p.shape.v);
+        VKOP_STATS(256, 1) VKOP_STATS(256, 2) VKOP_STATS(256, 4)
+        if constexpr (sizeof(T) == 4) { VKOP_STATS(256, 8) VKOP_STATS(1024, 8) }
+        else { VKOP_STATS(1024, 4) }
+#undef VKOP_STATS
+        if (!done) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_stats_kernel for %d x %d", p.shape.nt, p.shape.v);
+        // the most vectors a thread (four floats', two halves') that leave 2048 workgroups: with fewer in all
+        // their stores wait for each other, with smaller ones more of them combine the same chunks
+        const uint32_t vec = 16 / sizeof(T);
+        auto pieces = [&](uint32_t loads) { return (v.g.n + vkop::kSoftmaxScaleThreads * loads * vec - 1) / (vkop::kSoftmaxScaleThreads * loads * vec); };
+        uint32_t loads = 16 / vec;
+        while (loads > 1 && static_cast<uint64_t>(v.g.outer) * pieces(loads) < 2048) loads /= 2;
+        const uint32_t gs = pieces(loads);
+#define VKOP_SCALE(V) \
+    if (loads == V)   \
+        vkop::softmax_scale_kernel<T, V><<<v.g.outer * gs, vkop::kSoftmaxScaleThreads, 0, st>>>(in, out, stats, v.g.n, p.g, gs, nan_where, nan_value);
+        VKOP_SCALE(1) VKOP_SCALE(2)
+        if constexpr (sizeof(T) == 4) { VKOP_SCALE(4) }
+#undef VKOP_SCALE
         return launched("softmax_stats_kernel / softmax_scale_kernel");
     }
     case SoftmaxPlan::kStridedRegs: {
@@ -709,7 +703,7 @@ int launch_bigk(const T *in, T *values, int32_t *indices, const View &v, int k, 
         constexpr bool AL = decltype(al)::value;
         if constexpr (SOFTMAX) {
             auto *cs = reinterpret_cast<vkop::ChunkStat *>(base + l.chunkstats);
-            vkop::softmax_stats_kernel<T, NT, V, AL><<<blocks, NT, 0, st>>>(in, cs, n, c.g, c.per);
+            vkop::softmax_stats_kernel<T, NT, V><<<blocks, NT, 0, st>>>(in, cs, n, c.g);
             vkop::bigk_row_stats_kernel<<<rows, vkop::kWave, 0, st>>>(cs, stats, c.g);
         }
         vkop::bigk_hist_kernel<T, V, SOFTMAX, AL, 0><<<blocks, NT, 0, st>>>(in, n, uk, c.g, c.per, flip, w);
