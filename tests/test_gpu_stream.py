@@ -490,3 +490,33 @@ def test_bench_timeline_leg_sees_every_lane(ops):
     assert out.get("lanes_seen") == 3, out
     assert 0.7 < out["us_per_call_from_the_log"] / out["us_per_step_by_hip_events_same_run"] < 1.3, out
     assert 1.0 < out["mean_kernels_running"] <= 3.2, out
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,n,k", [(5, 3, 2), (5, 7, 3), (5, 9, 4), (4, 1001, 5), (4, 1003, 40), (3, 1462, 225), (3, 4097, 64), (3, 8195, 64),
+                                      (3, 8201, 100), (20, 20003, 50), (2, 50257, 200), (3, 131075, 50), (2, 100001, 600),
+                                      (2, 131077, 1100), (2, 29467, 886)])
+def test_rows_that_start_off_sixteen_bytes(ops, rows, n, k, dtype):
+    """Every selection route (one wave, one workgroup, scan + pick, scan + gather + rank, the radix select) on rows
+    of odd length in a tensor that itself starts one element off 16 bytes, the row's largest and smallest elements
+    in its last and first vectors -- loaded 16 bytes at a time, the last vector moved back into the row."""
+    rng = np.random.default_rng(rows * n + k)
+    x = rng.standard_normal((rows, n)).astype(dtype)
+    m = min(n // 3, 11)
+    for r in range(rows):
+        ends = np.concatenate([np.arange(m), n - 1 - np.arange(m)])
+        x[r, ends] += np.where(rng.random(ends.size) < 0.5, -5, 5).astype(dtype)
+    buf = torch.empty(rows * n + 1, dtype=torch.float16 if dtype == np.float16 else torch.float32, device="cuda")
+    view = buf[1:].view(rows, n)
+    view.copy_(dev(x))
+    bits = np.uint16 if dtype == np.float16 else np.uint32
+    for largest in (True, False):
+        v, ix = ops.topk(view, k, largest=largest)
+        ev, eix = oracle.topk(x, k, -1, largest)
+        assert np.array_equal(host(ix), eix) and np.array_equal(host(v).view(bits), ev.view(bits)), largest
+    for scale, top_p in ((1.0, None), (1.25, 0.9)):
+        # the aligned copy of the same rows takes the same kernels' other form: the same bits from either
+        got, want = ((ops.softmax_topk(t, k) if top_p is None else ops.softmax_topk_sampling(t, k, scale, top_p))
+                     for t in (view, dev(x)))
+        for g, w in zip(got, want):
+            assert np.array_equal(host(g), host(w)), (scale, top_p)

@@ -120,7 +120,7 @@ __device__ __forceinline__ void resolve_digit(const uint32_t *hist, uint32_t nee
 
 // Striped chunk: vector i of thread t starts at c0 + (i * NT + t) * VEC.
 template <typename T, int V, bool ALIGNED>
-__device__ __forceinline__ void bigk_load_striped(Vec128<T> (&q)[V], const T *rowp, uint32_t c0, uint32_t c1) {
+__device__ __forceinline__ void bigk_load_striped(Vec128<T> (&q)[V], const T *rowp, uint32_t n, uint32_t c0, uint32_t c1) {
     constexpr int VEC = Vec128<T>::N;
 #pragma unroll
     for (int i = 0; i < V; i++) {
@@ -129,8 +129,18 @@ __device__ __forceinline__ void bigk_load_striped(Vec128<T> (&q)[V], const T *ro
         if constexpr (ALIGNED) {
             q[i].load(rowp + (e0 < c1 ? e0 : 0u));
         } else {
+            load_vec_any<false>(q[i], rowp, e0, n);
+        }
+    }
+}
+
+// (before the first use of a chunk of vectors loaded at any alignment)
+template <typename T, int V, bool ALIGNED>
+__device__ __forceinline__ void bigk_settle(Vec128<T> (&q)[V], uint32_t n, uint32_t first, uint32_t step, bool last_chunk) {
+    if constexpr (!ALIGNED) {
+        if (last_chunk) {
 #pragma unroll
-            for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < c1 ? e0 + c : 0u));
+            for (int i = 0; i < V; i++) settle_vec(q[i], first + static_cast<uint32_t>(i) * step, n);
         }
     }
 }
@@ -153,7 +163,7 @@ __global__ __launch_bounds__(kBigThreads) void bigk_hist_kernel(const T *__restr
     const uint32_t c0 = min(chunk * per, n), c1 = min(c0 + per, n);
     const T *rowp = in + static_cast<size_t>(row) * n;
     Vec128<T> q[V];
-    bigk_load_striped<T, V, ALIGNED>(q, rowp, c0, c1);
+    bigk_load_striped<T, V, ALIGNED>(q, rowp, n, c0, c1);
     for (uint32_t b = tid; b < BINS; b += kBigThreads) lh[b] = 0;
 
     uint32_t *state = ws.state + static_cast<size_t>(row) * 8;
@@ -179,6 +189,7 @@ __global__ __launch_bounds__(kBigThreads) void bigk_hist_kernel(const T *__restr
     __syncthreads();  // lh is cleared
     LineStats st{0.f, 0.f, 0.0};
     if constexpr (SOFTMAX) st = ws.stats[row];
+    bigk_settle<T, V, ALIGNED>(q, n, c0 + tid * VEC, kBigThreads * VEC, c1 == n);
 #pragma unroll
     for (int i = 0; i < V; i++) {
         const uint32_t e0 = c0 + (static_cast<uint32_t>(i) * kBigThreads + tid) * VEC;
@@ -216,7 +227,7 @@ __global__ __launch_bounds__(kBigThreads) void bigk_count_kernel(const T *__rest
     const uint32_t c0 = min(chunk * per, n), c1 = min(c0 + per, n);
     const T *rowp = in + static_cast<size_t>(row) * n;
     Vec128<T> q[V];
-    bigk_load_striped<T, V, ALIGNED>(q, rowp, c0, c1);
+    bigk_load_striped<T, V, ALIGNED>(q, rowp, n, c0, c1);
     uint32_t *state = ws.state + static_cast<size_t>(row) * 8;
     const uint32_t d0 = state[0], d1 = state[2], need1 = state[3];
     uint32_t d2, need_eq;
@@ -229,6 +240,7 @@ __global__ __launch_bounds__(kBigThreads) void bigk_count_kernel(const T *__rest
     LineStats st{0.f, 0.f, 0.0};
     if constexpr (SOFTMAX) st = ws.stats[row];
     uint32_t gt = 0, eq = 0;
+    bigk_settle<T, V, ALIGNED>(q, n, c0 + tid * VEC, kBigThreads * VEC, c1 == n);
 #pragma unroll
     for (int i = 0; i < V; i++) {
         const uint32_t e0 = c0 + (static_cast<uint32_t>(i) * kBigThreads + tid) * VEC;
@@ -271,8 +283,7 @@ __global__ __launch_bounds__(kBigThreads) void bigk_gather_kernel(const T *__res
         if constexpr (ALIGNED) {
             q[i].load(rowp + (e0 < c1 ? e0 : 0u));
         } else {
-#pragma unroll
-            for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < c1 ? e0 + c : 0u));
+            load_vec_any<false>(q[i], rowp, e0, n);
         }
     }
     const uint32_t *state = ws.state + static_cast<size_t>(row) * 8;
@@ -297,6 +308,7 @@ __global__ __launch_bounds__(kBigThreads) void bigk_gather_kernel(const T *__res
 
     LineStats st{0.f, 0.f, 0.0};
     if constexpr (SOFTMAX) st = ws.stats[row];
+    bigk_settle<T, V, ALIGNED>(q, n, t0, VEC, c1 == n);
     uint32_t keys[V * VEC];
     uint32_t gt = 0, eq = 0;
 #pragma unroll

@@ -470,15 +470,12 @@ __global__ __launch_bounds__(kBigPickThreads) void bigpick_gather_kernel(const T
             e0[u] = b * BE + (j % kBlockLanes) * VEC;
             cend[u] = j < items ? n : 0u;
             r[u].v = make_uint4(0, 0, 0, 0);
-            if constexpr (ALIGNED) {
-                r[u].load(rowp + (e0[u] < cend[u] ? e0[u] : 0u));
-            } else {
-#pragma unroll
-                for (int c = 0; c < VEC; c++) r[u].set(c, load_elem(rowp, e0[u] + c < cend[u] ? e0[u] + c : 0u));
-            }
+            if constexpr (ALIGNED) r[u].load(rowp + (e0[u] < cend[u] ? e0[u] : 0u));
+            else load_vec_any<false>(r[u], rowp, e0[u], n);
         }
 #pragma unroll
         for (int u = 0; u < U; u++) {
+            if constexpr (!ALIGNED) settle_vec(r[u], e0[u], n);
             float vm = -INFINITY;
             bool any_nan = false;
 #pragma unroll

@@ -585,6 +585,45 @@ template <> struct Vec128<uint16_t> {
     }
 };
 
+// Vectors of a row that starts on any element: load_vec_any issues the load -- 16 bytes from element
+// e0 on, or, where the row ends inside them or before, its last 16 bytes -- and settle_vec, called
+// where the data is first used (not earlier: it waits for the load), moves a vector that the row's
+// end cut short into place: element c of it is then element e0 + c of the row for every e0 + c < n.
+// FEW: the row may be shorter than a vector (its elements are then loaded one by one).
+// (What it replaces -- one load an element -- made such rows up to twice as slow as aligned ones.  Fused
+// softmax -> top-k: [103,211004] f16 k = 21 35.0 -> 18.6 us, [166,70338] k = 8 f16 24.5 -> 15.3, f32
+// 23.0 -> 17.4, [32,50257] f16 k = 40 13.8 -> 11.7.)
+template <bool FEW, typename T> __device__ __forceinline__ void load_vec_any(Vec128<T> &q, const T *rowp, uint32_t e0, uint32_t n) {
+    constexpr uint32_t VEC = Vec128<T>::N;
+    if constexpr (FEW) {
+        if (n < VEC) {  // (the same in every thread)
+            q.v = make_uint4(0, 0, 0, 0);
+#pragma unroll
+            for (uint32_t c = 0; c < VEC; c++) q.set(static_cast<int>(c), load_elem(rowp, e0 + c < n ? e0 + c : 0u));
+            return;
+        }
+    }
+    q.load_any(rowp + min(e0, n - VEC));
+}
+template <typename T> __device__ __forceinline__ void settle_vec(Vec128<T> &q, uint32_t e0, uint32_t n) {
+    constexpr uint32_t VEC = Vec128<T>::N;
+    if (n >= VEC && e0 > n - VEC && e0 < n) {
+        const uint32_t s = e0 - (n - VEC);  // elements loaded before e0: 1 .. VEC - 1
+        if constexpr (sizeof(T) == 4) {
+            const uint4 v = q.v;
+            q.v.x = s == 1 ? v.y : s == 2 ? v.z : v.w;
+            q.v.y = s == 1 ? v.z : v.w;
+            q.v.z = v.w;
+        } else {
+            uint64_t lo = (static_cast<uint64_t>(q.v.y) << 32) | q.v.x, hi = (static_cast<uint64_t>(q.v.w) << 32) | q.v.z;
+            const uint32_t bits = (s & 3u) * 16u;
+            if (s >= 4) lo = hi, hi = 0;
+            lo = (lo >> bits) | (hi << 1 << (63u - bits));
+            q.v = make_uint4(static_cast<uint32_t>(lo), static_cast<uint32_t>(lo >> 32), static_cast<uint32_t>(hi >> bits), static_cast<uint32_t>(hi >> bits >> 32));
+        }
+    }
+}
+
 // The first `places` elements of a row, in index order, whose order key lies in
 // [xlo, xhi]: the row is read from its start, NT * 4 elements at a time, until enough
 // are found -- soon, when they are many, which is when this is used.  emit(pos, j) is
@@ -1401,7 +1440,7 @@ __device__ __forceinline__ void merge_row(RowsShared &sh, SelectShared &exact, f
 // SOFTMAX = true : fused softmax -> top-k (values are probabilities)
 // SOFTMAX = false: plain top-k, largest first (values are copies of the input)
 // ALIGNED: every row start is 16-byte aligned and n is a multiple of the vector
-// width, so chunks are read with 128-bit loads.
+// width (otherwise the vectors start on any element: load_vec_any).
 // MERGE: kMergeSplit    -- rows_merge_kernel must follow on the same stream;
 //        kMergeByTicket -- the workgroup that publishes a row's last chunk (found
 //                          with one counter per row) merges the row before it exits;
@@ -1469,8 +1508,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
         if constexpr (ALIGNED) {
             q[i].load(rowp + (e0 < c1 ? e0 : 0u));
         } else {
-#pragma unroll
-            for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < c1 ? e0 + c : 0u));
+            load_vec_any<V == 1>(q[i], rowp, e0, n);
         }
     }
 
@@ -1479,6 +1517,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
     auto body = [&](auto full_tag) {
         constexpr bool FULL = decltype(full_tag)::value;
         auto in_range = [&](uint32_t e) { return FULL || e < c1; };
+        if constexpr (!FULL && !ALIGNED) {
+            // (the row's last chunk, and of its vectors the one that holds the row's end: the same in every thread)
+            const uint32_t i_end = c1 == n ? (n - 1u - c0) / (NT * VEC) : static_cast<uint32_t>(V);
+#pragma unroll
+            for (int i = 0; i < V; i++)
+                if (static_cast<uint32_t>(i) == i_end) settle_vec(q[i], e_first + static_cast<uint32_t>(i) * NT * VEC, n);
+        }
 
         // ---- 2. per vector, in arrival order: maximum and sum of exp(x - ref) -----------
         // vmax[i]: float max of vector i (NaN dropped) for the softmax variant; for the

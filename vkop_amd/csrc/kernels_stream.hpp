@@ -102,8 +102,7 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
         if constexpr (ALIGNED) {
             q[i].load(rowp + (e0 < c1 ? e0 : 0u));
         } else {
-#pragma unroll
-            for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < c1 ? e0 + c : 0u));
+            load_vec_any<false>(q[i], rowp, e0, n);
         }
     };
     static_for<0, V>(issue_load);
@@ -134,6 +133,7 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
         double acc = 0.0;  // every term is added in double: a dominant term must not swallow what follows it
         static_for<0, V>([&](auto i_tag) {
             constexpr int i = decltype(i_tag)::value;
+            if constexpr (!FULL && !ALIGNED) settle_vec(q[i], e_first + static_cast<uint32_t>(i) * NT * VEC, n);
             float xv[VEC];
             float vm = -INFINITY;
 #pragma unroll
@@ -531,12 +531,8 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
             // (a slot past the wave's items reads the row's start and is marked by an index past the row's end)
             e0[u] = j < items ? b * BE + (j % kBlockLanes) * VEC : 0xFFFFFFFFu;
             r[u].v = make_uint4(0, 0, 0, 0);
-            if constexpr (ALIGNED) {
-                r[u].load(rowp + (e0[u] < n ? e0[u] : 0u));
-            } else {
-#pragma unroll
-                for (int c = 0; c < VEC; c++) r[u].set(c, load_elem(rowp, e0[u] < n && e0[u] + c < n ? e0[u] + c : 0u));
-            }
+            if constexpr (ALIGNED) r[u].load(rowp + (e0[u] < n ? e0[u] : 0u));
+            else load_vec_any<false>(r[u], rowp, e0[u], n);
         };
         static_for<0, U>(issue);
         const bool second_half = items > static_cast<uint32_t>(U) * kWave;  // wave-uniform
@@ -548,6 +544,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         uint32_t nv = 0;  // wave-uniform
         auto sift = [&](auto u_tag) __attribute__((always_inline)) {
             constexpr int u = decltype(u_tag)::value;
+            if constexpr (!ALIGNED) settle_vec(r[u], e0[u], n);
             float vm = -INFINITY;
             bool any_nan = false;
 #pragma unroll
@@ -821,17 +818,14 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                 e0[u] = b * BE + (j % kBlockLanes) * VEC;
                 cend[u] = j < items ? n : 0u;  // (0: nothing of this slot counts)
                 r[u].v = make_uint4(0, 0, 0, 0);
-                if constexpr (ALIGNED) {
-                    r[u].load(rowp + (e0[u] < cend[u] ? e0[u] : 0u));
-                } else {
-#pragma unroll
-                    for (int c = 0; c < VEC; c++) r[u].set(c, load_elem(rowp, e0[u] + c < cend[u] ? e0[u] + c : 0u));
-                }
+                if constexpr (ALIGNED) r[u].load(rowp + (e0[u] < cend[u] ? e0[u] : 0u));
+                else load_vec_any<false>(r[u], rowp, e0[u], n);
             }
             const float lo_f = ordered_to_float(lo);  // (lo > key of -inf: a number or +inf)
 #pragma unroll
             for (int u = 0; u < U; u++) {
                 // a vector without an element at or above lo (15 of a block's 16) costs one test
+                if constexpr (!ALIGNED) settle_vec(r[u], e0[u], n);
                 float vm = -INFINITY;
                 bool any_nan = false;
 #pragma unroll

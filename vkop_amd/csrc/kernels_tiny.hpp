@@ -82,8 +82,7 @@ __device__ __forceinline__ void tiny_row(TinyShared &smem, float *fscratch, doub
         if constexpr (ALIGNED) {
             q[i].load(rowp + (e0 < n ? e0 : 0u));
         } else {
-#pragma unroll
-            for (int c = 0; c < VEC; c++) q[i].set(c, load_elem(rowp, e0 + c < n ? e0 + c : 0u));
+            load_vec_any<V == 1>(q[i], rowp, e0, n);
         }
     }
     // ---- 2. keys, maximum, sum of fast terms
@@ -92,6 +91,7 @@ __device__ __forceinline__ void tiny_row(TinyShared &smem, float *fscratch, doub
     float m = -INFINITY;
 #pragma unroll
     for (int i = 0; i < V; i++) {
+        if constexpr (!ALIGNED) settle_vec(q[i], (static_cast<uint32_t>(i) * kWave + lane) * VEC, n);
 #pragma unroll
         for (int c = 0; c < VEC; c++) {
             const uint32_t e = (static_cast<uint32_t>(i) * kWave + lane) * VEC + static_cast<uint32_t>(c);

@@ -422,7 +422,7 @@ RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false) 
     if (wide >= 0 && (k > vkop::kMergeThreads - 1 || (k > kWideRowMinK && !forced_nt))) {
         c.nt = shapes[wide][0], c.v = shapes[wide][1], c.g = 1;
     } else if (forced_nt) {
-        if (!fits(forced_nt, forced_v, static_cast<uint32_t>(forced_g))) return c;
+        if (!fits(forced_nt, forced_v, static_cast<uint32_t>(forced_g)) || (n < vec && forced_v > 1)) return c;
         c.nt = forced_nt, c.v = forced_v, c.g = static_cast<uint32_t>(forced_g);
     } else if (k <= kWaveRowMaxK && wave_loads <= (dtype == VKOP_HIP_F32 ? 8u : 4u)) {
         c.nt = 64, c.g = 1;
