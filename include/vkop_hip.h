@@ -110,7 +110,7 @@ int vkop_hip_softmax(const void *in, void *out, int dtype, const int *shape,
  * +inf.  With sorted == 0 (the reference parses the attribute and ignores it,
  * ops/Topk.hpp:73-75; ONNX leaves the order open then) the same k elements
  * come in an order the library chooses, the same from run to run: on the
- * multi-pass radix select (smallest first on long rows, and rows no other
+ * multi-pass radix select (smallest first with a large k, and rows no other
  * route takes) as that select lists them, which saves its last step; on
  * every other route in sorted order, which costs nothing there.
  * 1 <= k <= min(extent of axis, VKOP_HIP_MAX_K). */

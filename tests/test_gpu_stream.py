@@ -520,3 +520,32 @@ def test_rows_that_start_off_sixteen_bytes(ops, rows, n, k, dtype):
                      for t in (view, dev(x)))
         for g, w in zip(got, want):
             assert np.array_equal(host(g), host(w)), (scale, top_p)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("n,k", [(4096, 64), (8400, 300), (8401, 300), (32000, 40), (50257, 200), (100000, 600), (131076, 1025)])
+def test_smallest_first_on_reversed_elements(ops, n, k, dtype):
+    """k smallest on long rows: the kernels of the other direction on reversed elements.  NaN (largest: last, behind
+    +inf) and +inf -- the reversed -inf that never becomes a candidate -- alone and side by side, where they fill the
+    last places and where they do not; zeros of both signs; rows of one value, of levels, in order."""
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((12, n)).astype(dtype)
+    x[1, rng.random(n) < 0.3] = np.nan
+    x[2, rng.random(n) < 0.9] = np.inf
+    few = rng.choice(n, k // 2, replace=False)
+    x[3, :], x[3, few] = np.inf, -1.5
+    x[4, :], x[4, few] = np.nan, rng.standard_normal(few.size)
+    x[5, 0::2], x[5, 1::2], x[5, few] = np.nan, np.inf, 2.0          # both kinds behind the candidates, mixed
+    x[6, :], x[6, few[: k // 4]] = np.nan, np.inf                    # fewer +inf than places, then NaN
+    x[7, :] = np.where(rng.random(n) < 0.5, dtype(0.0), dtype(-0.0))
+    x[8, :] = 0.75
+    x[9, :] = np.round(x[9].astype(np.float32) * 4) / 4
+    x[10, :] = np.sort(x[10])[::-1]
+    x[11, rng.choice(n, 5, replace=False)] = -np.inf
+    for rows in (x, np.tile(x, (2, 1))):                               # up to 16 rows, and more: other routes
+        v, ix = ops.topk(dev(rows), k, largest=False)
+        ev, eix = oracle.topk(rows, k, -1, False)
+        for r in range(rows.shape[0]):
+            assert np.array_equal(host(ix[r]), eix[r]), r
+        bits = np.uint16 if dtype == np.float16 else np.uint32
+        assert np.array_equal(host(v).view(bits), ev.view(bits))

@@ -21,11 +21,31 @@ template <> __device__ __forceinline__ float load_elem<uint16_t>(const uint16_t 
     return __half2float(__ushort_as_half(p[i]));
 }
 
+// Element of a float or half tensor whose order is turned round: it reads as its negative, and what is
+// stored is turned back, so a kernel written for the k largest gives the k smallest, ties by lower index
+// as before.  NaN still ranks as the largest value, which is last now: a loaded vector gives -inf for it
+// (Vec128, kernels_rows.hpp), which never becomes a candidate; where -inf itself is placed -- fewer than
+// k+1 other elements -- and in the exact selects, NaN comes behind it (plain_key).
+template <typename B> struct Reversed {
+    B bits;
+};
+template <typename T> constexpr bool kReversed = false;
+template <typename B> constexpr bool kReversed<Reversed<B>> = true;
+template <> __device__ __forceinline__ float load_elem<Reversed<float>>(const Reversed<float> *p, size_t i) { return -p[i].bits; }
+template <> __device__ __forceinline__ float load_elem<Reversed<uint16_t>>(const Reversed<uint16_t> *p, size_t i) {
+    return -__half2float(__ushort_as_half(p[i].bits));
+}
+
 // Round-to-nearest-even store of a float into a float or half tensor.
 template <typename T> __device__ __forceinline__ void store_elem(T *p, size_t i, float v);
 template <> __device__ __forceinline__ void store_elem<float>(float *p, size_t i, float v) { p[i] = v; }
 template <> __device__ __forceinline__ void store_elem<uint16_t>(uint16_t *p, size_t i, float v) {
     p[i] = __half_as_ushort(__float2half_rn(v));
+}
+
+template <> __device__ __forceinline__ void store_elem<Reversed<float>>(Reversed<float> *p, size_t i, float v) { p[i].bits = -v; }
+template <> __device__ __forceinline__ void store_elem<Reversed<uint16_t>>(Reversed<uint16_t> *p, size_t i, float v) {
+    p[i].bits = __half_as_ushort(__float2half_rn(-v));
 }
 
 // Value as the tensor type would hold it (float stays, half is rounded to
@@ -96,6 +116,13 @@ __device__ __forceinline__ uint32_t order_key(float v) {
     if (v != v) return 0xFFFFFFFFu;
     uint32_t u = __float_as_uint(v + 0.0f);  // -0 + +0 = +0
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+
+// The key plain top-k ranks an element by: order_key, and for a reversed element NaN below everything
+// (above 0, "no element").
+template <typename T> __device__ __forceinline__ uint32_t plain_key(float v) {
+    if constexpr (kReversed<T>) return v != v ? 1u : order_key(v);
+    else return order_key(v);
 }
 
 // Composite of key and position: larger composite = ranks earlier; among equal

@@ -482,7 +482,7 @@ __global__ __launch_bounds__(kBigPickThreads) void bigpick_gather_kernel(const T
             for (int c = 0; c < VEC; c++) {
                 const float x = r[u].get(c);
                 vm = fmaxf(vm, x);
-                if constexpr (!SOFTMAX) any_nan = any_nan || x != x;
+                if constexpr (!SOFTMAX && !kReversed<T>) any_nan = any_nan || x != x;
             }
             if (!(vm < lo_f) || any_nan) {
 #pragma unroll
@@ -622,7 +622,7 @@ __device__ __forceinline__ void bigpick_exact_row(SelectShared &ex, const T *row
             oi[r] = static_cast<int32_t>(idx);
         }
     } else {
-        select_topk_line<NT>(ex, n, kk, [&](uint32_t j) { return order_key(load_elem(rowp, j)); });
+        select_topk_line<NT>(ex, n, kk, [&](uint32_t j) { return plain_key<T>(load_elem(rowp, j)); });
         for (uint32_t r = tid; r < kk; r += NT) {
             const uint32_t idx = composite_index(ex.sel[r]);
             ov[r] = rowp[idx];
@@ -869,9 +869,21 @@ __global__ __launch_bounds__(kBigPickThreads) void bigpick_rank_kernel(const T *
 #ifdef VKOP_STAMPS
     const unsigned long long walk_t0 = wall_clock64();
 #endif
-    const uint32_t found = (row_aligned && xhi != 0xFFFFFFFFu) ? first_members_by_vectors<T, NT>(walk_counts, rowp, n, places, xlo, xhi, place)
-                                       : first_members_by_scan<T, NT>(walk_counts, rowp, n, places, xlo, xhi, 1.f,
-                                                                      [&](uint32_t pos, uint32_t j) { place(pos, j, load_elem(rowp, j)); });
+    auto walk_by_scan = [&](uint32_t from, uint32_t lo_key, uint32_t hi_key) -> uint32_t {
+        return first_members_by_scan<T, NT>(walk_counts, rowp, n, places - from, lo_key, hi_key, 1.f,
+                                            [&](uint32_t pos, uint32_t j) { place(from + pos, j, load_elem(rowp, j)); });
+    };
+    uint32_t found;
+    if (kReversed<T> && xlo == kKeyNegInf) {
+        // (a vector of a reversed row gives -inf for NaN: here the two are told apart, NaN behind -inf)
+        found = walk_by_scan(0, kKeyNegInf, kKeyNegInf);
+        __syncthreads();
+        if (found < places) found += walk_by_scan(found, 0xFFFFFFFFu, 0xFFFFFFFFu);
+    } else if (row_aligned && xhi != 0xFFFFFFFFu) {
+        found = first_members_by_vectors<T, NT>(walk_counts, rowp, n, places, xlo, xhi, place);
+    } else {
+        found = walk_by_scan(0, xlo, xhi);
+    }
 #ifdef VKOP_STAMPS
     if (tid == 0 && row < 8) {  // per row: (found << 40 | places << 20 | n_above), nanoseconds
         g_bp_stamps[32 + 2 * row] = (static_cast<unsigned long long>(found) << 40) | (static_cast<unsigned long long>(places) << 20) | n_above;

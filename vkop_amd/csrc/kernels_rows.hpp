@@ -585,6 +585,19 @@ template <> struct Vec128<uint16_t> {
     }
 };
 
+// (a reversed element: its negative, NaN as -inf)
+__device__ __forceinline__ float negated_or_neg_inf(float x) {
+    float r;
+    asm("v_max_f32_e64 %0, -%1, %2" : "=v"(r) : "v"(x), "s"(-INFINITY));
+    return r;
+}
+template <typename B> struct Vec128<Reversed<B>> : Vec128<B> {
+    __device__ __forceinline__ void load(const Reversed<B> *p) { Vec128<B>::load(&p->bits); }
+    __device__ __forceinline__ void load_any(const Reversed<B> *p) { Vec128<B>::load_any(&p->bits); }
+    __device__ __forceinline__ float get(int c) const { return negated_or_neg_inf(Vec128<B>::get(c)); }
+    __device__ __forceinline__ void set(int c, float f) { Vec128<B>::set(c, -f); }
+};
+
 // Vectors of a row that starts on any element: load_vec_any issues the load -- 16 bytes from element
 // e0 on, or, where the row ends inside them or before, its last 16 bytes -- and settle_vec, called
 // where the data is first used (not earlier: it waits for the load), moves a vector that the row's
@@ -801,12 +814,12 @@ __device__ __forceinline__ uint32_t first_members_by_vectors(uint32_t *counts, c
 // Places g0 .. kk-1 of a row's result go to the lowest-index elements whose order
 // key lies in [xlo, xhi] (a group of equal rank too large to collect).  SOFTMAX:
 // every member's value is tie_value (the group's probability); otherwise the element
-// itself.  All NT threads call.
+// itself.  All NT threads call; returns how many were found (first_members_by_scan).
 template <typename T, int NT, bool SOFTMAX>
-__device__ __forceinline__ void fill_group_by_scan(uint32_t *counts, const T *rowp, T *ov, int32_t *oi, uint32_t n,
+__device__ __forceinline__ uint32_t fill_group_by_scan(uint32_t *counts, const T *rowp, T *ov, int32_t *oi, uint32_t n,
                                                    uint32_t g0, uint32_t kk, uint32_t xlo, uint32_t xhi, float tie_value,
                                                    float scale = 1.f) {
-    first_members_by_scan<T, NT>(counts, rowp, n, kk - g0, xlo, xhi, scale, [&](uint32_t pos, uint32_t j) {
+    return first_members_by_scan<T, NT>(counts, rowp, n, kk - g0, xlo, xhi, scale, [&](uint32_t pos, uint32_t j) {
         if constexpr (SOFTMAX) store_elem(ov, g0 + pos, tie_value);
         else ov[g0 + pos] = rowp[j];
         oi[g0 + pos] = static_cast<int32_t>(j);
@@ -997,9 +1010,15 @@ __device__ __forceinline__ void finish_row(RowsShared &sh, uint32_t C2, bool par
             tie_g0 = settle_tie<T, NT>(sh, add_missing, rowp, ov, oi, n, kk, sh.prob[kk], M, rinv, scale);
         }
     } else if (partial) {
-        // the -inf elements follow the candidates, lowest indices first
+        // the -inf elements follow the candidates, lowest indices first (and, in a reversed row, NaN behind them)
         tie_g0 = C2;
-        fill_group_by_scan<T, NT, false>(sh.scan_counts, rowp, ov, oi, n, C2, kk, kKeyNegInf, kKeyNegInf, 0.f);
+        const uint32_t infs = fill_group_by_scan<T, NT, false>(sh.scan_counts, rowp, ov, oi, n, C2, kk, kKeyNegInf, kKeyNegInf, 0.f);
+        if constexpr (kReversed<T>) {
+            if (C2 + infs < kk) {  // (the same in every thread)
+                __syncthreads();
+                fill_group_by_scan<T, NT, false>(sh.scan_counts, rowp, ov, oi, n, C2 + infs, kk, 0xFFFFFFFFu, 0xFFFFFFFFu, 0.f);
+            }
+        }
     }
 
     BPS(34);
@@ -1428,7 +1447,7 @@ __device__ __forceinline__ void merge_row(RowsShared &sh, SelectShared &exact, f
             }
         }
     } else {
-        select_topk_line<NT>(exact, n, kk, [&](uint32_t j) { return order_key(load_elem(rowp, j)); });
+        select_topk_line<NT>(exact, n, kk, [&](uint32_t j) { return plain_key<T>(load_elem(rowp, j)); });
         for (uint32_t r = tid; r < kk; r += NT) {
             const uint32_t idx = composite_index(exact.sel[r]);
             ov[r] = rowp[idx];

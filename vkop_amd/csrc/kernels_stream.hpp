@@ -166,7 +166,7 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
                 // the sum so far exists HERE, under the loads still in flight (or the
                 // compiler moves all of it behind the last load)
                 asm volatile("" : "+v"(acc));
-            } else {
+            } else if constexpr (!kReversed<T>) {
                 // NaN ranks first in a plain top-k: the vector's maximum is then NaN
                 bool has_nan = false;
 #pragma unroll
@@ -187,7 +187,7 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
             for (int j = 0; j < kBlockLanes / 4; j++) {
                 const float4 v4 = src[j ^ ((lane >> 2) & 3)];  // (the block of vector lane / 4: its words are in the order 0..3 ^ that vector's number mod 4)
                 bm = fmaxf(fmaxf(bm, fmaxf(v4.x, v4.y)), fmaxf(v4.z, v4.w));
-                if constexpr (!SOFTMAX) b_nan = b_nan || __builtin_isunordered(v4.x, v4.y) || __builtin_isunordered(v4.z, v4.w);
+                if constexpr (!SOFTMAX && !kReversed<T>) b_nan = b_nan || __builtin_isunordered(v4.x, v4.y) || __builtin_isunordered(v4.z, v4.w);
             }
             // the wave's block L = vector L / 4, lane row L % 4 starts at element
             // c0 + ((L / 4) * NT + wave * 64 + (L % 4) * 16) * VEC of the row
@@ -551,7 +551,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
             for (int c = 0; c < VEC; c++) {
                 const float x = times_scale(r[u].get(c));
                 vm = fmaxf(vm, x);
-                if constexpr (!SOFTMAX) any_nan = any_nan || x != x;
+                if constexpr (!SOFTMAX && !kReversed<T>) any_nan = any_nan || x != x;
             }
             const bool pv = e0[u] < n && (!(vm < lo_f) || any_nan);
             const uint64_t mask = __ballot(pv);
@@ -580,7 +580,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                 const float x = times_scale(sv.get(c));
                 // (softmax: a NaN never passes, and thr is the key of a number, so the floats compare as the keys do)
                 bool pass;
-                if constexpr (SOFTMAX) pass = x >= lo_f;
+                if constexpr (SOFTMAX || kReversed<T>) pass = x >= lo_f;
                 else pass = order_key(x) >= thr;
                 pass = pass && lane < nv && (ALIGNED || eb + static_cast<uint32_t>(c) < n);
                 pbits |= pass ? (1u << c) : 0u;
@@ -832,7 +832,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                 for (int c = 0; c < VEC; c++) {
                     const float x = scaled(r[u].get(c), scale);
                     vm = fmaxf(vm, x);
-                    if constexpr (!SOFTMAX) any_nan = any_nan || x != x;
+                    if constexpr (!SOFTMAX && !kReversed<T>) any_nan = any_nan || x != x;
                 }
                 if (!(vm < lo_f) || any_nan) {
 #pragma unroll
@@ -1056,7 +1056,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
             }
         }
     } else {
-        select_topk_line<NT>(exact, n, kk, [&](uint32_t j) { return order_key(load_elem(rowp, j)); });
+        select_topk_line<NT>(exact, n, kk, [&](uint32_t j) { return plain_key<T>(load_elem(rowp, j)); });
         for (uint32_t r = tid; r < kk; r += NT) {
             const uint32_t idx = composite_index(exact.sel[r]);
             ov[r] = rowp[idx];

@@ -1,5 +1,5 @@
 // One (element type, variant) slice of the one-pass row kernels (chunk, merge, one wave per row):
-//   hipcc -DVKOP_ROWS_T=float|uint16_t -DVKOP_ROWS_SOFTMAX=true|false -c rows_inst.hip
+//   hipcc -DVKOP_ROWS_T=float|uint16_t|Reversed<..> -DVKOP_ROWS_SOFTMAX=true|false -c rows_inst.hip
 // (the scan / pick / large-k kernels of the same slice: stream_inst.hip)
 #include "rows_launch.hpp"
 
@@ -16,6 +16,27 @@ template <typename T, bool SOFTMAX> bool launch_rows_chunk(const RowsLaunch &a) 
 #define VKOP_ROWS_LAUNCH(NT, V, AL, MERGE)                       \
     rows_chunk_kernel<T, NT, V, SOFTMAX, AL, MERGE>              \
         <<<blocks, NT, 0, a.stream>>>(in, values, a.indices, a.n, a.k, a.g, a.per, a.ws)
+#define VKOP_ROWS_LOCAL(NT, V)                                               \
+    if (a.nt == NT && a.v == V) {                                            \
+        if (a.aligned) VKOP_ROWS_LAUNCH(NT, V, true, kMergeLocal);           \
+        else VKOP_ROWS_LAUNCH(NT, V, false, kMergeLocal);                    \
+        return true;                                                         \
+    }
+    if constexpr (kReversed<T>) {
+        if (a.merge != kMergeLocal) return false;
+        VKOP_ROWS_LOCAL(256, 1)
+        VKOP_ROWS_LOCAL(256, 2)
+        VKOP_ROWS_LOCAL(256, 4)
+        VKOP_ROWS_LOCAL(512, 4)
+        VKOP_ROWS_LOCAL(1024, 4)
+        if constexpr (sizeof(T) == 4) {
+            VKOP_ROWS_LOCAL(256, 8)
+            VKOP_ROWS_LOCAL(512, 8)
+            VKOP_ROWS_LOCAL(1024, 8)
+        }
+        return false;
+    } else {
+#undef VKOP_ROWS_LOCAL
 #define VKOP_ROWS_CASE(NT, V)                                                                  \
     if (a.nt == NT && a.v == V) {                                                              \
         if (a.aligned && a.merge == kMergeLocal) VKOP_ROWS_LAUNCH(NT, V, true, kMergeLocal);   \
@@ -85,6 +106,7 @@ template <typename T, bool SOFTMAX> bool launch_rows_chunk(const RowsLaunch &a) 
 #undef VKOP_ROWS_CASE
 #undef VKOP_ROWS_LAUNCH
     return false;
+    }
 }
 
 template <typename T, bool SOFTMAX> void launch_rows_merge(const RowsLaunch &a) {
@@ -145,9 +167,11 @@ template <typename T, bool SOFTMAX> bool launch_rows_tiny(const TinyLaunch &a) {
     return false;
 }
 
-template bool launch_rows_tiny<VKOP_ROWS_T, VKOP_ROWS_SOFTMAX>(const TinyLaunch &);
 template bool launch_rows_chunk<VKOP_ROWS_T, VKOP_ROWS_SOFTMAX>(const RowsLaunch &);
+#ifndef VKOP_ROWS_REVERSED  // (the one-wave kernel turns its keys round itself; rows of several chunks are never reversed)
+template bool launch_rows_tiny<VKOP_ROWS_T, VKOP_ROWS_SOFTMAX>(const TinyLaunch &);
 template void launch_rows_merge<VKOP_ROWS_T, VKOP_ROWS_SOFTMAX>(const RowsLaunch &);
+#endif
 
 }  // namespace vkop
 

@@ -57,6 +57,8 @@ extern template bool launch_rows_scan<float, true>(const ScanLaunch &);
 extern template bool launch_rows_scan<float, false>(const ScanLaunch &);
 extern template bool launch_rows_scan<uint16_t, true>(const ScanLaunch &);
 extern template bool launch_rows_scan<uint16_t, false>(const ScanLaunch &);
+extern template bool launch_rows_scan<Reversed<float>, false>(const ScanLaunch &);
+extern template bool launch_rows_scan<Reversed<uint16_t>, false>(const ScanLaunch &);
 
 // Enqueues rows_tiny_kernel (one wave per row, v 128-bit loads per lane); false if no kernel is built for v.
 struct TinyLaunch {
@@ -79,7 +81,8 @@ extern template bool launch_rows_tiny<float, false>(const TinyLaunch &);
 extern template bool launch_rows_tiny<uint16_t, true>(const TinyLaunch &);
 extern template bool launch_rows_tiny<uint16_t, false>(const TinyLaunch &);
 
-// Enqueues rows_chunk_kernel; false if no kernel is built for (nt, v).
+// Enqueues rows_chunk_kernel; false if no kernel is built for (nt, v) (reversed elements: only for rows that
+// one workgroup holds).
 template <typename T, bool SOFTMAX> bool launch_rows_chunk(const RowsLaunch &a);
 // Enqueues rows_merge_kernel (after a chunk kernel launched with kMergeSplit).
 template <typename T, bool SOFTMAX> void launch_rows_merge(const RowsLaunch &a);
@@ -88,6 +91,8 @@ extern template bool launch_rows_chunk<float, true>(const RowsLaunch &);
 extern template bool launch_rows_chunk<float, false>(const RowsLaunch &);
 extern template bool launch_rows_chunk<uint16_t, true>(const RowsLaunch &);
 extern template bool launch_rows_chunk<uint16_t, false>(const RowsLaunch &);
+extern template bool launch_rows_chunk<Reversed<float>, false>(const RowsLaunch &);
+extern template bool launch_rows_chunk<Reversed<uint16_t>, false>(const RowsLaunch &);
 extern template void launch_rows_merge<float, true>(const RowsLaunch &);
 extern template void launch_rows_merge<float, false>(const RowsLaunch &);
 extern template void launch_rows_merge<uint16_t, true>(const RowsLaunch &);

@@ -813,9 +813,11 @@ int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, 
             return fail(VKOP_HIP_ERR_UNSUPPORTED, "no rows_chunk_kernel for %d threads x %d loads", c.nt, c.v);
         if (int rc = launched("rows_chunk_kernel")) return rc;
     }
-    if (a.merge == vkop::kMergeSplit && (stages & 2)) {
-        vkop::launch_rows_merge<T, SOFTMAX>(a);
-        return launched("rows_merge_kernel");
+    if constexpr (!vkop::kReversed<T>) {
+        if (a.merge == vkop::kMergeSplit && (stages & 2)) {
+            vkop::launch_rows_merge<T, SOFTMAX>(a);
+            return launched("rows_merge_kernel");
+        }
     }
     return VKOP_HIP_OK;
 }
@@ -826,8 +828,21 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
               size_t ws_bytes, hipStream_t st) {
     // (the one-wave kernel serves both directions: it turns its order keys round)
     if (const int tiny = choose_tiny_loads(v, k, dtype)) return launch_tiny<T, false>(in, values, indices, v, k, tiny, st, !largest);
-    const ScanCfg sc = largest ? choose_scan_cfg(v, k, dtype) : ScanCfg{};
-    const RowsCfg c = (largest && !sc.ok) ? choose_rows_cfg(v, k, dtype) : RowsCfg{};
+    // Smallest first runs the kernels of the other direction on reversed elements wherever those are the scan
+    // kernels or one workgroup a row (with rows.path = 1, which switches the former off: the radix select): two
+    // launches or one for the select's seven, one read of the row for five.  [64,32000] f32 k = 40 41 -> 8.8 us,
+    // [64,128256] k = 50 61 -> 12.9, [8,262144] k = 1024 46.8 -> 21.2, [1024,4096] k = 64 29.7 -> 10.2.
+    const bool routed = largest || g_rows_path.load() != 1;
+    ScanCfg sc = routed ? choose_scan_cfg(v, k, dtype) : ScanCfg{};
+    // (without an order, the rows of the large-k kernels keep the select and the listing it has always given)
+    if (!largest && !sorted && sc.g2 != 0) sc = ScanCfg{};
+    RowsCfg c = (routed && !sc.ok) ? choose_rows_cfg(v, k, dtype) : RowsCfg{};
+    if (!largest && (c.g != 1 || c.nt < 256 || c.cap > static_cast<uint32_t>(vkop::kLocalCap))) c = RowsCfg{};
+    // Fewer vectors than places: their maxima bound nothing, and every row would take that kernel's second list
+    // ([2000,1462] f16 k = 225: 225 us, 32 with a workgroup's exact select a row).  Smallest first, where that
+    // select ran before, it stays the faster one up to twice as many ([2000,600] f32 k = 100: 15.3 against 17.9 us).
+    const uint32_t vectors = (v.g.n + 16 / sizeof(T) - 1) / (16 / sizeof(T));
+    if (c.ok && g_rows_path.load() != 1 && vectors < (largest ? 1u : 2u) * (static_cast<uint32_t>(k) + 1u)) c = RowsCfg{};
     const BigKCfg b = (c.ok || sc.ok) ? BigKCfg{} : choose_bigk_cfg(v, k, dtype);
     if (sc.ok || c.ok || b.ok) {
         const RowsLayout l = rows_layout(v, c, b, sc);
@@ -835,8 +850,15 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
             return fail(VKOP_HIP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", ws_bytes, l.total);
         if ((reinterpret_cast<uintptr_t>(ws) & (kAlign - 1)) != 0)
             return fail(VKOP_HIP_ERR_WORKSPACE, "workspace must be %zu-byte aligned", kAlign);
-        if (sc.ok) return launch_scan<T, false>(in, values, indices, v, k, sc, ws, l, st);
-        if (c.ok) return launch_rows<T, false>(in, values, indices, v, k, c, ws, l, st);
+        if (sc.ok && largest) return launch_scan<T, false>(in, values, indices, v, k, sc, ws, l, st);
+        if (c.ok && largest) return launch_rows<T, false>(in, values, indices, v, k, c, ws, l, st);
+        if (sc.ok || c.ok) {
+            using R = vkop::Reversed<T>;
+            const R *rin = reinterpret_cast<const R *>(in);
+            R *rvalues = reinterpret_cast<R *>(values);
+            if (sc.ok) return launch_scan<R, false>(rin, rvalues, indices, v, k, sc, ws, l, st);
+            return launch_rows<R, false>(rin, rvalues, indices, v, k, c, ws, l, st);
+        }
         // (sorted == 0: the one route where an order costs a step of its own leaves it out; every other route's
         // result is in order by construction, which satisfies "any order" too)
         return launch_bigk<T, false>(in, values, indices, v, k, largest, b, ws, l, st, sorted != 0);
