@@ -147,3 +147,16 @@ def test_route_planner_without_a_gpu(lib):
     # the workspace a call is told to bring covers the headline shape with room in the static scratch's 4 MiB
     need = capi.softmax_topk_workspace_bytes(F32, (64, 128256), -1, 50)
     assert 64 * 1024 < need <= 4 << 20
+
+
+def test_native_front_end_refuses_what_the_operators_refuse():
+    """vkop_amd.ops reaches the C ABI through its native front end, which is built with the library; a tensor that is not on
+    a GPU, and what is no tensor, are TypeErrors before anything else happens."""
+    torch = pytest.importorskip("torch")
+    from vkop_amd import ops
+    x = torch.zeros(2, 5)
+    for call in (lambda t: ops.softmax(t), lambda t: ops.topk(t, 2), lambda t: ops.softmax_topk(t, 2),
+                 lambda t: ops.softmax_topk_sampling(t, 2, 1.0, 0.9), lambda t: ops.softmax_reduce_max(t, 1), lambda t: ops.reduce_max(t, 1)):
+        for bad in (x, x.numpy(), None):
+            with pytest.raises(TypeError, match="GPU"):
+                call(bad)

@@ -3,13 +3,35 @@
 torch is used for device memory and streams only; every computation goes
 through the C ABI (vkop_amd.capi).  Inputs must be contiguous CUDA/HIP tensors
 of float32 or float16; results are new tensors on the same device, enqueued on
-torch's current stream.
+torch's current stream.  What a call does on the host -- checks, results,
+workspace, stream -- is native code (vkop_amd/host/python/native.cpp, built
+into vkop_amd/_native.so); there is no fallback: if that is not built, the first
+call raises.
 """
+import ctypes
+
 import torch
 
 from . import capi
 
 _DTYPES = {torch.float32: capi.F32, torch.float16: capi.F16}
+_native = None
+
+
+def _load():
+    """The native front end, bound to the library capi has loaded (on the first call: capi may be pointed at
+    another build of the library before it)."""
+    global _native
+    L = capi.lib()
+    try:
+        from . import _native as module
+    except ImportError as e:
+        raise FileNotFoundError("vkop_amd/_native.so is not built (%s); run `python -c 'import __graft_entry__ as g; g.build()'` "
+                                "or `make -C vkop_amd/host`" % e) from e
+    names = [n for n in L._signatures if not n.endswith(("tune", "measure_stages", "measure_path"))]
+    module.bind({n[len("vkop_hip_"):]: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in names}, capi.VkopHipError)
+    _native = module
+    return module
 
 
 def _prep(x):
@@ -34,17 +56,18 @@ class Workspace:
 
     def __init__(self):
         self.buf = None
+        self.ptr = self.size = 0  # the 256-byte aligned part of buf that calls use
 
     def get(self, nbytes):
         nbytes = int(nbytes)
         if nbytes == 0:
             return 0, 0
-        if self.buf is None or self.buf.numel() < nbytes:
+        if self.size < nbytes:
             self.buf = torch.empty(nbytes + 256, dtype=torch.uint8, device="cuda")
-            self._off = (-self.buf.data_ptr()) % 256
-            self._size = (self.buf.numel() - self._off) // 4 * 4
-            capi.workspace_init(self.buf.data_ptr() + self._off, self._size, _stream())
-        return self.buf.data_ptr() + self._off, self._size
+            off = (-self.buf.data_ptr()) % 256
+            self.ptr, self.size = self.buf.data_ptr() + off, (self.buf.numel() - off) // 4 * 4
+            capi.workspace_init(self.ptr, self.size, _stream())
+        return self.ptr, self.size
 
 
 _default_ws = Workspace()
@@ -52,86 +75,34 @@ _default_ws = Workspace()
 
 def softmax(x, axis=-1, nan_where=False, nan_value=0.0, out=None, workspace=None):
     """ops/Softmax.hpp:61-141 -- same shape and dtype as x."""
-    x, dt = _prep(x)
-    if out is None:
-        out = torch.empty_like(x)
-    ws = workspace or _default_ws
-    ptr, size = ws.get(capi.softmax_workspace_bytes(dt, x.shape, axis))
-    capi.softmax(x.data_ptr(), out.data_ptr(), dt, x.shape, axis, int(bool(nan_where)), nan_value, ptr, size, _stream())
-    return out
-
-
-def _out_shape(x, axis, k):
-    shape = list(x.shape)
-    shape[axis if axis >= 0 else axis + x.dim()] = int(k)
-    return shape
+    return (_native or _load()).softmax(x, axis, nan_where, nan_value, out, workspace or _default_ws)
 
 
 def topk(x, k, axis=-1, largest=True, sorted=True, workspace=None):
     """ops/Topk.hpp:95-218 -- (values like x, int32 indices), [axis] = k."""
-    x, dt = _prep(x)
-    shape = _out_shape(x, axis, k)
-    values = torch.empty(shape, dtype=x.dtype, device=x.device)
-    indices = torch.empty(shape, dtype=torch.int32, device=x.device)
-    ws = workspace or _default_ws
-    ptr, size = ws.get(capi.topk_workspace_bytes(dt, x.shape, axis, k))
-    capi.topk(x.data_ptr(), values.data_ptr(), indices.data_ptr(), dt, x.shape, axis, k, int(bool(largest)),
-              int(bool(sorted)), ptr, size, _stream())
-    return values, indices
+    return (_native or _load()).topk(x, k, axis, largest, sorted, workspace or _default_ws)
 
 
 def softmax_topk(x, k, axis=-1, largest=True, return_probs=False, workspace=None):
     """The registered post-proc pair of benchmark/main.cpp:85-101 in one call:
     top-k of softmax(x) along `axis`, without materialising the softmax tensor
     unless return_probs is set."""
-    x, dt = _prep(x)
-    shape = _out_shape(x, axis, k)
-    values = torch.empty(shape, dtype=x.dtype, device=x.device)
-    indices = torch.empty(shape, dtype=torch.int32, device=x.device)
-    probs = torch.empty_like(x) if return_probs else None
-    ws = workspace or _default_ws
-    ptr, size = ws.get(capi.softmax_topk_workspace_bytes(dt, x.shape, axis, k))
-    capi.softmax_topk(x.data_ptr(), probs.data_ptr() if return_probs else 0, values.data_ptr(), indices.data_ptr(),
-                      dt, x.shape, axis, k, int(bool(largest)), ptr, size, _stream())
-    return (values, indices, probs) if return_probs else (values, indices)
+    return (_native or _load()).softmax_topk(x, k, axis, largest, return_probs, workspace or _default_ws)
 
 
 def softmax_topk_sampling(x, k, scale=1.0, top_p=None, axis=-1, workspace=None):
     """Sampling-style fused call: top-k of softmax(fl32(x * scale)); with top_p also the nucleus count per row.
     -> (values, indices) or (values, indices, counts)."""
-    x, dt = _prep(x)
-    shape = _out_shape(x, axis, k)
-    values = torch.empty(shape, dtype=x.dtype, device=x.device)
-    indices = torch.empty(shape, dtype=torch.int32, device=x.device)
-    cshape = list(x.shape)
-    del cshape[axis if axis >= 0 else axis + x.dim()]
-    counts = torch.empty(cshape, dtype=torch.int32, device=x.device) if top_p is not None else None
-    ws = workspace or _default_ws
-    ptr, size = ws.get(capi.softmax_topk_workspace_bytes(dt, x.shape, axis, k))
-    capi.softmax_topk_sampling(x.data_ptr(), values.data_ptr(), indices.data_ptr(), counts.data_ptr() if counts is not None else 0,
-                               dt, x.shape, axis, k, scale, top_p if top_p is not None else 0.0, ptr, size, _stream())
-    return (values, indices, counts) if top_p is not None else (values, indices)
+    return (_native or _load()).softmax_topk_sampling(x, k, scale, top_p, axis, workspace or _default_ws)
 
 
 def softmax_reduce_max(x, axis, workspace=None):
     """max over `axis` of softmax along `axis`, in one read (bit-equal to reduce_max(softmax(x, axis), axis))."""
-    x, dt = _prep(x)
-    shape = list(x.shape)
-    del shape[axis if axis >= 0 else axis + x.dim()]
-    out = torch.empty(shape, dtype=x.dtype, device=x.device)
-    ws = workspace or _default_ws
-    ptr, size = ws.get(capi.softmax_reduce_max_workspace_bytes(dt, x.shape, axis))
-    capi.softmax_reduce_max(x.data_ptr(), out.data_ptr(), dt, x.shape, axis, ptr, size, _stream())
-    return out
+    return (_native or _load()).softmax_reduce_max(x, axis, workspace or _default_ws)
 
 
 def reduce_max(x, axis):
-    x, dt = _prep(x)
-    shape = list(x.shape)
-    del shape[axis if axis >= 0 else axis + x.dim()]
-    out = torch.empty(shape, dtype=x.dtype, device=x.device)
-    capi.reduce_max(x.data_ptr(), out.data_ptr(), dt, x.shape, axis, _stream())
-    return out
+    return (_native or _load()).reduce_max(x, axis)
 
 
 def topp_count(values, p):
