@@ -151,6 +151,40 @@ def test_softmax_axes(ops, shape, axis):
     assert_softmax_close(host(ops.softmax(dev(xh), axis)), xh, axis, str((shape, axis)) + " half")
 
 
+@pytest.mark.parametrize("outer,n,inner,dtype",
+                         [(3, n, 1 + (1 << 19) // n // 2, np.float32) for n in (1, 2, 5, 15, 16, 17, 32, 33, 48, 63, 64, 65, 100, 127, 128)] +
+                         [(1, 16, 40003, np.float32), (7, 80, 999, np.float32), (40, 128, 4096, np.float32)] +
+                         [(o, n, i, dt) for dt in (np.float32, np.float16)
+                          for o, n, i in ((2, 129, 33), (1, 200, 1003), (5, 255, 65), (16, 256, 8), (30, 257, 9), (3, 513, 3137), (16, 511, 785),
+                                          (300, 600, 12), (33, 777, 65), (2, 1000, 4100), (9, 1023, 520), (1, 1024, 8193), (2, 1025, 64))] +
+                         [(3, 17, 110001, np.float16), (5, 32, 40000, np.float16), (3, 33, 170003, np.float16), (8, 64, 32769, np.float16),
+                          (4, 65, 130001, np.float16), (33, 128, 8001, np.float16)])
+def test_softmax_lines_in_registers(ops, outer, n, inner, dtype):
+    """Lines along the middle axis that lanes, waves and workgroups hold in registers: line lengths
+    around the elements a lane, the lanes and the waves of a line, rows that are no whole number of
+    16-byte vectors and a tensor off 16 bytes; special lines; in place; the replacement of NaN; and the
+    largest probability alone, bit for bit the maximum of the tensor."""
+    rng = np.random.default_rng(outer + n + inner)
+    x = (rng.standard_normal((outer, n, inner), dtype=np.float32) * 3).astype(dtype)
+    x[0, n - 1, inner - 1], x[0, 0, 1], x[0, :, 2], x[-1, n // 2, 0] = np.nan, np.inf, -np.inf, np.nan
+    buf = torch.empty(x.size + 1, dtype=torch.float16 if dtype == np.float16 else torch.float32, device="cuda")
+    view = buf[1:].view(x.shape)
+    view.copy_(dev(x))
+    out = torch.full((x.size + 2,), 7.0, dtype=buf.dtype, device="cuda")
+    ops.softmax(view, axis=1, out=out[1:-1].view(x.shape))
+    o = host(out)
+    got = o[1:-1].reshape(x.shape)
+    assert o[0] == 7.0 and o[-1] == 7.0
+    assert_softmax_close(got, x, 1, str((outer, n, inner)))
+    nan = np.isnan(got)
+    fixed = host(ops.softmax(view, axis=1, nan_where=True, nan_value=0.25))
+    assert np.array_equal(fixed[~nan], got[~nan]) and np.all(fixed[nan] == dtype(0.25))
+    best = host(ops.softmax_reduce_max(view, 1))
+    assert np.array_equal(best, got.max(axis=1), equal_nan=True)
+    ops.softmax(view, axis=1, out=view)  # in place
+    assert np.array_equal(host(view), got, equal_nan=True)
+
+
 @pytest.mark.parametrize("shape,axis", [((4096, 64), -1), ((4096, 1024), -1), ((8192, 512), -1), ((300, 2048), -1), ((64, 40000), -1),
                                         ((16, 80, 840), 1), ((2, 1000, 64), 1), ((8, 4096, 64), 1)])
 def test_softmax_half_near_rounding_boundaries(ops, shape, axis):

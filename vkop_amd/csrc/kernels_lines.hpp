@@ -1,0 +1,215 @@
+// Softmax along a non-last axis, lines of up to kLinesMaxN elements: one read, one write.
+//
+// A tensor is [outer][n][inner]; a line is the n elements that lie inner apart.  A lane holds L
+// neighbouring lines (a 16-byte vector of the inner axis, at any alignment), of every line the
+// elements part, part + parts, ..., K of them at most.  The parts of a line are P groups of lanes of
+// a wave times W waves of a workgroup: maxima and sums cross the lanes by register exchanges and,
+// with W > 1, the waves through LDS (three barriers).
+// What bounds it: with wide rows the memory system ([8,21,262144] f32 81.5 -> 66.3 us, 5.3 TB/s; the
+// largest probability alone, one read, 65.6 -> 42.2), with long lines the workgroups that hold them --
+// 1024 elements are 8 waves of 100 registers, two a CU, and loads, exponentials and stores of two
+// overlap little ([8,1000,8000] f32 192 -> 113 us, 4.5 TB/s, where three passes of 4-byte accesses
+// ran before).  The rule that picks P, W and K, with what it was measured on: plan_lines.
+#pragma once
+
+#include "kernels_softmax.hpp"
+
+namespace vkop {
+
+constexpr int kLinesWavesMax = 16;
+
+// The value of the lane whose number differs in bit STRIDE.
+template <int STRIDE> __device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+    if constexpr (STRIDE == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return (threadIdx.x & 32u) ? r[0] : r[1];
+    } else if constexpr (STRIDE == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return (threadIdx.x & 16u) ? r[0] : r[1];
+    } else if constexpr (STRIDE == 8) {
+        return dpp_u32<0x128>(v);  // (a rotation of sixteen by eight)
+    } else {
+        return static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), STRIDE, kWave));
+    }
+}
+// Larger / sum over the P lanes of a wave that look at the same lines (lanes 64 / P apart).  The sum
+// adds both lanes of a pair in the same order, so every lane ends with the same bits.
+template <int P, typename F> __device__ __forceinline__ uint32_t join_parts(uint32_t v, F op) {
+    if constexpr (P >= 2) v = op(v, lane_xor<32>(v));
+    if constexpr (P >= 4) v = op(v, lane_xor<16>(v));
+    if constexpr (P >= 8) v = op(v, lane_xor<8>(v));
+    if constexpr (P >= 16) v = op(v, lane_xor<4>(v));
+    return v;
+}
+template <int P> __device__ __forceinline__ float parts_max(float v) {
+    return __uint_as_float(join_parts<P>(__float_as_uint(v), [](uint32_t a, uint32_t b) { return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b))); }));
+}
+template <int STRIDE> __device__ __forceinline__ double add_lane_xor(double v) {
+    const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
+    const uint64_t o = (static_cast<uint64_t>(lane_xor<STRIDE>(static_cast<uint32_t>(u >> 32))) << 32) | lane_xor<STRIDE>(static_cast<uint32_t>(u));
+    return v + __longlong_as_double(static_cast<long long>(o));
+}
+template <int P> __device__ __forceinline__ double parts_sum(double v) {
+    if constexpr (P >= 2) v = add_lane_xor<32>(v);
+    if constexpr (P >= 4) v = add_lane_xor<16>(v);
+    if constexpr (P >= 8) v = add_lane_xor<8>(v);
+    if constexpr (P >= 16) v = add_lane_xor<4>(v);
+    return v;
+}
+
+// MAX_ONLY: instead of the softmax tensor write each line's largest probability to out[line]: from
+// the same sums, so bit-equal to the maximum of what the other form writes.
+// K = ceil(n / (P * W)): every element but a lane's last exists.
+// Launch: blockDim = teams * W waves, a team of W waves per 64 / P vectors; LDS for W > 1:
+// 64 / P * L * (W * teams) doubles.
+template <typename T, int K, int P, bool MAX_ONLY>
+__global__ __launch_bounds__(kLinesWavesMax *kWave) void softmax_lines_reg_kernel(const T *in, T *out, LineGeom g, uint32_t W,
+                                                                                int nan_where, float nan_value) {
+    constexpr int L = Vec128<T>::N;
+    constexpr uint32_t LPW = kWave / P;  // vectors (of L lines) a wave
+    extern __shared__ double lines_lds[];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave)));
+    const uint32_t teams = blockDim.x / kWave / W, team = wave / W, tw = wave - team * W;
+    const uint32_t vpo = (g.inner + L - 1u) / L, total = g.outer * vpo;  // vectors an outer index, and in all
+    const uint32_t slot = lane & (LPW - 1u), part = tw * P + lane / LPW, parts = W * P;
+    // (neighbouring vectors share cache lines where rows of the slab start off a line boundary)
+    const uint32_t vec = (xcd_grouped_block() * teams + team) * LPW + slot;
+    const bool live = vec < total;
+    const uint32_t o = (live ? vec : 0u) / vpo, iv = (live ? vec : 0u) - o * vpo;  // (idle lanes shadow the first vector and store nothing)
+    const uint32_t col = min(iv * L, g.inner - L);  // the last vector of a row is moved back to end with it ...
+    const uint32_t skip = iv * L - col;             // ... and this many of its lines are the one's before
+    const size_t base = static_cast<size_t>(o) * g.n * g.inner + col;
+    const uint32_t n = g.n;
+    const bool last_ok = (K - 1) * parts + part < n;
+    Vec128<T> q[K];
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+        const uint32_t j = static_cast<uint32_t>(i) * parts + part;
+        q[i].v = load16_stream(in + base + static_cast<size_t>(i < K - 1 || last_ok ? j : n - 1u) * g.inner);
+    }
+    float m[L];
+    if constexpr (sizeof(T) == 2) {
+        uint32_t pk[4] = {q[0].v.x, q[0].v.y, q[0].v.z, q[0].v.w};
+#pragma unroll
+        for (int i = 0; i < K; i++) {  // (q[0] again: max_half2 drops NaN only against a number)
+            pk[0] = max_half2(pk[0], q[i].v.x), pk[1] = max_half2(pk[1], q[i].v.y);
+            pk[2] = max_half2(pk[2], q[i].v.z), pk[3] = max_half2(pk[3], q[i].v.w);
+        }
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            pk[w] = join_parts<P>(max_half2(pk[w], 0xFC00FC00u), [](uint32_t a, uint32_t b) { return max_half2(a, b); });
+            m[2 * w] = __half2float(__ushort_as_half(static_cast<uint16_t>(pk[w] & 0xFFFFu)));
+            m[2 * w + 1] = __half2float(__ushort_as_half(static_cast<uint16_t>(pk[w] >> 16)));
+        }
+    } else {
+#pragma unroll
+        for (int c = 0; c < L; c++) {
+            m[c] = -INFINITY;
+#pragma unroll
+            for (int i = 0; i + 1 < K; i += 2) m[c] = max3(m[c], q[i].get(c), q[i + 1].get(c));  // (drops NaN)
+            if constexpr (K % 2 != 0) m[c] = max3(m[c], m[c], q[K - 1].get(c));
+            m[c] = parts_max<P>(m[c]);
+        }
+    }
+    if (W > 1) {
+        // a wave's maxima are in each of its parts: the first writes them, and each part reads its share of the waves
+        float *fl = reinterpret_cast<float *>(lines_lds) + team * (W * LPW * L);
+        if (lane < LPW) {
+#pragma unroll
+            for (int c = 0; c < L; c++) fl[(tw * L + c) * LPW + slot] = m[c];
+        }
+        __syncthreads();
+        for (uint32_t w = lane / LPW; w < W; w += P) {
+#pragma unroll
+            for (int c = 0; c < L; c++) m[c] = fmaxf(m[c], fl[(w * L + c) * LPW + slot]);
+        }
+#pragma unroll
+        for (int c = 0; c < L; c++) m[c] = parts_max<P>(m[c]);
+        __syncthreads();  // (the sums take the same place)
+    }
+    float e[K][L];
+    TermSum<T> acc[L];
+#pragma unroll
+    for (int c = 0; c < L; c++) acc[c] = 0;
+#pragma unroll
+    for (int i = 0; i < K; i++) {
+        // (a vector after the other: scheduled together, the terms of sixteen do not fit the registers)
+        asm volatile("" : "+v"(q[i].v.x), "+v"(q[i].v.y), "+v"(q[i].v.z), "+v"(q[i].v.w));
+#pragma unroll
+        for (int c = 0; c < L; c++) {
+            e[i][c] = softmax_term_as<T>(q[i].get(c), m[c]);
+            acc[c] += static_cast<TermSum<T>>(i < K - 1 || last_ok ? e[i][c] : 0.f);
+        }
+    }
+    double s[L];
+#pragma unroll
+    for (int c = 0; c < L; c++) s[c] = parts_sum<P>(static_cast<double>(acc[c]));
+    if (W > 1) {
+        double *dl = lines_lds + team * (W * LPW * L);
+        if (lane < LPW) {
+#pragma unroll
+            for (int c = 0; c < L; c++) dl[(tw * L + c) * LPW + slot] = s[c];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < L; c++) s[c] = 0.0;
+        for (uint32_t w = lane / LPW; w < W; w += P) {  // fixed order: run-to-run stable
+#pragma unroll
+            for (int c = 0; c < L; c++) s[c] += dl[(w * L + c) * LPW + slot];
+        }
+#pragma unroll
+        for (int c = 0; c < L; c++) s[c] = parts_sum<P>(s[c]);
+    }
+    if constexpr (MAX_ONLY) {
+        if (live && part == 0) {
+            // the line's maximum has the term exp(0) = 1 (NaN where there is none, as the tensor would hold)
+            const size_t at = static_cast<size_t>(o) * g.inner + col;
+            Vec128<T> r;
+            r.v = make_uint4(0, 0, 0, 0);
+            float p[L];
+#pragma unroll
+            for (int c = 0; c < L; c++) {
+                p[c] = scale_term<T>(softmax_term_as<T>(m[c], m[c]), reciprocal_of_sum(s[c]));
+                r.set(c, p[c]);
+            }
+            if (skip == 0) store16_stream(out + at, r.v);
+            else {
+#pragma unroll
+                for (int c = 1; c < L; c++)
+                    if (static_cast<uint32_t>(c) >= skip) store_elem(out, at + c, p[c]);
+            }
+        }
+        return;
+    }
+    double rinv[L];
+#pragma unroll
+    for (int c = 0; c < L; c++) rinv[c] = reciprocal_of_sum(s[c]);
+    size_t at = base + static_cast<size_t>(part) * g.inner;
+    asm volatile("" : "+v"(at));  // (places again: sixteen of them kept from the loads are 32 registers)
+#pragma unroll
+    for (int i = 0; i < K; i++, at += static_cast<size_t>(parts) * g.inner) {
+        float p[L];
+        Vec128<T> r;
+        r.v = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < L; c++) asm volatile("" : "+v"(e[i][c]));
+#pragma unroll
+        for (int c = 0; c < L; c++) {
+            p[c] = scale_term<T>(e[i][c], rinv[c]);
+            if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
+            r.set(c, p[c]);
+        }
+        if (live && (i < K - 1 || last_ok)) {
+            if (skip == 0) store16_stream(out + at, r.v);
+            else {
+                // (its own lines alone: the others are another wave's, which may have stored them, in place, already)
+#pragma unroll
+                for (int c = 1; c < L; c++)
+                    if (static_cast<uint32_t>(c) >= skip) store_elem(out, at + c, p[c]);
+            }
+        }
+    }
+}
+
+}  // namespace vkop

@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "kernels_general.hpp"
 #include "kernels_rows.hpp"
 #include "kernels_bigpick.hpp"
 #include "kernels_stream.hpp"
@@ -97,5 +98,22 @@ extern template void launch_rows_merge<float, true>(const RowsLaunch &);
 extern template void launch_rows_merge<float, false>(const RowsLaunch &);
 extern template void launch_rows_merge<uint16_t, true>(const RowsLaunch &);
 extern template void launch_rows_merge<uint16_t, false>(const RowsLaunch &);
+
+// Softmax (or, max_only, each line's largest probability) along a non-last axis in registers
+// (kernels_lines.hpp); false if no kernel is built for (k, p).
+constexpr uint32_t kLinesMaxN = 1024;
+struct LinesLaunch {
+    const void *in;
+    void *out;
+    LineGeom g;
+    uint32_t k, p, w;  // elements of a line a lane, lane groups of a wave a line, waves a line
+    bool max_only;
+    int nan_where;
+    float nan_value;
+    hipStream_t stream;
+};
+template <typename T> bool launch_softmax_lines(const LinesLaunch &a);
+extern template bool launch_softmax_lines<float>(const LinesLaunch &);
+extern template bool launch_softmax_lines<uint16_t>(const LinesLaunch &);
 
 }  // namespace vkop

@@ -157,9 +157,10 @@ struct RowShape {
 };
 
 struct SoftmaxPlan {
-    enum Kind { kGeneralLines, kGeneralStrided, kThread, kGroup, kRow, kChunked, kStridedRegs, kStridedTile } kind = kGeneralLines;
+    enum Kind { kGeneralLines, kGeneralStrided, kThread, kGroup, kRow, kChunked, kLinesRegs, kStridedRegs, kStridedTile } kind = kGeneralLines;
     RowShape shape{0, 0};  // kChunked; kGroup: lanes a row and vectors a lane; kRow: threads and vectors a thread
     uint32_t g = 1, per = 0;
+    uint32_t lines_k = 0, lines_p = 0, lines_w = 0;  // kLinesRegs: LinesLaunch
     uint32_t ti_shift = 0;  // kStridedTile: log2 of the lines a tile
     size_t workspace = 0;
 };
@@ -187,11 +188,54 @@ void launch_strided_reg(const T *in, T *out, const View &v, int nan_where, float
 #undef VKOP_STRIDED_CASE
 }
 
+// The register kernel for lines along a non-last axis (kernels_lines.hpp) and its shape: lane groups of a
+// wave a line (P), waves a line (W) and elements a lane (K).  False: the kernels of one element a load.
+// us a call, those against this one: f32 [8,21,262144] 81.5 -> 66.3, [16,80,8400] max only 19.1 -> 15.1,
+// [16,512,784] 28.6 -> 14.3, [8,1000,8000] 192 -> 113, [32,1000,64] 18.4 -> 10.0; f16 [8,21,262144] 49.9 ->
+// 38.6, [2,512,3136] 20.9 -> 9.8, [8,200,65536] 179 -> 96.
+bool plan_lines(const View &v, uint32_t vec, SoftmaxPlan *p) {
+    const uint32_t n = v.g.n;
+    if (v.g.inner < vec || n > vkop::kLinesMaxN) return false;
+    const bool half = vec == 8;
+    const uint64_t vectors = static_cast<uint64_t>(v.g.outer) * ((v.g.inner + vec - 1) / vec);
+    // Short lines of few elements in all have too few lanes with 16 bytes each (f32 [1,4,65536] 3.1 against 3.2 us
+    // here, [1,80,8400] 5.8 against 4.9).  Halves, twice as many lines a lane: [1,80,8400] 4.2 against 6.1,
+    // [4,91,12345] 7.6 against 9.9, but [4,24,65536] 8.6 against 8.1, [8,48,65536] 30.4 against 22.5 and
+    // [8,100,65536] 64 against 60; their lines of up to 16 never gain more than they lose ([8,16,262144] 26.9 / 28.3).
+    if (n <= 128) {
+        if (v.elems < (1u << 19)) return false;
+        if (half && (n <= 16 || v.elems < (n <= 32 ? 5ull << 20 : n <= 64 ? 1ull << 24 : 1ull << 25))) return false;
+    } else if (vectors < 32) {  // ([1,1000,64] f16 10.2 against 11.9, f32 max only 8.3 against 9.2)
+        return false;
+    }
+    // As many elements a lane as its registers hold (f32 16, f16 8: their 64 terms either way), and pieces of a row
+    // of 128 bytes at least (P = 8) before a line takes several waves: a workgroup of many holds a CU on its
+    // barriers ([8,1000,8000] f32 with P = 4 126, 8 113, 16 157 us).  With too few workgroups for the chip, more of
+    // them: P = 16, half the lines ([32,1000,64] f32 13.0 -> 10.5, f16 17.5 -> 12.0).
+    const uint32_t kmax = half ? 8 : 16, need = (n + kmax - 1) / kmax;
+    uint32_t P = 1;
+    while (P < 8 && P < need) P *= 2;
+    if (half && n > 64 && n <= 128) P = 16;  // ([8,100,65536] max only: 36.1 us, with P = 8 41.8)
+    if (n > 128 && vectors / 8 < (half ? 512u : 128u)) P = 16;
+    uint32_t W = (need + P - 1) / P, K = (n + P * W - 1) / (P * W);
+    // fewer than 512 waves: fewer elements a lane, while that is more than 4 and a line has at most 4 waves
+    // ([1,80,8400] f32 6.3 -> 4.9, [1,200,1000] 8.2 -> 5.7; [32,777,65] f16 with 14 waves 14.7, with 7 12.6)
+    while (K > 4 && W <= 4 && vectors * P * W < 512ull * vkop::kWave) {
+        if (P < 16) P *= 2;
+        else W *= 2;
+        K = (n + P * W - 1) / (P * W);
+    }
+    p->kind = SoftmaxPlan::kLinesRegs;
+    p->lines_k = K, p->lines_p = P, p->lines_w = W;
+    return true;
+}
+
 SoftmaxPlan plan_softmax(const View &v, int dtype) {
     SoftmaxPlan p;
     const uint32_t vec = dtype == VKOP_HIP_F32 ? 4u : 8u;
     const uint32_t n = v.g.n, rows = v.g.outer;
     if (v.g.inner != 1) {
+        if (plan_lines(v, vec, &p)) return p;
         if (n <= static_cast<uint32_t>(vkop::kStridedMaxN)) p.kind = SoftmaxPlan::kStridedRegs;
         else {
             // a tile of TI lines (the power of two at or above min(inner, 64)) per workgroup; with too
@@ -325,6 +369,12 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
         if constexpr (sizeof(T) == 4) { VKOP_SCALE(4) }
 #undef VKOP_SCALE
         return launched("softmax_stats_kernel / softmax_scale_kernel");
+    }
+    case SoftmaxPlan::kLinesRegs: {
+        const vkop::LinesLaunch a{in, out, v.g, p.lines_k, p.lines_p, p.lines_w, false, nan_where, nan_value, st};
+        if (!vkop::launch_softmax_lines<T>(a))
+            return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
+        return launched("softmax_lines_reg_kernel");
     }
     case SoftmaxPlan::kStridedRegs: {
         launch_strided_reg<T, false>(in, out, v, nan_where, nan_value, st);
@@ -927,13 +977,19 @@ size_t selection_workspace(const View &v, int k, int dtype) {
 template <typename T>
 int softmax_reduce_max_impl(const T *in, T *out, const View &v, void *ws, size_t ws_bytes, hipStream_t st) {
     const uint32_t lines = v.g.outer * v.g.inner;
+    const SoftmaxPlan p = plan_softmax(v, sizeof(T) == 4 ? VKOP_HIP_F32 : VKOP_HIP_F16);
+    if (p.kind == SoftmaxPlan::kLinesRegs) {
+        const vkop::LinesLaunch a{in, out, v.g, p.lines_k, p.lines_p, p.lines_w, true, 0, 0.f, st};
+        if (!vkop::launch_softmax_lines<T>(a))
+            return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
+        return launched("softmax_lines_reg_kernel (max)");
+    }
     if (v.g.n <= static_cast<uint32_t>(vkop::kStridedMaxN)) {
         launch_strided_reg<T, true>(in, out, v, 0, 0.f, st);
         return launched("softmax_strided_reg_kernel");
     }
     if (v.g.inner != 1) {
         // long lines along a non-last axis: the statistics of the tile kernel, as the softmax itself takes them
-        const SoftmaxPlan p = plan_softmax(v, sizeof(T) == 4 ? VKOP_HIP_F32 : VKOP_HIP_F16);
         const uint32_t tiles = v.g.outer * ((v.g.inner + (1u << p.ti_shift) - 1) >> p.ti_shift);
         if (p.g == 1) {
             vkop::softmax_strided_tile_kernel<T, vkop::kTileWholeMax>
