@@ -1081,6 +1081,48 @@ def test_nms_random_configurations(ops):
         capi.tune("nms.threads", 0)
 
 
+@pytest.mark.parametrize("power", [-80, -41, -39, 0, 39, 41, 62])
+def test_nms_overlap_beside_the_threshold(ops, power):
+    """The quotient of the areas is compared without being formed where products decide: thresholds 2^-20 and 2^-18
+    beside some pair's own overlap -- the products decide from 2^-21 on, and 2^-22 bounds what a fused product
+    moves in the areas -- with boxes scaled by powers of two up to areas near the largest float and down to ones
+    that underflow to nothing."""
+    rng = np.random.default_rng(100 + power)
+    boxes = _nms_boxes(rng, 1, 96, 0.6) * np.float32(2.0 ** power)
+    scores = rng.random((1, 3, 96)).astype(np.float32)
+    a, b = boxes[0, :48], boxes[0, 48:]
+    f = np.float32
+    w, h = np.minimum(a[:, 2], b[:, 2]) - np.maximum(a[:, 0], b[:, 0]), np.minimum(a[:, 3], b[:, 3]) - np.maximum(a[:, 1], b[:, 1])
+    inter = (np.maximum(w, f(0)) * np.maximum(h, f(0))).astype(f)
+    area = lambda t: ((t[:, 2] - t[:, 0]) * (t[:, 3] - t[:, 1])).astype(f)
+    union = ((area(a) + area(b)).astype(f) - inter).astype(f)
+    iou = (inter[union > 0] / union[union > 0]).astype(f)
+    pool = iou[iou > 0][:6] if (iou > 0).any() else np.array([0.3], f)
+    for t in pool:
+        for thr in (t * f(1 + 2.0 ** -20), t * f(1 - 2.0 ** -20), t * f(1 + 2.0 ** -18), t * f(1 - 2.0 ** -18)):
+            got, _ = ops.nms(dev(boxes), dev(scores), float(thr), 0.1)
+            assert np.array_equal(host(got), oracle.nms(boxes, scores, float(thr), 0.1, 0, max_candidates=2048)), (power, thr)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_nms_rows_of_any_length_and_alignment(ops, dtype):
+    """Scores are read four at a time from any element on: rows shorter than that, rows that end inside a load, a
+    tensor off 16 bytes, and the numbers of pairs on both sides of the change of workgroup size."""
+    rng = np.random.default_rng(12)
+    for B, C, N in [(1, 1, 1), (1, 3, 2), (2, 2, 3), (1, 2, 5), (2, 3, 7), (1, 5, 1023), (2, 2, 1917), (1, 2, 9217), (3, 1, 12291),
+                    (2, 256, 77), (3, 171, 78), (9, 57, 1025)]:
+        boxes = _nms_boxes(rng, B, N, 0.3).astype(dtype)
+        scores = rng.random((B, C, N)).astype(dtype)
+        buf = torch.empty(scores.size + 1, dtype=torch.float16 if dtype == np.float16 else torch.float32, device="cuda")
+        view = buf[1:].view(scores.shape)
+        view.copy_(dev(scores))
+        thr = 0.9 if N > 1000 else 0.2
+        want = oracle.nms(boxes.astype(np.float32), scores.astype(np.float32), 0.45, thr, 0, max_candidates=2048)
+        for t in (dev(scores), view):
+            got, over = ops.nms(dev(boxes), t, 0.45, thr)
+            assert not over and np.array_equal(host(got), want), (B, C, N, dtype)
+
+
 def test_nms_detection_workload_full_size(ops):
     """The detection-shaped case of the operator benchmark, and a dense one with a per-class limit, against the oracle."""
     c5 = synth.detection_scores(16, 80, 8400, synth.SEEDS["C5"])
