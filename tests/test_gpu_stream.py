@@ -401,6 +401,33 @@ def test_sampling_variant_against_the_oracle(ops, shape, k, dtype):
                 assert np.array_equal(ix.reshape(-1, k)[r], oix.reshape(-1, k)[r]), (what, r)
 
 
+@pytest.mark.parametrize("k", [1, 5, 20, 31, 32, 40, 63, 64, 100, 150, 200, 255])
+@pytest.mark.parametrize("n", [50257, 131072])
+def test_sampling_half_rows_whose_probabilities_tie(ops, n, k):
+    """Long half rows under a temperature: the probabilities near the k-th place are subnormal halves, and elements
+    of different logits share one.  They are in order of index, whether the candidates at hand settle the group at
+    the k-th place or the row has to be read again: rows spread out, of a coarse grid, and ones whose tail all
+    rounds to the smallest half or to nothing."""
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((12, n)).astype(np.float32)
+    x[np.arange(12), rng.integers(0, n, 12)] += np.linspace(3, 16, 12, dtype=np.float32)
+    x[4:7] = np.round(x[4:7] * 16) / 16
+    x[7, rng.integers(0, n, 4 * k)] += np.float32(2.0)
+    x = np.ascontiguousarray((x * np.float32(1.25)).astype(np.float16))
+    for scale, top_p in ((1.25, 0.9), (1.0, 0.5), (0.75, 0.95)):
+        v, ix, c = (host(t) for t in ops.softmax_topk_sampling(dev(x), k, scale, top_p))
+        ov, oix, oc = oracle.softmax_topk_sampling(x, k, scale, top_p)
+        # Sums agree to 2^-22, so a probability that close to the boundary between two normal halves, 2^-11 apart, may
+        # fall on either side of it: one in 2^-10 of the values, a unit each, and where it joins or leaves the group at the
+        # k-th place the row's indices move with it.
+        assert half_ulp_diff(v, ov).max() <= 1 and (v.view(np.uint16) != ov.view(np.uint16)).sum() <= max(2, v.size >> 9)
+        assert ((ix == oix).all(axis=-1) | (v.view(np.uint16) != ov.view(np.uint16)).any(axis=-1)).sum() >= 11, (n, k, scale)
+        assert np.array_equal(c, oracle.topp_count(v.astype(np.float32), top_p))
+        # equal probabilities in order of index, in every row
+        equal = v[:, 1:] == v[:, :-1]
+        assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])
+
+
 @pytest.mark.parametrize("n", [50000, 8192, 1000, 8400])
 def test_sampling_variant_ties_special_rows_and_errors(ops, n):
     """(n = 50000: the scan + pick kernels; the shorter rows: one workgroup, or one wave, per row)"""

@@ -709,6 +709,29 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                     if (base == 0) p_first = p0;
                 }
                 tie = __ballot(tie) != 0ull;
+                bool by_index = false;  // (the same in every thread, as `tie` is)
+                if (tie) {
+                    // Where some candidate's probability lies below the k-th, every element of the row with a
+                    // probability of the first k is in the list (probabilities fall with the logits, and what is
+                    // not listed has a smaller logit than all that is): ranked once more by (probability, index)
+                    // the list gives their order.  Half-precision probabilities of long rows are small, some of
+                    // them subnormal, and nearly every call has such a row: f16 at a scale of 1.25 [32,50257] k = 40
+                    // 16.6 -> 15.4 us a call (17.2 -> 13.6 over other inputs), k = 90 20.7 -> 16.0, [8,32000] k = 40
+                    // 14.2 -> 12.0, [16,200000] k = 64 16.4 -> 13.6; where the groups are larger than what the list holds
+                    // beyond k -- [128,50257] k = 20 -- 23.6 as before, and a lower threshold did not change that.
+                    const float p_own = tid < C2 ? round_to_storage<T>(static_cast<float>(static_cast<double>(term) * rinv)) : 0.f;
+                    const float p_cut = round_to_storage<T>(static_cast<float>(static_cast<double>(sh.prob[k - 1u]) * rinv));
+                    by_index = __syncthreads_or(tid < C2 && p_own < p_cut) != 0;
+                    if (by_index) {
+                        const uint32_t idx = composite_index(mine);
+                        if (tid < C2) sh.cand[tid] = p_own >= p_cut ? composite(__float_as_uint(p_own), idx) : 0ull;
+                        sh.rank[tid] = 0;
+                        __syncthreads();
+                        block_rank_padded<NT>(sh, max(C2, 33u));
+                        if (tid < C2 && p_own >= p_cut && sh.rank[tid] < k) oi[sh.rank[tid]] = static_cast<int32_t>(idx);
+                        tie = false;
+                    }
+                }
                 if (!tie) {
                     // (the waves take the ranks 64 at a time, in turn)
                     for (uint32_t base = wave * kWave; base < k; base += NW * kWave) {
@@ -717,7 +740,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                                                    : round_to_storage<T>(static_cast<float>(static_cast<double>(sh.prob[r < k ? r : 0u]) * rinv));
                         if (r < k) {
                             store_elem(ov, r, p0);
-                            oi[r] = static_cast<int32_t>(sh.pidx[r]);
+                            if (!by_index) oi[r] = static_cast<int32_t>(sh.pidx[r]);
                         }
                     }
                 }
