@@ -33,10 +33,11 @@
 namespace vkop {
 
 constexpr int kNmsThreadsWide = 1024;   // few (batch, class) pairs
-constexpr int kNmsThreadsNarrow = 256;  // more than the chip holds wide workgroups at a time, two a CU
-// (us a call at f32, wide / narrow: [4,80,8400] 15.0 / 17.9, [8,80,8400] 20.9 / 20.6, [8,91,1917] 16.0 / 12.6,
-// [12,80,8400] 24.9 / 23.2, [16,80,8400] 31.7 / 26.5)
-constexpr int kNmsNarrowMinPairs = 513;
+constexpr int kNmsThreadsNarrow = 256;  // twice as many as the chip holds wide workgroups at a time, two a CU
+// (us a call at f32, wide / narrow: [4,80,8400] 15.0 / 17.9, [8,80,8400] 20.9 / 20.6, [8,91,1917] 15.2 / 12.6,
+// [12,80,8400] 24.1 / 22.4, [16,80,8400] 31.3 / 25.3.  From 513 pairs on narrow ones gain where candidates are
+// few, but where all of 2048 are they lose more: [8,80,2048] 285 / 424)
+constexpr int kNmsNarrowMinPairs = 1024;
 constexpr int kNmsMaxCandidates = 2048;  // per (batch, class); the reference's shader holds 1024
 constexpr int kNmsRankSortMax = 512;     // up to here a counting sort beats the bitonic network's barriers
 
@@ -58,10 +59,22 @@ __device__ __forceinline__ float4 nms_load4(const uint16_t *p) {
                        __half2float(__ushort_as_half(static_cast<unsigned short>(w.y >> 16))));
 }
 
+__device__ __forceinline__ float nms_iou(const float4 &a, const float4 &b) {
+    const float x1 = fmaxf(a.x, b.x), y1 = fmaxf(a.y, b.y), x2 = fminf(a.z, b.z), y2 = fminf(a.w, b.w);
+    if (x2 <= x1 || y2 <= y1) return 0.f;
+    const float inter = __fmul_rn(__fsub_rn(x2, x1), __fsub_rn(y2, y1));
+    const float area_a = __fmul_rn(__fsub_rn(a.z, a.x), __fsub_rn(a.w, a.y));
+    const float area_b = __fmul_rn(__fsub_rn(b.z, b.x), __fsub_rn(b.w, b.y));
+    const float uni = __fsub_rn(__fadd_rn(area_a, area_b), inter);
+    return uni > 0.f ? __fdiv_rn(inter, uni) : 0.f;
+}
+
 // IoU(a, b) > threshold, the division left out where the comparison does not need it: with t = threshold
 // and f = fl(t * uni), away from underflow and overflow inter > f (1 + 2^-21) means a quotient above t (1 + 2^-22)
 // (f is within 2^-24 of t * uni), whose rounding lies above t, and inter < f (1 - 2^-21) one below t, whose
-// rounding does not.  It is a third of the instructions of the whole, paid for every pair of a block.
+// rounding does not.  It is a third of the instructions of the whole, paid for every pair of a block.  (The walk of
+// more than kNmsRankSortMax candidates divides: its loop ends at the first overlap, and the branches around the
+// division cost it more than that -- [8,80,2048] all candidates 288 us, by products 325; [1,1,2048] 698 / 747.)
 __device__ __forceinline__ bool nms_overlap(const float4 &a, const float4 &b, float threshold) {
     const float x1 = fmaxf(a.x, b.x), y1 = fmaxf(a.y, b.y), x2 = fminf(a.z, b.z), y2 = fminf(a.w, b.w);
     if (x2 <= x1 || y2 <= y1) return 0.f > threshold;
@@ -86,7 +99,7 @@ __device__ __forceinline__ bool nms_overlap(const float4 &a, const float4 &b, fl
 // What bounds it: each workgroup's own chain -- scores from HBM (half of the call), a sort,
 // the blocks of the walk -- with five of them a CU to overlap.  us a call with the pack
 // kernel, 0.25 / 0.45, 51 kept a pair: [16,80,8400] f32 34.6 -> 26.3 (walk 16 -> 8), f16
-// 33.2 -> 24.6; [1,80,8400] f32 18.7 -> 11.2; [8,91,1917] f32 16.0 -> 12.5.
+// 33.2 -> 24.6; [1,80,8400] f32 18.7 -> 11.2; [8,91,1917] f32 16.2 -> 15.2; [8,80,400] all candidates 52 -> 32.
 // WHOLE: N is a multiple of four, and no load needs the step for a row's end ([16,80,8400] f32 26.3 us, before
 // that step was kept to the wave it concerns 29.0; [16,91,8399] f16, score by score before, 30.4 -> 24.4).
 template <typename T, int NT, bool WHOLE>
@@ -347,7 +360,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
 #pragma unroll
         for (int r = 0; r < JP; r++) {
             const uint32_t j = wave * JP + static_cast<uint32_t>(r);
-            if (lane > j && nms_overlap(bi, box[j], iou_threshold)) bits |= 1u << r;
+            if (lane > j && nms_iou(bi, box[j]) > iou_threshold) bits |= 1u << r;
         }
         if (bits != 0) atomicOr(&block_cols[lane], static_cast<unsigned long long>(bits) << (wave * JP));
         __syncthreads();  // (also: the bits cleared by the block before are in place)
@@ -367,7 +380,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
             if (p >= base + kWave && p < K && ((active[p / 64] >> (p % 64)) & 1ull)) {
                 bool dead = false;
                 for (uint64_t kk = keep; kk != 0 && !dead; kk &= kk - 1)
-                    dead = nms_overlap(mine[e], box[static_cast<uint32_t>(__builtin_ctzll(kk))], iou_threshold);
+                    dead = nms_iou(mine[e], box[static_cast<uint32_t>(__builtin_ctzll(kk))]) > iou_threshold;
                 if (dead) atomicAnd(&active[p / 64], ~(1ull << (p % 64)));
             }
         }
