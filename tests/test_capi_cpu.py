@@ -160,3 +160,21 @@ def test_native_front_end_refuses_what_the_operators_refuse():
         for bad in (x, x.numpy(), None):
             with pytest.raises(TypeError, match="GPU"):
                 call(bad)
+
+
+@pytest.mark.parametrize("transform", ["vmap", "jvp", "vjp"])
+def test_a_tensor_without_storage_is_an_exception(transform):
+    """Inside torch.vmap, jvp and vjp an operator sees a wrapper without storage.  Its pointer is asked for, and the error
+    raised, while the interpreter's lock is held and before the stream is (a GPU is not needed to get there)."""
+    torch = pytest.importorskip("torch")
+    from torch._subclasses import FakeTensorMode
+    from vkop_amd import ops
+    with FakeTensorMode():
+        t = torch.empty(2, 5, device="cuda")
+    out = torch.empty(2, 5)
+    run = {"vmap": lambda f: torch.vmap(f)(t), "jvp": lambda f: torch.func.jvp(f, (t,), (t,)), "vjp": lambda f: torch.func.vjp(f, t)}[transform]
+    for op in (lambda x: ops.softmax(x), lambda x: ops.softmax(x, out=out), lambda x: ops.topk(x, 2), lambda x: ops.softmax_topk(x, 2),
+               lambda x: ops.softmax_topk(x, 2, return_probs=True), lambda x: ops.softmax_topk_sampling(x, 2, 1.0, 0.9),
+               lambda x: ops.softmax_reduce_max(x, 0), lambda x: ops.reduce_max(x, 0)):
+        with pytest.raises(RuntimeError, match="storage"):
+            run(op)

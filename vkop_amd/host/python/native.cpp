@@ -42,6 +42,7 @@ struct PythonError {};
 // The tensor, its shape and element type as the C ABI takes them.
 struct Input {
     at::Tensor x;
+    const void *data = nullptr;
     int dtype = 0, ndim = 0, shape[4] = {0, 0, 0, 0};
     explicit Input(PyObject *o) {
         if (!THPVariable_Check(o) || !THPVariable_Unpack(o).is_cuda())
@@ -61,6 +62,7 @@ struct Input {
         x = t.is_contiguous() ? t : t.contiguous();
         ndim = static_cast<int>(x.dim());
         for (int d = 0; d < ndim; d++) shape[d] = static_cast<int>(x.size(d));
+        data = x.data_ptr();
     }
     // position of `axis` in the shape, negative ones from its end
     int place(long axis) const {
@@ -123,11 +125,22 @@ struct Scratch {
 
 void *stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
-// A C ABI call without the interpreter's lock (a launch may wait for room in the queue).
-template <typename F> void call(F &&f) {
-    int rc = 0;
-    Py_BEGIN_ALLOW_THREADS rc = f();
-    Py_END_ALLOW_THREADS if (rc == VKOP_HIP_OK) return;
+// The interpreter's lock is let go while this lives.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    Unlocked() = default;
+    Unlocked(const Unlocked &) = delete;
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// A C ABI call without the interpreter's lock (a launch may wait for room in the queue).  Its arguments are plain
+// values taken before: a tensor without storage (inside torch.vmap, jvp, grad) throws where its pointer is asked for.
+template <typename Function, typename... Args> void call(Function function, Args... args) {
+    const int rc = [&] {
+        const Unlocked unlocked;
+        return function(args...);
+    }();
+    if (rc == VKOP_HIP_OK) return;
     PyObject *e = PyObject_CallFunction(error_class, "is", rc, fn.last_error());
     if (e != nullptr) {
         PyErr_SetObject(error_class, e);
@@ -181,10 +194,8 @@ PyObject *softmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
         }
         const Scratch ws(a[5], fn.softmax_workspace_bytes(in.dtype, in.shape, in.ndim, static_cast<int>(axis)));
         void *st = stream();
-        call([&] {
-            return fn.softmax(in.x.data_ptr(), result, in.dtype, in.shape, in.ndim, static_cast<int>(axis), nan_where ? 1 : 0,
-                              nan_value, ws.ptr, ws.size, st);
-        });
+        call(fn.softmax, in.data, result, in.dtype, in.shape, in.ndim, static_cast<int>(axis), nan_where ? 1 : 0, nan_value, ws.ptr,
+             ws.size, st);
         if (a[4] == Py_None) return THPVariable_Wrap(out);
         Py_INCREF(a[4]);
         return a[4];
@@ -195,11 +206,15 @@ PyObject *softmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
 struct Selection {
     at::DimVector sizes;
     at::Tensor values, indices;
+    void *value_data = nullptr;
+    int32_t *index_data = nullptr;
     Selection(const Input &in, long axis, long k) : sizes(in.x.sizes().begin(), in.x.sizes().end()) {
         sizes[static_cast<size_t>(in.place(axis))] = k;
         if (k < 0) raise(PyExc_RuntimeError, "k = %ld must be at least 1", k);
         values = in.empty(sizes, in.x.scalar_type());
         indices = in.empty(sizes, at::kInt);
+        value_data = values.data_ptr();
+        index_data = static_cast<int32_t *>(indices.data_ptr());
     }
 };
 
@@ -213,10 +228,8 @@ PyObject *topk(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const int ik = static_cast<int>(k), ia = static_cast<int>(axis);
         const Scratch ws(a[5], fn.topk_workspace_bytes(in.dtype, in.shape, in.ndim, ia, ik));
         void *st = stream();
-        call([&] {
-            return fn.topk(in.x.data_ptr(), s.values.data_ptr(), static_cast<int32_t *>(s.indices.data_ptr()), in.dtype, in.shape,
-                           in.ndim, ia, ik, largest ? 1 : 0, sorted ? 1 : 0, ws.ptr, ws.size, st);
-        });
+        call(fn.topk, in.data, s.value_data, s.index_data, in.dtype, in.shape, in.ndim, ia, ik, largest ? 1 : 0, sorted ? 1 : 0,
+             ws.ptr, ws.size, st);
         return tuple_of({s.values, s.indices});
     });
 }
@@ -229,15 +242,16 @@ PyObject *softmax_topk(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const bool largest = as_bool(a[3]), return_probs = as_bool(a[4]);
         const Selection s(in, axis, k);
         at::Tensor probs;
-        if (return_probs) probs = in.empty(in.x.sizes(), in.x.scalar_type());
+        void *prob_data = nullptr;
+        if (return_probs) {
+            probs = in.empty(in.x.sizes(), in.x.scalar_type());
+            prob_data = probs.data_ptr();
+        }
         const int ik = static_cast<int>(k), ia = static_cast<int>(axis);
         const Scratch ws(a[5], fn.softmax_topk_workspace_bytes(in.dtype, in.shape, in.ndim, ia, ik));
         void *st = stream();
-        call([&] {
-            return fn.softmax_topk(in.x.data_ptr(), return_probs ? probs.data_ptr() : nullptr, s.values.data_ptr(),
-                                   static_cast<int32_t *>(s.indices.data_ptr()), in.dtype, in.shape, in.ndim, ia, ik,
-                                   largest ? 1 : 0, ws.ptr, ws.size, st);
-        });
+        call(fn.softmax_topk, in.data, prob_data, s.value_data, s.index_data, in.dtype, in.shape, in.ndim, ia, ik, largest ? 1 : 0,
+             ws.ptr, ws.size, st);
         return return_probs ? tuple_of({s.values, s.indices, probs}) : tuple_of({s.values, s.indices});
     });
 }
@@ -261,15 +275,16 @@ PyObject *softmax_topk_sampling(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const float top_p = counted ? static_cast<float>(as_double(a[3])) : 0.f;
         const Selection s(in, axis, k);
         at::Tensor counts;
-        if (counted) counts = in.empty(without(in, axis), at::kInt);
+        int32_t *count_data = nullptr;
+        if (counted) {
+            counts = in.empty(without(in, axis), at::kInt);
+            count_data = static_cast<int32_t *>(counts.data_ptr());
+        }
         const int ik = static_cast<int>(k), ia = static_cast<int>(axis);
         const Scratch ws(a[5], fn.softmax_topk_workspace_bytes(in.dtype, in.shape, in.ndim, ia, ik));
         void *st = stream();
-        call([&] {
-            return fn.softmax_topk_sampling(in.x.data_ptr(), s.values.data_ptr(), static_cast<int32_t *>(s.indices.data_ptr()),
-                                            counted ? static_cast<int32_t *>(counts.data_ptr()) : nullptr, in.dtype, in.shape,
-                                            in.ndim, ia, ik, scale, top_p, ws.ptr, ws.size, st);
-        });
+        call(fn.softmax_topk_sampling, in.data, s.value_data, s.index_data, count_data, in.dtype, in.shape, in.ndim, ia, ik, scale,
+             top_p, ws.ptr, ws.size, st);
         return counted ? tuple_of({s.values, s.indices, counts}) : tuple_of({s.values, s.indices});
     });
 }
@@ -281,11 +296,10 @@ PyObject *softmax_reduce_max(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const long axis = as_long(a[1]);
         const int ia = static_cast<int>(axis);
         at::Tensor out = in.empty(without(in, axis), in.x.scalar_type());
+        void *result = out.data_ptr();
         const Scratch ws(a[2], fn.softmax_reduce_max_workspace_bytes(in.dtype, in.shape, in.ndim, ia));
         void *st = stream();
-        call([&] {
-            return fn.softmax_reduce_max(in.x.data_ptr(), out.data_ptr(), in.dtype, in.shape, in.ndim, ia, ws.ptr, ws.size, st);
-        });
+        call(fn.softmax_reduce_max, in.data, result, in.dtype, in.shape, in.ndim, ia, ws.ptr, ws.size, st);
         return THPVariable_Wrap(out);
     });
 }
@@ -296,8 +310,9 @@ PyObject *reduce_max(PyObject *, PyObject *const *a, Py_ssize_t n) {
         const Input in(a[0]);
         const long axis = as_long(a[1]);
         at::Tensor out = in.empty(without(in, axis), in.x.scalar_type());
+        void *result = out.data_ptr();
         void *st = stream();
-        call([&] { return fn.reduce_max(in.x.data_ptr(), out.data_ptr(), in.dtype, in.shape, in.ndim, static_cast<int>(axis), st); });
+        call(fn.reduce_max, in.data, result, in.dtype, in.shape, in.ndim, static_cast<int>(axis), st);
         return THPVariable_Wrap(out);
     });
 }
