@@ -178,3 +178,22 @@ def test_a_tensor_without_storage_is_an_exception(transform):
                lambda x: ops.softmax_reduce_max(x, 0), lambda x: ops.reduce_max(x, 0)):
         with pytest.raises(RuntimeError, match="storage"):
             run(op)
+
+
+def test_native_front_end_takes_whole_numbers_only():
+    """k and axis are whole numbers (Python's, numpy's, one-element integer tensors): anything else is a TypeError, as ctypes
+    has it, and not rounded or parsed."""
+    torch = pytest.importorskip("torch")
+    import numpy as np
+    from torch._subclasses import FakeTensorMode
+    from vkop_amd import ops
+    with FakeTensorMode():
+        t = torch.empty(2, 5, device="cuda")
+    for bad in (2.5, "1", np.float64(1), None, torch.tensor(1.5)):
+        for call in (lambda: ops.softmax(t, bad), lambda: ops.topk(t, bad), lambda: ops.topk(t, 2, axis=bad), lambda: ops.softmax_topk(t, bad),
+                     lambda: ops.softmax_topk_sampling(t, bad), lambda: ops.softmax_reduce_max(t, bad), lambda: ops.reduce_max(t, bad)):
+            with pytest.raises(TypeError):
+                call()
+    for k in (2, np.int64(2), torch.tensor(2)):  # taken, the axis outside the tensor refused
+        with pytest.raises(IndexError):
+            ops.topk(t, k, axis=np.int32(7))

@@ -76,7 +76,7 @@ struct Input {
 };
 
 long as_long(PyObject *o) {
-    PyObject *i = PyNumber_Long(o);  // (as int() does: numbers of numpy and one-element tensors too)
+    PyObject *i = PyNumber_Index(o);  // (whole numbers, those of numpy and one-element tensors too; 2.5 or "2" is a TypeError)
     if (i == nullptr) throw PythonError{};
     const long v = PyLong_AsLong(i);
     Py_DECREF(i);
