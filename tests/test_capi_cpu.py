@@ -197,3 +197,42 @@ def test_native_front_end_takes_whole_numbers_only():
     for k in (2, np.int64(2), torch.tensor(2)):  # taken, the axis outside the tensor refused
         with pytest.raises(IndexError):
             ops.topk(t, k, axis=np.int32(7))
+
+
+def test_native_front_end_takes_any_object_with_get_as_workspace():
+    """A workspace is what its get(nbytes) returns: an object with nothing else, and a class derived from ops.Workspace with a
+    get() of its own.  (The rest of the call needs a GPU; get() is called before.)"""
+    torch = pytest.importorskip("torch")
+    from torch._subclasses import FakeTensorMode
+    from vkop_amd import capi, ops
+    with FakeTensorMode():
+        t = torch.empty(2, 100000, device="cuda")
+    out = torch.empty(2, 100000)
+    need = capi.softmax_workspace_bytes(capi.F32, (2, 100000), -1)
+    assert need > 0
+
+    class Asked(Exception):
+        pass
+
+    class Plain:
+        def get(self, nbytes):
+            raise Asked(nbytes)
+
+    class Derived(ops.Workspace):
+        def get(self, nbytes):
+            raise Asked(nbytes)
+
+    for ws in (Plain(), Derived()):
+        with pytest.raises(Asked, match=str(need)):
+            ops.softmax(t, out=out, workspace=ws)
+
+    class Wrong:
+        def __init__(self, answer):
+            self.answer = answer
+
+        def get(self, nbytes):
+            return self.answer
+
+    for answer in ((1, 2, 3), ("x", 1), (1.5, 1), 7):
+        with pytest.raises((TypeError, ValueError)):
+            ops.softmax(t, out=out, workspace=Wrong(answer))

@@ -27,6 +27,7 @@ struct Functions {
 #undef VKOP_NATIVE_MEMBER
 } fn;
 PyObject *error_class = nullptr;                             // vkop_amd.capi.VkopHipError(code, message)
+PyObject *workspace_class = nullptr;                         // vkop_amd.ops.Workspace
 PyObject *name_ptr = nullptr, *name_size = nullptr, *name_get = nullptr;
 
 // A failed Python call inside a function: unwinds to guarded(), which lets the exception set stand.
@@ -96,29 +97,47 @@ bool as_bool(PyObject *o) {
     return v != 0;
 }
 
-// What ops.Workspace holds, grown by its own get() when it is too small.
+// Scratch memory of at least `need` bytes.  ops.Workspace: its two attributes say what it holds, and its get() is called
+// only where that is too little.  Any other object, a class derived from it among them: whatever its get(need) returns.
 struct Scratch {
     void *ptr = nullptr;
     size_t size = 0;
     Scratch(PyObject *workspace, size_t need) {
-        if (need == 0) return;
-        size = number(workspace, name_size);
-        if (size < need) {
-            PyObject *want = PyLong_FromSize_t(need);
-            PyObject *r = want == nullptr ? nullptr : PyObject_CallMethodObjArgs(workspace, name_get, want, nullptr);
-            Py_XDECREF(want);
-            if (r == nullptr) throw PythonError{};
-            Py_DECREF(r);
-            size = number(workspace, name_size);
+        if (reinterpret_cast<PyObject *>(Py_TYPE(workspace)) == workspace_class) {
+            if (need == 0) return;
+            size = attribute(workspace, name_size);
+            if (size >= need) {
+                ptr = reinterpret_cast<void *>(attribute(workspace, name_ptr));
+                return;
+            }
         }
-        ptr = reinterpret_cast<void *>(number(workspace, name_ptr));
+        PyObject *want = PyLong_FromSize_t(need);
+        PyObject *r = want == nullptr ? nullptr : PyObject_CallMethodObjArgs(workspace, name_get, want, nullptr);
+        Py_XDECREF(want);
+        PyObject *pair = r == nullptr ? nullptr : PySequence_Tuple(r);
+        Py_XDECREF(r);
+        if (pair == nullptr) throw PythonError{};
+        const bool two = PyTuple_GET_SIZE(pair) == 2;
+        if (two) {
+            ptr = reinterpret_cast<void *>(number(PyTuple_GET_ITEM(pair, 0)));
+            size = PyErr_Occurred() ? 0 : number(PyTuple_GET_ITEM(pair, 1));
+        }
+        Py_DECREF(pair);
+        if (!two) raise(PyExc_ValueError, "workspace.get(nbytes): an address and a size expected");
+        if (PyErr_Occurred()) throw PythonError{};
     }
-    static size_t number(PyObject *o, PyObject *name) {
+    static size_t number(PyObject *v) {  // (an error is left set)
+        PyObject *i = v == Py_None ? PyLong_FromLong(0) : PyNumber_Index(v);  // (None: the null pointer, as ctypes has it)
+        const size_t n = i == nullptr ? 0 : PyLong_AsSize_t(i);
+        Py_XDECREF(i);
+        return n;
+    }
+    static size_t attribute(PyObject *o, PyObject *name) {
         PyObject *v = PyObject_GetAttr(o, name);
         if (v == nullptr) throw PythonError{};
-        const size_t n = PyLong_AsSize_t(v);
+        const size_t n = number(v);
         Py_DECREF(v);
-        if (n == static_cast<size_t>(-1) && PyErr_Occurred()) throw PythonError{};
+        if (PyErr_Occurred()) throw PythonError{};
         return n;
     }
 };
@@ -317,9 +336,9 @@ PyObject *reduce_max(PyObject *, PyObject *const *a, Py_ssize_t n) {
     });
 }
 
-// bind({name without vkop_hip_: address}, VkopHipError)
+// bind({name without vkop_hip_: address}, VkopHipError, Workspace)
 PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
-    if (n != 2 || !PyDict_Check(a[0])) return PyErr_Format(PyExc_TypeError, "bind(addresses, error class)");
+    if (n != 3 || !PyDict_Check(a[0])) return PyErr_Format(PyExc_TypeError, "bind(addresses, error class, workspace class)");
     Functions f;
     auto address = [&](const char *name) -> void * {
         PyObject *v = PyDict_GetItemString(a[0], name);  // (borrowed)
@@ -333,6 +352,9 @@ PyObject *bind(PyObject *, PyObject *const *a, Py_ssize_t n) {
     Py_INCREF(a[1]);
     Py_XDECREF(error_class);
     error_class = a[1];
+    Py_INCREF(a[2]);
+    Py_XDECREF(workspace_class);
+    workspace_class = a[2];
     fn = f;
     Py_RETURN_NONE;
 }

@@ -29,7 +29,7 @@ def _load():
         raise FileNotFoundError("vkop_amd/_native.so is not built (%s); run `python -c 'import __graft_entry__ as g; g.build()'` "
                                 "or `make -C vkop_amd/host`" % e) from e
     names = [n for n in L._signatures if not n.endswith(("tune", "measure_stages", "measure_path"))]
-    module.bind({n[len("vkop_hip_"):]: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in names}, capi.VkopHipError)
+    module.bind({n[len("vkop_hip_"):]: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in names}, capi.VkopHipError, Workspace)
     _native = module
     return module
 
