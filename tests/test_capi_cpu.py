@@ -236,3 +236,12 @@ def test_native_front_end_takes_any_object_with_get_as_workspace():
     for answer in ((1, 2, 3), ("x", 1), (1.5, 1), 7):
         with pytest.raises((TypeError, ValueError)):
             ops.softmax(t, out=out, workspace=Wrong(answer))
+
+
+def test_native_front_end_knows_what_it_was_built_for(monkeypatch):
+    torch = pytest.importorskip("torch")
+    from vkop_amd import ops
+    monkeypatch.setattr(ops, "_native", None)
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    with pytest.raises(ImportError, match="built for torch"):
+        ops.softmax(torch.zeros(2, 5))

@@ -9,10 +9,14 @@
 // functions: bind() takes them from the library that vkop_amd.capi has loaded.
 #include <Python.h>
 
+#include <cstdarg>
+#include <cstring>
+
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "vkop_hip.h"
 
@@ -367,10 +371,21 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", "Native front end of vko
 
 }  // namespace
 
+#define VKOP_NATIVE_TEXT2(x) #x
+#define VKOP_NATIVE_TEXT(x) VKOP_NATIVE_TEXT2(x)
 PyMODINIT_FUNC PyInit__native() {
+    // (the file's name does not say which interpreter it was built for)
+    constexpr char built_for[] = VKOP_NATIVE_TEXT(PY_MAJOR_VERSION) "." VKOP_NATIVE_TEXT(PY_MINOR_VERSION) ".";
+    if (std::strncmp(Py_GetVersion(), built_for, sizeof built_for - 1) != 0)
+        return PyErr_Format(PyExc_ImportError, "built for Python %sx, this is %s", built_for, Py_GetVersion());
     name_ptr = PyUnicode_InternFromString("ptr");
     name_size = PyUnicode_InternFromString("size");
     name_get = PyUnicode_InternFromString("get");
     if (name_ptr == nullptr || name_size == nullptr || name_get == nullptr) return nullptr;
-    return PyModule_Create(&module);
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

@@ -28,6 +28,9 @@ def _load():
     except ImportError as e:
         raise FileNotFoundError("vkop_amd/_native.so is not built (%s); run `python -c 'import __graft_entry__ as g; g.build()'` "
                                 "or `make -C vkop_amd/host`" % e) from e
+    if torch.__version__.split("+")[0] != module.torch_version:
+        raise ImportError("vkop_amd/_native.so was built for torch %s, this is %s: build it again (`make -C vkop_amd/host -B`)"
+                          % (module.torch_version, torch.__version__))
     names = [n for n in L._signatures if not n.endswith(("tune", "measure_stages", "measure_path"))]
     module.bind({n[len("vkop_hip_"):]: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in names}, capi.VkopHipError, Workspace)
     _native = module
