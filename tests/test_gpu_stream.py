@@ -576,3 +576,28 @@ def test_smallest_first_on_reversed_elements(ops, n, k, dtype):
             assert np.array_equal(host(ix[r]), eix[r]), r
         bits = np.uint16 if dtype == np.float16 else np.uint32
         assert np.array_equal(host(v).view(bits), ev.view(bits))
+
+
+@pytest.mark.parametrize("n,k", [(1000, 5), (4096, 64), (8400, 300), (8401, 300), (32000, 40), (50257, 200), (100000, 600), (131076, 1025)])
+def test_signalling_nan_ranks_as_nan(ops, n, k):
+    """A NaN is a NaN whether it is quiet or signalling: last among the smallest, first among the largest, of either sign,
+    alone, among +inf, and where NaN fills the last places; values are copies of the input's bits."""
+    rng = np.random.default_rng(n + k)
+    x = rng.standard_normal((20, n)).astype(np.float32)
+    bits = x.view(np.uint32)
+    kinds = np.array([0x7F800001, 0xFF800001, 0x7FBFFFFF, 0xFFBFFFFF, 0x7FC00000], np.uint32)
+    bits[0, n // 2] = kinds[0]
+    bits[1, 0], bits[1, n - 1] = kinds[0], kinds[1]
+    at = rng.random(n) < 0.3
+    bits[2, at] = rng.choice(kinds, at.sum())
+    few = rng.choice(n, k // 2, replace=False)
+    bits[3, :], x[3, few] = kinds[1], -1.5
+    bits[4, :] = rng.choice(kinds, n)
+    x[5, :], bits[5, 0::2], x[5, few] = np.inf, kinds[0], 2.0
+    for largest in (False, True):
+        for rows in (x[:12], x):
+            v, ix = ops.topk(dev(rows), k, largest=largest)
+            ev, eix = oracle.topk(rows, k, -1, largest)
+            for r in range(rows.shape[0]):
+                assert np.array_equal(host(ix[r]), eix[r]), (largest, r)
+            assert np.array_equal(host(v).view(np.uint32), ev.view(np.uint32)), largest

@@ -77,8 +77,10 @@ template <typename T> __device__ __forceinline__ void store16_stream(T *p, const
     __builtin_nontemporal_store(v, reinterpret_cast<vec16_any *>(p));
 }
 
-// Larger of three floats, NaN dropped (fmaxf on loaded values costs one more instruction an operand:
-// the compiler first turns every value that may be a signalling NaN into a quiet one).
+// Larger of three floats, quiet NaN dropped (fmaxf on loaded values costs one more instruction an operand:
+// the compiler first turns every value that may be a signalling NaN into a quiet one).  A signalling NaN
+// may come out as a quiet one: for callers whose result is NaN wherever an operand was -- a softmax's
+// maximum, the smallest value of a chunk whose sum is NaN either way.
 __device__ __forceinline__ float max3(float a, float b, float c) {
     float r;
     asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
@@ -89,7 +91,7 @@ __device__ __forceinline__ float min3(float a, float b, float c) {
     asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
-// Larger halves of two pairs, NaN dropped.
+// Larger halves of two pairs, quiet NaN dropped (signalling: as above).
 __device__ __forceinline__ uint32_t max_half2(uint32_t a, uint32_t b) {
     uint32_t r;
     asm("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));

@@ -585,16 +585,20 @@ template <> struct Vec128<uint16_t> {
     }
 };
 
-// (a reversed element: its negative, NaN as -inf)
-__device__ __forceinline__ float negated_or_neg_inf(float x) {
+// (a reversed element: its negative, NaN as -inf.  In IEEE mode v_max_f32 drops a quiet NaN but turns a signalling one into
+// a quiet one and keeps it: where there may be one -- a float, not what a half was converted to -- a first instruction makes it
+// quiet.  In assembly because the compiler may treat a signalling NaN as a quiet one: it folds fmaxf(m, fmaxf(-x, -inf)) into
+// one v_max3_f32, which loses m at a signalling x)
+template <bool QUIET> __device__ __forceinline__ float negated_or_neg_inf(float x) {
     float r;
-    asm("v_max_f32_e64 %0, -%1, %2" : "=v"(r) : "v"(x), "s"(-INFINITY));
+    if constexpr (QUIET) asm("v_max_f32_e64 %0, -%1, %2" : "=v"(r) : "v"(x), "s"(-INFINITY));
+    else asm("v_max_f32_e64 %0, -%1, -%1\n\tv_max_f32_e64 %0, %0, %2" : "=v"(r) : "v"(x), "s"(-INFINITY));
     return r;
 }
 template <typename B> struct Vec128<Reversed<B>> : Vec128<B> {
     __device__ __forceinline__ void load(const Reversed<B> *p) { Vec128<B>::load(&p->bits); }
     __device__ __forceinline__ void load_any(const Reversed<B> *p) { Vec128<B>::load_any(&p->bits); }
-    __device__ __forceinline__ float get(int c) const { return negated_or_neg_inf(Vec128<B>::get(c)); }
+    __device__ __forceinline__ float get(int c) const { return negated_or_neg_inf<sizeof(B) == 2>(Vec128<B>::get(c)); }
     __device__ __forceinline__ void set(int c, float f) { Vec128<B>::set(c, -f); }
 };
 
