@@ -1209,3 +1209,22 @@ def test_model_files_drive_the_operators(ops, dtype):
     got = runtime.run_model(tail, {"boxes": dev(boxes), "scores": dev(scores)})["selected"]
     want = oracle.nms(boxes.astype(np.float32), scores.astype(np.float32), 0.5, 0.25, 0, max_candidates=2048)
     assert np.array_equal(host(got), want) and len(want) > 0
+
+
+def test_softmax_more_threads_than_one_launch(ops):
+    """Rows x threads beyond 2^32: launched in slices of rows.  103 GB of halves in place."""
+    rows, n = (1 << 25) + 4096, 1537  # 128 threads a row
+    if torch.cuda.mem_get_info()[0] < 130 << 30:
+        pytest.skip("needs 130 GiB of GPU memory")
+    rng = np.random.default_rng(1)
+    pattern = dev(rng.standard_normal((4096, n)).astype(np.float16))
+    x = torch.empty((rows // 4096, 4096, n), dtype=torch.float16, device="cuda")
+    x[:] = pattern
+    want = ops.softmax(pattern)
+    x = x.view(rows, n)
+    ops.softmax(x, out=x)
+    last = rows // 4096 - 1
+    for i in (0, last // 2, last - 1, last):  # (the second slice begins in the last but one)
+        assert torch.equal(x[i * 4096:(i + 1) * 4096], want), i
+    del x
+    torch.cuda.empty_cache()

@@ -156,6 +156,16 @@ struct RowShape {
     int nt, v;
 };
 
+// HIP takes no grid of 2^32 threads or more: launch(first, count) for as many of `units` -- rows, or blocks of them -- at a
+// time as stay below that, the last workgroup's idle threads among them (all units in every case but tensors of tens of gigabytes).
+template <typename F> int in_slices(uint64_t units, uint64_t threads_per_unit, F &&launch) {
+    constexpr uint64_t kGridThreads = 0xFFFFFFFFull - 1024;
+    const uint64_t most = std::max<uint64_t>(1, kGridThreads / threads_per_unit);
+    for (uint64_t first = 0; first < units; first += most)
+        if (const int rc = launch(first, static_cast<uint32_t>(std::min(most, units - first)))) return rc;
+    return VKOP_HIP_OK;
+}
+
 struct SoftmaxPlan {
     enum Kind { kGeneralLines, kGeneralStrided, kThread, kGroup, kRow, kChunked, kLinesRegs, kStridedRegs, kStridedTile } kind = kGeneralLines;
     RowShape shape{0, 0};  // kChunked; kGroup: lanes a row and vectors a lane; kRow: threads and vectors a thread
@@ -186,6 +196,11 @@ void launch_strided_reg(const T *in, T *out, const View &v, int nan_where, float
     VKOP_STRIDED_CASE(96, 4)
     VKOP_STRIDED_CASE(128, 4)
 #undef VKOP_STRIDED_CASE
+}
+
+// Threads that the register kernel for lines takes for one outer index.
+uint64_t lines_threads(const View &v, uint32_t vec, uint32_t P, uint32_t W) {
+    return static_cast<uint64_t>((v.g.inner + vec - 1) / vec) * P * W;
 }
 
 // The register kernel for lines along a non-last axis (kernels_lines.hpp) and its shape: lane groups of a
@@ -225,6 +240,7 @@ bool plan_lines(const View &v, uint32_t vec, SoftmaxPlan *p) {
         else W *= 2;
         K = (n + P * W - 1) / (P * W);
     }
+    if (lines_threads(v, vec, P, W) > 0xFFFFFFFFull - 1024) return false;  // (an outer index of 2^31 lines)
     p->kind = SoftmaxPlan::kLinesRegs;
     p->lines_k = K, p->lines_p = P, p->lines_w = W;
     return true;
@@ -304,6 +320,19 @@ SoftmaxPlan plan_softmax(const View &v, int dtype) {
 }
 
 template <typename T>
+int launch_lines(const T *in, T *out, const View &v, const SoftmaxPlan &p, bool max_only, int nan_where, float nan_value,
+                 hipStream_t st) {
+    return in_slices(v.g.outer, lines_threads(v, 16 / sizeof(T), p.lines_p, p.lines_w), [&](uint64_t first, uint32_t outer) {
+        vkop::LinesLaunch a{in + first * v.g.n * v.g.inner, out + first * (max_only ? 1u : v.g.n) * v.g.inner, v.g, p.lines_k, p.lines_p,
+                            p.lines_w, max_only, nan_where, nan_value, st};
+        a.g.outer = outer;
+        if (!vkop::launch_softmax_lines<T>(a))
+            return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
+        return launched("softmax_lines_reg_kernel");
+    });
+}
+
+template <typename T>
 int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, float nan_value, void *ws,
                  size_t ws_bytes, hipStream_t st) {
     const SoftmaxPlan p = plan_softmax(v, dtype);
@@ -316,45 +345,42 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
     }
     case SoftmaxPlan::kGroup: {
         const uint32_t per_block = static_cast<uint32_t>(vkop::kSoftmaxGroupThreads / p.shape.nt);
-        const uint32_t blocks = (lines + per_block - 1) / per_block;
-#define VKOP_GROUP(G, V)                                                                                                     \
-    if (p.shape.nt == G && p.shape.v == V) {                                                                                 \
-        vkop::softmax_group_kernel<T, G, V><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value); \
-        return launched("softmax_group_kernel");                                                                             \
+        return in_slices((lines + per_block - 1) / per_block, vkop::kSoftmaxGroupThreads, [&](uint64_t first, uint32_t blocks) {
+            const uint64_t row0 = first * per_block;
+            const T *from = in + row0 * v.g.n;
+            T *to = out + row0 * v.g.n;
+            const uint32_t rows = static_cast<uint32_t>(std::min<uint64_t>(lines - row0, static_cast<uint64_t>(blocks) * per_block));
+#define VKOP_GROUP(G, V)                                                                                                       \
+    if (p.shape.nt == G && p.shape.v == V) {                                                                                   \
+        vkop::softmax_group_kernel<T, G, V><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(from, to, rows, v.g.n, nan_where, nan_value); \
+        return launched("softmax_group_kernel");                                                                               \
     }
 #define VKOP_GROUPS(G) VKOP_GROUP(G, 1) VKOP_GROUP(G, 2) VKOP_GROUP(G, 3) if constexpr (sizeof(T) == 4) { VKOP_GROUP(G, 4) }
-        VKOP_GROUPS(8) VKOP_GROUPS(16) VKOP_GROUPS(32) VKOP_GROUPS(64)
+            VKOP_GROUPS(8) VKOP_GROUPS(16) VKOP_GROUPS(32) VKOP_GROUPS(64)
 #undef VKOP_GROUPS
 #undef VKOP_GROUP
-        return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_group_kernel for %d lanes x %d", p.shape.nt, p.shape.v);
+            return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_group_kernel for %d lanes x %d", p.shape.nt, p.shape.v);
+        });
     }
     case SoftmaxPlan::kRow: {
-#define VKOP_ROW(V)                                                                                                  \
-    if (p.shape.v == V) {                                                                                            \
-        vkop::softmax_row_kernel<T, V><<<lines, p.shape.nt, 0, st>>>(in, out, v.g.n, nan_where, nan_value);          \
-        return launched("softmax_row_kernel");                                                                       \
+        return in_slices(lines, p.shape.nt, [&](uint64_t row0, uint32_t rows) {
+            const T *from = in + row0 * v.g.n;
+            T *to = out + row0 * v.g.n;
+#define VKOP_ROW(V)                                                                                     \
+    if (p.shape.v == V) {                                                                               \
+        vkop::softmax_row_kernel<T, V><<<rows, p.shape.nt, 0, st>>>(from, to, v.g.n, nan_where, nan_value); \
+        return launched("softmax_row_kernel");                                                          \
     }
-        VKOP_ROW(1) VKOP_ROW(2) VKOP_ROW(3) VKOP_ROW(4)
-        if constexpr (sizeof(T) == 4) { VKOP_ROW(5) VKOP_ROW(6) VKOP_ROW(7) VKOP_ROW(8) }
+            VKOP_ROW(1) VKOP_ROW(2) VKOP_ROW(3) VKOP_ROW(4)
+            if constexpr (sizeof(T) == 4) { VKOP_ROW(5) VKOP_ROW(6) VKOP_ROW(7) VKOP_ROW(8) }
 #undef VKOP_ROW
-        return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_row_kernel for %d x %d", p.shape.nt, p.shape.v);
+            return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_row_kernel for %d x %d", p.shape.nt, p.shape.v);
+        });
     }
     case SoftmaxPlan::kChunked: {
         if (ws == nullptr || ws_bytes < p.workspace)
             return fail(VKOP_HIP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", ws_bytes, p.workspace);
         auto *stats = reinterpret_cast<vkop::ChunkStat *>(static_cast<unsigned char *>(ws) + kTicketBytes);
-        const uint32_t blocks = v.g.outer * p.g;
-        bool done = false;
-#define VKOP_STATS(NT, V)                                                                              \
-    if (!done && p.shape.nt == NT && p.shape.v == V) {                                                 \
-        vkop::softmax_stats_kernel<T, NT, V><<<blocks, NT, 0, st>>>(in, stats, v.g.n, p.g);            \
-        done = true;                                                                                   \
-    }
-        VKOP_STATS(256, 1) VKOP_STATS(256, 2) VKOP_STATS(256, 4)
-        if constexpr (sizeof(T) == 4) { VKOP_STATS(256, 8) VKOP_STATS(1024, 8) }
-        else { VKOP_STATS(1024, 4) }
-#undef VKOP_STATS
-        if (!done) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_stats_kernel for %d x %d", p.shape.nt, p.shape.v);
         // the most vectors a thread (four floats', two halves') that leave 2048 workgroups: with fewer in all
         // their stores wait for each other, with smaller ones more of them combine the same chunks
         const uint32_t vec = 16 / sizeof(T);
@@ -362,19 +388,33 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
         uint32_t loads = 16 / vec;
         while (loads > 1 && static_cast<uint64_t>(v.g.outer) * pieces(loads) < 2048) loads /= 2;
         const uint32_t gs = pieces(loads);
+        const uint64_t threads = std::max<uint64_t>(static_cast<uint64_t>(p.g) * p.shape.nt, static_cast<uint64_t>(gs) * vkop::kSoftmaxScaleThreads);
+        return in_slices(v.g.outer, threads, [&](uint64_t row0, uint32_t rows) {
+            const T *from = in + row0 * v.g.n;
+            T *to = out + row0 * v.g.n;
+            auto *row_stats = stats + row0 * p.g;
+            bool done = false;
+#define VKOP_STATS(NT, V)                                                                                \
+    if (!done && p.shape.nt == NT && p.shape.v == V) {                                                   \
+        vkop::softmax_stats_kernel<T, NT, V><<<rows * p.g, NT, 0, st>>>(from, row_stats, v.g.n, p.g);    \
+        done = true;                                                                                     \
+    }
+            VKOP_STATS(256, 1) VKOP_STATS(256, 2) VKOP_STATS(256, 4)
+            if constexpr (sizeof(T) == 4) { VKOP_STATS(256, 8) VKOP_STATS(1024, 8) }
+            else { VKOP_STATS(1024, 4) }
+#undef VKOP_STATS
+            if (!done) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_stats_kernel for %d x %d", p.shape.nt, p.shape.v);
 #define VKOP_SCALE(V) \
     if (loads == V)   \
-        vkop::softmax_scale_kernel<T, V><<<v.g.outer * gs, vkop::kSoftmaxScaleThreads, 0, st>>>(in, out, stats, v.g.n, p.g, gs, nan_where, nan_value);
-        VKOP_SCALE(1) VKOP_SCALE(2)
-        if constexpr (sizeof(T) == 4) { VKOP_SCALE(4) }
+        vkop::softmax_scale_kernel<T, V><<<rows * gs, vkop::kSoftmaxScaleThreads, 0, st>>>(from, to, row_stats, v.g.n, p.g, gs, nan_where, nan_value);
+            VKOP_SCALE(1) VKOP_SCALE(2)
+            if constexpr (sizeof(T) == 4) { VKOP_SCALE(4) }
 #undef VKOP_SCALE
-        return launched("softmax_stats_kernel / softmax_scale_kernel");
+            return launched("softmax_stats_kernel / softmax_scale_kernel");
+        });
     }
     case SoftmaxPlan::kLinesRegs: {
-        const vkop::LinesLaunch a{in, out, v.g, p.lines_k, p.lines_p, p.lines_w, false, nan_where, nan_value, st};
-        if (!vkop::launch_softmax_lines<T>(a))
-            return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
-        return launched("softmax_lines_reg_kernel");
+        return launch_lines(in, out, v, p, false, nan_where, nan_value, st);
     }
     case SoftmaxPlan::kStridedRegs: {
         launch_strided_reg<T, false>(in, out, v, nan_where, nan_value, st);
@@ -882,7 +922,8 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
     // kernels or one workgroup a row (with rows.path = 1, which switches the former off: the radix select): two
     // launches or one for the select's seven, one read of the row for five.  [64,32000] f32 k = 40 41 -> 8.8 us,
     // [64,128256] k = 50 61 -> 12.9, [8,262144] k = 1024 46.8 -> 21.2, [1024,4096] k = 64 29.7 -> 10.2.
-    const bool routed = largest || g_rows_path.load() != 1;
+    // (2^22 rows and more: a grid of a thousand threads a row is more than HIP takes, the select's is not.)
+    const bool routed = largest || (g_rows_path.load() != 1 && v.g.outer < (1u << 22));
     ScanCfg sc = routed ? choose_scan_cfg(v, k, dtype) : ScanCfg{};
     // (without an order, the rows of the large-k kernels keep the select and the listing it has always given)
     if (!largest && !sorted && sc.g2 != 0) sc = ScanCfg{};
@@ -979,10 +1020,7 @@ int softmax_reduce_max_impl(const T *in, T *out, const View &v, void *ws, size_t
     const uint32_t lines = v.g.outer * v.g.inner;
     const SoftmaxPlan p = plan_softmax(v, sizeof(T) == 4 ? VKOP_HIP_F32 : VKOP_HIP_F16);
     if (p.kind == SoftmaxPlan::kLinesRegs) {
-        const vkop::LinesLaunch a{in, out, v.g, p.lines_k, p.lines_p, p.lines_w, true, 0, 0.f, st};
-        if (!vkop::launch_softmax_lines<T>(a))
-            return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
-        return launched("softmax_lines_reg_kernel (max)");
+        return launch_lines(in, out, v, p, true, 0, 0.f, st);
     }
     if (v.g.n <= static_cast<uint32_t>(vkop::kStridedMaxN)) {
         launch_strided_reg<T, true>(in, out, v, 0, 0.f, st);
