@@ -1228,3 +1228,19 @@ def test_softmax_more_threads_than_one_launch(ops):
         assert torch.equal(x[i * 4096:(i + 1) * 4096], want), i
     del x
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("rows,n", [(2000, 200), (300, 4000), (40, 100000)])
+def test_softmax_subnormal_terms_are_rounded_once(ops, rows, n):
+    """Exponentials below 2^-126: the double polynomial is scaled before it is rounded to the subnormal grid.  One element
+    of 0 makes the sum 1 to the last bit, so the probabilities are the terms; float(exp(d)) in 64 bits is what they round
+    to but for arguments within 2^-36 of a rounding midpoint, fewer than one in 2^20 here."""
+    rng = np.random.default_rng(rows + n)
+    x = -rng.uniform(87.4, 103.9, (rows, n)).astype(np.float32)
+    x[:, n // 3] = 0.0
+    want = np.exp(x.astype(np.float64)).astype(np.float32)
+    a = host(ops.softmax(dev(x)))
+    b = host(ops.softmax(dev(x.T), axis=0)).T
+    for got in (a, b):
+        bad = (got.view(np.uint32) != want.view(np.uint32)).sum()
+        assert ulp_diff(got, want).max() <= 1 and bad <= max(1, x.size >> 20), (bad, x.size)

@@ -232,9 +232,10 @@ template <int NT> __device__ __forceinline__ double block_sum(double v, double *
 // It is the one thing a float softmax tensor computes per element, and what costs there are the
 // conversions and the double rounding and scaling instructions, not the multiply-adds: the
 // multiple of ln 2 is found in single precision (any integer near d log2 e serves: |r| <= 0.34662
-// covers the rounding of d * log2 e), the power of two goes onto the float, and the polynomial is
+// covers the rounding of d * log2 e), the power of two goes into the double's exponent as an integer --
+// before the one rounding to float, which a subnormal result needs -- and the polynomial is
 // the minimax one of degree 8 on that interval (2^-39.8; the Taylor polynomial of degree 9 it
-// replaces: 2^-37).  18.8 against 30.6 issue slots an element (a loop of nothing else, 2.1 M threads).
+// replaces: 2^-37).
 __device__ __forceinline__ float exp_accurate(float d) {
     d = d < -104.0f ? -104.0f : d;  // (a comparison, not a maximum: NaN stays)
     const float n = rintf(d * 1.44269504088896341f);
@@ -248,7 +249,8 @@ __device__ __forceinline__ float exp_accurate(float d) {
     p = fma(p, r, 0x1.fffffffff71a8p-2);
     p = fma(p, r, 0x1.ffffffffd37fep-1);
     p = fma(p, r, 1.0);
-    return ldexpf(static_cast<float>(p), __float2int_rn(n));
+    const int hi = __double2hiint(p) + __float2int_rn(n) * (1 << 20);  // (0.7 <= p <= 1.5, -150 <= n: still a normal double)
+    return static_cast<float>(__hiloint2double(hi, __double2loint(p)));
 }
 
 // One softmax term: exp of the single-precision difference x - m.
