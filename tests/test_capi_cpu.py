@@ -245,3 +245,44 @@ def test_native_front_end_knows_what_it_was_built_for(monkeypatch):
     monkeypatch.setattr(torch, "__version__", "1.0.0")
     with pytest.raises(ImportError, match="built for torch"):
         ops.softmax(torch.zeros(2, 5))
+
+
+def test_polynomial_of_the_exponential():
+    """exp_accurate's polynomial interpolates e^r at the nine Chebyshev points of [-0.34662, 0.34662], the coefficients rounded
+    to double: made again from that sentence in 60 digits, bit for bit, and its relative error on the interval is below 2^-39."""
+    import re
+    from decimal import Decimal as D, getcontext
+    getcontext().prec = 60
+    text = open(os.path.join(os.path.dirname(os.path.dirname(__file__)), "vkop_amd", "csrc", "device_utils.hpp")).read()
+    body = text[text.index("float exp_accurate(float d)"):]
+    body = body[:body.index("__double2hiint")]
+    have = [float.fromhex(h) for h in re.findall(r"0x1\.[0-9a-f]+p-?\d+", body)]
+    have.append(float(re.findall(r"p = fma\(p, r, (1\.0)\);", body)[0]))
+    have.reverse()
+    assert len(have) == 9
+
+    def cos(x):
+        s, t, i = D(0), D(1), 0
+        while abs(t) > D(10) ** -58:
+            s, i = s + t, i + 2
+            t = -t * x * x / (i * (i - 1))
+        return s
+    pi = D("3.14159265358979323846264338327950288419716939937510582097494459")
+    r_max = D("0.34662")
+    pts = [r_max * cos(pi * (2 * i + 1) / 18) for i in range(9)]
+    table = [p.exp() for p in pts]  # Newton's divided differences, then the powers' coefficients
+    for step in range(1, 9):
+        for i in range(8, step - 1, -1):
+            table[i] = (table[i] - table[i - 1]) / (pts[i] - pts[i - step])
+    coeff = [table[8]] + [D(0)] * 8
+    for i in range(7, -1, -1):
+        coeff = [table[i] - pts[i] * coeff[0]] + [coeff[j - 1] - pts[i] * coeff[j] for j in range(1, 9)]
+    assert [float(c) for c in coeff] == have
+    worst = D(0)
+    for i in range(2001):
+        r = r_max * (D(i) / 1000 - 1)
+        p = D(0)
+        for c in reversed(have):
+            p = p * r + D(c)
+        worst = max(worst, abs(p / r.exp() - 1))
+    assert worst < D(2) ** -39

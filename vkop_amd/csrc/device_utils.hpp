@@ -234,8 +234,8 @@ template <int NT> __device__ __forceinline__ double block_sum(double v, double *
 // multiple of ln 2 is found in single precision (any integer near d log2 e serves: |r| <= 0.34662
 // covers the rounding of d * log2 e), the power of two goes into the double's exponent as an integer --
 // before the one rounding to float, which a subnormal result needs -- and the polynomial is
-// the minimax one of degree 8 on that interval (2^-39.8; the Taylor polynomial of degree 9 it
-// replaces: 2^-37).
+// the one of degree 8 that interpolates e^r at the nine Chebyshev points of that interval, its
+// coefficients rounded to double (2^-39.7; the Taylor polynomial of degree 9 it replaces: 2^-37).
 __device__ __forceinline__ float exp_accurate(float d) {
     d = d < -104.0f ? -104.0f : d;  // (a comparison, not a maximum: NaN stays)
     const float n = rintf(d * 1.44269504088896341f);
