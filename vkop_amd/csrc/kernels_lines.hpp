@@ -62,8 +62,12 @@ template <int P> __device__ __forceinline__ double parts_sum(double v) {
 // K = ceil(n / (P * W)): every element but a lane's last exists.
 // Launch: blockDim = teams * W waves, a team of W waves per 64 / P vectors; LDS for W > 1:
 // 64 / P * L * (W * teams) doubles.
-template <typename T, int K, int P, bool MAX_ONLY>
-__global__ __launch_bounds__(kLinesWavesMax *kWave) void softmax_lines_reg_kernel(const T *in, T *out, LineGeom g, uint32_t W,
+// WIDE: a lane adds its terms in double.  Halves in one wave a line add up to eight of them in float (TermSum), which
+// [8,21,262144] is worth 2 %; longer lines, more of them in all, do not.
+// (the largest probability of halves is held to 64 registers, which K = 8 exceeds by one: two workgroups of 16 waves a CU
+// instead of one, [8,1000,8000] 47 against 61 us)
+template <typename T, int K, int P, bool MAX_ONLY, bool WIDE>
+__global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && MAX_ONLY ? 8 : 4))) void softmax_lines_reg_kernel(const T *in, T *out, LineGeom g, uint32_t W,
                                                                                 int nan_where, float nan_value) {
     constexpr int L = Vec128<T>::N;
     constexpr uint32_t LPW = kWave / P;  // vectors (of L lines) a wave
@@ -129,7 +133,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) void softmax_lines_reg_kerne
         __syncthreads();  // (the sums take the same place)
     }
     float e[K][L];
-    TermSum<T> acc[L];
+    std::conditional_t<WIDE, double, TermSum<T>> acc[L];
 #pragma unroll
     for (int c = 0; c < L; c++) acc[c] = 0;
 #pragma unroll
@@ -139,7 +143,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) void softmax_lines_reg_kerne
 #pragma unroll
         for (int c = 0; c < L; c++) {
             e[i][c] = softmax_term_as<T>(q[i].get(c), m[c]);
-            acc[c] += static_cast<TermSum<T>>(i < K - 1 || last_ok ? e[i][c] : 0.f);
+            acc[c] += i < K - 1 || last_ok ? e[i][c] : 0.f;
         }
     }
     double s[L];

@@ -150,18 +150,26 @@ template <typename T, int V> struct RowPiece {
         }
         return m;
     }
-    // the terms, and their sum over this lane's elements
-    __device__ __forceinline__ double terms(float m) {
-        TermSum<T> acc = 0;
+    // the terms, and their sum over this lane's elements: halves' terms added in float SUM at a time (TermSum)
+    template <int SUM> __device__ __forceinline__ double terms(float m) {
+        static_assert(VEC % SUM == 0, "a vector's terms in equal parts");
+        double acc = 0.0;
 #pragma unroll
         for (int i = 0; i < V; i++) {
+            TermSum<T> part = 0;
 #pragma unroll
             for (int c = 0; c < VEC; c++) {
                 e[i][c] = softmax_term_as<T>(q[i].get(c), m);
-                acc += static_cast<TermSum<T>>(i < V - 1 || static_cast<uint32_t>(c) >= dup ? e[i][c] : 0.f);
+                const float counted = i < V - 1 || static_cast<uint32_t>(c) >= dup ? e[i][c] : 0.f;
+                if constexpr (sizeof(T) == 4) {
+                    acc += static_cast<double>(counted);
+                } else {
+                    part = c % SUM == 0 ? counted : part + counted;
+                    if (c % SUM == SUM - 1) acc += static_cast<double>(part);
+                }
             }
         }
-        return static_cast<double>(acc);
+        return acc;
     }
     __device__ __forceinline__ void store(T *orow, double rinv, bool live, int nan_where, float nan_value) {
 #pragma unroll
@@ -193,7 +201,9 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(con
     RowPiece<T, V> p;
     p.load(in + row0, n, threadIdx.x % G, G);
     const float m = group_max<G>(p.largest());
-    const double rinv = reciprocal_of_sum(group_sum<G>(p.terms(m)));
+    // (halves: the shorter the row, the fewer terms are added in float -- n up to 64: 1, 128: 2, 256: 4, else 8)
+    constexpr int SUM = G == 8 ? (V == 1 ? 1 : V == 2 ? 2 : 4) : G == 16 && V <= 2 ? 4 : 8;
+    const double rinv = reciprocal_of_sum(group_sum<G>(p.template terms<SUM < RowPiece<T, V>::VEC ? SUM : RowPiece<T, V>::VEC>(m)));
     p.store(out + row0, rinv, live, nan_where, nan_value);
 }
 
@@ -219,7 +229,7 @@ __global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel
         const uint32_t w = lane & (kSoftmaxRowWavesMax - 1);
         m = group_max<kSoftmaxRowWavesMax>(w < waves ? fscratch[w] : -INFINITY);
     }
-    double s = group_sum<kWave>(p.terms(m));
+    double s = group_sum<kWave>(p.template terms<RowPiece<T, V>::VEC>(m));
     if (waves > 1) {
         if (lane == 0) dscratch[wave] = s;
         __syncthreads();
@@ -243,13 +253,13 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_thread_kernel(co
         x[j] = load_elem(rowp, j < n ? j : 0u);
         if (j < n) m = fmaxf(m, x[j]);
     }
-    TermSum<T> acc = 0;
+    double acc = 0.0;
 #pragma unroll
     for (uint32_t j = 0; j < VEC - 1; j++) {
         x[j] = j < n ? softmax_term_as<T>(x[j], m) : 0.f;
-        acc += static_cast<TermSum<T>>(x[j]);
+        acc += static_cast<double>(x[j]);
     }
-    const double rinv = reciprocal_of_sum(static_cast<double>(acc));
+    const double rinv = reciprocal_of_sum(acc);
     T *orow = out + static_cast<size_t>(row) * n;
 #pragma unroll
     for (uint32_t j = 0; j < VEC - 1; j++) {

@@ -14,11 +14,14 @@ template <typename T> bool launch_softmax_lines(const LinesLaunch &a) {
     const size_t lds = a.w > 1 ? static_cast<size_t>(teams) * a.w * per_team * L * sizeof(double) : 0;
     const T *in = static_cast<const T *>(a.in);
     T *out = static_cast<T *>(a.out);
-#define VKOP_LINES(K, P)                                                                                                            \
-    if (a.k == K && a.p == P) {                                                                                                     \
-        if (a.max_only) softmax_lines_reg_kernel<T, K, P, true><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, 0, 0.f);      \
-        else softmax_lines_reg_kernel<T, K, P, false><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, a.nan_where, a.nan_value); \
-        return true;                                                                                                                \
+#define VKOP_LINES_LAUNCH(K, P, WIDE)                                                                                                      \
+    if (a.max_only) softmax_lines_reg_kernel<T, K, P, true, WIDE><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, 0, 0.f);          \
+    else softmax_lines_reg_kernel<T, K, P, false, WIDE><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, a.nan_where, a.nan_value)
+#define VKOP_LINES(K, P)                                                                                                                   \
+    if (a.k == K && a.p == P) {                                                                                                            \
+        if (sizeof(T) == 4 || a.w > 1) VKOP_LINES_LAUNCH(K, P, true);                                                                      \
+        else VKOP_LINES_LAUNCH(K, P, (sizeof(T) == 4));                                                                                    \
+        return true;                                                                                                                       \
     }
 #define VKOP_LINES_5_8(P) VKOP_LINES(5, P) VKOP_LINES(6, P) VKOP_LINES(7, P) VKOP_LINES(8, P)
 #define VKOP_LINES_9_16(P)                                                                                     \
@@ -35,6 +38,7 @@ template <typename T> bool launch_softmax_lines(const LinesLaunch &a) {
 #undef VKOP_LINES_9_16
 #undef VKOP_LINES_5_8
 #undef VKOP_LINES
+#undef VKOP_LINES_LAUNCH
     return false;
 }
 
