@@ -158,7 +158,10 @@ def test_softmax_axes(ops, shape, axis):
                           for o, n, i in ((2, 129, 33), (1, 200, 1003), (5, 255, 65), (16, 256, 8), (30, 257, 9), (3, 513, 3137), (16, 511, 785),
                                           (300, 600, 12), (33, 777, 65), (2, 1000, 4100), (9, 1023, 520), (1, 1024, 8193), (2, 1025, 64))] +
                          [(3, 17, 110001, np.float16), (5, 32, 40000, np.float16), (3, 33, 170003, np.float16), (8, 64, 32769, np.float16),
-                          (4, 65, 130001, np.float16), (33, 128, 8001, np.float16)])
+                          (4, 65, 130001, np.float16), (33, 128, 8001, np.float16)] +
+                         # large enough for ordinary stores off the cache lines, a kilobyte of a row a wave and less, one wave a line and more
+                         [(8, 16, 82001, np.float32), (8, 80, 13107, np.float32), (5, 600, 4099, np.float32), (8, 24, 131075, np.float16),
+                          (8, 64, 50001, np.float16), (8, 300, 8001, np.float16)])
 def test_softmax_lines_in_registers(ops, outer, n, inner, dtype):
     """Lines along the middle axis that lanes, waves and workgroups hold in registers: line lengths
     around the elements a lane, the lanes and the waves of a line, rows that are no whole number of

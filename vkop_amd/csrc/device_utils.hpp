@@ -77,6 +77,12 @@ template <typename T> __device__ __forceinline__ void store16_stream(T *p, const
     __builtin_nontemporal_store(v, reinterpret_cast<vec16_any *>(p));
 }
 
+template <typename T> __device__ __forceinline__ void store16_any(T *p, const uint4 &u) {
+    vec16_any v;
+    v.x = u.x, v.y = u.y, v.z = u.z, v.w = u.w;
+    *reinterpret_cast<vec16_any *>(p) = v;
+}
+
 // Larger of three floats, quiet NaN dropped (fmaxf on loaded values costs one more instruction an operand:
 // the compiler first turns every value that may be a signalling NaN into a quiet one).  A signalling NaN
 // may come out as a quiet one: for callers whose result is NaN wherever an operand was -- a softmax's

@@ -217,9 +217,17 @@ bool plan_lines(const View &v, uint32_t vec, SoftmaxPlan *p) {
     // here, [1,80,8400] 5.8 against 4.9).  Halves, twice as many lines a lane: [1,80,8400] 4.2 against 6.1,
     // [4,91,12345] 7.6 against 9.9, but [4,24,65536] 8.6 against 8.1, [8,48,65536] 30.4 against 22.5 and
     // [8,100,65536] 64 against 60; their lines of up to 16 never gain more than they lose ([8,16,262144] 26.9 / 28.3).
+    // Halves' rows off 16 bytes, or off the cache lines, ask for more of them: [8,32,81921] 18.1 against 23.0, [8,64,40961]
+    // 18.8 / 25.4, [8,48,54612] 18.4 / 22.2, but [8,32,131073] 36.3 / 31.9, [8,64,65537] 46.8 / 35.2.
+    // (The largest probability alone takes the same kernel as the tensor, whose maximum it is bit for bit, whichever of the two
+    // is the better one for it: [8,128,65536] 42.8 against 39.2, [8,65,129055] 49 / 55.)
     if (n <= 128) {
         if (v.elems < (1u << 19)) return false;
-        if (half && (n <= 16 || v.elems < (n <= 32 ? 5ull << 20 : n <= 64 ? 1ull << 24 : 1ull << 25))) return false;
+        if (half) {
+            const bool off16 = v.g.inner % 8 != 0, off128 = v.g.inner % 64 != 0;
+            const uint64_t least = n <= 32 ? (off16 && n > 20 ? 3ull << 23 : 5ull << 20) : n <= 64 ? (off128 ? 3ull << 23 : 1ull << 24) : 1ull << 25;
+            if (n <= 16 || v.elems < least) return false;
+        }
     } else if (vectors < 32) {  // ([1,1000,64] f16 10.2 against 11.9, f32 max only 8.3 against 9.2)
         return false;
     }
@@ -324,7 +332,7 @@ int launch_lines(const T *in, T *out, const View &v, const SoftmaxPlan &p, bool 
                  hipStream_t st) {
     return in_slices(v.g.outer, lines_threads(v, 16 / sizeof(T), p.lines_p, p.lines_w), [&](uint64_t first, uint32_t outer) {
         vkop::LinesLaunch a{in + first * v.g.n * v.g.inner, out + first * (max_only ? 1u : v.g.n) * v.g.inner, v.g, p.lines_k, p.lines_p,
-                            p.lines_w, max_only, nan_where, nan_value, st};
+                            p.lines_w, max_only, v.elems * sizeof(T), nan_where, nan_value, st};
         a.g.outer = outer;
         if (!vkop::launch_softmax_lines<T>(a))
             return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
