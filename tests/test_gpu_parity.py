@@ -1247,3 +1247,24 @@ def test_softmax_subnormal_terms_are_rounded_once(ops, rows, n):
     for got in (a, b):
         bad = (got.view(np.uint32) != want.view(np.uint32)).sum()
         assert ulp_diff(got, want).max() <= 1 and bad <= max(1, x.size >> 20), (bad, x.size)
+
+
+@pytest.mark.parametrize("lanes", [1, 7, 15, 16, 40])
+def test_softmax_value_held_by_few_lanes_of_every_wave(ops, lanes):
+    """A row whose smallest value sits in every 64th 16-byte vector, or in up to 40 of each 64: its copies are set apart from the
+    sum whatever number of a wave's lanes hold them, and counted with the term as it is defined, rounded to float, so the
+    hardware exponential's error for that one value is not in the row's sum a thousand times over.  What is left is the average of
+    that error over values that all differ, 3.2e-9 of the sum at most on these 64 rows; a quarter of a row with one value's
+    error brought 1.5e-8."""
+    n, rows = 131072, 64
+    rng = np.random.default_rng(lanes)
+    lane = (np.arange(n) // 4) % 64
+    floor = np.linspace(-9.3, -5.1, rows).astype(np.float32)[:, None]
+    x = floor + rng.uniform(0.05, 0.5, (rows, n)).astype(np.float32)
+    x = np.where(lane[None] < lanes, floor, x).astype(np.float32)
+    x[:, 77] = 0.0
+    got = host(ops.softmax(dev(x)))
+    e = np.exp(x.astype(np.float64)).astype(np.float32).astype(np.float64)
+    # the sum's relative error, from the other elements: their results' own roundings average to 1e-10, the copies' share one
+    off = (got / (e / e.sum(-1, keepdims=True)) - 1)[:, lane >= lanes].mean(-1)
+    assert np.abs(off).max() < 6e-9, np.abs(off).max()

