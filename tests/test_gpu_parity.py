@@ -1087,9 +1087,8 @@ def test_nms_random_configurations(ops):
 @pytest.mark.parametrize("power", [-80, -41, -39, 0, 39, 41, 62])
 def test_nms_overlap_beside_the_threshold(ops, power):
     """The quotient of the areas is compared without being formed where products decide: thresholds 2^-20 and 2^-18
-    beside some pair's own overlap -- the products decide from 2^-21 on, and 2^-22 bounds what a fused product
-    moves in the areas -- with boxes scaled by powers of two up to areas near the largest float and down to ones
-    that underflow to nothing."""
+    beside some pair's own overlap -- the products decide from 2^-21 on -- with boxes scaled by powers of two up to areas
+    near the largest float and down to ones that underflow to nothing."""
     rng = np.random.default_rng(100 + power)
     boxes = _nms_boxes(rng, 1, 96, 0.6) * np.float32(2.0 ** power)
     scores = rng.random((1, 3, 96)).astype(np.float32)
@@ -1268,3 +1267,34 @@ def test_softmax_value_held_by_few_lanes_of_every_wave(ops, lanes):
     # the sum's relative error, from the other elements: their results' own roundings average to 1e-10, the copies' share one
     off = (got / (e / e.sum(-1, keepdims=True)) - 1)[:, lane >= lanes].mean(-1)
     assert np.abs(off).max() < 6e-9, np.abs(off).max()
+
+
+@pytest.mark.parametrize("others", [0, 300, 700])
+def test_nms_overlap_equal_to_the_threshold(ops, others):
+    """The comparison with the threshold is the host's bit for bit, every operation rounded on its own: thresholds that are a
+    pair's own overlap, and its neighbours, for pairs whose overlap comes out otherwise when one of the two areas goes into
+    their sum unrounded -- alone, in a list of up to 512 and in a longer one."""
+    f, d = np.float32, np.float64
+    rng = np.random.default_rng(17)
+    a, b = (_nms_boxes(rng, 1, 4000, 0.5)[0] for _ in range(2))
+    side = lambda t: (t[:, 2] - t[:, 0], t[:, 3] - t[:, 1])
+    w, h = np.minimum(a[:, 2], b[:, 2]) - np.maximum(a[:, 0], b[:, 0]), np.minimum(a[:, 3], b[:, 3]) - np.maximum(a[:, 1], b[:, 1])
+    keep = (w > 0.02) & (h > 0.02)
+    a, b, inter = a[keep], b[keep], (w * h)[keep]
+    (aw, ah), (bw, bh) = side(a), side(b)
+    apart = inter / ((aw * ah + bw * bh) - inter)
+    fused = [inter / ((x.astype(d) * y + z).astype(f) - inter) for x, y, z in ((aw, ah, bw * bh), (bw, bh, aw * ah))]
+    assert apart.dtype == f
+    pick = np.flatnonzero((fused[0] != apart) | (fused[1] != apart))[:24]
+    assert pick.size == 24
+    # far from the two and from each other
+    k = np.arange(others)
+    rest = np.stack([10 + k, 10 + k, 10.5 + k, 10.5 + k], -1).astype(f)
+    scores = np.concatenate([[0.9, 0.8], 0.7 - 0.0005 * k]).astype(f)[None, None]
+    for i in pick:
+        boxes = np.concatenate([a[i][None], b[i][None], rest])[None]
+        for thr in (np.nextafter(apart[i], f(0)), apart[i], np.nextafter(apart[i], f(1)), fused[0][i], fused[1][i]):
+            for bx in (boxes, boxes[:, [1, 0] + list(range(2, 2 + others))]):
+                got, _ = ops.nms(dev(bx), dev(scores), float(thr), 0.0)
+                want = others + (1 if apart[i] > thr else 2)
+                assert got.shape[0] == want and np.array_equal(host(got), oracle.nms(bx, scores, float(thr), 0.0, 0, max_candidates=2048)), (i, thr)

@@ -10,9 +10,9 @@
 //      corner coordinates of its own sorted positions into registers;
 //   3. the sorted list is walked in blocks of 64: all waves compute, for every
 //      candidate of the block, which earlier ones of the block would suppress it
-//      (IoU as in shaders/nms.comp:61-72; the compiler fuses products of the areas
-//      into their sums, so an overlap within 2^-22 of the threshold may compare
-//      otherwise than with every operation rounded); the first wave finds the kept set with a few ballots (a fixed-point
+//      (IoU as in shaders/nms.comp:61-72, every operation rounded on its own so
+//      that the comparison with the threshold is the same bit for bit on the
+//      host); the first wave finds the kept set with a few ballots (a fixed-point
 //      iteration instead of one step per kept box).  Up to 512 candidates, the
 //      usual case, have their boxes in LDS: the waves share a block's tests
 //      against the boxes kept so far as they share those within it, and the kept
@@ -59,13 +59,23 @@ __device__ __forceinline__ float4 nms_load4(const uint16_t *p) {
                        __half2float(__ushort_as_half(static_cast<unsigned short>(w.y >> 16))));
 }
 
-__device__ __forceinline__ float nms_iou(const float4 &a, const float4 &b) {
+// Areas of the intersection and of the union of two boxes that overlap (false: they do not), every operation rounded on
+// its own.  (Plain operators without contraction: __fmul_rn is an ordinary product to this compiler, which fused that of one
+// area into the sum of both -- IoU(a, b) was not IoU(b, a).  It costs an instruction a pair: [16,80,8400] 26.0 us either way.)
+__device__ __forceinline__ bool nms_areas(const float4 &a, const float4 &b, float &inter, float &uni) {
+#pragma clang fp contract(off)
     const float x1 = fmaxf(a.x, b.x), y1 = fmaxf(a.y, b.y), x2 = fminf(a.z, b.z), y2 = fminf(a.w, b.w);
-    if (x2 <= x1 || y2 <= y1) return 0.f;
-    const float inter = __fmul_rn(__fsub_rn(x2, x1), __fsub_rn(y2, y1));
-    const float area_a = __fmul_rn(__fsub_rn(a.z, a.x), __fsub_rn(a.w, a.y));
-    const float area_b = __fmul_rn(__fsub_rn(b.z, b.x), __fsub_rn(b.w, b.y));
-    const float uni = __fsub_rn(__fadd_rn(area_a, area_b), inter);
+    if (x2 <= x1 || y2 <= y1) return false;
+    inter = (x2 - x1) * (y2 - y1);
+    const float area_a = (a.z - a.x) * (a.w - a.y);
+    const float area_b = (b.z - b.x) * (b.w - b.y);
+    uni = (area_a + area_b) - inter;
+    return true;
+}
+
+__device__ __forceinline__ float nms_iou(const float4 &a, const float4 &b) {
+    float inter, uni;
+    if (!nms_areas(a, b, inter, uni)) return 0.f;
     return uni > 0.f ? __fdiv_rn(inter, uni) : 0.f;
 }
 
@@ -76,12 +86,8 @@ __device__ __forceinline__ float nms_iou(const float4 &a, const float4 &b) {
 // more than kNmsRankSortMax candidates divides: its loop ends at the first overlap, and the branches around the
 // division cost it more than that -- [8,80,2048] all candidates 288 us, by products 325; [1,1,2048] 698 / 747.)
 __device__ __forceinline__ bool nms_overlap(const float4 &a, const float4 &b, float threshold) {
-    const float x1 = fmaxf(a.x, b.x), y1 = fmaxf(a.y, b.y), x2 = fminf(a.z, b.z), y2 = fminf(a.w, b.w);
-    if (x2 <= x1 || y2 <= y1) return 0.f > threshold;
-    const float inter = __fmul_rn(__fsub_rn(x2, x1), __fsub_rn(y2, y1));
-    const float area_a = __fmul_rn(__fsub_rn(a.z, a.x), __fsub_rn(a.w, a.y));
-    const float area_b = __fmul_rn(__fsub_rn(b.z, b.x), __fsub_rn(b.w, b.y));
-    const float uni = __fsub_rn(__fadd_rn(area_a, area_b), inter);
+    float inter, uni;
+    if (!nms_areas(a, b, inter, uni)) return 0.f > threshold;
     const float f = __fmul_rn(threshold, uni);
     const bool plain = threshold > 0x1p-20f && threshold < 0x1p20f && f > 0x1p-80f && f < 0x1p80f;
     const bool above = inter > __fmul_rn(f, 1.f + 0x1p-21f), below = inter < __fmul_rn(f, 1.f - 0x1p-21f);
@@ -251,11 +257,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
     }
     // corners of the candidate at sorted position p
     auto corners = [&](uint32_t p) {
+#pragma clang fp contract(off)
         const T *r = brow + static_cast<size_t>(composite_index(comp[p])) * 4;
         float4 b = make_float4(load_elem(r, 0), load_elem(r, 1), load_elem(r, 2), load_elem(r, 3));
         if (center_point_box) {  // (x_center, y_center, width, height), shaders/nms.comp:55-58
             const float hw = b.z * 0.5f, hh = b.w * 0.5f;
-            b = make_float4(__fsub_rn(b.x, hw), __fsub_rn(b.y, hh), __fadd_rn(b.x, hw), __fadd_rn(b.y, hh));
+            b = make_float4(b.x - hw, b.y - hh, b.x + hw, b.y + hh);
         }
         return b;
     };
