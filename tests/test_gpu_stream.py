@@ -601,3 +601,38 @@ def test_signalling_nan_ranks_as_nan(ops, n, k):
             for r in range(rows.shape[0]):
                 assert np.array_equal(host(ix[r]), eix[r]), (largest, r)
             assert np.array_equal(host(v).view(np.uint32), ev.view(np.uint32)), largest
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,n,k", [(9, 4096, 64), (9, 4001, 64), (20, 8192, 100), (16, 8400, 300), (9, 1100, 100)])
+def test_rows_of_few_values_whose_keys_end_in_ones(ops, rows, n, k, dtype):
+    """One workgroup a row, rows of one value, two or a dozen: the bound from the lane maxima holds the leading 16 bits of a
+    key, the low bits of which are ones for -0.75 and anything for 0.1, and is raised to the value itself where fewer than k+1
+    lanes exceed it.  k - 1, k, k + 1 elements above the value, -inf beside it, and -inf alone; both directions and fused."""
+    rng = np.random.default_rng(n + k)
+    x = np.empty((rows, n), np.float32)
+    for r in range(rows):
+        v = (-0.75, 0.1, -0.1, 0.75, -3.3e-5, 1e4, -1e4)[r % 7]
+        x[r] = v
+        if r % 9 == 7:
+            x[r, rng.permutation(n)[:n // 2]] = -np.inf
+        if r % 9 == 8:
+            x[r] = (np.round(rng.standard_normal(n) * 2) / 2 * 0.1)
+        if r % 3 == 1:
+            at = rng.choice(n, k + r % 5 - 1, replace=False)
+            x[r, at] = v + np.abs(v) * (1 + rng.random(at.size))
+        if r % 3 == 2:
+            at = rng.choice(n, k + r % 4 - 1, replace=False)
+            x[r, at] = v - np.abs(v) * (1 + rng.random(at.size))
+    x[rows - 1] = -np.inf
+    x[rows - 1, :k // 2] = 0.1
+    x = x.astype(dtype)
+    bits = np.uint16 if dtype == np.float16 else np.uint32
+    for largest in (True, False):
+        v, ix = ops.topk(dev(x), k, largest=largest)
+        ev, eix = oracle.topk(x, k, -1, largest)
+        assert np.array_equal(host(ix), eix) and np.array_equal(host(v).view(bits), ev.view(bits)), largest
+    v, ix = (host(t) for t in ops.softmax_topk(dev(x), k))
+    ev, eix = oracle.softmax_topk(x, k)
+    assert np.array_equal(ix, eix)
+    assert (half_ulp_diff(v, ev) if dtype == np.float16 else ulp_diff(v, ev)).max() <= (1 if dtype == np.float16 else 2)

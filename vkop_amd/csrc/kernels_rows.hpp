@@ -279,7 +279,7 @@ template <int NT> struct ChunkShared {  // chunk phase
     uint4 stage_v[NT];     // per wave: up to 64 vectors holding an element at or above the threshold ...
     uint32_t stage_e[NT];  // ... and the index of their first element
     uint32_t wave_thr[16];
-    uint32_t refine[40];  // element counts per bit of the exact threshold search; [32], [33]: smallest key at or above a bound / elements
+    uint32_t refine[42];  // element counts per bit of the exact threshold search; [32], [33]: smallest key at or above a bound / elements
                           // above that key, and the same in [34] ... [39] for the next two distinct values up
     uint32_t thr, total, over;
 };
@@ -1827,7 +1827,24 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
             // bound, everything at or above it is listed straight away if that fits (first turn of the loop
             // below), and only otherwise the exact cut is looked for (second turn).
             bool tight = false;
-            if (tid < 40) cs.refine[tid] = (tid >= 32 && (tid & 1u) == 0u) ? 0xFFFFFFFFu : 0u;
+            if (tid < 42) cs.refine[tid] = (tid >= 32 && (tid & 1u) == 0u) ? 0xFFFFFFFFu : 0u;
+            // The bound has the lane maxima's (k+1)-th largest in its leading 16 bits alone.  Where many lane maxima are
+            // equal -- a row of one value -- and the low bits of their key are not zero (of a negative value they are
+            // rarely: a row of 0.75 with the largest first has zeros, with the smallest first ones), it lies below that
+            // value, and everything that follows looks for what the smallest lane maximum at or above the bound says at
+            // once, if fewer than k+1 lanes exceed it.
+            __syncthreads();
+            {
+                const uint32_t least = ~wave_max_u32(~(lkey >= thr ? lkey : 0xFFFFFFFFu));
+                if (lane == 0) atomicMin(&cs.refine[40], least);
+                __syncthreads();
+                const uint32_t t0 = cs.refine[40];
+                const uint32_t above = static_cast<uint32_t>(__popcll(__ballot(lkey > t0)));
+                if (lane == 0 && above) atomicAdd(&cs.refine[41], above);
+                __syncthreads();
+                // (thr is that bound, which k+1 lanes reach, not the one that keeps -inf out)
+                if (thr == thr_block && t0 != 0xFFFFFFFFu && cs.refine[41] < want) thr = t0;
+            }
             {
                 uint32_t a = 0;
 #pragma unroll
