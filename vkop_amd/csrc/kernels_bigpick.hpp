@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kBigPickThreads) void bigpick_gather_kernel(const T
     __shared__ uint32_t wtot[NW];
     __shared__ uint32_t cslots[2][NW];
     __shared__ uint32_t lcount, zcount, lbase[kBigPickLists];
-    __shared__ uint64_t lcand[kBigPickLocalCap];
+    __shared__ __align__(16) uint64_t lcand[kBigPickLocalCap];
     __shared__ uint64_t zcand[kBigPickZoneQuota];
     __shared__ float lterm[SOFTMAX ? kBigPickLocalCap : 1];
     __shared__ float fscratch[NW];
@@ -383,9 +383,11 @@ __global__ __launch_bounds__(kBigPickThreads) void bigpick_gather_kernel(const T
         const uint32_t both = bigpick_count_sum(c2, cslots[flip]);
         const uint32_t nfull = both >> 16, nhit = both & 0xFFFFu;
         if (nfull * BE + (nhit - nfull) > static_cast<uint32_t>(kBigPickCap)) {  // (the same for every thread of every workgroup of the row)
-            // the largest value (its low ten bits aside) that k+1 elements are KNOWN to reach
-            uint32_t tmin = 0;
-            for (int bit = 31; bit >= 10; bit--) {
+            // the largest value (its low ten bits aside) that k+1 elements are KNOWN to reach: of the bits in which the
+            // largest key differs from thr, which they are known to reach already
+            const uint32_t differ = thr ^ kmax;
+            uint32_t tmin = differ == 0u ? thr : thr & ~((2u << (31 - __clz(static_cast<int>(differ)))) - 1u);
+            for (int bit = differ == 0u ? 0 : 31 - __clz(static_cast<int>(differ)); bit >= 10; bit--) {
                 const uint32_t trial = tmin | (1u << bit);
                 uint32_t c = 0;
 #pragma unroll
@@ -412,24 +414,26 @@ __global__ __launch_bounds__(kBigPickThreads) void bigpick_gather_kernel(const T
             for (uint32_t b = static_cast<uint32_t>(GE) * NT + tid; b < 8192u; b += NT) known[b] = 0;
             if (tid == 0) answer[0] = 0xFFFFFFFFu;
             __syncthreads();
-            if (tid < static_cast<uint32_t>(kWave)) {
-                // lane L owns blocks 128 L .. 128 L + 127 (summed in rotated order: lanes on different banks)
-                uint32_t sum = 0;
-                for (uint32_t j = 0; j < 128u; j++) sum += known[lane * 128u + ((j + 2u * lane) & 127u)];
-                uint32_t incl = sum;  // sum over lanes <= this one
+            // thread t owns blocks 32 t .. 32 t + 31
+            const uint4 *own = reinterpret_cast<const uint4 *>(known) + tid * 4u;
+            uint32_t sum = 0;
 #pragma unroll
-                for (int o = 1; o < kWave; o <<= 1) {
-                    const uint32_t t = __shfl_up(incl, o, kWave);
-                    if (lane >= static_cast<uint32_t>(o)) incl += t;
-                }
-                uint32_t before = incl - sum;
-                if (before < want && want <= incl) {
-                    for (uint32_t j = 0; j < 128u; j++) {
-                        before += known[lane * 128u + j];
-                        if (before >= want) {
-                            answer[0] = lane * 128u + j;
-                            break;
-                        }
+            for (int j = 0; j < 4; j++) {
+                const uint4 w = own[j];
+                sum += (w.x & 0xFFFFu) + (w.x >> 16) + (w.y & 0xFFFFu) + (w.y >> 16) + (w.z & 0xFFFFu) + (w.z >> 16) + (w.w & 0xFFFFu) + (w.w >> 16);
+            }
+            const uint32_t incl = wave_inclusive_sum_u32(sum);
+            if (lane == kWave - 1) wtot[wave] = incl;
+            __syncthreads();
+            uint32_t before = incl - sum;
+#pragma unroll
+            for (int w = 0; w < NW; w++) before += static_cast<uint32_t>(w) < wave ? wtot[w] : 0u;
+            if (before < want && want <= before + sum) {
+                for (uint32_t j = 0; j < 32u; j++) {
+                    before += known[tid * 32u + j];
+                    if (before >= want) {
+                        answer[0] = tid * 32u + j;
+                        break;
                     }
                 }
             }
