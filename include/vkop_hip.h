@@ -256,11 +256,14 @@ int vkop_hip_nms(const void *boxes, const void *scores, int32_t *out, int out_ca
  * Unknown names return VKOP_HIP_ERR_INVALID. */
 int vkop_hip_tune(const char *name, int value);
 
-/* Launch shape the fused / top-k entry points would use for this tensor:
+/* Launch shape the fused entry point, largest first, would use for this tensor:
  * threads per workgroup, 128-bit loads per thread and workgroups per row of the
  * streaming kernel (a second kernel per row follows when chunks > 1); all three
- * are 0 when the general one-workgroup-per-line kernels would run.  Any out
- * pointer may be NULL. */
+ * are 0 when the radix select or the general one-workgroup-per-line kernels would
+ * run.  The plain top-k takes the same shape, except on a row that one workgroup
+ * of this kernel holds and that has fewer 16-byte vectors than k + 1 (smallest
+ * first: fewer than 2 (k + 1)): it runs an exact select there.  Any out pointer
+ * may be NULL. */
 int vkop_hip_rows_plan(int dtype, const int *shape, int ndim, int axis, int k,
                        int *threads, int *loads, int *chunks);
 

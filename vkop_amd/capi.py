@@ -329,13 +329,15 @@ def measure_stages(stages):
 
 
 def measure_path(dtype, shape, axis, k):
-    """Benchmarks only: 2 = scan + pick kernels, 1 = chunk (+ merge) kernels, 0 = other kernels for this tensor."""
+    """Which kernels a fused call on this tensor takes: 4 = one wave per row, 3 = scan + gather + rank, 2 = scan + pick,
+    1 = chunk (+ merge), 0 = radix select or general kernels.  The plain top-k takes the same ones, except where path 1 has
+    fewer 16-byte vectors a row than k + 1 (smallest first: than 2 (k + 1)): an exact select.  Benchmarks and tests only."""
     arr, nd = _shape(shape)
     return lib().vkop_hip_measure_path(dtype, arr, nd, axis, int(k))
 
 
 def rows_plan(dtype, shape, axis, k):
-    """(threads, loads, chunks) of the streaming kernel for this tensor; zeros = general kernels."""
+    """(threads, loads, chunks) of a fused call's streaming kernel for this tensor, as measure_path; zeros = path 0."""
     arr, nd = _shape(shape)
     t, l, c = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
     check(lib().vkop_hip_rows_plan(dtype, arr, nd, axis, k, ctypes.byref(t), ctypes.byref(l), ctypes.byref(c)))

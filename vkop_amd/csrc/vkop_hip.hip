@@ -940,6 +940,7 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
     // Fewer vectors than places: their maxima bound nothing, and every row would take that kernel's second list
     // ([2000,1462] f16 k = 225: 225 us, 32 with a workgroup's exact select a row).  Smallest first, where that
     // select ran before, it stays the faster one up to twice as many ([2000,600] f32 k = 100: 15.3 against 17.9 us).
+    // (The fused call and vkop_hip_rows_plan do not know this rule.)
     const uint32_t vectors = (v.g.n + 16 / sizeof(T) - 1) / (16 / sizeof(T));
     if (c.ok && g_rows_path.load() != 1 && vectors < (largest ? 1u : 2u) * (static_cast<uint32_t>(k) + 1u)) c = RowsCfg{};
     const BigKCfg b = (c.ok || sc.ok) ? BigKCfg{} : choose_bigk_cfg(v, k, dtype);
