@@ -603,6 +603,26 @@ def test_softmax_then_max_in_one_pass(ops, shape, axis, dtype):
         assert ulp_diff(fused[ok], want[ok]).max() <= 2
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,n", [(200000, 1), (200000, 5), (200000, 8), (200000, 13), (200000, 16), (200000, 17), (200000, 40), (200000, 64), (150000, 100), (131072, 128),
+                                    (85163, 197), (32768, 512), (16777, 1000), (8192, 2049), (600, 20001), (64, 9001), (83, 200000),
+                                    (3, 600000)])
+def test_softmax_then_max_of_last_axis_rows(ops, rows, n, dtype):
+    """Bit for bit the maximum of the softmax operator's tensor on the last axis too, whatever kernels the row length takes
+    (a thread, lanes of a wave or a workgroup a row, chunks): in half precision a sum taken in another order gave another
+    half in one line of ten thousand."""
+    x = torch.from_numpy((np.random.default_rng(n).standard_normal((rows, n), dtype=np.float32) * 2).astype(dtype))
+    x[0, n // 2] = float("nan")
+    x[1, :] = float("-inf")
+    x[2, n - 1] = float("inf")
+    xd = x.cuda()
+    fused = host(ops.softmax_reduce_max(xd, 1))
+    chain = host(ops.reduce_max(ops.softmax(xd, 1), 1))
+    bits = np.uint16 if dtype == np.float16 else np.uint32
+    assert np.isnan(chain[:3]).all() and np.isnan(fused[:3]).all()
+    assert np.array_equal(fused[3:].view(bits), chain[3:].view(bits))
+
+
 def test_workspace_too_small_is_an_error(ops):
     from vkop_amd import capi
     x = dev(synth.classifier_logits(4, 1000, 1))

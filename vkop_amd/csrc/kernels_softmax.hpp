@@ -12,6 +12,7 @@
 //                           read of the input comes from the Infinity Cache for
 //                           tensors that fit it.
 //   softmax_thread_kernel   rows of fewer elements than a vector.
+//   (each also without the tensor: the row's largest probability alone, from the same sum)
 // Strided lines (another axis, long lines):
 //   softmax_strided_tile_kernel  a tile of up to 64 neighbouring lines per workgroup of 16 waves,
 //                           rows dealt to the waves, three passes over the tile; with few
@@ -190,9 +191,14 @@ template <typename T, int V> struct RowPiece {
         }
     }
 };
+// The MAX_ONLY forms below write, instead of the tensor, each row's largest probability to out[row]: the term of the row's
+// maximum over the same sum, so bit for bit the maximum of what the other form writes (NaN where that is NaN).
+template <typename T> __device__ __forceinline__ void store_largest(T *out, size_t row, float m, double rinv) {
+    store_elem(out, row, round_to_storage<T>(scale_term<T>(softmax_term_as<T>(m, m), rinv)));
+}
 
 constexpr int kSoftmaxGroupThreads = 256;
-template <typename T, int G, int V>
+template <typename T, int G, int V, bool MAX_ONLY>
 __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(const T *in, T *out, uint32_t rows, uint32_t n,
                                                                             int nan_where, float nan_value) {
     const uint32_t row = blockIdx.x * (kSoftmaxGroupThreads / G) + threadIdx.x / G;
@@ -204,7 +210,11 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(con
     // (halves: the shorter the row, the fewer terms are added in float -- n up to 64: 1, 128: 2, 256: 4, else 8)
     constexpr int SUM = G == 8 ? (V == 1 ? 1 : V == 2 ? 2 : 4) : G == 16 && V <= 2 ? 4 : 8;
     const double rinv = reciprocal_of_sum(group_sum<G>(p.template terms<SUM < RowPiece<T, V>::VEC ? SUM : RowPiece<T, V>::VEC>(m)));
-    p.store(out + row0, rinv, live, nan_where, nan_value);
+    if constexpr (MAX_ONLY) {
+        if (live && threadIdx.x % G == 0) store_largest(out, row, m, rinv);
+    } else {
+        p.store(out + row0, rinv, live, nan_where, nan_value);
+    }
 }
 
 // ---- a row per workgroup ----------------------------------------------------------------------
@@ -213,7 +223,7 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(con
 // half of it idle.  One read, one write, two barriers.  [9872,8296] f32 241 -> 114 us, f16 88 -> 61;
 // [2000,20001] f32 225 -> 60 us, f16 133 -> 39 (element by element before); [256,8192] f32 8.4 -> 5.5.
 constexpr int kSoftmaxRowWavesMax = 16;
-template <typename T, int V>
+template <typename T, int V, bool MAX_ONLY>
 __global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel(const T *in, T *out, uint32_t n, int nan_where,
                                                                                 float nan_value) {
     __shared__ float fscratch[kSoftmaxRowWavesMax];
@@ -236,36 +246,49 @@ __global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel
         const uint32_t w = lane & (kSoftmaxRowWavesMax - 1);
         s = group_sum<kSoftmaxRowWavesMax>(w < waves ? dscratch[w] : 0.0);
     }
-    p.store(out + row0, reciprocal_of_sum(s), true, nan_where, nan_value);
+    if constexpr (MAX_ONLY) {
+        if (tid == 0) store_largest(out, blockIdx.x, m, reciprocal_of_sum(s));
+    } else {
+        p.store(out + row0, reciprocal_of_sum(s), true, nan_where, nan_value);
+    }
 }
 
 // ---- rows shorter than a vector: a thread each ------------------------------------------------
-template <typename T>
+// MAX_ONLY: rows of up to 16 elements, where a thread a row is still the faster one ([200000,13] f16 5.5 us, by the group
+// kernel 9.8; f32 7.8 / 9.0).  The sum is taken as the kernel that writes the tensor takes it: rows longer than a vector a
+// vector at a time, and those as the group kernel's lanes join (V = 1, terms in double).
+constexpr uint32_t kSoftmaxThreadMaxN = 16;
+template <typename T, bool MAX_ONLY>
 __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_thread_kernel(const T *in, T *out, uint32_t rows, uint32_t n,
                                                                              int nan_where, float nan_value) {
-    constexpr uint32_t VEC = Vec128<T>::N;
+    constexpr uint32_t VEC = Vec128<T>::N, NMAX = MAX_ONLY ? kSoftmaxThreadMaxN : VEC - 1;
+    static_assert(kSoftmaxThreadMaxN <= 4 * VEC, "vectors' sums");
     const uint32_t row = blockIdx.x * kSoftmaxGroupThreads + threadIdx.x;
     if (row >= rows) return;
     const T *rowp = in + static_cast<size_t>(row) * n;
-    float x[VEC - 1], m = -INFINITY;
+    float x[NMAX], m = -INFINITY;
 #pragma unroll
-    for (uint32_t j = 0; j < VEC - 1; j++) {
+    for (uint32_t j = 0; j < NMAX; j++) {
         x[j] = load_elem(rowp, j < n ? j : 0u);
         if (j < n) m = fmaxf(m, x[j]);
     }
-    double acc = 0.0;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (uint32_t j = 0; j < VEC - 1; j++) {
+    for (uint32_t j = 0; j < NMAX; j++) {
         x[j] = j < n ? softmax_term_as<T>(x[j], m) : 0.f;
-        acc += static_cast<double>(x[j]);
+        acc[j / VEC] += static_cast<double>(x[j]);
     }
-    const double rinv = reciprocal_of_sum(acc);
-    T *orow = out + static_cast<size_t>(row) * n;
+    const double rinv = reciprocal_of_sum((acc[0] + acc[1]) + (acc[2] + acc[3]));
+    if constexpr (MAX_ONLY) {
+        store_largest(out, row, m, rinv);
+    } else {
+        T *orow = out + static_cast<size_t>(row) * n;
 #pragma unroll
-    for (uint32_t j = 0; j < VEC - 1; j++) {
-        float p = round_to_storage<T>(scale_term<T>(x[j], rinv));
-        if (nan_where && p != p) p = nan_value;
-        if (j < n) store_elem(orow, j, p);
+        for (uint32_t j = 0; j < NMAX; j++) {
+            float p = round_to_storage<T>(scale_term<T>(x[j], rinv));
+            if (nan_where && p != p) p = nan_value;
+            if (j < n) store_elem(orow, j, p);
+        }
     }
 }
 
@@ -364,32 +387,12 @@ __global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__
     if (tid == 0) stats[blockIdx.x] = ChunkStat{acc, m, ref, mn, copies};
 }
 
-// ---- chunked rows: exp(x - M) / S -----------------------------------------------------
-// Launch: rows * GS workgroups of 256, V vectors a thread, GS = ceil(n / (256 * V * VEC)); G: the
-// chunks a row of the statistics kernel.  In-place calls are fine: see the moved vector.
-// [64,128256] f32, both kernels: 24.9 -> 22.3 us (2 reads and 1 write of 33 MB: 4.4 TB/s);
-// [63,132402] (rows off 16 bytes) f32 35.9 -> 24.3, f16 34.8 -> 17.3; [32,50257] f16 10.1 -> 8.0.
-constexpr int kSoftmaxScaleThreads = 256;
-template <typename T, int V>
-__global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(const T *in, T *out, const ChunkStat *__restrict__ stats,
-                                                                            uint32_t n, uint32_t G, uint32_t GS, int nan_where,
-                                                                            float nan_value) {
-    constexpr uint32_t VEC = Vec128<T>::N, NT = kSoftmaxScaleThreads;
-    __shared__ LineStats row_stats;
-    __shared__ float wave_m[NT / kWave];
-    __shared__ double wave_s[NT / kWave];
+// A row's maximum and the reciprocal of its sum (in thread 0) from its G chunks.  Up to 64 of them are combined by the first
+// wave, a chunk a lane; with more each wave takes its share (two barriers more, a quarter of the exponentials).
+template <typename T, uint32_t NT>
+__device__ __forceinline__ LineStats combine_chunks(const ChunkStat *cs, uint32_t G, float *wave_m, double *wave_s) {
     static_assert(NT / kWave == 4, "the two combinations below");
     const uint32_t tid = threadIdx.x;
-    const uint32_t row = blockIdx.x / GS, chunk = blockIdx.x - row * GS;
-    const uint32_t e_first = chunk * (NT * V * VEC) + tid * VEC;
-    const size_t row0 = static_cast<size_t>(row) * n;
-    const T *rowp = in + row0;
-    Vec128<T> q[V];
-#pragma unroll
-    for (int i = 0; i < V; i++) q[i].v = load16_stream(rowp + min(e_first + static_cast<uint32_t>(i) * NT * VEC, n - VEC));
-    // A row of up to 64 chunks is combined by the first wave, a chunk a lane, under everyone's loads;
-    // with more chunks each wave takes its share of them (two barriers more, a quarter of the exponentials).
-    const ChunkStat *cs = stats + static_cast<size_t>(row) * G;
     const uint32_t takers = G <= static_cast<uint32_t>(kWave) ? static_cast<uint32_t>(kWave) : NT;
     float M = -INFINITY;
     double part = 0.0;
@@ -415,7 +418,34 @@ __global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(con
         __syncthreads();
         part = (wave_s[0] + wave_s[1]) + (wave_s[2] + wave_s[3]);
     }
-    if (tid == 0) row_stats = LineStats{M, 0.f, 1.0 / part};
+    return LineStats{M, 0.f, 1.0 / part};
+}
+
+// ---- chunked rows: exp(x - M) / S -----------------------------------------------------
+// Launch: rows * GS workgroups of 256, V vectors a thread, GS = ceil(n / (256 * V * VEC)); G: the
+// chunks a row of the statistics kernel.  In-place calls are fine: see the moved vector.
+// [64,128256] f32, both kernels: 24.9 -> 22.3 us (2 reads and 1 write of 33 MB: 4.4 TB/s);
+// [63,132402] (rows off 16 bytes) f32 35.9 -> 24.3, f16 34.8 -> 17.3; [32,50257] f16 10.1 -> 8.0.
+constexpr int kSoftmaxScaleThreads = 256;
+template <typename T, int V>
+__global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(const T *in, T *out, const ChunkStat *__restrict__ stats,
+                                                                            uint32_t n, uint32_t G, uint32_t GS, int nan_where,
+                                                                            float nan_value) {
+    constexpr uint32_t VEC = Vec128<T>::N, NT = kSoftmaxScaleThreads;
+    __shared__ LineStats row_stats;
+    __shared__ float wave_m[NT / kWave];
+    __shared__ double wave_s[NT / kWave];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t row = blockIdx.x / GS, chunk = blockIdx.x - row * GS;
+    const uint32_t e_first = chunk * (NT * V * VEC) + tid * VEC;
+    const size_t row0 = static_cast<size_t>(row) * n;
+    const T *rowp = in + row0;
+    Vec128<T> q[V];
+#pragma unroll
+    for (int i = 0; i < V; i++) q[i].v = load16_stream(rowp + min(e_first + static_cast<uint32_t>(i) * NT * VEC, n - VEC));
+    // (under everyone's loads)
+    const LineStats combined = combine_chunks<T, NT>(stats + static_cast<size_t>(row) * G, G, wave_m, wave_s);
+    if (tid == 0) row_stats = combined;
     __syncthreads();
     const LineStats ls = row_stats;
     T *orow = out + row0;
@@ -442,6 +472,16 @@ __global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(con
                 if (static_cast<uint32_t>(c) >= dup) store_elem(orow, n - VEC + static_cast<uint32_t>(c), p[c]);
         }
     }
+}
+
+// The largest probability of each row, out[row], in place of the above.  Launch: a workgroup a row.
+template <typename T>
+__global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_fold_max_kernel(T *__restrict__ out, const ChunkStat *__restrict__ stats, uint32_t G) {
+    constexpr uint32_t NT = kSoftmaxScaleThreads;
+    __shared__ float wave_m[NT / kWave];
+    __shared__ double wave_s[NT / kWave];
+    const LineStats st = combine_chunks<T, NT>(stats + static_cast<size_t>(blockIdx.x) * G, G, wave_m, wave_s);
+    if (threadIdx.x == 0) store_elem(out, blockIdx.x, round_to_storage<T>(softmax_prob_as<T>(st.m, st)));
 }
 
 // ---- long strided lines: a tile of neighbouring lines per workgroup -----------------------------

@@ -340,15 +340,17 @@ int launch_lines(const T *in, T *out, const View &v, const SoftmaxPlan &p, bool 
     });
 }
 
-template <typename T>
-int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, float nan_value, void *ws,
+// The softmax of last-axis rows, or (MAX_ONLY) each row's largest probability: the kernels of kThread ... kChunked.
+template <typename T, bool MAX_ONLY>
+int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int nan_where, float nan_value, void *ws,
                  size_t ws_bytes, hipStream_t st) {
-    const SoftmaxPlan p = plan_softmax(v, dtype);
-    const uint32_t lines = v.g.outer * v.g.inner;
-    switch (p.kind) {
+    const uint32_t lines = v.g.outer;
+    const uint64_t out_row = MAX_ONLY ? 1u : v.g.n;
+    const auto kind = MAX_ONLY && v.g.n <= vkop::kSoftmaxThreadMaxN ? SoftmaxPlan::kThread : p.kind;
+    switch (kind) {
     case SoftmaxPlan::kThread: {
         const uint32_t blocks = (lines + vkop::kSoftmaxGroupThreads - 1) / vkop::kSoftmaxGroupThreads;
-        vkop::softmax_thread_kernel<T><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value);
+        vkop::softmax_thread_kernel<T, MAX_ONLY><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(in, out, lines, v.g.n, nan_where, nan_value);
         return launched("softmax_thread_kernel");
     }
     case SoftmaxPlan::kGroup: {
@@ -356,11 +358,11 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
         return in_slices((lines + per_block - 1) / per_block, vkop::kSoftmaxGroupThreads, [&](uint64_t first, uint32_t blocks) {
             const uint64_t row0 = first * per_block;
             const T *from = in + row0 * v.g.n;
-            T *to = out + row0 * v.g.n;
+            T *to = out + row0 * out_row;
             const uint32_t rows = static_cast<uint32_t>(std::min<uint64_t>(lines - row0, static_cast<uint64_t>(blocks) * per_block));
 #define VKOP_GROUP(G, V)                                                                                                       \
     if (p.shape.nt == G && p.shape.v == V) {                                                                                   \
-        vkop::softmax_group_kernel<T, G, V><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(from, to, rows, v.g.n, nan_where, nan_value); \
+        vkop::softmax_group_kernel<T, G, V, MAX_ONLY><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(from, to, rows, v.g.n, nan_where, nan_value); \
         return launched("softmax_group_kernel");                                                                               \
     }
 #define VKOP_GROUPS(G) VKOP_GROUP(G, 1) VKOP_GROUP(G, 2) VKOP_GROUP(G, 3) if constexpr (sizeof(T) == 4) { VKOP_GROUP(G, 4) }
@@ -373,10 +375,10 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
     case SoftmaxPlan::kRow: {
         return in_slices(lines, p.shape.nt, [&](uint64_t row0, uint32_t rows) {
             const T *from = in + row0 * v.g.n;
-            T *to = out + row0 * v.g.n;
+            T *to = out + row0 * out_row;
 #define VKOP_ROW(V)                                                                                     \
     if (p.shape.v == V) {                                                                               \
-        vkop::softmax_row_kernel<T, V><<<rows, p.shape.nt, 0, st>>>(from, to, v.g.n, nan_where, nan_value); \
+        vkop::softmax_row_kernel<T, V, MAX_ONLY><<<rows, p.shape.nt, 0, st>>>(from, to, v.g.n, nan_where, nan_value); \
         return launched("softmax_row_kernel");                                                          \
     }
             VKOP_ROW(1) VKOP_ROW(2) VKOP_ROW(3) VKOP_ROW(4)
@@ -399,7 +401,7 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
         const uint64_t threads = std::max<uint64_t>(static_cast<uint64_t>(p.g) * p.shape.nt, static_cast<uint64_t>(gs) * vkop::kSoftmaxScaleThreads);
         return in_slices(v.g.outer, threads, [&](uint64_t row0, uint32_t rows) {
             const T *from = in + row0 * v.g.n;
-            T *to = out + row0 * v.g.n;
+            T *to = out + row0 * out_row;
             auto *row_stats = stats + row0 * p.g;
             bool done = false;
 #define VKOP_STATS(NT, V)                                                                                \
@@ -412,6 +414,10 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
             else { VKOP_STATS(1024, 4) }
 #undef VKOP_STATS
             if (!done) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_stats_kernel for %d x %d", p.shape.nt, p.shape.v);
+            if constexpr (MAX_ONLY) {
+                vkop::softmax_fold_max_kernel<T><<<rows, vkop::kSoftmaxScaleThreads, 0, st>>>(to, row_stats, p.g);
+                return launched("softmax_stats_kernel / softmax_fold_max_kernel");
+            }
 #define VKOP_SCALE(V) \
     if (loads == V)   \
         vkop::softmax_scale_kernel<T, V><<<rows * gs, vkop::kSoftmaxScaleThreads, 0, st>>>(from, to, row_stats, v.g.n, p.g, gs, nan_where, nan_value);
@@ -421,6 +427,22 @@ int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, f
             return launched("softmax_stats_kernel / softmax_scale_kernel");
         });
     }
+    default:
+        return fail(VKOP_HIP_ERR_UNSUPPORTED, "not a plan of last-axis rows");
+    }
+}
+
+template <typename T>
+int softmax_impl(const T *in, T *out, const View &v, int dtype, int nan_where, float nan_value, void *ws,
+                 size_t ws_bytes, hipStream_t st) {
+    const SoftmaxPlan p = plan_softmax(v, dtype);
+    const uint32_t lines = v.g.outer * v.g.inner;
+    switch (p.kind) {
+    case SoftmaxPlan::kThread:
+    case SoftmaxPlan::kGroup:
+    case SoftmaxPlan::kRow:
+    case SoftmaxPlan::kChunked:
+        return softmax_rows<T, false>(in, out, v, p, nan_where, nan_value, ws, ws_bytes, st);
     case SoftmaxPlan::kLinesRegs: {
         return launch_lines(in, out, v, p, false, nan_where, nan_value, st);
     }
@@ -1031,7 +1053,8 @@ int softmax_reduce_max_impl(const T *in, T *out, const View &v, void *ws, size_t
     if (p.kind == SoftmaxPlan::kLinesRegs) {
         return launch_lines(in, out, v, p, true, 0, 0.f, st);
     }
-    if (v.g.n <= static_cast<uint32_t>(vkop::kStridedMaxN)) {
+    if (v.g.inner == 1 && p.kind != SoftmaxPlan::kGeneralLines) return softmax_rows<T, true>(in, out, v, p, 0, 0.f, ws, ws_bytes, st);
+    if (p.kind == SoftmaxPlan::kStridedRegs) {
         launch_strided_reg<T, true>(in, out, v, 0, 0.f, st);
         return launched("softmax_strided_reg_kernel");
     }
@@ -1052,7 +1075,7 @@ int softmax_reduce_max_impl(const T *in, T *out, const View &v, void *ws, size_t
             <<<tiles * p.g, vkop::kStridedTileThreads, 0, st>>>(in, out, cstats, v.g, p.ti_shift, p.g, p.per, 0, 0.f);
         return launched("softmax_strided_tile_kernel (split, max)");
     }
-    // long rows: the line statistics, then exp_accurate(0) / S per line
+    // rows of more than 2^25 elements: the line statistics, then exp_accurate(0) / S per line
     const size_t need = kTicketBytes + align_up(static_cast<size_t>(lines) * sizeof(vkop::LineStats));
     if (ws == nullptr || ws_bytes < need)
         return fail(VKOP_HIP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", ws_bytes, need);
@@ -1575,9 +1598,9 @@ int vkop_hip_rows_plan(int dtype, const int *shape, int ndim, int axis, int k, i
 size_t vkop_hip_softmax_reduce_max_workspace_bytes(int dtype, const int *shape, int ndim, int axis) {
     View v;
     if (check_dtype(dtype) || make_view(shape, ndim, axis, &v)) return 0;
-    if (v.g.n <= static_cast<uint32_t>(vkop::kStridedMaxN)) return 0;
-    if (v.g.inner != 1) return plan_softmax(v, dtype).workspace;
-    return kTicketBytes + align_up(static_cast<size_t>(v.g.outer) * v.g.inner * sizeof(vkop::LineStats));
+    const SoftmaxPlan p = plan_softmax(v, dtype);
+    if (p.kind != SoftmaxPlan::kGeneralLines) return p.workspace;
+    return kTicketBytes + align_up(static_cast<size_t>(v.g.outer) * sizeof(vkop::LineStats));
 }
 
 int vkop_hip_softmax_reduce_max(const void *in, void *out, int dtype, const int *shape, int ndim, int axis,
