@@ -238,6 +238,20 @@ def test_native_front_end_takes_any_object_with_get_as_workspace():
             ops.softmax(t, out=out, workspace=Wrong(answer))
 
 
+@pytest.mark.parametrize("shape,axis", [((0, 5000, 7), 1), ((3, 5000, 0), 1), ((3, 300, 0), 1), ((0, 200000), 1), ((0, 100), 1),
+                                        ((3, 0), 1), ((3, 0, 5), 1), ((0, 1000, 5), 1), ((0,), 0), ((2, 0, 3, 4), 2)])
+def test_tensors_without_elements(lib, shape, axis):
+    """No scratch is asked for and nothing launched (a plan that divided by its number of tiles ended the process)."""
+    for dt in (capi.F32, capi.F16):
+        assert capi.softmax_workspace_bytes(dt, shape, axis) == 0
+        assert capi.softmax_reduce_max_workspace_bytes(dt, shape, axis) == 0
+        capi.softmax(0, 0, dt, shape, axis)
+        if shape[axis] != 0:
+            capi.softmax_reduce_max(0, 0, dt, shape, axis)
+            capi.topk(0, 0, 0, dt, shape, axis, min(5, shape[axis]))
+            capi.softmax_topk(0, 0, 0, 0, dt, shape, axis, min(5, shape[axis]))
+
+
 def test_native_front_end_knows_what_it_was_built_for(monkeypatch):
     torch = pytest.importorskip("torch")
     from vkop_amd import ops

@@ -256,6 +256,7 @@ bool plan_lines(const View &v, uint32_t vec, SoftmaxPlan *p) {
 
 SoftmaxPlan plan_softmax(const View &v, int dtype) {
     SoftmaxPlan p;
+    if (v.elems == 0) return p;  // (nothing to launch; no tiles or rows to divide by)
     const uint32_t vec = dtype == VKOP_HIP_F32 ? 4u : 8u;
     const uint32_t n = v.g.n, rows = v.g.outer;
     if (v.g.inner != 1) {
@@ -1598,6 +1599,7 @@ int vkop_hip_rows_plan(int dtype, const int *shape, int ndim, int axis, int k, i
 size_t vkop_hip_softmax_reduce_max_workspace_bytes(int dtype, const int *shape, int ndim, int axis) {
     View v;
     if (check_dtype(dtype) || make_view(shape, ndim, axis, &v)) return 0;
+    if (v.elems == 0) return 0;
     const SoftmaxPlan p = plan_softmax(v, dtype);
     if (p.kind != SoftmaxPlan::kGeneralLines) return p.workspace;
     return kTicketBytes + align_up(static_cast<size_t>(v.g.outer) * sizeof(vkop::LineStats));
