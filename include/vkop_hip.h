@@ -260,10 +260,9 @@ int vkop_hip_tune(const char *name, int value);
  * threads per workgroup, 128-bit loads per thread and workgroups per row of the
  * streaming kernel (a second kernel per row follows when chunks > 1); all three
  * are 0 when the radix select or the general one-workgroup-per-line kernels would
- * run.  The plain top-k takes the same shape, except on a row that one workgroup
- * of this kernel holds and that has fewer 16-byte vectors than k + 1 (smallest
- * first: fewer than 2 (k + 1)): it runs an exact select there.  Any out pointer
- * may be NULL. */
+ * run.  The plain top-k takes the same shape, except on rows that one workgroup
+ * of this kernel holds but an exact select ranks sooner (many short rows for a large
+ * k): it runs that there.  Any out pointer may be NULL. */
 int vkop_hip_rows_plan(int dtype, const int *shape, int ndim, int axis, int k,
                        int *threads, int *loads, int *chunks);
 

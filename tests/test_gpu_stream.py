@@ -578,6 +578,26 @@ def test_smallest_first_on_reversed_elements(ops, n, k, dtype):
         assert np.array_equal(host(v).view(bits), ev.view(bits))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,n,k", [(1023, 400, 44), (1024, 400, 57), (4096, 801, 75), (256, 1000, 150), (257, 1000, 150), (300, 1500, 219),
+                                      (300, 1505, 219), (256, 2400, 271), (257, 2400, 271), (5, 1500, 393), (9, 999, 249), (9, 1031, 249)])
+def test_rows_of_one_workgroup_or_of_an_exact_select(ops, rows, n, k, dtype):
+    """Rows on either side of the line between the one-workgroup kernel and the exact select, both directions, spread out and
+    with values equal en masse."""
+    rng = np.random.default_rng(rows + n + k)
+    bits = np.uint16 if dtype == np.float16 else np.uint32
+    for step in (0, 0.25):
+        x = rng.standard_normal((rows, n)).astype(np.float32)
+        if step:
+            x = np.round(x / np.float32(step)) * np.float32(step)
+        x = x.astype(dtype)
+        x[1, n // 2] = np.nan
+        for largest in (True, False):
+            v, ix = ops.topk(dev(x), k, largest=largest)
+            ev, eix = oracle.topk(x, k, largest=largest)
+            assert np.array_equal(host(ix), eix) and np.array_equal(host(v).view(bits), ev.view(bits)), (step, largest)
+
+
 @pytest.mark.parametrize("n,k", [(1000, 5), (4096, 64), (8400, 300), (8401, 300), (32000, 40), (50257, 200), (100000, 600), (131076, 1025)])
 def test_signalling_nan_ranks_as_nan(ops, n, k):
     """A NaN is a NaN whether it is quiet or signalling: last among the smallest, first among the largest, of either sign,

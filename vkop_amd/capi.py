@@ -330,8 +330,8 @@ def measure_stages(stages):
 
 def measure_path(dtype, shape, axis, k):
     """Which kernels a fused call on this tensor takes: 4 = one wave per row, 3 = scan + gather + rank, 2 = scan + pick,
-    1 = chunk (+ merge), 0 = radix select or general kernels.  The plain top-k takes the same ones, except where path 1 has
-    fewer 16-byte vectors a row than k + 1 (smallest first: than 2 (k + 1)): an exact select.  Benchmarks and tests only."""
+    1 = chunk (+ merge), 0 = radix select or general kernels.  The plain top-k takes the same ones, except where an
+    exact select is faster than path 1 (many short rows, large k).  Benchmarks and tests only."""
     arr, nd = _shape(shape)
     return lib().vkop_hip_measure_path(dtype, arr, nd, axis, int(k))
 

@@ -944,6 +944,27 @@ int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, 
 }
 
 // ------------------------------------------------------------------ top-k ----
+// Rows that one workgroup of the chunk kernel holds, but that a workgroup's exact select (topk_lines_kernel) ranks sooner.
+// (vec: elements a vector.)  The line lies where the two were the same, within 10 % on either side, over 375 shapes of normal rows
+// (8 to 30000 of 200 to 20000 elements, f32 and f16, 0.4 to 8 vectors a place, either direction); us a call, chunk kernel / select:
+//  * fewer vectors than places, whose maxima bound nothing, in rows that the list does not hold whole: [8,1500] f16 k = 196 29 / 19,
+//    [1500,1500] 167 / 28;
+//  * smallest first up to two vectors a place, where the select ran before and its time does not depend on the data;
+//  * 256 threads, short rows by the thousand, which the select reads again from the cache: [6000,400] f32 k = 44 40 / 30, k = 104
+//    52 / 36, [30000,800] f16 k = 104 275 / 207; but [300,400] f32 k = 104 9.3 / 10.8, [1500,800] f16 k = 75 18 / 20;
+//  * 512 and 1024 threads, more rows than CUs (a workgroup each at a time) of few elements for so many threads: [300,1500] f32 k = 219
+//    18.5 / 17.3, [1500,2400] k = 132 50 / 28, [6000,5564] f16 k = 290 339 / 194; but [64,800] f32 k = 152 11.4 / 13.6, [300,4000]
+//    k = 221 18 / 27, [1500,8000] k = 249 55 / 77.
+bool select_is_faster(const View &v, int k, const RowsCfg &c, uint32_t vec, bool largest) {
+    const uint32_t n = v.g.n, rows = v.g.outer;
+    if (c.g != 1 || c.nt < 256) return false;
+    const uint32_t vectors = (n + vec - 1) / vec, places = static_cast<uint32_t>(k) + 1u;
+    if (vectors < places && n > static_cast<uint32_t>(vkop::kLocalCap)) return true;
+    if (!largest && vectors < 2u * places) return true;
+    if (c.nt == 256) return rows >= 1024 && n < (vec == 4 || rows >= 4096 ? 1000u : 600u);
+    return rows > 256 && (c.nt == 512 ? n <= 4500 && rows >= n / 5 : n <= 6500 && rows >= n / 11);
+}
+
 template <typename T>
 int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, int largest, int sorted, int dtype, void *ws,
               size_t ws_bytes, hipStream_t st) {
@@ -960,12 +981,7 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
     if (!largest && !sorted && sc.g2 != 0) sc = ScanCfg{};
     RowsCfg c = (routed && !sc.ok) ? choose_rows_cfg(v, k, dtype) : RowsCfg{};
     if (!largest && (c.g != 1 || c.nt < 256 || c.cap > static_cast<uint32_t>(vkop::kLocalCap))) c = RowsCfg{};
-    // Fewer vectors than places: their maxima bound nothing, and every row would take that kernel's second list
-    // ([2000,1462] f16 k = 225: 225 us, 32 with a workgroup's exact select a row).  Smallest first, where that
-    // select ran before, it stays the faster one up to twice as many ([2000,600] f32 k = 100: 15.3 against 17.9 us).
-    // (The fused call and vkop_hip_rows_plan do not know this rule.)
-    const uint32_t vectors = (v.g.n + 16 / sizeof(T) - 1) / (16 / sizeof(T));
-    if (c.ok && g_rows_path.load() != 1 && vectors < (largest ? 1u : 2u) * (static_cast<uint32_t>(k) + 1u)) c = RowsCfg{};
+    if (c.ok && g_rows_path.load() != 1 && select_is_faster(v, k, c, 16 / sizeof(T), largest != 0)) c = RowsCfg{};
     const BigKCfg b = (c.ok || sc.ok) ? BigKCfg{} : choose_bigk_cfg(v, k, dtype);
     if (sc.ok || c.ok || b.ok) {
         const RowsLayout l = rows_layout(v, c, b, sc);
