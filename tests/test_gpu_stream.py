@@ -580,10 +580,10 @@ def test_smallest_first_on_reversed_elements(ops, n, k, dtype):
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
 @pytest.mark.parametrize("rows,n,k", [(1023, 400, 44), (1024, 400, 57), (4096, 801, 75), (256, 1000, 150), (257, 1000, 150), (300, 1500, 219),
-                                      (300, 1505, 219), (256, 2400, 271), (257, 2400, 271), (5, 1500, 393), (9, 999, 249), (9, 1031, 249)])
+                                      (300, 1505, 219), (257, 1576, 393), (300, 1577, 394), (300, 1681, 394), (256, 2400, 271), (257, 2400, 271), (5, 1500, 393), (9, 999, 249), (9, 1031, 249), (9, 1383, 345), (1025, 8196, 23)])
 def test_rows_of_one_workgroup_or_of_an_exact_select(ops, rows, n, k, dtype):
     """Rows on either side of the line between the one-workgroup kernel and the exact select, both directions, spread out and
-    with values equal en masse."""
+    with values equal en masse; and the fused call, whose line lies elsewhere."""
     rng = np.random.default_rng(rows + n + k)
     bits = np.uint16 if dtype == np.float16 else np.uint32
     for step in (0, 0.25):
@@ -596,6 +596,15 @@ def test_rows_of_one_workgroup_or_of_an_exact_select(ops, rows, n, k, dtype):
             v, ix = ops.topk(dev(x), k, largest=largest)
             ev, eix = oracle.topk(x, k, largest=largest)
             assert np.array_equal(host(ix), eix) and np.array_equal(host(v).view(bits), ev.view(bits)), (step, largest)
+        x[1, n // 2] = 0.5
+        v, ix = ops.softmax_topk(dev(x), k)
+        v, ix = host(v), host(ix)
+        ev, eix, ep = oracle.softmax_topk(x, k, return_probs=True)
+        assert (half_ulp_diff(v, ev).max() <= 1) if dtype == np.float16 else (ulp_diff(v, ev).max() <= 2), step
+        for r in range(0, rows, 37):
+            check_fused_invariants(x[r].astype(np.float32), v[r].astype(np.float32), ix[r])
+            if well_separated_cut(ep[r].astype(np.float32), x[r].astype(np.float32), k, 4 if dtype == np.float32 else 1 << 14):
+                assert np.array_equal(ix[r], eix[r]), (step, r)
 
 
 @pytest.mark.parametrize("n,k", [(1000, 5), (4096, 64), (8400, 300), (8401, 300), (32000, 40), (50257, 200), (100000, 600), (131076, 1025)])

@@ -1024,6 +1024,15 @@ FusedPlan plan_fused(const View &v, int k, int dtype, int largest, bool want_pro
     if (want_probs) return p;  // the softmax tensor is written by the general kernels
     if (largest) p.scan = choose_scan_cfg(v, k, dtype);
     if (largest && !p.scan.ok) p.rows = choose_rows_cfg(v, k, dtype);
+    // A k whose places are about as many as a row's vectors, on more rows than CUs or in rows that the list does not hold whole:
+    // every row would take the one-workgroup kernel's second list; the general kernels (line statistics, an exact select of probabilities) rank it sooner.  us a call:
+    // [300,1500] f32 k = 393 76 / 26, f16 k = 196 62 / 35, [1500,800] f32 k = 209 74 / 27, [8,1500] f32 k = 393 38 / 24; but at
+    // 1.3 vectors a place [300,2400] f16 k = 229 30 / 48, and [64,800] f32 k = 209 14 / 18.
+    const uint32_t vec = dtype == VKOP_HIP_F32 ? 4u : 8u, places = static_cast<uint32_t>(k) + 1u;
+    if (p.rows.ok && g_rows_path.load() != 1 && p.rows.nt >= 512 && p.rows.g == 1 &&
+        (v.g.outer > 256 || v.g.n > static_cast<uint32_t>(vkop::kLocalCap)) &&
+        (v.g.n + vec - 1) / vec <= places + places / 16)
+        p.rows = RowsCfg{};
     if (!p.scan.ok && !p.rows.ok) p.big = choose_bigk_cfg(v, k, dtype);
     return p;
 }
@@ -1575,7 +1584,7 @@ int vkop_hip_measure_path(int dtype, const int *shape, int ndim, int axis, int k
     if (choose_tiny_loads(v, k, dtype) != 0) return 4;
     const ScanCfg sc = choose_scan_cfg(v, k, dtype);
     if (sc.ok) return sc.g2 != 0 ? 3 : 2;
-    if (choose_rows_cfg(v, k, dtype).ok) return 1;
+    if (plan_fused(v, k, dtype, 1, false).rows.ok) return 1;
     return 0;
 }
 
@@ -1605,7 +1614,7 @@ int vkop_hip_rows_plan(int dtype, const int *shape, int ndim, int axis, int k, i
         if (chunks != nullptr) *chunks = static_cast<int>(sc.g);
         return VKOP_HIP_OK;
     }
-    const RowsCfg c = k >= 1 ? choose_rows_cfg(v, k, dtype) : RowsCfg{};
+    const RowsCfg c = k >= 1 ? plan_fused(v, k, dtype, 1, false).rows : RowsCfg{};
     if (threads != nullptr) *threads = c.ok ? c.nt : 0;
     if (loads != nullptr) *loads = c.ok ? c.v : 0;
     if (chunks != nullptr) *chunks = c.ok ? static_cast<int>(c.g) : 0;
