@@ -947,9 +947,10 @@ int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, 
 // Rows that one workgroup of the chunk kernel holds, but that a workgroup's exact select (topk_lines_kernel) ranks sooner.
 // (vec: elements a vector.)  The line lies where the two were the same, within 10 % on either side, over 375 shapes of normal rows
 // (8 to 30000 of 200 to 20000 elements, f32 and f16, 0.4 to 8 vectors a place, either direction); us a call, chunk kernel / select:
-//  * fewer vectors than places, whose maxima bound nothing, in rows that the list does not hold whole: [8,1500] f16 k = 196 29 / 19,
-//    [1500,1500] 167 / 28;
-//  * smallest first up to two vectors a place, where the select ran before and its time does not depend on the data;
+//  * about as many vectors as places, or fewer, whose maxima bound nothing, in rows that the list does not hold whole: [8,1500] f16
+//    k = 196 29 / 19, [1500,1500] 167 / 28;
+//  * smallest first up to two vectors a place, where the select ran before and its time does not depend on the data, and by the
+//    thousand of rows just past what 256 threads hold: [3300,8196] k = 23 f16 189 / 124, f32 132 / 121, [3300,10094] f16 191 / 161;
 //  * 256 threads, short rows by the thousand, which the select reads again from the cache: [6000,400] f32 k = 44 40 / 30, k = 104
 //    52 / 36, [30000,800] f16 k = 104 275 / 207; but [300,400] f32 k = 104 9.3 / 10.8, [1500,800] f16 k = 75 18 / 20;
 //  * 512 and 1024 threads, more rows than CUs (a workgroup each at a time) of few elements for so many threads: [300,1500] f32 k = 219
@@ -959,8 +960,9 @@ bool select_is_faster(const View &v, int k, const RowsCfg &c, uint32_t vec, bool
     const uint32_t n = v.g.n, rows = v.g.outer;
     if (c.g != 1 || c.nt < 256) return false;
     const uint32_t vectors = (n + vec - 1) / vec, places = static_cast<uint32_t>(k) + 1u;
-    if (vectors < places && n > static_cast<uint32_t>(vkop::kLocalCap)) return true;
+    if (vectors <= places + places / 16 && n > static_cast<uint32_t>(vkop::kLocalCap)) return true;
     if (!largest && vectors < 2u * places) return true;
+    if (!largest && c.nt >= 512 && rows > 1024 && n < (vec == 8 && n % 8 == 0 ? 9000u : 11000u)) return true;
     if (c.nt == 256) return rows >= 1024 && n < (vec == 4 || rows >= 4096 ? 1000u : 600u);
     return rows > 256 && (c.nt == 512 ? n <= 4500 && rows >= n / 5 : n <= 6500 && rows >= n / 11);
 }
