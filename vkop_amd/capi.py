@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libvkop_hip.so")
 # the same library built with the benchmark's hook (vkop_hip_measure_stages): bench.py's per-kernel legs load
 # this one instead, in a process of their own (use_bench_library() before the first lib())
 BENCH_LIB_PATH = os.path.join(_HERE, "libvkop_hip_bench.so")
-BENCH_ONLY = ("vkop_hip_measure_stages",)
+BENCH_ONLY = ("vkop_hip_measure_stages", "vkop_hip_measure_polls")
 HEADER_PATH = os.path.join(ROOT, "include", "vkop_hip.h")
 
 OK, ERR_INVALID, ERR_DEVICE, ERR_WORKSPACE, ERR_UNSUPPORTED = 0, 1, 2, 3, 4
@@ -143,6 +143,7 @@ def lib():
         "vkop_hip_softmax_reduce_max": (i, [vp, vp, i, ip, i, i, vp, sz, vp]),
         "vkop_hip_tune": (i, [ctypes.c_char_p, i]),
         "vkop_hip_measure_stages": (i, [i]),
+        "vkop_hip_measure_polls": (i, [i]),
         "vkop_hip_measure_path": (i, [i, ip, i, i, i]),
         "vkop_hip_rows_plan": (i, [i, ip, i, i, i, ip, ip, ip]),
     }

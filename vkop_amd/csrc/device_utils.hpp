@@ -97,10 +97,16 @@ __device__ __forceinline__ float min3(float a, float b, float c) {
     asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
-// Larger halves of two pairs, quiet NaN dropped (signalling: as above).
+// Larger and smaller halves of two pairs, quiet NaN dropped (signalling: as above).
 __device__ __forceinline__ uint32_t max_half2(uint32_t a, uint32_t b) {
     uint32_t r;
     asm("v_pk_max_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+
+__device__ __forceinline__ uint32_t min_half2(uint32_t a, uint32_t b) {
+    uint32_t r;
+    asm("v_pk_min_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
 

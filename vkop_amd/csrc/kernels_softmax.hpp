@@ -10,7 +10,8 @@
 //                           chunk, the second combines a row's chunk results and
 //                           writes exp(x - M) / S for its chunk.  The second
 //                           read of the input comes from the Infinity Cache for
-//                           tensors that fit it.
+//                           tensors that fit it.  (Most such tensors, not in place: both in
+//                           one launch and one read, kernels_joined.hpp.)
 //   softmax_thread_kernel   rows of fewer elements than a vector.
 //   (each also without the tensor: the row's largest probability alone, from the same sum)
 // Strided lines (another axis, long lines):
@@ -22,7 +23,7 @@
 //                           contiguous inner axis; the line's elements stay in
 //                           registers, so the input is read once.
 // All of them produce what kernels_general.hpp defines: terms exp_accurate(x - M),
-// the sum in double, one rounding of term * (1 / sum).  The chunked variant sums
+// the sum in double, one rounding of term * (1 / sum).  The chunked variants sum
 // hardware-exp terms (argument scaled with a two-part log2 e, so the scaling adds
 // no bias); the sum's relative error of ~1e-8 is far below a float ulp.
 #pragma once
@@ -293,50 +294,69 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_thread_kernel(co
 }
 
 // ---- chunked rows: statistics ---------------------------------------------------------
-// Launch: rows * G workgroups; per = NT * V * VEC elements a chunk, whose vectors start on any
-// element (n >= VEC).  A row that is no whole number of vectors has its last one moved back to end
-// with the row; the leading elements it repeats -- of the chunk before, possibly -- count for the
-// chunk's maximum and minimum, which does no harm, and for nothing else.
-// The loads are ordinary ones: the scale kernel reads the same bytes again and finds them in the
-// Infinity Cache.
+// A chunk is NT * V * VEC elements of a row, what a workgroup of NT threads holds: vector i of thread tid is elements
+// ((chunk * V + i) * NT + tid) * VEC and on, from any element (n >= VEC).  A row that is no whole
+// number of vectors has its last one moved back to end with the row; the leading elements it repeats -- of the chunk
+// before, possibly -- count for the chunk's maximum and minimum, which does no harm, and for nothing else.
+template <typename T, int NT, int V> struct Chunk {
+    static constexpr uint32_t VEC = Vec128<T>::N;
+    Vec128<T> q[V];
+    static __device__ __forceinline__ uint32_t first(uint32_t chunk) { return (chunk * (V * NT) + threadIdx.x) * VEC; }
+    // KEPT: ordinary loads, for what is read again; else non-temporal ones
+    template <bool KEPT> __device__ __forceinline__ void load(const T *rowp, uint32_t chunk, uint32_t n) {
+        const uint32_t e_first = first(chunk);
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+            const uint32_t at = min(e_first + static_cast<uint32_t>(i) * (NT * VEC), n - VEC) * static_cast<uint32_t>(sizeof(T));  // (bytes: below 2^27)
+            const T *p = reinterpret_cast<const T *>(reinterpret_cast<const char *>(rowp) + at);
+            q[i].v = KEPT ? load16_any(p) : load16_stream(p);
+        }
+    }
+};
+template <int NT> struct ChunkScratch {
+    static constexpr int NW = NT / kWave;
+    static_assert(NW <= kSoftmaxRowWavesMax && kSoftmaxRowWavesMax % NW == 0, "waves a workgroup");
+    float m[NW], mn[NW];
+    double s[NW];
+    uint32_t n[NW];
+};
+// The chunk's statistics, in every lane of the first wave.  All threads call; two barriers.
 template <typename T, int NT, int V>
-__global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__ in, ChunkStat *__restrict__ stats,
-                                                           uint32_t n, uint32_t G) {
+__device__ __forceinline__ ChunkStat chunk_stats(const Chunk<T, NT, V> &ch, uint32_t chunk, uint32_t n, ChunkScratch<NT> &sh) {
     constexpr uint32_t VEC = Vec128<T>::N;
     constexpr int NW = NT / kWave;
-    __shared__ float fscratch[NW];
-    __shared__ float fscratch2[NW];
-    __shared__ double dscratch[NW];
-    __shared__ uint32_t uscratch[NW];
     const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const uint32_t row = blockIdx.x / G, chunk = blockIdx.x - row * G;
-    const uint32_t e_first = chunk * (NT * V * VEC) + tid * VEC;
-    const T *rowp = in + static_cast<size_t>(row) * n;
-    Vec128<T> q[V];
-#pragma unroll
-    for (int i = 0; i < V; i++) q[i].load_any(rowp + min(e_first + static_cast<uint32_t>(i) * NT * VEC, n - VEC));
+    const uint32_t e_first = ch.first(chunk);
     // Maximum and minimum in one pass and one reduction.
-    float m = -INFINITY, mn = INFINITY;
+    float m = -INFINITY, mn = INFINITY;  // (NaN is dropped)
+    if constexpr (sizeof(T) == 2) {
+        uint32_t pm = 0xFC00FC00u, pn = 0x7C007C00u;
 #pragma unroll
-    for (int i = 0; i < V; i++) {
+        for (int i = 0; i < V; i++) {
+            const uint4 &v = ch.q[i].v;
+            pm = max_half2(max_half2(pm, max_half2(v.x, v.y)), max_half2(v.z, v.w));
+            pn = min_half2(min_half2(pn, min_half2(v.x, v.y)), min_half2(v.z, v.w));
+        }
+        auto half = [](uint32_t h) { return __half2float(__ushort_as_half(static_cast<uint16_t>(h))); };
+        m = fmaxf(half(pm & 0xFFFFu), half(pm >> 16));
+        mn = fminf(half(pn & 0xFFFFu), half(pn >> 16));
+    } else {
 #pragma unroll
-        for (int c = 0; c < static_cast<int>(VEC); c += 2) {
-            m = max3(m, q[i].get(c), q[i].get(c + 1));  // (drops NaN)
-            mn = min3(mn, q[i].get(c), q[i].get(c + 1));
+        for (int i = 0; i < V; i++) {
+            m = max3(max3(m, ch.q[i].get(0), ch.q[i].get(1)), ch.q[i].get(2), ch.q[i].get(3));
+            mn = min3(min3(mn, ch.q[i].get(0), ch.q[i].get(1)), ch.q[i].get(2), ch.q[i].get(3));
         }
     }
     const float own_min = mn;
     m = group_max<kWave>(m);
     mn = -group_max<kWave>(-mn);
-    if constexpr (NW > 1) {
-        if (lane == 0) {
-            fscratch[wave] = m;
-            fscratch2[wave] = mn;
-        }
-        __syncthreads();
-        m = group_max<kSoftmaxRowWavesMax>(fscratch[lane % NW]);
-        mn = -group_max<kSoftmaxRowWavesMax>(-fscratch2[lane % NW]);
+    if (lane == 0) {
+        sh.m[wave] = m;
+        sh.mn[wave] = mn;
     }
+    __syncthreads();
+    m = group_max<kSoftmaxRowWavesMax>(sh.m[lane % NW]);
+    mn = -group_max<kSoftmaxRowWavesMax>(-sh.mn[lane % NW]);
     // reference of the chunk's sum: its maximum, or 0 when that is not finite
     // (then every term is 0, inf or NaN, and NaN / inf must reach the sum)
     const float ref = (m > -INFINITY && m < INFINITY) ? m : 0.f;
@@ -352,11 +372,11 @@ __global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__
     auto sum = [&](auto full_tag) {
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            const uint32_t e0 = e_first + static_cast<uint32_t>(i) * NT * VEC;
+            const uint32_t e0 = e_first + static_cast<uint32_t>(i) * (NT * VEC);
             const uint32_t dup = decltype(full_tag)::value || e0 <= n - VEC ? 0u : min(e0 - (n - VEC), VEC);
 #pragma unroll
             for (int c = 0; c < static_cast<int>(VEC); c++) {
-                const float x = q[i].get(c);
+                const float x = ch.q[i].get(c);
                 const double t = static_cast<double>(fast_term_unbiased(x, ref));
                 const bool counts = decltype(full_tag)::value || static_cast<uint32_t>(c) >= dup;
                 acc += counts ? t : 0.0;
@@ -370,21 +390,33 @@ __global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__
     if (apart) acc -= static_cast<double>(copies) * static_cast<double>(fast_term_unbiased(mn, ref));
     acc = group_sum<kWave>(acc);
     copies = wave_sum(copies);
-    if constexpr (NW > 1) {
-        if (lane == 0) {
-            dscratch[wave] = acc;
-            uscratch[wave] = copies;
-        }
-        __syncthreads();
-        acc = dscratch[0];
-        copies = uscratch[0];
+    if (lane == 0) {
+        sh.s[wave] = acc;
+        sh.n[wave] = copies;
+    }
+    __syncthreads();
+    if (tid < static_cast<uint32_t>(kWave)) {
+        acc = sh.s[0];
+        copies = sh.n[0];
 #pragma unroll
         for (int w = 1; w < NW; w++) {  // fixed order: run-to-run stable
-            acc += dscratch[w];
-            copies += uscratch[w];
+            acc += sh.s[w];
+            copies += sh.n[w];
         }
     }
-    if (tid == 0) stats[blockIdx.x] = ChunkStat{acc, m, ref, mn, copies};
+    return ChunkStat{acc, m, ref, mn, copies};
+}
+
+// Launch: rows * G workgroups.  The scale kernel reads the same bytes again and finds them in the Infinity Cache.
+template <typename T, int NT, int V>
+__global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__ in, ChunkStat *__restrict__ stats, uint32_t n,
+                                                           uint32_t G) {
+    __shared__ ChunkScratch<NT> sh;
+    const uint32_t row = blockIdx.x / G, chunk = blockIdx.x - row * G;
+    Chunk<T, NT, V> ch;
+    ch.template load<true>(in + static_cast<size_t>(row) * n, chunk, n);
+    const ChunkStat st = chunk_stats(ch, chunk, n, sh);
+    if (threadIdx.x == 0) stats[blockIdx.x] = st;
 }
 
 // A row's maximum and the reciprocal of its sum (in thread 0) from its G chunks.  Up to 64 of them are combined by the first

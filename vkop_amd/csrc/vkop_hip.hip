@@ -15,6 +15,7 @@
 #include "kernels_general.hpp"
 #include "kernels_rows.hpp"
 #include "rows_launch.hpp"
+#include "kernels_joined.hpp"
 #include "kernels_softmax.hpp"
 #include "kernels_bigk.hpp"
 #include "kernels_nms.hpp"
@@ -134,9 +135,16 @@ std::atomic<int> g_rows_threads{0}, g_rows_loads{0}, g_rows_chunks{0}, g_rows_fu
 #ifdef VKOP_BENCH_HOOKS
 std::atomic<int> g_rows_stages{3};
 inline int measured_stages() { return g_rows_stages.load(); }
+std::atomic<uint32_t> g_joined_polls{100};
+inline uint32_t joined_polls() { return g_joined_polls.load(); }
 #else
 inline int measured_stages() { return 3; }
+// How often a workgroup of softmax_joined_kernel looks for its row's other chunks before it reads what it misses: a look takes
+// about a microsecond, the wait for a row whose workgroups run a few of them.
+constexpr uint32_t joined_polls() { return 100; }
 #endif
+// (what tells the records of a call of softmax_joined_kernel from whatever the workspace held before)
+std::atomic<uint32_t> g_joined_calls{0};
 
 // The per-row arrival counters of the one-kernel top-k variant sit at a fixed
 // place, the first kTicketRows words of every workspace, whatever the operator
@@ -170,6 +178,7 @@ struct SoftmaxPlan {
     enum Kind { kGeneralLines, kGeneralStrided, kThread, kGroup, kRow, kChunked, kLinesRegs, kStridedRegs, kStridedTile } kind = kGeneralLines;
     RowShape shape{0, 0};  // kChunked; kGroup: lanes a row and vectors a lane; kRow: threads and vectors a thread
     uint32_t g = 1, per = 0;
+    bool joined = false;  // kChunked: in one launch where the tensors do not overlap
     uint32_t lines_k = 0, lines_p = 0, lines_w = 0;  // kLinesRegs: LinesLaunch
     uint32_t ti_shift = 0;  // kStridedTile: log2 of the lines a tile
     size_t workspace = 0;
@@ -254,6 +263,31 @@ bool plan_lines(const View &v, uint32_t vec, SoftmaxPlan *p) {
     return true;
 }
 
+// The shape of softmax_joined_kernel for rows of a tensor, false where the pair of kernels is the faster one: 512 threads of as
+// many vectors (eight floats', four halves') as leave 150 workgroups, a row's in at most 16 chunks, or 8 of smaller
+// ones and of fewer than 32 rows of halves -- every workgroup of a row reads the records of all, again and again until they are there.  us, the pair / this: f32
+// [16,262144] 13.4 / 12.8 with 16 chunks, [16,65536] 7.8 / 8.0 with 8 in 128 workgroups, 9.1 with 16; [8,262144] 9.6 / 10.7 with
+// 32; [32,33001] 8.5 / 7.7; f16 [32,200000] 14.9 / 12.9, [32,65536] 8.3 / 7.9, [64,262144] 25.2 / 24.6,
+// [16,262144] 10.5 / 11.3.
+// More workgroups than the chip takes at once, and a last chunk left mostly empty: 256 threads of ten (five) vectors, in at most
+// 20 chunks, where they leave 3 % less empty.  us, 512 threads / 256: f32 [500,50257] 49.5 / 43.7, [64,200000] 28.5 / 24.8; f16
+// [500,33001] 30.1 / 24.5, [500,100003] 65.9 / 57.4; at once, [64,50257] f32 10.9 / 12.9.
+bool plan_joined(const View &v, uint32_t vec, RowShape *shape) {
+    const uint64_t n = v.g.n, rows = v.g.outer;
+    const int half = vec == 8 ? 2 : 1;
+    auto chunks = [&](const RowShape &c) { return (n + c.nt * c.v * vec - 1) / (c.nt * c.v * vec); };
+    auto held = [&](const RowShape &c) { return chunks(c) * c.nt * c.v; };
+    const RowShape wide{512, 8 / half}, fitted{256, 10 / half};
+    RowShape s = wide;
+    while (s.v > 2 / half && rows * chunks(s) < 150) s.v /= 2;
+    if (rows * chunks(s) < 150) return false;
+    uint32_t most = s.v == wide.v && (half == 1 || rows >= 32) ? 16 : 8;
+    if (rows * chunks(wide) > 256 && held(fitted) * 103 < held(wide) * 100) s = fitted, most = most == 16 ? 20 : 8;
+    if (chunks(s) > most) return false;
+    *shape = s;
+    return true;
+}
+
 SoftmaxPlan plan_softmax(const View &v, int dtype) {
     SoftmaxPlan p;
     if (v.elems == 0) return p;  // (nothing to launch; no tiles or rows to divide by)
@@ -311,15 +345,19 @@ SoftmaxPlan plan_softmax(const View &v, int dtype) {
         p.shape = RowShape{static_cast<int>(nt), static_cast<int>((nvec + nt - 1) / nt)};
         return p;
     }
-    // chunked: the largest chunk that still leaves 512 workgroups, else the smallest; beyond
-    // 1024 chunks a row, workgroups of 1024 threads ([8,262144] f32 with 512 / 1024: 10.0 / 10.5 us;
-    // [4,1048576] 14.4 / 15.4: every workgroup of the scale kernel combines all chunks of its row)
     if (n > (1u << 25)) return p;  // (the general kernel)
-    const uint32_t loads_max = 32u / vec;
-    uint32_t nt = 256, loads = loads_max;
+    p.joined = plan_joined(v, vec, &p.shape);
+    uint32_t nt = static_cast<uint32_t>(p.shape.nt), loads = static_cast<uint32_t>(p.shape.v);
     auto chunks = [&] { return (n + nt * loads * vec - 1) / (nt * loads * vec); };
-    while (loads > 1 && static_cast<uint64_t>(rows) * chunks() < 512) loads /= 2;
-    if (chunks() > 1024) nt = 1024, loads = loads_max;
+    if (!p.joined) {
+        // the largest chunk that still leaves 512 workgroups, else the smallest; beyond
+        // 1024 chunks a row, workgroups of 1024 threads ([8,262144] f32 with 512 / 1024: 10.0 / 10.5 us;
+        // [4,1048576] 14.4 / 15.4: every workgroup of the scale kernel combines all chunks of its row)
+        const uint32_t loads_max = 32u / vec;
+        nt = 256, loads = loads_max;
+        while (loads > 1 && static_cast<uint64_t>(rows) * chunks() < 512) loads /= 2;
+        if (chunks() > 1024) nt = 1024, loads = loads_max;
+    }
     p.per = nt * loads * vec;
     p.g = chunks();
     p.kind = SoftmaxPlan::kChunked;
@@ -339,6 +377,41 @@ int launch_lines(const T *in, T *out, const View &v, const SoftmaxPlan &p, bool 
             return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
         return launched("softmax_lines_reg_kernel");
     });
+}
+
+// Whether two tensors of `elems` elements share no byte.
+template <typename T> bool apart(const T *a, const T *b, uint64_t elems) {
+    const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+    return (x < y ? y - x : x - y) >= elems * sizeof(T);
+}
+
+template <typename T>
+int launch_joined(const T *in, T *out, const View &v, const SoftmaxPlan &p, int nan_where, float nan_value, void *ws, hipStream_t st) {
+    auto *done = static_cast<uint32_t *>(ws);
+    auto *recs = reinterpret_cast<uint64_t *>(static_cast<unsigned char *>(ws) + kTicketBytes);
+    // (a counter a row: as many rows a launch as there are of them)
+    for (uint64_t row0 = 0; row0 < v.g.outer; row0 += kTicketRows) {
+        const uint32_t rows = static_cast<uint32_t>(std::min<uint64_t>(kTicketRows, v.g.outer - row0));
+        const uint32_t call = g_joined_calls.fetch_add(1, std::memory_order_relaxed);
+        const uint32_t tag = ((call % 0xFFFFFFu + 1u) * 0x9E3779u) & 0xFFFFFFu;  // (not 0; another one for each of 2^24 - 1 calls)
+        const T *from = in + row0 * v.g.n;
+        T *to = out + row0 * v.g.n;
+        auto launch = [&](auto kernel) {
+            kernel<<<rows * p.g, p.shape.nt, 0, st>>>(from, to, recs + row0 * p.g * vkop::kJoinedWords, done, v.g.n, p.g, tag,
+                                                      joined_polls(), nan_where, nan_value);
+            return launched("softmax_joined_kernel");
+        };
+        int rc = -1;
+#define VKOP_JOINED(NT, V) \
+    if (p.shape.nt == NT && p.shape.v == V) rc = launch(vkop::softmax_joined_kernel<T, NT, V>);
+        VKOP_JOINED(512, 2) VKOP_JOINED(512, 4)
+        if constexpr (sizeof(T) == 4) { VKOP_JOINED(256, 10) VKOP_JOINED(512, 8) }
+        else { VKOP_JOINED(256, 5) VKOP_JOINED(512, 1) }
+#undef VKOP_JOINED
+        if (rc < 0) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_joined_kernel for %d x %d", p.shape.nt, p.shape.v);
+        if (rc != VKOP_HIP_OK) return rc;
+    }
+    return VKOP_HIP_OK;
 }
 
 // The softmax of last-axis rows, or (MAX_ONLY) each row's largest probability: the kernels of kThread ... kChunked.
@@ -391,6 +464,8 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
     case SoftmaxPlan::kChunked: {
         if (ws == nullptr || ws_bytes < p.workspace)
             return fail(VKOP_HIP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", ws_bytes, p.workspace);
+        if (!MAX_ONLY && p.joined && apart(in, out, v.elems) && reinterpret_cast<uintptr_t>(ws) % sizeof(uint64_t) == 0)
+            return launch_joined(in, out, v, p, nan_where, nan_value, ws, st);
         auto *stats = reinterpret_cast<vkop::ChunkStat *>(static_cast<unsigned char *>(ws) + kTicketBytes);
         // the most vectors a thread (four floats', two halves') that leave 2048 workgroups: with fewer in all
         // their stores wait for each other, with smaller ones more of them combine the same chunks
@@ -410,9 +485,9 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
         vkop::softmax_stats_kernel<T, NT, V><<<rows * p.g, NT, 0, st>>>(from, row_stats, v.g.n, p.g);    \
         done = true;                                                                                     \
     }
-            VKOP_STATS(256, 1) VKOP_STATS(256, 2) VKOP_STATS(256, 4)
-            if constexpr (sizeof(T) == 4) { VKOP_STATS(256, 8) VKOP_STATS(1024, 8) }
-            else { VKOP_STATS(1024, 4) }
+            VKOP_STATS(256, 1) VKOP_STATS(256, 2) VKOP_STATS(256, 4) VKOP_STATS(512, 2) VKOP_STATS(512, 4)
+            if constexpr (sizeof(T) == 4) { VKOP_STATS(256, 8) VKOP_STATS(256, 10) VKOP_STATS(512, 8) VKOP_STATS(1024, 8) }
+            else { VKOP_STATS(256, 5) VKOP_STATS(512, 1) VKOP_STATS(1024, 4) }
 #undef VKOP_STATS
             if (!done) return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_stats_kernel for %d x %d", p.shape.nt, p.shape.v);
             if constexpr (MAX_ONLY) {
@@ -1594,6 +1669,12 @@ int vkop_hip_measure_path(int dtype, const int *shape, int ndim, int axis, int k
 int vkop_hip_measure_stages(int stages) {
     if (stages < 1 || stages > 3) return fail(VKOP_HIP_ERR_INVALID, "stages must be 1, 2 or 3");
     g_rows_stages = stages;
+    return VKOP_HIP_OK;
+}
+
+int vkop_hip_measure_polls(int polls) {
+    if (polls < 0) return fail(VKOP_HIP_ERR_INVALID, "polls must not be negative");
+    g_joined_polls = static_cast<uint32_t>(polls);
     return VKOP_HIP_OK;
 }
 #endif

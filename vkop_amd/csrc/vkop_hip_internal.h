@@ -1,8 +1,8 @@
 /*
  * Measurement hooks that are NOT part of the public interface (include/vkop_hip.h):
  * for this repository's benchmarks and tests only.  vkop_hip_measure_path is a pure
- * query and part of libvkop_hip.so; vkop_hip_measure_stages changes what a call
- * launches and exists only in the benchmark build of the library
+ * query and part of libvkop_hip.so; vkop_hip_measure_stages and vkop_hip_measure_polls
+ * change what a call launches or how it waits and exist only in the benchmark build of the library
  * (libvkop_hip_bench.so: the same objects, the C ABI source compiled with
  * -DVKOP_BENCH_HOOKS).
  */
@@ -22,6 +22,12 @@ extern "C" {
  * libvkop_hip_bench.so only. */
 #ifdef VKOP_BENCH_HOOKS
 int vkop_hip_measure_stages(int stages);
+
+/* How often a workgroup of the one-launch softmax of long rows looks for the row's
+ * other chunks before it reads what it misses itself (100 to start with); with 0 every
+ * workgroup that comes first does.  Results are the same bits.
+ * libvkop_hip_bench.so only. */
+int vkop_hip_measure_polls(int polls);
 #endif
 
 /* Which kernels a fused call (largest first) on this tensor would run -- and a plain
