@@ -237,20 +237,30 @@ template <int NT> __device__ __forceinline__ double block_sum(double v, double *
 
 // --------------------------------------------------------------- softmax ----
 
+// The larger of d and -104, below which a term is 0.  NAN_TOO: NaN stays NaN (else it is -104; half the cycles).
+template <bool NAN_TOO> __device__ __forceinline__ float at_least_minus_104(float d) {
+    float r;
+    if constexpr (NAN_TOO) asm("v_maximum3_f32 %0, %1, %2, %2" : "=v"(r) : "v"(d), "s"(-104.0f));
+    else asm("v_max_f32 %0, %2, %1" : "=v"(r) : "v"(d), "s"(-104.0f));
+    return r;
+}
+
 // exp(d) rounded to float, evaluated in double, for d up to 88 (a term's exponent is at most a
 // little above 0) or NaN: the relative error before the final rounding is below 2^-39, so the
 // result is the correctly rounded float except within that distance of a rounding midpoint,
 // where it is the other neighbour.  d below -104 (including -inf) gives 0; NaN gives NaN.
-// It is the one thing a float softmax tensor computes per element, and what costs there are the
-// conversions and the double rounding and scaling instructions, not the multiply-adds: the
-// multiple of ln 2 is found in single precision (any integer near d log2 e serves: |r| <= 0.34662
-// covers the rounding of d * log2 e), the power of two goes into the double's exponent as an integer --
+// It is the one thing a float softmax tensor computes per element.  Single-precision sums and products issue in 2.4
+// cycles a wave here, double ones, conversions and everything else in 4.4: the multiple of ln 2 is found in single precision
+// by adding and subtracting 1.5 2^23 (any integer near d log2 e serves: |r| <= 0.34662
+// covers the rounding of d * log2 e), the low bits of that sum go into the double's exponent as they are --
 // before the one rounding to float, which a subnormal result needs -- and the polynomial is
 // the one of degree 8 that interpolates e^r at the nine Chebyshev points of that interval, its
 // coefficients rounded to double (2^-39.7; the Taylor polynomial of degree 9 it replaces: 2^-37).
-__device__ __forceinline__ float exp_accurate(float d) {
-    d = d < -104.0f ? -104.0f : d;  // (a comparison, not a maximum: NaN stays)
-    const float n = rintf(d * 1.44269504088896341f);
+template <bool NAN_TOO = true> __device__ __forceinline__ float exp_accurate(float d) {
+    d = at_least_minus_104<NAN_TOO>(d);
+    constexpr float kMagic = 12582912.f;
+    const float nb = fmaf(d, 1.44269504088896341f, kMagic);
+    const float n = nb - kMagic;
     const double r = fma(-static_cast<double>(n), 0.69314718055994530942, static_cast<double>(d));
     double p = 0x1.a15a6596eb202p-16;
     p = fma(p, r, 0x1.a1aa9a9593b29p-13);
@@ -261,8 +271,8 @@ __device__ __forceinline__ float exp_accurate(float d) {
     p = fma(p, r, 0x1.fffffffff71a8p-2);
     p = fma(p, r, 0x1.ffffffffd37fep-1);
     p = fma(p, r, 1.0);
-    const int hi = __double2hiint(p) + __float2int_rn(n) * (1 << 20);  // (0.7 <= p <= 1.5, -150 <= n: still a normal double)
-    return static_cast<float>(__hiloint2double(hi, __double2loint(p)));
+    const uint32_t hi = static_cast<uint32_t>(__double2hiint(p)) + (__float_as_uint(nb) << 20);  // (0.7 <= p <= 1.5, -150 <= n: still a normal double)
+    return static_cast<float>(__hiloint2double(static_cast<int>(hi), __double2loint(p)));
 }
 
 // One softmax term: exp of the single-precision difference x - m.
@@ -273,14 +283,14 @@ __device__ __forceinline__ float softmax_term(float x, float m) { return exp_acc
 // out as a first-order factor (2^(a + l) = 2^a (1 + l ln 2), |l| < 1e-6).  For results that are
 // stored in half precision: 2^-22 relative before a rounding to 11 bits moves one result in two
 // thousand by one unit of a half, and costs a third of exp_accurate.  Results below 2^-126 are 0.
-__device__ __forceinline__ float exp_half_grade(float d) {
+template <bool NAN_TOO = true> __device__ __forceinline__ float exp_half_grade(float d) {
     constexpr float kHi = 1.44269502162933349609375f;  // float(log2 e)
     constexpr float kLo = 1.925963033500011e-8f;       // log2 e - kHi
+    d = at_least_minus_104<NAN_TOO>(d);  // (there the hardware exponential is 0, and what follows is finite)
     const float a = d * kHi;
-    const float l = fmaf(d, kLo, fmaf(d, kHi, -a));  // (d = -inf: NaN, and so is the product below)
+    const float l = fmaf(d, kLo, fmaf(d, kHi, -a));
     const float e = __builtin_amdgcn_exp2f(a);
-    const float t = fmaf(e, l * 0.693147180559945309f, e);
-    return e > 0.f && e < INFINITY ? t : e;  // (0, inf and NaN as the hardware unit gives them)
+    return fmaf(e, l * 0.693147180559945309f, e);
 }
 
 // The term as the element type asks for it: float tensors get the correctly rounded exponential,
@@ -289,6 +299,13 @@ __device__ __forceinline__ float exp_half_grade(float d) {
 template <typename T> __device__ __forceinline__ float softmax_term_as(float x, float m) {
     if constexpr (sizeof(T) == 2) return exp_half_grade(x - m);
     else return exp_accurate(x - m);
+}
+
+// The same for kernels whose row's sum holds every term already, NaN included: whatever at a NaN element, since 1 / sum is NaN
+// with it.
+template <typename T> __device__ __forceinline__ float softmax_term_of_row(float x, float m) {
+    if constexpr (sizeof(T) == 2) return exp_half_grade<false>(x - m);
+    else return exp_accurate<false>(x - m);
 }
 
 // What a thread adds its own few terms up in, and how a term becomes a probability, in the same
@@ -302,6 +319,22 @@ template <typename T> __device__ __forceinline__ float scale_term(float e, doubl
     if constexpr (sizeof(T) == 2) return e * static_cast<float>(rinv);
     else return static_cast<float>(static_cast<double>(e) * rinv);
 }
+
+// scale_term for many terms of one row, without its conversions: 1 / sum in two floats, whose products with a float term add
+// up to the double product within 2^-48 (a result in 2^24 differs from the one rounding of that product).
+template <typename T> struct Quotient;
+template <> struct Quotient<float> {
+    float high, low;
+    Quotient() = default;
+    __device__ __forceinline__ explicit Quotient(double rinv) : high(static_cast<float>(rinv)), low(static_cast<float>(rinv - static_cast<double>(high))) {}
+    __device__ __forceinline__ float operator()(float e) const { return fmaf(e, high, e * low); }
+};
+template <> struct Quotient<uint16_t> {
+    float rinv;
+    Quotient() = default;
+    __device__ __forceinline__ explicit Quotient(double r) : rinv(static_cast<float>(r)) {}
+    __device__ __forceinline__ float operator()(float e) const { return e * rinv; }
+};
 
 // The nucleus cut of a sorted result, by all 64 lanes of one wave: the number of leading values whose
 // running sum -- added in order, in float, sum = fl(sum + v) -- first reaches p, or k if it never does

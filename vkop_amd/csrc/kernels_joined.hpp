@@ -131,7 +131,8 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
     uint32_t before = 0, same = 0;
     asm volatile("" : "+v"(same));
     if (tid == 0) before = __hip_atomic_fetch_add(done + row + same, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const LineStats ls = row_stats;
+    const Quotient<T> over_sum(row_stats.rinv);
+    const float m = row_stats.m;
     T *orow = out + row0;
     const uint32_t e_first = ch.first(own);
 #pragma unroll
@@ -142,7 +143,7 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
         r.v = make_uint4(0, 0, 0, 0);
 #pragma unroll
         for (int c = 0; c < static_cast<int>(VEC); c++) {
-            p[c] = softmax_prob_as<T>(ch.q[i].get(c), ls);
+            p[c] = over_sum(softmax_term_of_row<T>(ch.q[i].get(c), m));
             if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
             r.set(c, p[c]);
         }

@@ -190,9 +190,9 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         }
         return;
     }
-    double rinv[L];
+    Quotient<T> over_sum[L];
 #pragma unroll
-    for (int c = 0; c < L; c++) rinv[c] = reciprocal_of_sum(s[c]);
+    for (int c = 0; c < L; c++) over_sum[c] = Quotient<T>(reciprocal_of_sum(s[c]));
     size_t at = base + static_cast<size_t>(part) * g.inner;
     asm volatile("" : "+v"(at));  // (places again: sixteen of them kept from the loads are 32 registers)
 #pragma unroll
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         for (int c = 0; c < L; c++) asm volatile("" : "+v"(e[i][c]));
 #pragma unroll
         for (int c = 0; c < L; c++) {
-            p[c] = scale_term<T>(e[i][c], rinv[c]);
+            p[c] = over_sum[c](e[i][c]);
             if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
             r.set(c, p[c]);
         }

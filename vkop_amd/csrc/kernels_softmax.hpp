@@ -174,13 +174,14 @@ template <typename T, int V> struct RowPiece {
         return acc;
     }
     __device__ __forceinline__ void store(T *orow, double rinv, bool live, int nan_where, float nan_value) {
+        const Quotient<T> over_sum(rinv);
 #pragma unroll
         for (int i = 0; i < V; i++) {
             Vec128<T> r;
             r.v = make_uint4(0, 0, 0, 0);
 #pragma unroll
             for (int c = 0; c < VEC; c++) {
-                e[i][c] = scale_term<T>(e[i][c], rinv);
+                e[i][c] = over_sum(e[i][c]);
                 r.set(c, e[i][c]);
             }
             if (nan_where) {  // (the same in every thread)
@@ -479,7 +480,8 @@ __global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(con
     const LineStats combined = combine_chunks<T, NT>(stats + static_cast<size_t>(row) * G, G, wave_m, wave_s);
     if (tid == 0) row_stats = combined;
     __syncthreads();
-    const LineStats ls = row_stats;
+    const Quotient<T> over_sum(row_stats.rinv);
+    const float m = row_stats.m;
     T *orow = out + row0;
 #pragma unroll
     for (int i = 0; i < V; i++) {
@@ -489,7 +491,7 @@ __global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(con
         r.v = make_uint4(0, 0, 0, 0);
 #pragma unroll
         for (int c = 0; c < static_cast<int>(VEC); c++) {
-            p[c] = softmax_prob_as<T>(q[i].get(c), ls);
+            p[c] = over_sum(softmax_term_of_row<T>(q[i].get(c), m));
             if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
             r.set(c, p[c]);
         }
@@ -750,11 +752,12 @@ __global__ __launch_bounds__(kStridedThreads) void softmax_strided_reg_kernel(co
         if (live && part == 0) store_elem(out, line, p);
         return;
     }
+    const Quotient<T> over_sum(rinv);
 #pragma unroll
     for (int i = 0; i < NPER; i++) {
         const uint32_t j = static_cast<uint32_t>(i) * P + part;
         if (live && j < n) {
-            float p = round_to_storage<T>(scale_term<T>(x[i], rinv));
+            float p = round_to_storage<T>(over_sum(x[i]));
             if (nan_where && p != p) p = nan_value;
             store_elem(out, base + static_cast<size_t>(j) * g.inner, p);
         }
