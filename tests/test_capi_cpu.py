@@ -199,6 +199,13 @@ def test_native_front_end_takes_whole_numbers_only():
             ops.topk(t, k, axis=np.int32(7))
 
 
+@pytest.mark.parametrize("dtype,rows,n,chunk", [(capi.F32, 64, 128256, 16384), (capi.F32, 150, 8200, 16384), (capi.F16, 64, 65537, 16384),
+                                                (capi.F32, 32, 33001, 8192), (capi.F32, 64, 200000, 10240), (capi.F16, 500, 33001, 10240)])
+def test_softmax_of_long_rows_asks_for_a_record_a_chunk(lib, dtype, rows, n, chunk):
+    """32 bytes behind the 64 KiB of counters for every chunk that the one-launch softmax splits a row into."""
+    assert capi.softmax_workspace_bytes(dtype, (rows, n), -1) >= 65536 + rows * -(-n // chunk) * 32
+
+
 def test_native_front_end_takes_any_object_with_get_as_workspace():
     """A workspace is what its get(nbytes) returns: an object with nothing else, and a class derived from ops.Workspace with a
     get() of its own.  (The rest of the call needs a GPU; get() is called before.)"""

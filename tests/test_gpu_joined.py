@@ -97,6 +97,24 @@ def test_a_workgroup_that_does_not_wait_reads_the_other_chunks_itself(ops, rows,
         lib.vkop_hip_measure_polls(100)
 
 
+@pytest.mark.parametrize("rows,n", [(64, 128256), (32, 33001), (64, 200000)])
+def test_nothing_is_written_behind_the_workspace(ops, rows, n):
+    """With what the query asks for, and with what the pair of kernels' statistics take, 24 bytes a chunk."""
+    from vkop_amd import capi
+    x = torch.randn((rows, n), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    want = ops.softmax(x)
+    need = capi.softmax_workspace_bytes(capi.F32, (rows, n), -1)
+    pair = 65536 + -(-(need - 65536) * 3 // 4 // 256) * 256
+    for size in (need, pair):
+        ws = torch.zeros(need + 65536, dtype=torch.uint8, device="cuda")
+        ws[size:] = 0xA5
+        out = torch.zeros_like(x)
+        capi.softmax(x.data_ptr(), out.data_ptr(), capi.F32, (rows, n), -1, 0, 0.0, ws.data_ptr(), size,
+                     torch.cuda.current_stream().cuda_stream)
+        assert torch.equal(out, want)
+        assert bool((ws[size:] == 0xA5).all())
+
+
 def test_more_rows_than_counters(ops):
     """16384 counters: two launches.  540 M halves."""
     rows, n = 16384 + 40, 32776

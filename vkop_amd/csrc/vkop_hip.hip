@@ -182,6 +182,7 @@ struct SoftmaxPlan {
     uint32_t lines_k = 0, lines_p = 0, lines_w = 0;  // kLinesRegs: LinesLaunch
     uint32_t ti_shift = 0;  // kStridedTile: log2 of the lines a tile
     size_t workspace = 0;
+    size_t pair_workspace = 0;  // kChunked: what the pair of kernels needs, at most `workspace`
 };
 
 // Lines of up to kStridedMaxN elements along a non-last axis, held in registers: the
@@ -362,7 +363,11 @@ SoftmaxPlan plan_softmax(const View &v, int dtype) {
     p.g = chunks();
     p.kind = SoftmaxPlan::kChunked;
     p.shape = RowShape{static_cast<int>(nt), static_cast<int>(loads)};
-    p.workspace = kTicketBytes + align_up(static_cast<size_t>(rows) * p.g * sizeof(vkop::ChunkStat));
+    const size_t total = static_cast<size_t>(rows) * p.g;
+    constexpr size_t record = vkop::kJoinedWords * sizeof(uint64_t);
+    static_assert(record >= sizeof(vkop::ChunkStat), "the larger of the two");
+    p.pair_workspace = kTicketBytes + align_up(total * sizeof(vkop::ChunkStat));
+    p.workspace = p.joined ? kTicketBytes + align_up(total * record) : p.pair_workspace;
     return p;
 }
 
@@ -462,9 +467,11 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
         });
     }
     case SoftmaxPlan::kChunked: {
-        if (ws == nullptr || ws_bytes < p.workspace)
+        if (ws == nullptr || ws_bytes < p.pair_workspace)
             return fail(VKOP_HIP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", ws_bytes, p.workspace);
-        if (!MAX_ONLY && p.joined && apart(in, out, v.elems) && reinterpret_cast<uintptr_t>(ws) % sizeof(uint64_t) == 0)
+        // (a record is larger than a chunk's statistics: in a workspace that holds only those, the pair)
+        if (!MAX_ONLY && p.joined && ws_bytes >= p.workspace && apart(in, out, v.elems) &&
+            reinterpret_cast<uintptr_t>(ws) % sizeof(uint64_t) == 0)
             return launch_joined(in, out, v, p, nan_where, nan_value, ws, st);
         auto *stats = reinterpret_cast<vkop::ChunkStat *>(static_cast<unsigned char *>(ws) + kTicketBytes);
         // the most vectors a thread (four floats', two halves') that leave 2048 workgroups: with fewer in all
