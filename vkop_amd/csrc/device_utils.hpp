@@ -330,10 +330,10 @@ template <> struct Quotient<float> {
     __device__ __forceinline__ float operator()(float e) const { return fmaf(e, high, e * low); }
 };
 template <> struct Quotient<uint16_t> {
-    float rinv;
+    float high;
     Quotient() = default;
-    __device__ __forceinline__ explicit Quotient(double r) : rinv(static_cast<float>(r)) {}
-    __device__ __forceinline__ float operator()(float e) const { return e * rinv; }
+    __device__ __forceinline__ explicit Quotient(double rinv) : high(static_cast<float>(rinv)) {}
+    __device__ __forceinline__ float operator()(float e) const { return e * high; }
 };
 
 // The nucleus cut of a sorted result, by all 64 lanes of one wave: the number of leading values whose

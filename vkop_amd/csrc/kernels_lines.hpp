@@ -32,29 +32,85 @@ template <int STRIDE> __device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
         return static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), STRIDE, kWave));
     }
 }
-// Larger / sum over the P lanes of a wave that look at the same lines (lanes 64 / P apart).  The sum
-// adds both lanes of a pair in the same order, so every lane ends with the same bits.
-template <int P, typename F> __device__ __forceinline__ uint32_t join_parts(uint32_t v, F op) {
-    if constexpr (P >= 2) v = op(v, lane_xor<32>(v));
-    if constexpr (P >= 4) v = op(v, lane_xor<16>(v));
+// Maxima and sums over the P lanes of a wave that look at the same lines (lanes 64 / P apart), L values a lane.  The lanes share
+// the lines out: a step exchanges one half of the values for the other lane's other half (one swap and one operation for two
+// values), so that after the steps of 32 and 16 lanes a lane holds kOwned = L / min(P, 4) of the lines, from owned_line() on;
+// the steps of 8 and 4 leave both lanes of a pair with them.  (With every value to every lane each step costs four times as much:
+// exchanges, not terms, were 40 % of the instructions of a line's largest probability: [16,80,8400] f32 13.5 -> 12.2 us; the tensor [8,21,262144] 67.5 -> 66.5.)  The sum adds
+// both lanes of a pair in the same order, so every lane ends with the same bits.
+template <int STRIDE> __device__ __forceinline__ void swap_lanes(uint32_t &a, uint32_t &b) {
+    if constexpr (STRIDE == 32) {
+        const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+        a = r[0], b = r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = r[0], b = r[1];
+    }
+}
+template <int STRIDE> __device__ __forceinline__ void swap_lanes(double &a, double &b) {
+    uint64_t x = static_cast<uint64_t>(__double_as_longlong(a)), y = static_cast<uint64_t>(__double_as_longlong(b));
+    uint32_t xl = static_cast<uint32_t>(x), xh = static_cast<uint32_t>(x >> 32), yl = static_cast<uint32_t>(y), yh = static_cast<uint32_t>(y >> 32);
+    swap_lanes<STRIDE>(xl, yl);
+    swap_lanes<STRIDE>(xh, yh);
+    a = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(xh) << 32) | xl));
+    b = __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(yh) << 32) | yl));
+}
+template <int STRIDE> __device__ __forceinline__ double lane_xor(double v) {
+    const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
+    const uint64_t o = (static_cast<uint64_t>(lane_xor<STRIDE>(static_cast<uint32_t>(u >> 32))) << 32) | lane_xor<STRIDE>(static_cast<uint32_t>(u));
+    return __longlong_as_double(static_cast<long long>(o));
+}
+template <int STRIDE> __device__ __forceinline__ float lane_xor(float v) { return __uint_as_float(lane_xor<STRIDE>(__float_as_uint(v))); }
+template <int P> constexpr int kLineSharers = P < 4 ? P : 4;
+// The steps of 8 and 4 lanes.
+template <int P, typename V, typename F> __device__ __forceinline__ V join_rest(V v, F op) {
     if constexpr (P >= 8) v = op(v, lane_xor<8>(v));
     if constexpr (P >= 16) v = op(v, lane_xor<4>(v));
     return v;
 }
-template <int P> __device__ __forceinline__ float parts_max(float v) {
-    return __uint_as_float(join_parts<P>(__float_as_uint(v), [](uint32_t a, uint32_t b) { return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b))); }));
+// Afterwards v[0 .. L / kLineSharers<P>) are the lane's own.
+template <int P, int L, typename V, typename F> __device__ __forceinline__ void share_out(V (&v)[L], F op) {
+    if constexpr (P >= 2) {
+#pragma unroll
+        for (int i = 0; i < L / 2; i++) {
+            swap_lanes<32>(v[i], v[i + L / 2]);
+            v[i] = op(v[i], v[i + L / 2]);
+        }
+    }
+    if constexpr (P >= 4) {
+#pragma unroll
+        for (int i = 0; i < L / 4; i++) {
+            swap_lanes<16>(v[i], v[i + L / 4]);
+            v[i] = op(v[i], v[i + L / 4]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < L / kLineSharers<P>; i++) v[i] = join_rest<P>(v[i], op);
 }
-template <int STRIDE> __device__ __forceinline__ double add_lane_xor(double v) {
-    const uint64_t u = static_cast<uint64_t>(__double_as_longlong(v));
-    const uint64_t o = (static_cast<uint64_t>(lane_xor<STRIDE>(static_cast<uint32_t>(u >> 32))) << 32) | lane_xor<STRIDE>(static_cast<uint32_t>(u));
-    return v + __longlong_as_double(static_cast<long long>(o));
+// The way back: every lane's own values to all lanes of the same lines.
+template <int P, int L> __device__ __forceinline__ void hand_out(float (&f)[L]) {
+    uint32_t v[L];
+#pragma unroll
+    for (int i = 0; i < L / kLineSharers<P>; i++) v[i] = __float_as_uint(f[i]);
+    if constexpr (P >= 4) {
+#pragma unroll
+        for (int i = 0; i < L / 4; i++) {
+            v[i + L / 4] = v[i];
+            swap_lanes<16>(v[i], v[i + L / 4]);
+        }
+    }
+    if constexpr (P >= 2) {
+#pragma unroll
+        for (int i = 0; i < L / 2; i++) {
+            v[i + L / 2] = v[i];
+            swap_lanes<32>(v[i], v[i + L / 2]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < L; i++) f[i] = __uint_as_float(v[i]);
 }
-template <int P> __device__ __forceinline__ double parts_sum(double v) {
-    if constexpr (P >= 2) v = add_lane_xor<32>(v);
-    if constexpr (P >= 4) v = add_lane_xor<16>(v);
-    if constexpr (P >= 8) v = add_lane_xor<8>(v);
-    if constexpr (P >= 16) v = add_lane_xor<4>(v);
-    return v;
+template <int P, int L> __device__ __forceinline__ uint32_t owned_line(uint32_t lane) {
+    return (P >= 2 ? (lane >> 5) * (L / 2) : 0u) + (P >= 4 ? ((lane >> 4) & 1u) * (L / 4) : 0u);
 }
 
 // MAX_ONLY: instead of the softmax tensor write each line's largest probability to out[line]: from
@@ -96,6 +152,8 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         const uint32_t j = static_cast<uint32_t>(i) * parts + part;
         q[i].v = load16_stream(in + base + static_cast<size_t>(i < K - 1 || last_ok ? j : n - 1u) * g.inner);
     }
+    constexpr int C = L / kLineSharers<P>, EXTRA = P / kLineSharers<P>;  // lines a lane owns, lanes that own the same
+    const uint32_t own0 = owned_line<P, L>(lane), extra = (lane / LPW) % EXTRA;
     float m[L];
     if constexpr (sizeof(T) == 2) {
         uint32_t pk[4] = {q[0].v.x, q[0].v.y, q[0].v.z, q[0].v.w};
@@ -105,37 +163,48 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
             pk[2] = max_half2(pk[2], q[i].v.z), pk[3] = max_half2(pk[3], q[i].v.w);
         }
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
-            pk[w] = join_parts<P>(max_half2(pk[w], 0xFC00FC00u), [](uint32_t a, uint32_t b) { return max_half2(a, b); });
+        for (int w = 0; w < 4; w++) pk[w] = max_half2(pk[w], 0xFC00FC00u);
+        share_out<P>(pk, [](uint32_t a, uint32_t b) { return max_half2(a, b); });
+#pragma unroll
+        for (int w = 0; w < C / 2; w++) {
             m[2 * w] = __half2float(__ushort_as_half(static_cast<uint16_t>(pk[w] & 0xFFFFu)));
             m[2 * w + 1] = __half2float(__ushort_as_half(static_cast<uint16_t>(pk[w] >> 16)));
         }
     } else {
+        uint32_t mu[L];
 #pragma unroll
         for (int c = 0; c < L; c++) {
             m[c] = -INFINITY;
 #pragma unroll
             for (int i = 0; i + 1 < K; i += 2) m[c] = max3(m[c], q[i].get(c), q[i + 1].get(c));  // (drops NaN)
             if constexpr (K % 2 != 0) m[c] = max3(m[c], m[c], q[K - 1].get(c));
-            m[c] = parts_max<P>(m[c]);
+            mu[c] = __float_as_uint(m[c]);
         }
-    }
-    if (W > 1) {
-        // a wave's maxima are in each of its parts: the first writes them, and each part reads its share of the waves
-        float *fl = reinterpret_cast<float *>(lines_lds) + team * (W * LPW * L);
-        if (lane < LPW) {
+        share_out<P>(mu, [](uint32_t a, uint32_t b) { return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b))); });
 #pragma unroll
-            for (int c = 0; c < L; c++) fl[(tw * L + c) * LPW + slot] = m[c];
+        for (int c = 0; c < C; c++) m[c] = __uint_as_float(mu[c]);
+    }
+    auto larger = [](float a, float b) { return fmaxf(a, b); };
+    if (W > 1) {
+        // a wave's maxima go to LDS, and the lanes that own the same lines read their share of the waves
+        float *fl = reinterpret_cast<float *>(lines_lds) + team * (W * LPW * L);
+        if (extra == 0) {
+#pragma unroll
+            for (int c = 0; c < C; c++) fl[(tw * L + own0 + c) * LPW + slot] = m[c];
         }
         __syncthreads();
-        for (uint32_t w = lane / LPW; w < W; w += P) {
+        for (uint32_t w = extra; w < W; w += EXTRA) {
 #pragma unroll
-            for (int c = 0; c < L; c++) m[c] = fmaxf(m[c], fl[(w * L + c) * LPW + slot]);
+            for (int c = 0; c < C; c++) m[c] = fmaxf(m[c], fl[(w * L + own0 + c) * LPW + slot]);
         }
 #pragma unroll
-        for (int c = 0; c < L; c++) m[c] = parts_max<P>(m[c]);
+        for (int c = 0; c < C; c++) m[c] = join_rest<P>(m[c], larger);
         __syncthreads();  // (the sums take the same place)
     }
+    float own_m[C];
+#pragma unroll
+    for (int c = 0; c < C; c++) own_m[c] = m[c];
+    hand_out<P>(m);
     float e[K][L];
     std::conditional_t<WIDE, double, TermSum<T>> acc[L];
 #pragma unroll
@@ -150,49 +219,65 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
             acc[c] += i < K - 1 || last_ok ? e[i][c] : 0.f;
         }
     }
-    double s[L];
+    double s[L];  // (the lane's own C lines)
 #pragma unroll
-    for (int c = 0; c < L; c++) s[c] = parts_sum<P>(static_cast<double>(acc[c]));
+    for (int c = 0; c < L; c++) s[c] = static_cast<double>(acc[c]);
+    auto sum = [](double a, double b) { return a + b; };
+    share_out<P>(s, sum);
     if (W > 1) {
         double *dl = lines_lds + team * (W * LPW * L);
-        if (lane < LPW) {
+        if (extra == 0) {
 #pragma unroll
-            for (int c = 0; c < L; c++) dl[(tw * L + c) * LPW + slot] = s[c];
+            for (int c = 0; c < C; c++) dl[(tw * L + own0 + c) * LPW + slot] = s[c];
         }
         __syncthreads();
 #pragma unroll
-        for (int c = 0; c < L; c++) s[c] = 0.0;
-        for (uint32_t w = lane / LPW; w < W; w += P) {  // fixed order: run-to-run stable
+        for (int c = 0; c < C; c++) s[c] = 0.0;
+        for (uint32_t w = extra; w < W; w += EXTRA) {  // fixed order: run-to-run stable
 #pragma unroll
-            for (int c = 0; c < L; c++) s[c] += dl[(w * L + c) * LPW + slot];
+            for (int c = 0; c < C; c++) s[c] += dl[(w * L + own0 + c) * LPW + slot];
         }
 #pragma unroll
-        for (int c = 0; c < L; c++) s[c] = parts_sum<P>(s[c]);
+        for (int c = 0; c < C; c++) s[c] = join_rest<P>(s[c], sum);
     }
     if constexpr (MAX_ONLY) {
-        if (live && part == 0) {
+        if (live && extra == 0 && tw == 0) {
             // the line's maximum has the term exp(0) = 1 (NaN where there is none, as the tensor would hold)
             const size_t at = static_cast<size_t>(o) * g.inner + col;
             Vec128<T> r;
             r.v = make_uint4(0, 0, 0, 0);
-            float p[L];
+            float p[C];
 #pragma unroll
-            for (int c = 0; c < L; c++) {
-                p[c] = scale_term<T>(softmax_term_as<T>(m[c], m[c]), reciprocal_of_sum(s[c]));
-                r.set(c, p[c]);
+            for (int c = 0; c < C; c++) {
+                p[c] = scale_term<T>(softmax_term_as<T>(own_m[c], own_m[c]), reciprocal_of_sum(s[c]));
+                if constexpr (C == L) r.set(c, p[c]);
             }
-            if (skip == 0) store16_stream(out + at, r.v);
+            if (C == L && skip == 0) store16_stream(out + at, r.v);
             else {
 #pragma unroll
-                for (int c = 1; c < L; c++)
-                    if (static_cast<uint32_t>(c) >= skip) store_elem(out, at + c, p[c]);
+                for (int c = 0; c < C; c++)
+                    if (own0 + static_cast<uint32_t>(c) >= skip) store_elem(out, at + own0 + c, p[c]);
             }
         }
         return;
     }
     Quotient<T> over_sum[L];
+    {
+        float high[L], low[L];
 #pragma unroll
-    for (int c = 0; c < L; c++) over_sum[c] = Quotient<T>(reciprocal_of_sum(s[c]));
+        for (int c = 0; c < C; c++) {
+            const Quotient<T> own(reciprocal_of_sum(s[c]));
+            high[c] = own.high;
+            if constexpr (sizeof(T) == 4) low[c] = own.low;
+        }
+        hand_out<P>(high);
+        if constexpr (sizeof(T) == 4) hand_out<P>(low);
+#pragma unroll
+        for (int c = 0; c < L; c++) {
+            over_sum[c].high = high[c];
+            if constexpr (sizeof(T) == 4) over_sum[c].low = low[c];
+        }
+    }
     size_t at = base + static_cast<size_t>(part) * g.inner;
     asm volatile("" : "+v"(at));  // (places again: sixteen of them kept from the loads are 32 registers)
 #pragma unroll
