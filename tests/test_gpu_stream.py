@@ -284,6 +284,26 @@ def test_random_shapes_k_and_row_kinds_on_whatever_route_they_take(ops, seed):
         _compare_paths(ops, n, k, dtype, rows, kinds, path)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("n,k", [(1040, 128), (2048, 129), (4095, 255), (4096, 256), (4097, 200), (8192, 300), (8193, 300), (12288, 408), (12289, 256),
+                                 (16384, 409), (16385, 500), (32768, 511), (9000, 511), (2200, 511)])
+def test_wide_workgroups_with_the_vectors_a_row_needs(ops, n, k, dtype):
+    """A row in a workgroup of 512 or 1024 threads, at and just past what each number of vectors a thread holds, and as
+    many places as its list takes: plain top-k exactly, in either direction; the fused call to the bars."""
+    rng = np.random.default_rng(n + k)
+    bits = np.uint16 if dtype == np.float16 else np.uint32
+    for kind in ("llm", "levels", "sorted", "runs", "masked", "nan_and_inf", "signed_zeros", "tenth", "half_half"):
+        x = np.ascontiguousarray(_rows(kind, 17, n, rng).astype(dtype))
+        xd = dev(x)
+        for largest in (True, False):
+            t, tj = ops.topk(xd, k, largest=largest)
+            et, ej = oracle.topk(x, k, largest=largest)
+            assert np.array_equal(host(tj), ej) and np.array_equal(host(t).view(bits), et.view(bits)), (kind, largest)
+        v, ix = ops.softmax_topk(xd, k)
+        ov, oix = oracle.softmax_topk(x, k)
+        assert (half_ulp_diff if dtype == np.float16 else ulp_diff)(host(v), ov).max() <= (1 if dtype == np.float16 else 2), kind
+
+
 @pytest.mark.parametrize("rows,n,k", [(17, 20001, 16), (8, 20001, 16), (24, 50000, 40), (5, 131072, 64), (16, 16385, 5)])
 def test_flat_rows_with_dozens_of_peaks_on_the_chunk_and_merge_kernels(ops, rows, n, k):
     """The chunk + merge kernels over several chunks (rows.path = 1: no shape takes them by itself any

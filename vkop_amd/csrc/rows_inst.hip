@@ -22,6 +22,19 @@ template <typename T, bool SOFTMAX> bool launch_rows_chunk(const RowsLaunch &a) 
         else VKOP_ROWS_LAUNCH(NT, V, false, kMergeLocal);                    \
         return true;                                                         \
     }
+    // (wide workgroups on rows that fill a part of their most vectors a thread: fitted_loads)
+    if (a.merge == kMergeLocal && !a.sampling) {
+        VKOP_ROWS_LOCAL(512, 2)
+        VKOP_ROWS_LOCAL(1024, 2)
+        if constexpr (sizeof(T) == 4) {
+            VKOP_ROWS_LOCAL(512, 4)
+            VKOP_ROWS_LOCAL(1024, 3)
+            VKOP_ROWS_LOCAL(1024, 4)
+        } else {
+            VKOP_ROWS_LOCAL(512, 1)
+            VKOP_ROWS_LOCAL(1024, 1)
+        }
+    }
     if constexpr (kReversed<T>) {
         if (a.merge != kMergeLocal) return false;
         VKOP_ROWS_LOCAL(256, 1)

@@ -583,10 +583,13 @@ uint32_t rows_cap(int k) {
 }
 
 constexpr int kWaveRowMaxK = 32;  // largest k served by the one-wave-per-row launch
+constexpr int kTwoAndHalfListsMaxK = 408;  // largest k with rows_cap(k) <= kLocalCap
 constexpr int kWideRowMinK = 64;  // above it a row that fits one workgroup is given to one (of enough threads)
 
-// (for_size: what a call could use whatever rows.path says at that time)
-RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false) {
+// (for_size: what a call could use whatever rows.path says at that time.  full_list: also a k whose places the list of a
+// one-workgroup row holds less than 2.5 times, 409 to 511: usual rows list 1.2 to 1.4 times the places, and a second listing at most
+// 2 k + 1 elements, 1023 of the list's 1024.)
+RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false, bool full_list = false) {
     RowsCfg c;
     if (v.g.inner != 1 || k > vkop::kFastMaxK || v.g.n == 0 || v.g.outer == 0) return c;
     const uint32_t vec = dtype == VKOP_HIP_F32 ? 4u : 8u;
@@ -597,7 +600,7 @@ RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false) 
     int forced_nt = g_rows_threads.load(), forced_v = g_rows_loads.load(), forced_g = g_rows_chunks.load();
     if (forced_nt <= 0 || forced_v <= 0 || forced_g <= 0) forced_nt = 0;
     const uint32_t nvec = (n + vec - 1) / vec;
-    const uint32_t cap = rows_cap(k);
+    const uint32_t cap = full_list ? std::min(rows_cap(k), static_cast<uint32_t>(vkop::kLocalCap)) : rows_cap(k);
     auto fits = [&](int nt, int vv, uint32_t g) {
         const uint32_t nw = static_cast<uint32_t>(nt) / 64u;
         if (g < 1 || g > static_cast<uint32_t>(vkop::kMergeChunksMax)) return false;
@@ -966,6 +969,22 @@ int launch_scan(const T *in, T *values, int32_t *indices, const View &v, int k, 
     return launched("rows_scan_kernel / rows_pick_kernel");
 }
 
+// Vectors a thread of a workgroup that holds its row: of 512 and 1024 threads, which the plan takes by the places and whose shape
+// holds 16384 elements and more, as few as hold this row -- every vector costs its comparisons and counts in every wave, whether
+// there are elements in it or not.  us a call, top-k and fused, with eight vectors / these: [16,8400] f32 k = 300 14.5 / 13.4,
+// 17.8 / 15.4; [256,8000] k = 300 15.4 / 13.8, 18.6 / 15.8; [64,4000] k = 130 9.5 / 8.8, 11.3 / 9.9; [16,12000] k = 400 13.3 /
+// 12.1, 16.2 / 15.0.
+int fitted_loads(const RowsCfg &c, uint32_t n, uint32_t vec) {
+    if (c.nt < 512) return c.v;
+    static const int f32_wide[] = {2, 3, 4}, f32_less[] = {2, 4}, f16[] = {1, 2};
+    auto first = [&](const auto &loads) {
+        for (const int v : loads)
+            if (v < c.v && static_cast<uint64_t>(c.nt) * v * vec >= n) return v;
+        return c.v;
+    };
+    return vec == 8 ? first(f16) : c.nt == 1024 ? first(f32_wide) : first(f32_less);
+}
+
 template <typename T, bool SOFTMAX>
 int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, const RowsCfg &c, void *ws,
                 const RowsLayout &l, hipStream_t st, bool sampling = false, float scale = 1.f, int32_t *counts = nullptr,
@@ -1003,6 +1022,10 @@ int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, 
         w.cap_shift = 0;
         while ((1u << w.cap_shift) < w.cap) w.cap_shift++;
     }
+    if (a.merge == vkop::kMergeLocal && !sampling) {
+        a.v = static_cast<uint32_t>(fitted_loads(c, v.g.n, vec));
+        a.per = a.nt * a.v * vec;
+    }
     a.ws = w;
     a.stream = st;
     a.sampling = sampling;
@@ -1035,9 +1058,11 @@ int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, 
 //    thousand of rows just past what 256 threads hold: [3300,8196] k = 23 f16 189 / 124, f32 132 / 121, [3300,10094] f16 191 / 161;
 //  * 256 threads, short rows by the thousand, which the select reads again from the cache: [6000,400] f32 k = 44 40 / 30, k = 104
 //    52 / 36, [30000,800] f16 k = 104 275 / 207; but [300,400] f32 k = 104 9.3 / 10.8, [1500,800] f16 k = 75 18 / 20;
-//  * 512 and 1024 threads, more rows than CUs (a workgroup each at a time) of few elements for so many threads: [300,1500] f32 k = 219
-//    18.5 / 17.3, [1500,2400] k = 132 50 / 28, [6000,5564] f16 k = 290 339 / 194; but [64,800] f32 k = 152 11.4 / 13.6, [300,4000]
-//    k = 221 18 / 27, [1500,8000] k = 249 55 / 77.
+//  * 512 and 1024 threads, more rows than CUs (a workgroup each at a time) of few elements for so many threads, a line for each of the
+//    two (with the vectors fitted, fitted_loads): f32 [1200,1100] k = 240 25 / 18, [6000,1500] k = 130 76 / 66, but [700,1500] k = 130
+//    13 / 18, [2500,2200] k = 240 32 / 44, [6000,4000] k = 130 71 / 124; f32 [700,3000] k = 300 36 / 30, [1200,4000] 47 / 44,
+//    [6000,5500] 229 / 186, but [450,4000] 20 / 33, [700,4400] 30 / 39, [2500,6400] 98 / 105; f16 [700,3000] k = 300 49 / 38,
+//    [2500,5500] 125 / 102, but [450,4000] 27 / 42, [1200,6400] 64 / 71.
 bool select_is_faster(const View &v, int k, const RowsCfg &c, uint32_t vec, bool largest) {
     const uint32_t n = v.g.n, rows = v.g.outer;
     if (c.g != 1 || c.nt < 256) return false;
@@ -1046,7 +1071,9 @@ bool select_is_faster(const View &v, int k, const RowsCfg &c, uint32_t vec, bool
     if (!largest && vectors < 2u * places) return true;
     if (!largest && c.nt >= 512 && rows > 1024 && n < (vec == 8 && n % 8 == 0 ? 9000u : 11000u)) return true;
     if (c.nt == 256) return rows >= 1024 && n < (vec == 4 || rows >= 4096 ? 1000u : 600u);
-    return rows > 256 && (c.nt == 512 ? n <= 4500 && rows >= n / 5 : n <= 6500 && rows >= n / 11);
+    if (rows <= 256) return false;
+    if (c.nt == 512) return rows >= 1000 && n <= 1600;
+    return n <= (vec == 4 ? 2000u : 2600u) + std::min(rows, 2000u) * 11u / 5u && n <= (vec == 4 && rows < 4000 ? 5500u : 6500u);
 }
 
 template <typename T>
@@ -1066,6 +1093,19 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
     RowsCfg c = (routed && !sc.ok) ? choose_rows_cfg(v, k, dtype) : RowsCfg{};
     if (!largest && (c.g != 1 || c.nt < 256 || c.cap > static_cast<uint32_t>(vkop::kLocalCap))) c = RowsCfg{};
     if (c.ok && g_rows_path.load() != 1 && select_is_faster(v, k, c, 16 / sizeof(T), largest != 0)) c = RowsCfg{};
+    if (routed && !sc.ok && !c.ok && k > kTwoAndHalfListsMaxK && v.g.outer <= 256 && g_rows_path.load() != 1) {
+        // A k that the list holds less than 2.5 times, up to a row a CU.  Such a workgroup keeps everything in LDS: the call takes
+        // whatever workspace is given, as the kernels below that need none.  us a call, those below / this, f32: [16,16000] k = 500
+        // 30.9 / 13.2, of levels 49 / 19, sorted 28.7 / 25.3; [256,8400] k = 420 25.6 / 12.5, smallest first 25.8 / 12.4; [8,5000]
+        // k = 450 18.9 / 11.1; f16 [16,16000] k = 500 44.4 / 13.3; but [300,5000] f32 25.3 / 33.9, [300,9000] f16 42.1 / 44.1.
+        const RowsCfg full = choose_rows_cfg(v, k, dtype, false, true);
+        if (full.ok && full.g == 1 && !select_is_faster(v, k, full, 16 / sizeof(T), largest != 0)) {
+            const RowsLayout none;
+            if (largest) return launch_rows<T, false>(in, values, indices, v, k, full, nullptr, none, st);
+            using R = vkop::Reversed<T>;
+            return launch_rows<R, false>(reinterpret_cast<const R *>(in), reinterpret_cast<R *>(values), indices, v, k, full, nullptr, none, st);
+        }
+    }
     const BigKCfg b = (c.ok || sc.ok) ? BigKCfg{} : choose_bigk_cfg(v, k, dtype);
     if (sc.ok || c.ok || b.ok) {
         const RowsLayout l = rows_layout(v, c, b, sc);
