@@ -1104,6 +1104,42 @@ def test_nms_random_configurations(ops):
         capi.tune("nms.threads", 0)
 
 
+@pytest.mark.parametrize("threads", [256, 1024])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+def test_nms_candidates_at_the_edges_of_block_and_list(ops, threads, dtype):
+    """So many candidates that a block or the list is full, has one more or one less, ends in a block of 1, 2, 16, 17 ..
+    (lanes share a candidate's tests there), from rows of whole and of cut vectors; crowded boxes and equal scores."""
+    from vkop_amd import capi
+    capi.tune("nms.threads", threads)
+    try:
+        for count in (1, 2, 3, 15, 16, 17, 32, 33, 63, 64, 65, 66, 80, 81, 96, 97, 127, 128, 129, 257, 511, 512, 513, 2047, 2048, 2049, 2300):
+            rng = np.random.default_rng(count)
+            N = int(max(count, rng.choice([2304, 2305, 9216 + 3])))
+            boxes = _nms_boxes(rng, 1, N, 0.5 if count % 2 else 0.15).astype(dtype)
+            scores = (rng.integers(0, 100, (1, 3, N)) / 256).astype(dtype)      # at most 0.39, many of them equal
+            for c in range(3):
+                scores[0, c, rng.permutation(N)[:count]] += dtype(0.5)
+            for iou in (0.0, 0.45):
+                got, over = ops.nms(dev(boxes), dev(scores), iou, 0.45, 0)
+                want = oracle.nms(boxes.astype(np.float32), scores.astype(np.float32), iou, 0.45, 0, max_candidates=2048)
+                assert np.array_equal(host(got), want), (count, N, iou)
+                assert over == (count > 2048), count
+    finally:
+        capi.tune("nms.threads", 0)
+
+
+@pytest.mark.parametrize("B,C", [(1, 1), (1, 3), (1, 4), (1, 5), (3, 683), (5, 821)])
+def test_nms_records_of_any_number_of_pairs(ops, B, C):
+    """The pack kernel: four pairs a workgroup, 2048 counts a step; pairs without a record among them."""
+    rng = np.random.default_rng(B * C)
+    boxes = _nms_boxes(rng, B, 70, 0.3)
+    scores = rng.random((B, C, 70)).astype(np.float32)
+    scores[rng.random((B, C)) < 0.3] = 0.0
+    for per_class in (0, 2):
+        got, over = ops.nms(dev(boxes), dev(scores), 0.9, 0.1, per_class)
+        assert np.array_equal(host(got), oracle.nms(boxes, scores, 0.9, 0.1, per_class, max_candidates=2048)) and not over
+
+
 @pytest.mark.parametrize("power", [-80, -41, -39, 0, 39, 41, 62])
 def test_nms_overlap_beside_the_threshold(ops, power):
     """The quotient of the areas is compared without being formed where products decide: thresholds 2^-20 and 2^-18

@@ -1281,8 +1281,9 @@ int nms_impl(const T *boxes, const T *scores, int32_t *out, int out_capacity, in
     else VKOP_NMS_LAUNCH(vkop::kNmsThreadsWide, false);
 #undef VKOP_NMS_LAUNCH
     if (int rc = launched("nms_kernel")) return rc;
-    vkop::nms_pack_kernel<<<pairs, 256, 0, st>>>(selected, counts, out, out_count, pairs, static_cast<uint32_t>(C), max_sel,
-                                                 static_cast<uint32_t>(out_capacity));
+    const uint32_t packers = (pairs + vkop::kNmsPackPairs - 1) / vkop::kNmsPackPairs;
+    vkop::nms_pack_kernel<<<packers, 256, 0, st>>>(selected, counts, out, out_count, pairs, static_cast<uint32_t>(C), max_sel,
+                                                   static_cast<uint32_t>(out_capacity));
     return launched("nms_pack_kernel");
 }
 
