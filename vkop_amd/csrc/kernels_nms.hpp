@@ -185,9 +185,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
             // vectors of the lane within the row and the round: the first of them, as the row ends after them
             const int32_t reach = static_cast<int32_t>(min(N - min(N, wave_first), tiles * (kWave * 4))) - static_cast<int32_t>(lane * 4);
             word &= (1u << (reach > 0 ? (static_cast<uint32_t>(reach) + kWave * 4 - 1) / (kWave * 4) : 0u)) - 1u;
-            while (__ballot(word != 0u) != 0ull) {
-                const uint32_t first = word != 0u ? static_cast<uint32_t>(__builtin_ctz(word)) : ~0u;  // (none: zeros below, and no candidates)
+            uint32_t own_listed = 0;  // (0, but for all that the compiler knows another one in every lane: it would add up over the lanes)
+            asm("" : "+v"(own_listed));
+            for (;;) {
                 const bool any = word != 0u;
+                const uint64_t some = __builtin_amdgcn_ballot_w64(any);
+                if (some == 0ull) break;
+                const uint32_t first = any ? static_cast<uint32_t>(__builtin_ctz(word)) : ~0u;  // (none: zeros below)
                 word &= word - 1u;
                 // (bitwise selects: by conditions the scores go to scratch memory, to be indexed there)
                 uint32_t x[4] = {};
@@ -199,21 +203,39 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
                     x[2] |= on & __float_as_uint(s[u].z);
                     x[3] |= on & __float_as_uint(s[u].w);
                 }
-                uint64_t mask[4];
-                uint32_t n = 0, at = 0;
+                uint32_t above = 0;
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    mask[c] = __ballot(any && __uint_as_float(x[c]) > score_threshold);
-                    n += static_cast<uint32_t>(__popcll(mask[c]));
-                }
-                if (lane == 0) at = atomicAdd(&listed, n);
-                at = uniform_u32(at);
+                for (int c = 0; c < 4; c++) above |= __uint_as_float(x[c]) > score_threshold ? 1u << c : 0u;
+                above = any ? above : 0u;
+                const uint32_t box0 = wave_first + first * (kWave * 4) + lane * 4;
+                // room for n more, and this lane's place behind the lanes below it
+                auto reserve = [&](uint32_t n) -> uint32_t {
+                    uint32_t at = 0;
+                    if (lane == 0) at = atomicAdd(&listed + own_listed, n);
+                    return uniform_u32(at);
+                };
+                if (__builtin_amdgcn_ballot_w64((above & (above - 1u)) != 0u) == 0ull) {
+                    // one a lane, the rule (a quarter of the instructions behind the selects)
+                    const uint32_t at = reserve(static_cast<uint32_t>(__popcll(some))) + lanes_below(some);
+                    const uint32_t c = static_cast<uint32_t>(__builtin_ctz(above | 8u));
+                    const uint32_t v = c == 0u ? x[0] : c == 1u ? x[1] : c == 2u ? x[2] : x[3];
+                    if (any && at < static_cast<uint32_t>(kNmsMaxCandidates)) comp[at] = composite(order_key(__uint_as_float(v)), box0 + c);
+                } else {
+                    uint64_t mask[4];
+                    uint32_t n = 0;
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const uint32_t place = at + lanes_below(mask[c]);
-                    if (((mask[c] >> lane) & 1ull) && place < static_cast<uint32_t>(kNmsMaxCandidates))
-                        comp[place] = composite(order_key(__uint_as_float(x[c])), wave_first + first * (kWave * 4) + lane * 4 + static_cast<uint32_t>(c));
-                    at += static_cast<uint32_t>(__popcll(mask[c]));
+                    for (int c = 0; c < 4; c++) {
+                        mask[c] = __builtin_amdgcn_ballot_w64((above & (1u << c)) != 0u);
+                        n += static_cast<uint32_t>(__popcll(mask[c]));
+                    }
+                    uint32_t at = reserve(n);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const uint32_t place = at + lanes_below(mask[c]);
+                        if ((above & (1u << c)) != 0u && place < static_cast<uint32_t>(kNmsMaxCandidates))
+                            comp[place] = composite(order_key(__uint_as_float(x[c])), box0 + static_cast<uint32_t>(c));
+                        at += static_cast<uint32_t>(__popcll(mask[c]));
+                    }
                 }
             }
         }
