@@ -108,9 +108,9 @@ __device__ __forceinline__ bool nms_overlap(const float4 &a, const float4 &b, fl
 // boxes 1.3, the block's overlaps 1.5, its kept set 0.4 (a second block, one pair in twenty, 1.6).  A chain this
 // short is bound by instruction fetch as much as by anything: a launch finds none of its code in the CUs' caches,
 // and forms of these steps that run fewer instructions out of more code were slower, step by step.  us a call with the
-// pack kernel, 0.25 / 0.45, 51 kept a pair: [16,80,8400] f32 26.0 -> 18.5, f16 24.0 -> 16.2; [16,91,8399] f32
-// 27.2 -> 18.9; [1,80,8400] f32 11.6 -> 10.6; [8,91,1917] f32 15.2 -> 11.8; [16,20,8400], 400 candidates, 26.2 -> 24.4;
-// [8,80,400] all candidates 33.2 -> 29.2; more than 2048 of 8400 ([4,4,8400], the list made twice) 63.6 -> 64.5.
+// pack kernel, 0.25 / 0.45, 51 kept a pair: [16,80,8400] f32 26.1 -> 18.3, f16 24.1 -> 15.5; [16,91,8399] f32
+// 27.0 -> 18.4; [1,80,8400] f32 11.6 -> 10.8; [8,91,1917] f32 15.2 -> 11.6; [16,20,8400], 400 candidates, 26.1 -> 24.1;
+// [8,80,400] all candidates 33.4 -> 29.3; more than 2048 of 8400 ([4,4,8400], the list made twice) 64.2 -> 64.6.
 // WHOLE: N is a multiple of four, and no load needs the step for a row's end (it costs a row that has one 0.4 us).
 template <typename T, int NT, bool WHOLE>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ? 8 : 6))) void nms_kernel(
@@ -479,7 +479,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
 // had more candidates than kNmsMaxCandidates; a (-1,-1,-1) record follows the last
 // one when capacity allows.  Launch: a workgroup of 256 for every kNmsPackPairs pairs, a wave a pair.
 // What bounds it: its round trips to memory, so a thread's counts are loaded eight at a time, under them the
-// first selected boxes, and only the last workgroup asks for overflows ([16,80,8400]: a workgroup a pair, a count at a time 4.3 us, 2.6 so).
+// first selected boxes, and only the last workgroup asks for overflows ([16,80,8400], the shortest and the mean: a workgroup a pair, a count at a time 4.2 and 4.4 us, so 2.6 and 4.0).
 constexpr uint32_t kNmsPackPairs = 256 / kWave;
 __global__ __launch_bounds__(256) void nms_pack_kernel(const int32_t *__restrict__ selected,
                                                               const uint32_t *__restrict__ counts, int32_t *__restrict__ out,
