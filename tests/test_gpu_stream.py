@@ -448,6 +448,36 @@ def test_sampling_half_rows_whose_probabilities_tie(ops, n, k):
         assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])
 
 
+@pytest.mark.parametrize("k", [3, 20, 40, 90])
+def test_half_rows_with_a_tie_at_the_cut_where_the_list_may_end(ops, k):
+    """k + 5 elements above the rest, t + 1 neighbouring ones of them around the k-th place a last place of their logits apart, whose
+    probabilities are equal halves: the list of candidates may end with that group, and whether it holds all of it is
+    decided by the largest probability that is not listed -- of the group's own value in every other row, where an
+    element a few last places below goes on with it."""
+    rng = np.random.default_rng(k)
+    n, rows, scale = 32000, 64, 1.25
+    x = (rng.standard_normal((rows, n)) * 0.5).astype(np.float16)
+    for r in range(rows):
+        where = rng.permutation(n)[:k + 5]
+        x[r, where] = np.linspace(5.0, 4.0, k + 5).astype(np.float16)
+        x[r, where[0]] = 8.0 + rng.random() * 6.0   # the row's maximum: the others' probabilities are small halves
+        t = int(rng.integers(1, 5))
+        first = k - 1 - int(rng.integers(0, min(t, k - 1)))
+        group = where[first:first + t + 1]
+        top = x[r, group[0]]
+        x[r, group] = top - np.spacing(top) * rng.integers(0, 2, len(group)).astype(np.float16)
+        if r % 2:
+            x[r, where[-1]] = top - np.spacing(top) * np.float16(3)
+    v, ix, _ = (host(a) for a in ops.softmax_topk_sampling(dev(x), k, scale, 0.9))
+    ov, oix, _ = oracle.softmax_topk_sampling(x, k, scale, 0.9)
+    # sums agree to 2^-22: a probability that close to a boundary between two halves may fall on either side of it
+    assert half_ulp_diff(v, ov).max() <= 1
+    same = (v.view(np.uint16) == ov.view(np.uint16)).all(axis=-1)
+    assert same.sum() >= rows - 2 and np.array_equal(ix[same], oix[same])
+    equal = v[:, 1:] == v[:, :-1]
+    assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])
+
+
 @pytest.mark.parametrize("n", [50000, 8192, 1000, 8400])
 def test_sampling_variant_ties_special_rows_and_errors(ops, n):
     """(n = 50000: the scan + pick kernels; the shorter rows: one workgroup, or one wave, per row)"""

@@ -697,6 +697,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
             // wave decides alike whether the row is done, and no barrier is needed for that
             bool tie = false;
             if constexpr (SOFTMAX) {
+                bool cut = false;  // equal logits on both sides of the k-th place
                 double csum = 0.0;
                 for (uint32_t r = lane; r < want; r += kWave) csum += sh.corr[r];
                 const double rinv = 1.0 / (s_base + wave_sum_f64_uniform(csum));
@@ -705,11 +706,24 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                     const uint32_t r = base + lane;  // ranks r and r + 1 <= k
                     const float p0 = round_to_storage<T>(static_cast<float>(static_cast<double>(sh.prob[r < k ? r : 0u]) * rinv));
                     const float p1 = round_to_storage<T>(static_cast<float>(static_cast<double>(sh.prob[r < k ? r + 1u : 0u]) * rinv));
-                    tie = tie || (r < k && p0 == p1 && sh.pkey[r] != sh.pkey[r < k ? r + 1u : 0u]);
+                    if (r < k && p0 == p1) {
+                        if (sh.pkey[r] != sh.pkey[r + 1u]) tie = true;
+                        else cut = cut || r + 1u == k;
+                    }
                     if (base == 0) p_first = p0;
                 }
                 tie = __ballot(tie) != 0ull;
+                cut = __ballot(cut) != 0ull;
                 bool by_index = false;  // (the same in every thread, as `tie` is)
+                float p_own = 0.f, p_cut = 0.f, p_unlisted = 0.f;
+                if (tie || cut) {
+                    auto prob = [&](float of_term) { return round_to_storage<T>(static_cast<float>(static_cast<double>(of_term) * rinv)); };
+                    p_own = tid < C2 ? prob(term) : 0.f;
+                    p_cut = prob(sh.prob[k - 1u]);
+                    p_unlisted = prob(softmax_term(ordered_to_float(thr - 1u), M));  // the largest that an element which is not listed has
+                    // Equal logits at the cut are in index order, but a smaller one may have the same probability still
+                    if (!tie) tie = __syncthreads_or((tid < C2 && static_cast<uint32_t>(mine >> 32) < sh.pkey[k] && p_own >= p_cut) || p_unlisted >= p_cut) != 0;
+                }
                 if (tie) {
                     // Where some candidate's probability lies below the k-th, every element of the row with a
                     // probability of the first k is in the list (probabilities fall with the logits, and what is
@@ -719,9 +733,9 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                     // 16.6 -> 15.4 us a call (17.2 -> 13.6 over other inputs), k = 90 20.7 -> 16.0, [8,32000] k = 40
                     // 14.2 -> 12.0, [16,200000] k = 64 16.4 -> 13.6; where the groups are larger than what the list holds
                     // beyond k -- [128,50257] k = 20 -- 23.6 as before, and a lower threshold did not change that.
-                    const float p_own = tid < C2 ? round_to_storage<T>(static_cast<float>(static_cast<double>(term) * rinv)) : 0.f;
-                    const float p_cut = round_to_storage<T>(static_cast<float>(static_cast<double>(sh.prob[k - 1u]) * rinv));
-                    by_index = __syncthreads_or(tid < C2 && p_own < p_cut) != 0;
+                    // So it does where the largest key that is not listed, the one below thr, has a probability below the k-th
+                    // (a list of hardly more than k + 1 may hold none).
+                    by_index = __syncthreads_or((tid < C2 && p_own < p_cut) || p_unlisted < p_cut) != 0;
                     if (by_index) {
                         const uint32_t idx = composite_index(mine);
                         if (tid < C2) sh.cand[tid] = p_own >= p_cut ? composite(__float_as_uint(p_own), idx) : 0ull;
