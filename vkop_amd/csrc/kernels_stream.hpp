@@ -486,6 +486,11 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     // -inf never becomes a candidate: a row with k+1 larger elements does not need it,
     // and finish_row fills any other row's last places from the row itself
     thr = max(thr, kKeyNegInf + 1u);
+    // Half-precision probabilities of logits closer than this are often equal: with a list that goes on a little below, the
+    // group at the k-th place nearly always ends inside it (probabilities from 100 of the smallest half on), and E1 can
+    // tell.  It is one candidate in a hundred more: sampling
+    // [32,50257] k = 40 by the inputs 14.0 / 14.0 / 19.3 us, with the threshold as found 13.8 to 22.2.
+    if constexpr (SOFTMAX && sizeof(T) == 2) thr = max(min(thr, order_key(ordered_to_float(thr) - 1e-2f)), kKeyNegInf + 1u);
 
     // ---- D1. the first gather, wave by wave ------------------------------------------------
     // Every wave reads again ITS threads' blocks that reach thr (a list of its own in LDS: no
