@@ -257,6 +257,32 @@ def test_softmax_special_values_and_nan_option(ops):
     assert np.all(host(ops.softmax(dev(c))) == np.float32(1.0 / 777))
 
 
+@pytest.mark.parametrize("shape,axis", [((3000, 3), 1), ((3000, 12), 1), ((3000, 197), 1), ((300, 1000), 1), ((300, 4000), 1), ((600, 20001), 1),
+                                        ((40, 100000), 1), ((3, 600000), 1), ((300, 21, 65), 1), ((16, 80, 840), 1), ((3, 1000, 4100), 1),
+                                        ((300, 70, 5), 1), ((8, 4096, 64), 1), ((300, 1100, 64), 1), ((4, 2500, 3), 1), ((300, 40), 0)])
+def test_softmax_nan_of_any_payload(ops, shape, axis):
+    """A NaN is a NaN whatever its sign and payload, and so is the line that holds one: every kernel that sums the accurate
+    terms, and those that sum others.  Its largest probability and the replacement of NaN likewise."""
+    rng = np.random.default_rng(sum(shape))
+    for dtype, bits, kinds in ((np.float32, np.uint32, (0x7FC00001, 0x7F800001, 0x7FFFFFFF, 0xFFFFFFFF, 0xFF800001, 0x7FC00ABC, 0x7FC00F6A, 0xFFC00001)),
+                               (np.float16, np.uint16, (0x7E01, 0x7C01, 0x7FFF, 0xFFFF, 0xFC01))):
+        x = (rng.standard_normal(shape, dtype=np.float32) * 2).astype(dtype)
+        lines = np.moveaxis(x, axis, -1)
+        at = np.unravel_index(rng.choice(lines[..., 0].size, min(lines[..., 0].size - 1, 2 * len(kinds)), replace=False), lines.shape[:-1])
+        held = np.zeros(lines.shape[:-1], bool)
+        held[at] = True
+        b = np.moveaxis(x.view(bits), axis, -1)
+        for i, line in enumerate(zip(*at)):
+            b[line + (rng.integers(0, shape[axis]),)] = kinds[i % len(kinds)]
+        xd = torch.from_numpy(x.view(np.int32 if dtype == np.float32 else np.int16)).cuda().view(torch.float32 if dtype == np.float32 else torch.float16)
+        got = np.moveaxis(host(ops.softmax(xd, axis)), axis, -1)
+        assert np.isnan(got[held]).all() and not np.isnan(got[~held]).any(), dtype
+        put = np.moveaxis(host(ops.softmax(xd, axis, nan_where=True, nan_value=0.25)), axis, -1)
+        assert np.all(put[held] == dtype(0.25)) and np.array_equal(put[~held], got[~held]), dtype
+        best = host(ops.softmax_reduce_max(xd, axis))
+        assert np.array_equal(np.isnan(best), held) and np.array_equal(best[~held], got[~held].max(-1)), dtype
+
+
 def test_softmax_in_place(ops):
     x = synth.classifier_logits(16, 1000, seed=3)
     xd = dev(x)

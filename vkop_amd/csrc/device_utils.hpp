@@ -272,7 +272,9 @@ template <bool NAN_TOO = true> __device__ __forceinline__ float exp_accurate(flo
     p = fma(p, r, 0x1.ffffffffd37fep-1);
     p = fma(p, r, 1.0);
     const uint32_t hi = static_cast<uint32_t>(__double2hiint(p)) + (__float_as_uint(nb) << 20);  // (0.7 <= p <= 1.5, -150 <= n: still a normal double)
-    return static_cast<float>(__hiloint2double(static_cast<int>(hi), __double2loint(p)));
+    const float e = static_cast<float>(__hiloint2double(static_cast<int>(hi), __double2loint(p)));
+    // (a NaN's low bits have gone into that exponent: e may be any number, and is NaN again with d * 0; else e + 0)
+    return NAN_TOO ? fmaf(d, 0.f, e) : e;
 }
 
 // One softmax term: exp of the single-precision difference x - m.
