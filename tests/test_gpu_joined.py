@@ -168,3 +168,47 @@ def test_workspace_with_other_contents_and_replays(ops):
                 assert torch.equal(out, want[(i + 1) % 3])
     finally:
         capi.graph_destroy(graph)
+
+
+@pytest.mark.parametrize("rows,n", [(64, 65537), (300, 20483), (32, 33001), (150, 8200)])
+def test_a_workspace_whose_counters_do_not_start_at_zero_ends_every_wait(ops, rows, n):
+    """A workspace nobody cleared: at each of these counts some workgroup takes itself for the row's last one and clears the
+    records while others still look for them.  They run out of looks and read the chunks themselves: same bits."""
+    from vkop_amd import capi
+    x = torch.randn((rows, n), generator=torch.Generator(device="cuda").manual_seed(n), device="cuda")
+    want = ops.softmax(x)
+    need = capi.softmax_workspace_bytes(capi.F32, (rows, n), -1)
+    ws = torch.zeros(need + 256, dtype=torch.uint8, device="cuda")
+    at = -ws.data_ptr() % 256
+    stream = torch.cuda.current_stream().cuda_stream
+    for count in (0, 1, 2, 3, 4, 7, 11, 1 << 30):
+        ws[at:at + 65536].view(torch.int32).fill_(count)
+        for _ in range(2):
+            out = torch.zeros_like(x)
+            capi.softmax(x.data_ptr(), out.data_ptr(), capi.F32, (rows, n), -1, 0, 0.0, ws.data_ptr() + at, need, stream)
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), count
+
+
+def test_two_streams_on_one_workspace_end(ops):
+    """Against the rules: their records and counters replace each other's.  Nothing is said about the values of the first ten
+    calls, but every one ends, and the workspace serves again once it is cleared."""
+    from vkop_amd import capi
+    rows, n = 64, 65537
+    x = torch.randn((rows, n), generator=torch.Generator(device="cuda").manual_seed(5), device="cuda")
+    want = ops.softmax(x)
+    need = capi.softmax_workspace_bytes(capi.F32, (rows, n), -1)
+    ws = torch.zeros(need + 256, dtype=torch.uint8, device="cuda")
+    at = ws.data_ptr() + (-ws.data_ptr()) % 256
+    outs, streams = [torch.zeros_like(x) for _ in range(2)], [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(5):
+        for out, stream in zip(outs, streams):
+            capi.softmax(x.data_ptr(), out.data_ptr(), capi.F32, (rows, n), -1, 0, 0.0, at, need, stream.cuda_stream)
+    torch.cuda.synchronize()
+    stream = torch.cuda.current_stream().cuda_stream
+    capi.workspace_init(at, need // 4 * 4, stream)
+    out = torch.zeros_like(x)
+    capi.softmax(x.data_ptr(), out.data_ptr(), capi.F32, (rows, n), -1, 0, 0.0, at, need, stream)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
     constexpr uint32_t VEC = Vec128<T>::N;
     static_assert(NT * V * VEC < (1 << 16), "a record's count");
     __shared__ ChunkScratch<NT> sh;
-    __shared__ ChunkStat own_stats[kJoinedMaxChunks];  // of the chunks that this workgroup had to read itself
+    __shared__ ChunkStat stats[kJoinedMaxChunks];  // where this workgroup has to read chunks itself
     __shared__ LineStats row_stats;
     __shared__ uint64_t sh_missing;
     const uint32_t tid = threadIdx.x;
@@ -83,22 +83,25 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
     const ChunkStat mine = chunk_stats(ch, own, n, sh);
     if (tid < static_cast<uint32_t>(kWave)) {
         if (tid == 0) publish_chunk(rrecs + own * kJoinedWords, mine, tag);
+        // (its own record is not looked for: what a call that breaks the rules for a workspace does to it ends no wait late)
         ChunkWords w;
         uint64_t missing;
         for (uint32_t poll = 0;; poll++) {
             bool absent = false;
             if (tid < G) {
                 w.read(rrecs + tid * kJoinedWords);
-                absent = !w.arrived(tag);
+                absent = tid != own && !w.arrived(tag);
             }
             missing = __ballot(absent);
-            // (its own record always arrives)
-            if (missing == 0ull || (poll >= polls && ((missing >> own) & 1ull) == 0ull)) break;
+            if (missing == 0ull || poll >= polls) break;
             __builtin_amdgcn_s_sleep(1);
         }
+        const ChunkStat c = tid == own ? mine : w.stat();
         if (missing == 0ull) {
-            const LineStats st = combine_wave<T>(w.stat(), tid < G);
+            const LineStats st = combine_wave<T>(c, tid < G);
             if (tid == 0) row_stats = st;
+        } else if (tid < G) {
+            stats[tid] = c;  // (those of the missing chunks are written below)
         }
         if (tid == 0) sh_missing = missing;
     }
@@ -108,17 +111,11 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
             const uint32_t c = static_cast<uint32_t>(__builtin_ctzll(left));
             ch.template load<false>(rowp, c, n);
             const ChunkStat st = chunk_stats(ch, c, n, sh);
-            if (tid == 0) own_stats[c] = st;
+            if (tid == 0) stats[c] = st;
         }
         __syncthreads();
         if (tid < static_cast<uint32_t>(kWave)) {
-            ChunkStat c = own_stats[tid < G ? tid : 0u];
-            if (tid < G && ((sh_missing >> tid) & 1ull) == 0ull) {
-                ChunkWords w;
-                w.read(rrecs + tid * kJoinedWords);
-                c = w.stat();
-            }
-            const LineStats st = combine_wave<T>(c, tid < G);
+            const LineStats st = combine_wave<T>(stats[tid < G ? tid : 0u], tid < G);
             if (tid == 0) row_stats = st;
         }
         uint32_t again = own;
@@ -126,10 +123,11 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
         ch.template load<false>(rowp, again, n);
         __syncthreads();
     }
-    // This workgroup has read what it needs of the row's records.  (Whose answer is not waited for here: at an address the
-    // compiler takes for the same in every lane it would be, before the lanes that ask share it out.)
+    // This workgroup has read what it needs of the row's records, and its own is in memory: whoever clears them clears that too.
+    // (Whose answer is not waited for here: at an address the compiler takes for the same in every lane it would be, before
+    // the lanes that ask share it out.)
     uint32_t before = 0, same = 0;
-    asm volatile("" : "+v"(same));
+    asm volatile("s_waitcnt vmcnt(0)" : "+v"(same) : : "memory");
     if (tid == 0) before = __hip_atomic_fetch_add(done + row + same, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const Quotient<T> over_sum(row_stats.rinv);
     const float m = row_stats.m;
