@@ -206,6 +206,24 @@ def test_softmax_of_long_rows_asks_for_a_record_a_chunk(lib, dtype, rows, n, chu
     assert capi.softmax_workspace_bytes(dtype, (rows, n), -1) >= 65536 + rows * -(-n // chunk) * 32
 
 
+def test_no_record_tag_is_that_of_a_cleared_word(lib):
+    """The one-launch softmax takes a word with the launch's tag for arrived: none of a launch's four may be 0, which a cleared
+    word has, nor alike, and a launch's are not those of the one before.  All launches until the tags come again, and across
+    the counter's wrap."""
+    import ctypes
+    import numpy as np
+    f = ctypes.CDLL(capi.BENCH_LIB_PATH).vkop_hip_measure_tags
+    f.argtypes = [ctypes.c_uint, ctypes.c_uint, ctypes.c_void_p]
+    at_once = 1 << 20
+    tags = np.zeros((at_once, 4), np.uint32)
+    for first in [i * at_once for i in range(18)] + [(1 << 32) - at_once // 2]:
+        assert f(first, at_once, tags.ctypes.data) == 0
+        assert tags.min() > 0 and tags.max() < 1 << 24, first
+        for w in range(4):
+            assert not np.any(tags[:, w] == tags[:, (w + 1) % 4]) and not np.any(tags[:, w] == tags[:, (w + 2) % 4]), first
+            assert not np.any(tags[1:, w] == tags[:-1, w]), first
+
+
 def test_native_front_end_takes_any_object_with_get_as_workspace():
     """A workspace is what its get(nbytes) returns: an object with nothing else, and a class derived from ops.Workspace with a
     get() of its own.  (The rest of the call needs a GPU; get() is called before.)"""

@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libvkop_hip.so")
 # the same library built with the benchmark's hook (vkop_hip_measure_stages): bench.py's per-kernel legs load
 # this one instead, in a process of their own (use_bench_library() before the first lib())
 BENCH_LIB_PATH = os.path.join(_HERE, "libvkop_hip_bench.so")
-BENCH_ONLY = ("vkop_hip_measure_stages", "vkop_hip_measure_polls")
+BENCH_ONLY = ("vkop_hip_measure_stages", "vkop_hip_measure_polls", "vkop_hip_measure_tags")
 HEADER_PATH = os.path.join(ROOT, "include", "vkop_hip.h")
 
 OK, ERR_INVALID, ERR_DEVICE, ERR_WORKSPACE, ERR_UNSUPPORTED = 0, 1, 2, 3, 4
@@ -144,6 +144,7 @@ def lib():
         "vkop_hip_tune": (i, [ctypes.c_char_p, i]),
         "vkop_hip_measure_stages": (i, [i]),
         "vkop_hip_measure_polls": (i, [i]),
+        "vkop_hip_measure_tags": (i, [ctypes.c_uint, ctypes.c_uint, vp]),
         "vkop_hip_measure_path": (i, [i, ip, i, i, i]),
         "vkop_hip_rows_plan": (i, [i, ip, i, i, i, ip, ip, ip]),
     }

@@ -21,8 +21,10 @@ constexpr uint32_t kJoinedMaxChunks = kWave;
 constexpr int kJoinedWords = 4;  // 64-bit words of a chunk's record
 
 // A record is four words of 40 bits each under a tag of 24 that differs from launch to launch and from word to word: a word
-// with its tag has arrived, whatever lay there before, and no word needs to arrive before another.
-__device__ __forceinline__ uint32_t word_tag(uint32_t tag, int i) { return (tag + static_cast<uint32_t>(i) * 0x5BD1E9u) & 0xFFFFFFu; }
+// with its tag has arrived, whatever lay there before, and no word needs to arrive before another.  22 bits are the launch's,
+// which are not all 0 (a cleared word has not arrived) and come again after 2^22 - 1 launches; two are the word's.
+constexpr uint32_t launch_tag(uint32_t launch) { return ((launch % 0x3FFFFFu + 1u) * 0x9E3779u) & 0x3FFFFFu; }  // (an odd factor)
+__host__ __device__ constexpr uint32_t word_tag(uint32_t tag, int i) { return (tag << 2) | static_cast<uint32_t>(i); }
 __device__ __forceinline__ void publish_chunk(uint64_t *rec, const ChunkStat &c, uint32_t tag) {
     const uint64_t low40 = (1ull << 40) - 1u, s = static_cast<uint64_t>(__double_as_longlong(c.s));
     auto put = [&](int i, uint64_t bits) { publish(rec + i, (static_cast<uint64_t>(word_tag(tag, i)) << 40) | bits); };

@@ -397,8 +397,7 @@ int launch_joined(const T *in, T *out, const View &v, const SoftmaxPlan &p, int 
     // (a counter a row: as many rows a launch as there are of them)
     for (uint64_t row0 = 0; row0 < v.g.outer; row0 += kTicketRows) {
         const uint32_t rows = static_cast<uint32_t>(std::min<uint64_t>(kTicketRows, v.g.outer - row0));
-        const uint32_t call = g_joined_calls.fetch_add(1, std::memory_order_relaxed);
-        const uint32_t tag = ((call % 0xFFFFFFu + 1u) * 0x9E3779u) & 0xFFFFFFu;  // (not 0; another one for each of 2^24 - 1 calls)
+        const uint32_t tag = vkop::launch_tag(g_joined_calls.fetch_add(1, std::memory_order_relaxed));
         const T *from = in + row0 * v.g.n;
         T *to = out + row0 * v.g.n;
         auto launch = [&](auto kernel) {
@@ -1723,6 +1722,14 @@ int vkop_hip_measure_stages(int stages) {
 int vkop_hip_measure_polls(int polls) {
     if (polls < 0) return fail(VKOP_HIP_ERR_INVALID, "polls must not be negative");
     g_joined_polls = static_cast<uint32_t>(polls);
+    return VKOP_HIP_OK;
+}
+
+int vkop_hip_measure_tags(unsigned first, unsigned count, unsigned *tags) {
+    if (tags == nullptr) return fail(VKOP_HIP_ERR_INVALID, "tags is null");
+    for (size_t i = 0; i < count; i++)
+        for (int w = 0; w < vkop::kJoinedWords; w++)
+            tags[i * vkop::kJoinedWords + w] = vkop::word_tag(vkop::launch_tag(first + static_cast<unsigned>(i)), w);
     return VKOP_HIP_OK;
 }
 #endif

@@ -2,7 +2,7 @@
  * Measurement hooks that are NOT part of the public interface (include/vkop_hip.h):
  * for this repository's benchmarks and tests only.  vkop_hip_measure_path is a pure
  * query and part of libvkop_hip.so; vkop_hip_measure_stages and vkop_hip_measure_polls
- * change what a call launches or how it waits and exist only in the benchmark build of the library
+ * change what a call launches or how it waits and, like vkop_hip_measure_tags, exist only in the benchmark build of the library
  * (libvkop_hip_bench.so: the same objects, the C ABI source compiled with
  * -DVKOP_BENCH_HOOKS).
  */
@@ -28,6 +28,10 @@ int vkop_hip_measure_stages(int stages);
  * workgroup that comes first does.  Results are the same bits.
  * libvkop_hip_bench.so only. */
 int vkop_hip_measure_polls(int polls);
+
+/* The tags of the four words of a record, for launches first ... first + count - 1 of
+ * that softmax: tags[count][4].  A pure query.  libvkop_hip_bench.so only. */
+int vkop_hip_measure_tags(unsigned first, unsigned count, unsigned *tags);
 #endif
 
 /* Which kernels a fused call (largest first) on this tensor would run -- and a plain

@@ -31,7 +31,7 @@ def _load():
     if torch.__version__.split("+")[0] != module.torch_version:
         raise ImportError("vkop_amd/_native.so was built for torch %s, this is %s: build it again (`make -C vkop_amd/host -B`)"
                           % (module.torch_version, torch.__version__))
-    names = [n for n in L._signatures if not n.endswith(("tune", "measure_stages", "measure_polls", "measure_path"))]
+    names = [n for n in L._signatures if not n.endswith(("tune", "measure_stages", "measure_polls", "measure_tags", "measure_path"))]
     module.bind({n[len("vkop_hip_"):]: ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in names}, capi.VkopHipError, Workspace)
     _native = module
     return module
