@@ -649,6 +649,33 @@ def test_softmax_then_max_of_last_axis_rows(ops, rows, n, dtype):
     assert np.array_equal(fused[3:].view(bits), chain[3:].view(bits))
 
 
+# A line of one 0 and n - 1 times d: its sum 1 + (n - 1) exp(d) is exact in double, in any order.  With these d its reciprocal lies
+# so near a boundary between two floats that 1 / sum split in two floats, 48 bits of it, comes out as the other one.
+@pytest.mark.parametrize("n,d", [(3, 0xc00457d9), (12, 0xbf811cdd), (12, 0xc18825f0), (70, 0xbf58afe1), (70, 0xc0dca981), (80, 0xbf9df231),
+                                 (197, 0xbf3967a5), (1100, 0xc0889f64), (2500, 0xbfedfbfe), (4000, 0xbfee4c35), (4096, 0xbfac208c),
+                                 (20001, 0xbcee0490), (100000, 0xbf1af22d), (100000, 0xc1c6636a), (600000, 0xbfe751fe)])
+def test_float_probabilities_are_the_double_product_rounded_once(ops, n, d):
+    """Every kernel that scales a row's terms, and those that write its largest probability alone, bit for bit."""
+    d = np.array([d], np.uint32).view(np.float32)[0]
+    term = np.float64(np.float32(np.exp(np.float64(d))))
+    rinv = 1.0 / (1.0 + (n - 1) * term)
+    top, rest = np.float32(rinv), np.float32(term * rinv)
+    for rows, inner in ((2000, 1), (300, 1), (64, 1), (2, 1), (8, 65), (2, 4100), (8, 16384), (300, 5)):
+        if rows * n * inner > 1 << 26:
+            continue
+        x = torch.full((rows, n, inner), float(d), device="cuda")
+        x[:, n // 3] = 0.0
+        if inner == 1:
+            x = x.view(rows, n)
+        got, best = ops.softmax(x, 1), ops.softmax_reduce_max(x, 1)
+        assert bool((best == float(top)).all()), (rows, inner)
+        assert bool((got[:, n // 3] == float(top)).all()), (rows, inner)
+        assert int((got == float(rest)).sum()) == rows * (n - 1) * inner, (rows, inner)
+        if inner == 1:
+            y = x.clone()
+            assert torch.equal(ops.softmax(y, 1, out=y), got), rows
+
+
 def test_workspace_too_small_is_an_error(ops):
     from vkop_amd import capi
     x = dev(synth.classifier_logits(4, 1000, 1))

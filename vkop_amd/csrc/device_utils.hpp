@@ -322,14 +322,13 @@ template <typename T> __device__ __forceinline__ float scale_term(float e, doubl
     else return static_cast<float>(static_cast<double>(e) * rinv);
 }
 
-// scale_term for many terms of one row, without its conversions: 1 / sum in two floats, whose products with a float term add
-// up to the double product within 2^-48 (a result in 2^24 differs from the one rounding of that product).
+// scale_term for many terms of one row, bit for bit: what is the same for all of them is worked out once.
 template <typename T> struct Quotient;
 template <> struct Quotient<float> {
-    float high, low;
+    double rinv;
     Quotient() = default;
-    __device__ __forceinline__ explicit Quotient(double rinv) : high(static_cast<float>(rinv)), low(static_cast<float>(rinv - static_cast<double>(high))) {}
-    __device__ __forceinline__ float operator()(float e) const { return fmaf(e, high, e * low); }
+    __device__ __forceinline__ explicit Quotient(double r) : rinv(r) {}
+    __device__ __forceinline__ float operator()(float e) const { return scale_term<float>(e, rinv); }
 };
 template <> struct Quotient<uint16_t> {
     float high;

@@ -262,21 +262,25 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         return;
     }
     Quotient<T> over_sum[L];
-    {
-        float high[L], low[L];
+    if constexpr (sizeof(T) == 2) {
+        float high[L];
+#pragma unroll
+        for (int c = 0; c < C; c++) high[c] = Quotient<T>(reciprocal_of_sum(s[c])).high;
+        hand_out<P>(high);
+#pragma unroll
+        for (int c = 0; c < L; c++) over_sum[c].high = high[c];
+    } else {
+        // (a double's two words as two floats)
+        float low[L], high[L];
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            const Quotient<T> own(reciprocal_of_sum(s[c]));
-            high[c] = own.high;
-            if constexpr (sizeof(T) == 4) low[c] = own.low;
+            const double r = reciprocal_of_sum(s[c]);
+            low[c] = __int_as_float(__double2loint(r)), high[c] = __int_as_float(__double2hiint(r));
         }
+        hand_out<P>(low);
         hand_out<P>(high);
-        if constexpr (sizeof(T) == 4) hand_out<P>(low);
 #pragma unroll
-        for (int c = 0; c < L; c++) {
-            over_sum[c].high = high[c];
-            if constexpr (sizeof(T) == 4) over_sum[c].low = low[c];
-        }
+        for (int c = 0; c < L; c++) over_sum[c].rinv = __hiloint2double(__float_as_int(high[c]), __float_as_int(low[c]));
     }
     size_t at = base + static_cast<size_t>(part) * g.inner;
     asm volatile("" : "+v"(at));  // (places again: sixteen of them kept from the loads are 32 registers)
