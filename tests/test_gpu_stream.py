@@ -478,6 +478,82 @@ def test_half_rows_with_a_tie_at_the_cut_where_the_list_may_end(ops, k):
     assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])
 
 
+@pytest.mark.parametrize("k", [3, 40, 90])
+def test_float_rows_with_equal_logits_at_the_cut(ops, k):
+    """k + 4 equal logits around the k-th place, where the list of candidates may end; in two rows of three a logit one float below
+    with a lower index, whose difference to the row's maximum rounds to the same float (a maximum 8 above and more) or does not
+    (the others).  Maxima 2 to 100 above the group (the last: subnormal probabilities), groups at 5, -3, 0, 300 and 1e-3."""
+    rng = np.random.default_rng(k)
+    n, rows = 40000, 60
+    x = np.empty((rows, n), np.float32)
+    for r in range(rows):
+        v = np.float32((5.0, -3.0, 0.0, 300.0, 1e-3)[r % 5])
+        x[r] = v - 1 - np.abs(rng.standard_normal(n)).astype(np.float32)
+        where = np.sort(rng.permutation(n)[:k + 6])
+        x[r, where[1:k + 5]] = v
+        x[r, where[-1]] = v + np.float32((2.0, 8.5, 17.0, 40.0, 89.0, 100.0)[r // 5 % 6])
+        if r % 3:
+            x[r, where[0]] = np.nextafter(v, np.float32(-np.inf))
+        if r % 3 == 2:
+            x[r, where[2]] = np.nextafter(np.nextafter(v, np.float32(-np.inf)), np.float32(-np.inf))
+    v, ix = (host(t) for t in ops.softmax_topk(dev(x), k))
+    ev, eix = oracle.softmax_topk(x, k)
+    assert np.array_equal(ix, eix) and ulp_diff(v, ev).max() <= 2
+
+
+@pytest.mark.parametrize("spread", [2.0 ** -i for i in range(3, 22, 3)])
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+def test_rows_of_small_range_whose_list_goes_on_below_its_threshold(ops, spread, dtype):
+    """Rows so narrow that the stretch below the threshold (0.01 of halves, 2^-16 of floats) holds dozens, hundreds or all of
+    their elements, with and without a peak."""
+    rng = np.random.default_rng(int(1 / spread))
+    x = (rng.standard_normal((9, 50257)) * spread).astype(np.float32)
+    x[3:6] += np.float32(0.75)
+    x[0::3, 77] = 6.0
+    x = x.astype(dtype)
+    for k in (5, 40, 100):
+        v, ix = (host(t) for t in ops.softmax_topk(dev(x), k))
+        ev, eix = oracle.softmax_topk(x, k)
+        if dtype == np.float32:
+            assert ulp_diff(v, ev).max() <= 2, k
+        else:
+            assert half_ulp_diff(v, ev).max() <= 1, k
+        bits = np.uint32 if dtype == np.float32 else np.uint16
+        for r in range(9):
+            check_fused_invariants(x[r].astype(np.float32), v[r].astype(np.float32), ix[r])
+            # the sums agree to 2^-22: where no probability fell on the other side of a boundary, neither did an index
+            if np.array_equal(v[r].view(bits), ev[r].view(bits)) and (dtype == np.float16 or spread > 1e-3):
+                assert np.array_equal(ix[r], eix[r]), (k, r)
+
+
+def test_a_tie_at_the_cut_costs_no_second_look(ops):
+    """[64,128256] k = 50 with 70 logits of 5 behind the maximum of every row: where that is 13 the next float below 5 has the same
+    difference to it, rounded, where it is 13.3 it has not, and the one takes the time of the other (a row that starts over takes
+    6 us of 14 longer).  The least of nine means of 40 calls each, the two in turn."""
+    rng = np.random.default_rng(9)
+    rows, n, k = 64, 128256, 50
+    x = np.minimum(rng.standard_normal((rows, n)).astype(np.float32), np.float32(3.0))
+    where = np.stack([rng.permutation(n)[:71] for _ in range(rows)])
+    np.put_along_axis(x, where, np.float32(5.0), -1)
+    inputs = {}
+    for top in (13.0, 13.3):
+        x[np.arange(rows), where[:, 0]] = top
+        inputs[top] = dev(x)
+        assert np.array_equal(host(ops.softmax_topk(inputs[top], k)[1]), oracle.softmax_topk(x, k)[1])
+    best = dict.fromkeys(inputs, 1e9)
+    for _ in range(9):
+        for top, t in inputs.items():
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            ops.softmax_topk(t, k)
+            a.record()
+            for _ in range(40):
+                ops.softmax_topk(t, k)
+            b.record()
+            torch.cuda.synchronize()
+            best[top] = min(best[top], a.elapsed_time(b) / 40)
+    assert best[13.0] < 1.2 * best[13.3], best
+
+
 @pytest.mark.parametrize("n", [50000, 8192, 1000, 8400])
 def test_sampling_variant_ties_special_rows_and_errors(ops, n):
     """(n = 50000: the scan + pick kernels; the shorter rows: one workgroup, or one wave, per row)"""

@@ -486,11 +486,18 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     // -inf never becomes a candidate: a row with k+1 larger elements does not need it,
     // and finish_row fills any other row's last places from the row itself
     thr = max(thr, kKeyNegInf + 1u);
-    // Half-precision probabilities of logits closer than this are often equal: with a list that goes on a little below, the
-    // group at the k-th place nearly always ends inside it (probabilities from 100 of the smallest half on), and E1 can
-    // tell.  It is one candidate in a hundred more: sampling
+    // The list goes on a little below the threshold, so that the group of equal probabilities at the k-th place ends inside it
+    // and E1 can tell (else the row starts over below, 5 to 10 us of a call).  Floats: logits that far apart have different
+    // probabilities unless those are subnormal -- x - M is rounded by at most 2^-18 wherever its exponential is not 0, and terms
+    // of differences 2^-17 apart are 64 places of a float apart.  It lists next to nothing more, and the threshold is an element's
+    // value: of logits that went through bfloat16 the list ended with the group in a few rows of every call ([64,128256]
+    // k = 50 18.7 us, [64,32000] k = 40 15.4, [32,50257] k = 40 17.0; so 14.1, 10.3, 11.5).  Halves: the probabilities of logits closer
+    // than 0.01 are often equal, and seldom those of others (from 100 of the smallest half on).  It is one candidate in a hundred more: sampling
     // [32,50257] k = 40 by the inputs 14.0 / 14.0 / 19.3 us, with the threshold as found 13.8 to 22.2.
-    if constexpr (SOFTMAX && sizeof(T) == 2) thr = max(min(thr, order_key(ordered_to_float(thr) - 1e-2f)), kKeyNegInf + 1u);
+    if constexpr (SOFTMAX) {
+        constexpr float kBelow = sizeof(T) == 2 ? 1e-2f : 0x1p-16f;
+        thr = max(min(thr, order_key(ordered_to_float(thr) - kBelow)), kKeyNegInf + 1u);
+    }
 
     // ---- D1. the first gather, wave by wave ------------------------------------------------
     // Every wave reads again ITS threads' blocks that reach thr (a list of its own in LDS: no
@@ -689,12 +696,11 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
             BPS(31);
             if (tid < C2) {
                 const uint32_t rk = sh.rank[tid];
-                if (rk < want) {
-                    sh.pidx[rk] = composite_index(mine);
-                    sh.pkey[rk] = static_cast<uint32_t>(mine >> 32);
-                    sh.prob[rk] = term;
-                    sh.corr[rk] = cr;
-                }
+                // (the tables hold NT ranks; those past the first k + 1 say how the list goes on)
+                sh.pidx[rk] = composite_index(mine);
+                sh.pkey[rk] = static_cast<uint32_t>(mine >> 32);
+                sh.prob[rk] = term;
+                sh.corr[rk] = cr;
             }
             __syncthreads();
             BPS(32);
@@ -720,29 +726,32 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                 tie = __ballot(tie) != 0ull;
                 cut = __ballot(cut) != 0ull;
                 bool by_index = false;  // (the same in every thread, as `tie` is)
-                float p_own = 0.f, p_cut = 0.f, p_unlisted = 0.f;
+                float p_cut = 0.f;
+                auto prob = [&](float of_term) { return round_to_storage<T>(static_cast<float>(static_cast<double>(of_term) * rinv)); };
                 if (tie || cut) {
-                    auto prob = [&](float of_term) { return round_to_storage<T>(static_cast<float>(static_cast<double>(of_term) * rinv)); };
-                    p_own = tid < C2 ? prob(term) : 0.f;
+                    // Every element with a probability of the first k is in the list where the list's last has a smaller one, or
+                    // the largest key that is not listed, the one below thr (probabilities fall with the logits).
                     p_cut = prob(sh.prob[k - 1u]);
-                    p_unlisted = prob(softmax_term(ordered_to_float(thr - 1u), M));  // the largest that an element which is not listed has
-                    // Equal logits at the cut are in index order, but a smaller one may have the same probability still
-                    if (!tie) tie = __syncthreads_or((tid < C2 && static_cast<uint32_t>(mine >> 32) < sh.pkey[k] && p_own >= p_cut) || p_unlisted >= p_cut) != 0;
+                    const bool whole = prob(sh.prob[C2 - 1u]) < p_cut || prob(softmax_term(ordered_to_float(thr - 1u), M)) < p_cut;
+                    if (!tie) {
+                        // Equal logits at the cut are in index order, but a smaller one may have the same probability still
+                        bool smaller = false;
+                        for (uint32_t r = k + 1u + lane; r < C2; r += kWave)
+                            smaller = smaller || (sh.pkey[r] != sh.pkey[k] && prob(sh.prob[r]) >= p_cut);
+                        tie = !whole || __ballot(smaller) != 0ull;
+                    }
+                    by_index = tie && whole;
                 }
                 if (tie) {
-                    // Where some candidate's probability lies below the k-th, every element of the row with a
-                    // probability of the first k is in the list (probabilities fall with the logits, and what is
-                    // not listed has a smaller logit than all that is): ranked once more by (probability, index)
-                    // the list gives their order.  Half-precision probabilities of long rows are small, some of
+                    // Ranked once more by (probability, index) the list gives the order of the row's first k. Half-precision
+                    // probabilities of long rows are small, some of
                     // them subnormal, and nearly every call has such a row: f16 at a scale of 1.25 [32,50257] k = 40
                     // 16.6 -> 15.4 us a call (17.2 -> 13.6 over other inputs), k = 90 20.7 -> 16.0, [8,32000] k = 40
                     // 14.2 -> 12.0, [16,200000] k = 64 16.4 -> 13.6; where the groups are larger than what the list holds
                     // beyond k -- [128,50257] k = 20 -- 23.6 as before, and a lower threshold did not change that.
-                    // So it does where the largest key that is not listed, the one below thr, has a probability below the k-th
-                    // (a list of hardly more than k + 1 may hold none).
-                    by_index = __syncthreads_or((tid < C2 && p_own < p_cut) || p_unlisted < p_cut) != 0;
                     if (by_index) {
                         const uint32_t idx = composite_index(mine);
+                        const float p_own = tid < C2 ? prob(term) : 0.f;
                         if (tid < C2) sh.cand[tid] = p_own >= p_cut ? composite(__float_as_uint(p_own), idx) : 0ull;
                         sh.rank[tid] = 0;
                         __syncthreads();
