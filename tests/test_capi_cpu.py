@@ -149,6 +149,23 @@ def test_route_planner_without_a_gpu(lib):
     assert 64 * 1024 < need <= 4 << 20
 
 
+def test_rows_plan_tells_the_loads_that_run(lib):
+    """Rows that a wide workgroup holds are launched with as few vectors a thread as hold the row, unless the shape is forced."""
+    F32, F16 = capi.F32, capi.F16
+    for dt, n, k, want in ((F32, 8400, 300, (1024, 3, 1)), (F32, 8192, 300, (1024, 2, 1)), (F32, 16000, 300, (1024, 4, 1)),
+                           (F32, 16385, 300, (1024, 8, 1)), (F32, 4000, 130, (512, 2, 1)), (F32, 8190, 130, (512, 4, 1)),
+                           (F16, 8400, 300, (1024, 2, 1)), (F16, 8192, 300, (1024, 1, 1)), (F16, 20000, 300, (1024, 4, 1))):
+        assert capi.rows_plan(dt, (16, n), -1, k) == want, (dt, n, k)
+    try:
+        for shape in ((1024, 8, 1), (512, 8, 1), (1024, 4, 8)):
+            for name, value in zip(("rows.threads", "rows.loads", "rows.chunks"), shape):
+                capi.tune(name, value)
+            assert capi.rows_plan(F32, (16, 8400), -1, 100) == shape
+    finally:
+        for name in ("rows.threads", "rows.loads", "rows.chunks"):
+            capi.tune(name, 0)
+
+
 def test_native_front_end_refuses_what_the_operators_refuse():
     """vkop_amd.ops reaches the C ABI through its native front end, which is built with the library; a tensor that is not on
     a GPU, and what is no tensor, are TypeErrors before anything else happens."""

@@ -569,6 +569,9 @@ struct RowsCfg {
     int nt = 0, v = 0;
     uint32_t g = 0, per = 0;
     uint32_t cap = 0, cap_shift = 0;
+    bool forced = false;  // the shape that rows.threads, rows.loads and rows.chunks ask for
+    // a row that one workgroup holds never leaves it: list and records stay in LDS
+    bool local() const { return g == 1 && cap <= static_cast<uint32_t>(vkop::kLocalCap); }
 };
 
 // Candidate slots per chunk: 2.5 times the k+1 wanted elements (a chunk of
@@ -628,7 +631,7 @@ RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false, 
         c.nt = shapes[wide][0], c.v = shapes[wide][1], c.g = 1;
     } else if (forced_nt) {
         if (!fits(forced_nt, forced_v, static_cast<uint32_t>(forced_g)) || (n < vec && forced_v > 1)) return c;
-        c.nt = forced_nt, c.v = forced_v, c.g = static_cast<uint32_t>(forced_g);
+        c.nt = forced_nt, c.v = forced_v, c.g = static_cast<uint32_t>(forced_g), c.forced = true;
     } else if (k <= kWaveRowMaxK && wave_loads <= (dtype == VKOP_HIP_F32 ? 8u : 4u)) {
         c.nt = 64, c.g = 1;
         c.v = wave_loads <= 1 ? 1 : wave_loads <= 2 ? 2 : wave_loads <= 4 ? 4 : 8;
@@ -974,7 +977,7 @@ int launch_scan(const T *in, T *values, int32_t *indices, const View &v, int k, 
 // 17.8 / 15.4; [256,8000] k = 300 15.4 / 13.8, 18.6 / 15.8; [64,4000] k = 130 9.5 / 8.8, 11.3 / 9.9; [16,12000] k = 400 13.3 /
 // 12.1, 16.2 / 15.0.
 int fitted_loads(const RowsCfg &c, uint32_t n, uint32_t vec) {
-    if (c.nt < 512) return c.v;
+    if (c.nt < 512 || !c.local() || c.forced) return c.v;
     static const int f32_wide[] = {2, 3, 4}, f32_less[] = {2, 4}, f16[] = {1, 2};
     auto first = [&](const auto &loads) {
         for (const int v : loads)
@@ -1010,10 +1013,7 @@ int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, 
     a.g = c.g;
     a.per = c.per;
     a.aligned = (reinterpret_cast<uintptr_t>(in) % 16 == 0) && (v.g.n % vec == 0);
-    // a row that one workgroup holds never leaves it: list and records stay in LDS
-    a.merge = (c.g == 1 && c.cap <= static_cast<uint32_t>(vkop::kLocalCap)) ? vkop::kMergeLocal
-              : (c.g == 1 || by_ticket)                                         ? vkop::kMergeByTicket
-                                                                                : vkop::kMergeSplit;
+    a.merge = c.local() ? vkop::kMergeLocal : (c.g == 1 || by_ticket) ? vkop::kMergeByTicket : vkop::kMergeSplit;
     if (a.merge == vkop::kMergeLocal) {
         // the list is in LDS, where the kernel reserves kLocalCap entries whatever k is: all of them are the
         // list (an overflow -- values equal en masse at the cut -- makes the workgroup list a second time)
@@ -1754,7 +1754,7 @@ int vkop_hip_rows_plan(int dtype, const int *shape, int ndim, int axis, int k, i
     }
     const RowsCfg c = k >= 1 ? plan_fused(v, k, dtype, 1, false).rows : RowsCfg{};
     if (threads != nullptr) *threads = c.ok ? c.nt : 0;
-    if (loads != nullptr) *loads = c.ok ? c.v : 0;
+    if (loads != nullptr) *loads = c.ok ? fitted_loads(c, v.g.n, dtype == VKOP_HIP_F32 ? 4u : 8u) : 0;
     if (chunks != nullptr) *chunks = c.ok ? static_cast<int>(c.g) : 0;
     return VKOP_HIP_OK;
 }
