@@ -212,3 +212,35 @@ def test_two_streams_on_one_workspace_end(ops):
     capi.softmax(x.data_ptr(), out.data_ptr(), capi.F32, (rows, n), -1, 0, 0.0, at, need, stream)
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("rows,n", [(64, 65536), (64, 65540), (300, 20483), (32, 33001), (100, 9001), (150, 8200), (64, 200000), (64, 128256),
+                                    (64, 65537), (64, 65544), (64, 65543)])
+def test_in_place_while_other_chunks_are_written(ops, rows, n, dtype):
+    """In place, with looks limited to none, one and a few: workgroups read chunks whose own workgroups start and write over them
+    meanwhile.  Same bits as out of place; last vectors that reach back into the chunk before and ones that just do not."""
+    from vkop_amd import capi
+    lib = ctypes.CDLL(capi.BENCH_LIB_PATH)
+    f = lib.vkop_hip_softmax
+    f.argtypes = capi.lib()._signatures["vkop_hip_softmax"][1]
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.randn((rows, n), generator=gen, device="cuda").sub_(4.0).to(dtype)   # (a probability is above every logit of some chunks)
+    x[1, : n // 2] = float("-inf")
+    want = ops.softmax(x)
+    shape = (ctypes.c_int * 2)(rows, n)
+    dt = capi.F32 if dtype == torch.float32 else capi.F16
+    need = capi.lib().vkop_hip_softmax_workspace_bytes(dt, shape, 2, -1)
+    ws = torch.zeros(need + 256, dtype=torch.uint8, device="cuda")
+    at = ws.data_ptr() + (-ws.data_ptr()) % 256
+    stream = torch.cuda.current_stream().cuda_stream
+    try:
+        for polls in (0, 0, 0, 0, 1, 1, 3, 100):
+            assert lib.vkop_hip_measure_polls(polls) == 0
+            y = x.clone()
+            torch.cuda.synchronize()
+            assert f(y.data_ptr(), y.data_ptr(), dt, shape, 2, -1, 0, 0.0, at, need, stream) == 0
+            torch.cuda.synchronize()
+            assert torch.equal(y, want), polls
+    finally:
+        lib.vkop_hip_measure_polls(100)

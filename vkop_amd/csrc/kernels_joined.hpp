@@ -1,16 +1,18 @@
 // Softmax of long last-axis rows in one launch, one read and one write.
 //
-// A row is split into G <= 64 chunks, a workgroup each, as in the pair of kernels in kernels_softmax.hpp (statistics, scale),
-// which reads the tensor twice.  Here a workgroup keeps its chunk in registers, publishes the chunk's statistics, waits until
-// those of the row's other chunks are there and writes its probabilities.
+// A row is split into G chunks (plan_joined: at most 20; the reader of the records holds 64), a workgroup each, as in the pair of
+// kernels in kernels_softmax.hpp (statistics, scale), which reads the tensor twice.  Here a workgroup keeps its chunk in registers,
+// publishes the chunk's statistics, waits until those of the row's other chunks are there and writes its probabilities.
 // The wait needs no particular number of workgroups on the chip: workgroups start in order, so those of the rows before end
 // without this one's help, and after `polls` looks a workgroup that still misses a chunk (its workgroup has not started:
 // other streams' kernels hold the chip) reads that chunk itself.  Every wait ends, whatever else runs.
+// in == out is fine: a chunk is read by its own workgroup before that writes, and one that is read for another workgroup while its
+// own writes over it has its record in memory by then, which is looked for again after the read.  (Its last vector must not
+// reach back into the chunk before, which may have been written: the pair takes such rows in place.)
 // What bounds it: the arithmetic and the loads of the few workgroups a CU holds, half each -- [64,128256] f32 with neither
 // exponential takes 11.5 us, without the wait as long as with it -- and, with few rows, the wait.  us, the pair / this:
 // [64,128256] f32 22.1 / 16.2, f16 15.5 / 13.5; [500,128256] f32 119 / 105, f16 80 / 67; [500,50257] f32 56 / 44, f16 39 / 30.
-// The pair stays for calls in place (a chunk that is read for another workgroup must not have been overwritten), for rows of
-// more than 64 chunks, and for few rows of many chunks, where the wait is all there is ([8,262144] f32 8.8 / 10.2).
+// The pair stays for few rows of many chunks, where the wait is all there is.
 #pragma once
 
 #include "kernels_softmax.hpp"
@@ -66,9 +68,8 @@ template <typename T> __device__ __forceinline__ LineStats combine_wave(const Ch
 
 // Launch: rows * G workgroups, G = ceil(n / (NT * V * VEC)); recs: [rows][G] records, done: [rows], at zero before and after.
 template <typename T, int NT, int V>
-__global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict__ in, T *__restrict__ out, uint64_t *recs,
-                                                                          uint32_t *done, uint32_t n, uint32_t G, uint32_t tag,
-                                                                          uint32_t polls, int nan_where, float nan_value) {
+__global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *in, T *out, uint64_t *recs, uint32_t *done, uint32_t n, uint32_t G,
+                                                            uint32_t tag, uint32_t polls, int nan_where, float nan_value) {
     constexpr uint32_t VEC = Vec128<T>::N;
     static_assert(NT * V * VEC < (1 << 16), "a record's count");
     __shared__ ChunkScratch<NT> sh;
@@ -106,14 +107,24 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
             stats[tid] = c;  // (those of the missing chunks are written below)
         }
         if (tid == 0) sh_missing = missing;
+        // Its own record is in memory before the counter is raised -- whoever clears the records clears that too -- and before
+        // any of its probabilities is written.
+        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
     }
     __syncthreads();
     if (sh_missing != 0ull) {
         for (uint64_t left = sh_missing; left != 0ull; left &= left - 1ull) {
             const uint32_t c = static_cast<uint32_t>(__builtin_ctzll(left));
             ch.template load<false>(rowp, c, n);
-            const ChunkStat st = chunk_stats(ch, c, n, sh);
-            if (tid == 0) stats[c] = st;
+            ChunkStat st = chunk_stats(ch, c, n, sh);
+            if (tid < static_cast<uint32_t>(kWave)) {
+                // (in place the chunk's workgroup may have started and written over it by now: then its record came first)
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                ChunkWords w;
+                w.read(rrecs + c * kJoinedWords);
+                if (w.arrived(tag)) st = w.stat();
+                if (tid == 0) stats[c] = st;
+            }
         }
         __syncthreads();
         if (tid < static_cast<uint32_t>(kWave)) {
@@ -125,11 +136,10 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *__restrict_
         ch.template load<false>(rowp, again, n);
         __syncthreads();
     }
-    // This workgroup has read what it needs of the row's records, and its own is in memory: whoever clears them clears that too.
-    // (Whose answer is not waited for here: at an address the compiler takes for the same in every lane it would be, before
-    // the lanes that ask share it out.)
+    // This workgroup has read what it needs of the row's records.  (Whose answer is not waited for here: at an address the
+    // compiler takes for the same in every lane it would be, before the lanes that ask share it out.)
     uint32_t before = 0, same = 0;
-    asm volatile("s_waitcnt vmcnt(0)" : "+v"(same) : : "memory");
+    asm volatile("" : "+v"(same));
     if (tid == 0) before = __hip_atomic_fetch_add(done + row + same, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const Quotient<T> over_sum(row_stats.rinv);
     const float m = row_stats.m;

@@ -10,7 +10,7 @@
 //                           chunk, the second combines a row's chunk results and
 //                           writes exp(x - M) / S for its chunk.  The second
 //                           read of the input comes from the Infinity Cache for
-//                           tensors that fit it.  (Most such tensors, not in place: both in
+//                           tensors that fit it.  (Most such tensors: both in
 //                           one launch and one read, kernels_joined.hpp.)
 //   softmax_thread_kernel   rows of fewer elements than a vector.
 //   (each also without the tensor: the row's largest probability alone, from the same sum)

@@ -178,7 +178,7 @@ struct SoftmaxPlan {
     enum Kind { kGeneralLines, kGeneralStrided, kThread, kGroup, kRow, kChunked, kLinesRegs, kStridedRegs, kStridedTile } kind = kGeneralLines;
     RowShape shape{0, 0};  // kChunked; kGroup: lanes a row and vectors a lane; kRow: threads and vectors a thread
     uint32_t g = 1, per = 0;
-    bool joined = false;  // kChunked: in one launch where the tensors do not overlap
+    bool joined = false;  // kChunked: in one launch where the tensors allow it (joined_fits)
     uint32_t lines_k = 0, lines_p = 0, lines_w = 0;  // kLinesRegs: LinesLaunch
     uint32_t ti_shift = 0;  // kStridedTile: log2 of the lines a tile
     size_t workspace = 0;
@@ -384,10 +384,12 @@ int launch_lines(const T *in, T *out, const View &v, const SoftmaxPlan &p, bool 
     });
 }
 
-// Whether two tensors of `elems` elements share no byte.
-template <typename T> bool apart(const T *a, const T *b, uint64_t elems) {
-    const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
-    return (x < y ? y - x : x - y) >= elems * sizeof(T);
+// Whether softmax_joined_kernel may run on these tensors: they share no byte, or are the same and no row's last vector reaches
+// back into the chunk before its own.
+template <typename T> bool joined_fits(const T *in, const T *out, const View &v, const SoftmaxPlan &p) {
+    const auto x = reinterpret_cast<uintptr_t>(in), y = reinterpret_cast<uintptr_t>(out);
+    const uint32_t last = v.g.n % p.per;
+    return x == y ? last == 0 || last >= 16 / sizeof(T) : (x < y ? y - x : x - y) >= v.elems * sizeof(T);
 }
 
 template <typename T>
@@ -467,9 +469,9 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
     }
     case SoftmaxPlan::kChunked: {
         if (ws == nullptr || ws_bytes < p.pair_workspace)
-            return fail(VKOP_HIP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", ws_bytes, p.workspace);
+            return fail(VKOP_HIP_ERR_WORKSPACE, "workspace of %zu bytes given, %zu needed", ws_bytes, p.pair_workspace);
         // (a record is larger than a chunk's statistics: in a workspace that holds only those, the pair)
-        if (!MAX_ONLY && p.joined && ws_bytes >= p.workspace && apart(in, out, v.elems) &&
+        if (!MAX_ONLY && p.joined && ws_bytes >= p.workspace && joined_fits(in, out, v, p) &&
             reinterpret_cast<uintptr_t>(ws) % sizeof(uint64_t) == 0)
             return launch_joined(in, out, v, p, nan_where, nan_value, ws, st);
         auto *stats = reinterpret_cast<vkop::ChunkStat *>(static_cast<unsigned char *>(ws) + kTicketBytes);
