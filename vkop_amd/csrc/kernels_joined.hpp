@@ -86,20 +86,20 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *in, T *out,
     const ChunkStat mine = chunk_stats(ch, own, n, sh);
     if (tid < static_cast<uint32_t>(kWave)) {
         if (tid == 0) publish_chunk(rrecs + own * kJoinedWords, mine, tag);
-        // (its own record is not looked for: what a call that breaks the rules for a workspace does to it ends no wait late)
         ChunkWords w;
         uint64_t missing;
         for (uint32_t poll = 0;; poll++) {
             bool absent = false;
             if (tid < G) {
                 w.read(rrecs + tid * kJoinedWords);
-                absent = tid != own && !w.arrived(tag);
+                absent = !w.arrived(tag);
             }
             missing = __ballot(absent);
+            // (its own may be missing too: a call that breaks the rules for a workspace can take it away)
             if (missing == 0ull || poll >= polls) break;
             __builtin_amdgcn_s_sleep(1);
         }
-        const ChunkStat c = tid == own ? mine : w.stat();
+        const ChunkStat c = w.stat();
         if (missing == 0ull) {
             const LineStats st = combine_wave<T>(c, tid < G);
             if (tid == 0) row_stats = st;
