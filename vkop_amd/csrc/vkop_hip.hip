@@ -264,28 +264,46 @@ bool plan_lines(const View &v, uint32_t vec, SoftmaxPlan *p) {
     return true;
 }
 
-// The shape of softmax_joined_kernel for rows of a tensor, false where the pair of kernels is the faster one: 512 threads of as
-// many vectors (eight floats', four halves') as leave 150 workgroups, a row's in at most 16 chunks, or 8 of smaller
-// ones and of fewer than 32 rows of halves -- every workgroup of a row reads the records of all, again and again until they are there.  us, the pair / this: f32
+// The shape of softmax_joined_kernel for rows of a tensor, false where the pair of kernels is the faster one: below 150 workgroups,
+// and with a row in more chunks than 16, 20 of the narrow shape, or 8 of small ones and of fewer than 32 rows of halves -- every
+// workgroup of a row reads the records of all, again and again until they are there.  us, the pair / this: f32
 // [16,262144] 13.4 / 12.8 with 16 chunks, [16,65536] 7.8 / 8.0 with 8 in 128 workgroups, 9.1 with 16; [8,262144] 9.6 / 10.7 with
 // 32; [32,33001] 8.5 / 7.7; f16 [32,200000] 14.9 / 12.9, [32,65536] 8.3 / 7.9, [64,262144] 25.2 / 24.6,
 // [16,262144] 10.5 / 11.3.
-// More workgroups than the chip takes at once, and a last chunk left mostly empty: 256 threads of ten (five) vectors, in at most
-// 20 chunks, where they leave 3 % less empty.  us, 512 threads / 256: f32 [500,50257] 49.5 / 43.7, [64,200000] 28.5 / 24.8; f16
-// [500,33001] 30.1 / 24.5, [500,100003] 65.9 / 57.4; at once, [64,50257] f32 10.9 / 12.9.
+// Up to two of the widest shape a CU, the one whose workgroups end first (the narrow one where the widest leaves 150 too): so much a
+// call and so much for each one that a CU has to run, and every chunk that a workgroup reads a record of (in 0.01 us, fitted to 176 tensors of 64 to 510 rows of 8200 to 33000
+// elements in every shape).  With the widest ones that leave 150 workgroups instead, most of a chunk may be empty: f32 [150,12000] 9.9
+// / 7.7, [100,20000] 10.2 / 7.9, [300,12000] 13.6 / 10.9, [300,16400] 13.8 either way; f16 [150,20000] 9.6 / 8.6, [300,12000]
+// 11.4 / 9.9.
+// More: the widest, or the narrow one where it leaves 3 % less empty.  us, 512 threads / 256: f32 [500,50257] 49.5 / 43.7, [64,200000] 28.5 / 24.8; f16
+// [500,33001] 30.1 / 24.5, [500,100003] 65.9 / 57.4.
 bool plan_joined(const View &v, uint32_t vec, RowShape *shape) {
+    struct Candidate {
+        RowShape shape;
+        uint32_t call, each, most;
+    };
     const uint64_t n = v.g.n, rows = v.g.outer;
-    const int half = vec == 8 ? 2 : 1;
-    auto chunks = [&](const RowShape &c) { return (n + c.nt * c.v * vec - 1) / (c.nt * c.v * vec); };
-    auto held = [&](const RowShape &c) { return chunks(c) * c.nt * c.v; };
-    const RowShape wide{512, 8 / half}, fitted{256, 10 / half};
-    RowShape s = wide;
-    while (s.v > 2 / half && rows * chunks(s) < 150) s.v /= 2;
-    if (rows * chunks(s) < 150) return false;
-    uint32_t most = s.v == wide.v && (half == 1 || rows >= 32) ? 16 : 8;
-    if (rows * chunks(wide) > 256 && held(fitted) * 103 < held(wide) * 100) s = fitted, most = most == 16 ? 20 : 8;
-    if (chunks(s) > most) return false;
-    *shape = s;
+    const bool many = vec == 4 || rows >= 32;
+    const Candidate f32[] = {{{512, 8}, 520, 460, 16}, {{256, 10}, 690, 235, 20}, {{512, 4}, 540, 225, 8}, {{512, 2}, 480, 150, 8}};
+    const Candidate f16[] = {{{512, 4}, 490, 330, many ? 16u : 8u}, {{256, 5}, 630, 175, many ? 20u : 8u}, {{512, 2}, 480, 190, 8}, {{512, 1}, 500, 133, 8}};
+    const auto &of = vec == 4 ? f32 : f16;
+    auto chunks = [&](const Candidate &c) { return (n + c.shape.nt * c.shape.v * vec - 1) / (c.shape.nt * c.shape.v * vec); };
+    auto held = [&](const Candidate &c) { return chunks(c) * c.shape.nt * c.shape.v; };
+    const Candidate *best = nullptr;
+    if (rows * chunks(of[0]) > 512) {
+        best = held(of[1]) * 103 < held(of[0]) * 100 ? &of[1] : &of[0];
+        if (chunks(*best) > best->most) return false;
+    } else {
+        uint64_t least = 0;
+        for (const Candidate &c : of) {
+            const uint64_t groups = rows * chunks(c), cost = c.call + (groups + 255) / 256 * c.each + chunks(c) * 15;
+            if (groups < 150 || groups > 1024 || chunks(c) > c.most || (best != nullptr && cost >= least)) continue;
+            if (&c == &of[1] && rows * chunks(of[0]) < 150) continue;
+            best = &c, least = cost;
+        }
+        if (best == nullptr) return false;
+    }
+    *shape = best->shape;
     return true;
 }
 
