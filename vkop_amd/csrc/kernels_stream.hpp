@@ -268,6 +268,7 @@ struct PickShared {
     uint4 stage_v[kPickThreads / kWave][kWave];     // per wave: the vectors that hold an element at or above the threshold ...
     uint32_t stage_e[kPickThreads / kWave][kWave];  // ... and the index of their first element
     uint32_t trial_cnt[kPickThreads / kWave][kPickThreads / kWave];  // [wave][trial]: the wave's thread maxima that reach another wave's bound
+    uint32_t waves_above;  // waves whose list does not go on below the threshold
 };
 union PickSharedUnion {
     PickShared pick;
@@ -355,6 +356,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     if (tid == 0) {
         sh.count = 0;
         sh.wave_overflow = 0;
+        smem.pick.waves_above = 0;
     }
     auto combine_records = [&]() __attribute__((always_inline)) {
       if constexpr (SOFTMAX) {
@@ -486,18 +488,6 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     // -inf never becomes a candidate: a row with k+1 larger elements does not need it,
     // and finish_row fills any other row's last places from the row itself
     thr = max(thr, kKeyNegInf + 1u);
-    // The list goes on a little below the threshold, so that the group of equal probabilities at the k-th place ends inside it
-    // and E1 can tell (else the row starts over below, 5 to 10 us of a call).  Floats: logits that far apart have different
-    // probabilities unless those are subnormal -- x - M is rounded by at most 2^-18 wherever its exponential is not 0, and terms
-    // of differences 2^-17 apart are 64 places of a float apart.  It lists next to nothing more, and the threshold is an element's
-    // value: of logits that went through bfloat16 the list ended with the group in a few rows of every call ([64,128256]
-    // k = 50 18.7 us, [64,32000] k = 40 15.4, [32,50257] k = 40 17.0; so 14.1, 10.3, 11.5).  Halves: the probabilities of logits closer
-    // than 0.01 are often equal, and seldom those of others (from 100 of the smallest half on).  It is one candidate in a hundred more: sampling
-    // [32,50257] k = 40 by the inputs 14.0 / 14.0 / 19.3 us, with the threshold as found 13.8 to 22.2.
-    if constexpr (SOFTMAX) {
-        constexpr float kBelow = sizeof(T) == 2 ? 1e-2f : 0x1p-16f;
-        thr = max(min(thr, order_key(ordered_to_float(thr) - kBelow)), kKeyNegInf + 1u);
-    }
 
     // ---- D1. the first gather, wave by wave ------------------------------------------------
     // Every wave reads again ITS threads' blocks that reach thr (a list of its own in LDS: no
@@ -511,21 +501,45 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     constexpr uint32_t kWaveHitCap = 2 * U * (kWave / kBlockLanes);  // blocks a wave reads again in one go
     static_assert(NW * kWaveHitCap <= kPickHitCap, "every wave's list of blocks fits");
     static_assert(NW <= kPickThreads / kWave, "a stage per wave");
+    static_assert(NT <= kFastMaxK + 1, "a place by rank for every candidate of E1");
     // About 1.15 (k+1) blocks reach thr, a wave's share of them has to fit its list, and the shares are not alike:
     // from five eighths of the lists' total on, some wave of most rows has too many, and what the waves did is
     // thrown away (an unaligned row pays a load per element for it).  Such rows go the general way at once.
     const bool wave_lists = want <= NW * kWaveHitCap * 5u / 8u;
+    // The lists go on a little below the threshold, so that the group of equal probabilities at the k-th place ends inside them
+    // and E1 can tell (else the row starts over below, 5 to 10 us of a call).  Floats: logits that far apart have different
+    // probabilities unless those are subnormal -- x - M is rounded by at most 2^-18 wherever its exponential is not 0, and terms
+    // of differences 2^-17 apart are 64 places of a float apart.  The threshold is an element's
+    // value: of logits that went through bfloat16 the list ended with the group in a few rows of every call ([64,128256]
+    // k = 50 18.7 us, [64,32000] k = 40 15.4, [32,50257] k = 40 17.0; so 14.1, 10.3, 11.5).  Halves: the probabilities of logits closer
+    // than 0.01 are often equal, and seldom those of others (from 100 of the smallest half on).  It is one candidate in a hundred more: sampling
+    // [32,50257] k = 40 by the inputs 14.0 / 14.0 / 19.3 us, with the threshold as found 13.8 to 22.2.
+    // Not in rows so narrow that it is many more: a wave with four times its share of k + 1 blocks keeps to the threshold.
+    uint32_t low = thr;
+    if constexpr (SOFTMAX) {
+        constexpr float kBelow = sizeof(T) == 2 ? 1e-2f : 0x1p-16f;
+        low = max(min(thr, order_key(ordered_to_float(thr) - kBelow)), kKeyNegInf + 1u);
+    }
     if (wave_lists) {
-        uint32_t wave_n = 0;  // wave-uniform
+        uint32_t wave_n = 0, own_thr = low;  // wave-uniform
 #pragma unroll
-        for (int e = 0; e < GE; e++) wave_n += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= thr)));
+        for (int e = 0; e < GE; e++) wave_n += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= low)));
+        if constexpr (SOFTMAX) {
+            if (wave_n > min(want / (NW / 4) + 4u, kWaveHitCap)) {
+                own_thr = thr;
+                wave_n = 0;
+#pragma unroll
+                for (int e = 0; e < GE; e++) wave_n += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= thr)));
+                if (lane == 0) atomicAdd(&smem.pick.waves_above, 1u);
+            }
+        }
         const bool wave_ok = wave_n <= kWaveHitCap;
         uint32_t *whits = hits + wave * kWaveHitCap;
         if (wave_ok) {
             uint32_t pos = 0;
 #pragma unroll
             for (int e = 0; e < GE; e++) {
-                const bool pass = gk[e] >= thr;
+                const bool pass = gk[e] >= own_thr;
                 const uint64_t mask = __ballot(pass);
                 if (pass) whits[pos + lanes_below(mask)] = static_cast<uint32_t>(e) * NT + tid;
                 pos += static_cast<uint32_t>(__popcll(mask));
@@ -533,7 +547,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         }
         __builtin_amdgcn_wave_barrier();  // (the wave reads its own list: LDS keeps a wave's accesses in order)
         const uint32_t items = wave_ok ? wave_n * kBlockLanes : 0u;  // one per vector of a block that is read again
-        const float lo_f = ordered_to_float(thr);
+        const float lo_f = ordered_to_float(own_thr);
         Vec128<T> r[2 * U];
         uint32_t e0[2 * U];
         auto issue = [&](auto u_tag) __attribute__((always_inline)) {
@@ -593,7 +607,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                 // (softmax: a NaN never passes, and thr is the key of a number, so the floats compare as the keys do)
                 bool pass;
                 if constexpr (SOFTMAX || kReversed<T>) pass = x >= lo_f;
-                else pass = order_key(x) >= thr;
+                else pass = order_key(x) >= own_thr;
                 pass = pass && lane < nv && (ALIGNED || eb + static_cast<uint32_t>(c) < n);
                 pbits |= pass ? (1u << c) : 0u;
             }
@@ -625,6 +639,39 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         M = sh.row_max;
         s_base = sh.total;
     }
+    bool listed = wave_lists && sh.wave_overflow == 0u;  // every wave listed all of its elements at or above thr (the same in every thread)
+    if constexpr (SOFTMAX) {
+        // The list as far down as all waves went, and so far only where that leaves it within what the ranking of E1 takes at its
+        // quickest (past 128 entries 4 us more): what some waves listed below the threshold goes out again otherwise (about 1 us).
+        // us, [32,50257] k = 40, every list to the threshold / below it / so: f16 rows spread by 0.3 21.0 / 13.0 / 13.0, 0.05 22.2 /
+        // 14.9 / 14.8, 0.02 23.0 / 31.0 / 24.5, 0.001 32.4 / 38.5 / 34.2; f32 1e-4 12.5 / 16.6 / 12.7, 2e-5 12.4 / 24.0 / 12.3; k = 100
+        // f16 0.3 15.7 / 22.0 / 16.2; spread by 1 12.4 and 11.4 either way.
+        const uint32_t above = smem.pick.waves_above, have = sh.count;
+        if (listed && above == 0u && have <= (want <= 112u ? 128u : 256u)) {
+            thr = low;
+        } else if (listed && above != static_cast<uint32_t>(NW) && low < thr) {
+            listed = have <= static_cast<uint32_t>(kFastCap);
+            static_assert(kFastCap % NT == 0, "entries a thread");
+            uint64_t entry[kFastCap / NT];
+#pragma unroll
+            for (int e = 0; e < kFastCap / NT; e++) entry[e] = sh.cand[static_cast<uint32_t>(e) * NT + tid];
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < kFastCap / NT; e++) sh.cand[static_cast<uint32_t>(e) * NT + tid] = 0;
+            if (tid == 0) sh.count = 0;
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < kFastCap / NT; e++) {
+                const bool stays = static_cast<uint32_t>(e) * NT + tid < have && static_cast<uint32_t>(entry[e] >> 32) >= thr;
+                const uint64_t mask = __ballot(stays);
+                uint32_t at = 0;
+                if (lane == 0 && mask != 0ull) at = atomicAdd(&sh.count, static_cast<uint32_t>(__popcll(mask)));
+                at = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(at)));
+                if (stays) sh.cand[at + lanes_below(mask)] = entry[e];
+            }
+            __syncthreads();
+        }
+    }
     const uint32_t per_shift = 31u - static_cast<uint32_t>(__clz(per));
     // the scan-kernel wave that summed element idx (per = 256 * V vectors: a power of two)
     auto wave_of = [&](uint32_t idx) {
@@ -642,7 +689,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     // logit of rank k is in the list -- which is what logits that went through bfloat16 or int8 are full of.
     {
         const uint32_t C2 = sh.count;
-        bool common = wave_lists && sh.wave_overflow == 0u && C2 >= want && C2 <= static_cast<uint32_t>(NT) && kk == k;
+        bool common = listed && C2 >= want && C2 <= static_cast<uint32_t>(NT) && kk == k;
         if constexpr (SOFTMAX) common = common && s_base > 0.0 && s_base < static_cast<double>(INFINITY) && M > -INFINITY && M < INFINITY;
         if (__builtin_expect(common, 1)) {
             // A candidate's own part (its wave's record, its accurate term) and the ranking are two chains of
@@ -798,7 +845,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         // The general code: with the list the waves made, if every wave could list all of its blocks
         // (the list may still hold fewer than k+1 entries, or have dropped what came after its capacity:
         // sh.count says how many there were), else from an empty one.
-        have_list = wave_lists && sh.wave_overflow == 0u;
+        have_list = listed;
         __syncthreads();
         for (uint32_t t = tid; t < static_cast<uint32_t>(kFastCap); t += NT) sh.rank[t] = 0;
         if (!have_list && tid == 0) sh.count = 0;
