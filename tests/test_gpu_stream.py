@@ -299,9 +299,17 @@ def test_wide_workgroups_with_the_vectors_a_row_needs(ops, n, k, dtype):
             t, tj = ops.topk(xd, k, largest=largest)
             et, ej = oracle.topk(x, k, largest=largest)
             assert np.array_equal(host(tj), ej) and np.array_equal(host(t).view(bits), et.view(bits)), (kind, largest)
-        v, ix = ops.softmax_topk(xd, k)
+        v, ix = (host(t) for t in ops.softmax_topk(xd, k))
         ov, oix = oracle.softmax_topk(x, k)
-        assert (half_ulp_diff if dtype == np.float16 else ulp_diff)(host(v), ov).max() <= (1 if dtype == np.float16 else 2), kind
+        assert (half_ulp_diff if dtype == np.float16 else ulp_diff)(v, ov).max() <= (1 if dtype == np.float16 else 2), kind
+        xf, op = x.astype(np.float32), oracle.softmax(x).astype(np.float32)
+        for r in range(17):
+            if np.isfinite(v[r]).all():
+                check_fused_invariants(xf[r], v[r].astype(np.float32), ix[r])
+            else:
+                assert np.array_equal(ix[r], np.arange(k)), (kind, r)  # all-NaN row: lowest indices
+            if well_separated_cut(op[r], xf[r], k, 4 if dtype == np.float32 else 1 << 14):
+                assert np.array_equal(ix[r], oix[r]), (kind, r)
 
 
 @pytest.mark.parametrize("rows,n,k", [(17, 20001, 16), (8, 20001, 16), (24, 50000, 40), (5, 131072, 64), (16, 16385, 5)])
