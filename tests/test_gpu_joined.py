@@ -48,7 +48,7 @@ def test_rows_against_the_oracle_and_the_pair_of_kernels(ops, rows, n, dtype, st
     again = ops.softmax(t)
     replaced = ops.softmax(t, nan_where=True, nan_value=7.0)
     inplace = t.clone()
-    ops.softmax(inplace, out=inplace)    # (the pair: a chunk may be read for another workgroup)
+    ops.softmax(inplace, out=inplace)    # (the one launch too; the pair where the last vector reaches back into the chunk before)
     best = ops.softmax_reduce_max(t, -1)
     torch.cuda.synchronize()
     bits = torch.int32 if dtype == np.float32 else torch.int16
@@ -216,7 +216,7 @@ def test_two_streams_on_one_workspace_end(ops):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("rows,n", [(64, 65536), (64, 65540), (300, 20483), (32, 33001), (100, 9001), (150, 8200), (64, 200000), (64, 128256),
-                                    (64, 65537), (64, 65544), (64, 65543)])
+                                    (64, 65537), (64, 65544), (64, 65543), (300, 20484), (300, 20487), (300, 20488)])
 def test_in_place_while_other_chunks_are_written(ops, rows, n, dtype):
     """In place, with looks limited to none, one and a few: workgroups read chunks whose own workgroups start and write over them
     meanwhile.  Same bits as out of place; last vectors that reach back into the chunk before and ones that just do not."""
