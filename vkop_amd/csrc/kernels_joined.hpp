@@ -11,7 +11,7 @@
 // reach back into the chunk before, which may have been written: the pair takes such rows in place.)
 // What bounds it: the arithmetic and the loads of the few workgroups a CU holds, half each -- [64,128256] f32 with neither
 // exponential takes 11.5 us, without the wait as long as with it -- and, with few rows, the wait.  us, the pair / this:
-// [64,128256] f32 22.1 / 16.2, f16 15.5 / 13.5; [500,128256] f32 119 / 105, f16 80 / 67; [500,50257] f32 56 / 44, f16 39 / 30.
+// [64,128256] f32 21.9 / 16.3, f16 14.9 / 13.2; [500,50257] f32 55.3 / 43.5, f16 37.8 / 28.3; [32,33001] f32 8.7 / 8.0, f16 7.8 / 7.3.
 // The pair stays for few rows of many chunks, where the wait is all there is.
 #pragma once
 

@@ -36,7 +36,7 @@ template <int STRIDE> __device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
 // the lines out: a step exchanges one half of the values for the other lane's other half (one swap and one operation for two
 // values), so that after the steps of 32 and 16 lanes a lane holds kOwned = L / min(P, 4) of the lines, from owned_line() on;
 // the steps of 8 and 4 leave both lanes of a pair with them.  (With every value to every lane each step costs four times as much:
-// exchanges, not terms, were 40 % of the instructions of a line's largest probability: [16,80,8400] f32 13.5 -> 12.2 us; the tensor [8,21,262144] 67.5 -> 66.5.)  The sum adds
+// exchanges, not terms, were 40 % of the instructions of a line's largest probability: [16,80,8400] f32 13.5 -> 12.2 us; the tensor's time is the memory's and did not change.)  The sum adds
 // both lanes of a pair in the same order, so every lane ends with the same bits.
 template <int STRIDE> __device__ __forceinline__ void swap_lanes(uint32_t &a, uint32_t &b) {
     if constexpr (STRIDE == 32) {

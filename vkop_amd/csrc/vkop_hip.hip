@@ -267,8 +267,8 @@ bool plan_lines(const View &v, uint32_t vec, SoftmaxPlan *p) {
 // The shape of softmax_joined_kernel for rows of a tensor, false where the pair of kernels is the faster one: below 150 workgroups,
 // and with a row in more chunks than 16, 20 of the narrow shape, or 8 of small ones and of fewer than 32 rows of halves -- every
 // workgroup of a row reads the records of all, again and again until they are there.  us, the pair / this: f32
-// [16,262144] 13.4 / 12.8 with 16 chunks, [16,65536] 7.8 / 8.0 with 8 in 128 workgroups, 9.1 with 16; [8,262144] 9.6 / 10.7 with
-// 32; [32,33001] 8.5 / 7.7; f16 [32,200000] 14.9 / 12.9, [32,65536] 8.3 / 7.9, [64,262144] 25.2 / 24.6,
+// [16,262144] 14.0 / 13.2 with 16 chunks, [16,65536] 7.8 / 8.0 with 8 in 128 workgroups, 9.1 with 16; [8,262144] 9.6 / 10.2 with
+// 16, 10.7 with 32; [32,33001] 8.7 / 8.0; f16 [32,200000] 14.5 / 13.1, [32,65536] 8.4 / 7.8, [64,262144] 23.7 / 20.9,
 // [16,262144] 10.5 / 11.3.
 // Up to two of the widest shape a CU, the one whose workgroups end first (the narrow one where the widest leaves 150 too): so much a
 // call and so much for each one that a CU has to run, and every chunk that a workgroup reads a record of (in 0.01 us, fitted to 176 tensors of 64 to 510 rows of 8200 to 33000
