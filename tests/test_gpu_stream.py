@@ -512,8 +512,8 @@ def test_float_rows_with_equal_logits_at_the_cut(ops, k):
 @pytest.mark.parametrize("spread", [2.0 ** -i for i in (3, 4, 5, 6, 9, 12, 13, 14, 15, 18, 21)])
 @pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
 def test_rows_of_small_range_whose_list_goes_on_below_its_threshold(ops, spread, dtype):
-    """Rows so narrow that the stretch below the threshold (0.01 of halves, 2^-16 of floats) holds dozens, hundreds or all of
-    their elements, with and without a peak."""
+    """Rows so narrow that the stretch below the threshold (0.01 of halves, 2^-13 of a float threshold) holds dozens, hundreds or
+    all of their elements, with and without a peak."""
     rng = np.random.default_rng(int(1 / spread))
     x = (rng.standard_normal((9, 50257)) * spread).astype(np.float32)
     x[3:6] += np.float32(0.75)
@@ -563,8 +563,8 @@ def test_a_tie_at_the_cut_costs_no_second_look(ops):
 
 
 def test_a_row_of_small_range_costs_no_longer_list(ops):
-    """[32,50257] k = 40 of rows spread by 2e-5, where 2^-16 below the threshold lies most of the row, against rows spread by 0.3
-    (listed down there they took 2.1 times as long, 1.1 times where not).  These rows have no more than 128 elements at their
+    """[32,50257] k = 40 of rows spread by 2e-5 against rows spread by 0.3 (listed to 2^-16 below the threshold, where most of such a
+    row lies, they took 2.1 times as long; 1.1 times to 2^-13 of it).  These rows have no more than 128 elements at their
     thresholds, past which the ranking takes longer.  The least of nine means of 40 calls each, the two in turn."""
     x = np.random.default_rng(6).standard_normal((32, 50257)).astype(np.float32)
     inputs = {spread: dev(x * np.float32(spread)) for spread in (0.3, 2e-5)}

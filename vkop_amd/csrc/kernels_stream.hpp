@@ -507,24 +507,24 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     // thrown away (an unaligned row pays a load per element for it).  Such rows go the general way at once.
     const bool wave_lists = want <= NW * kWaveHitCap * 5u / 8u;
     // The lists go on a little below the threshold, so that the group of equal probabilities at the k-th place ends inside them
-    // and E1 can tell (else the row starts over below, 5 to 10 us of a call).  Floats: logits that far apart have different
-    // probabilities unless those are subnormal -- x - M is rounded by at most 2^-18 wherever its exponential is not 0, and terms
-    // of differences 2^-17 apart are 64 places of a float apart.  The threshold is an element's
-    // value: of logits that went through bfloat16 the list ended with the group in a few rows of every call ([64,128256]
-    // k = 50 18.7 us, [64,32000] k = 40 15.4, [32,50257] k = 40 17.0; so 14.1, 10.3, 11.5).  Halves: the probabilities of logits closer
+    // and E1 can tell (else the row starts over below, 5 to 10 us of a call).  Floats: by 2^-13 of the threshold, whose own last
+    // place is 2^-9 of it, so rows of any scale list next to nothing more.  Logits 2^-17 apart have different probabilities unless
+    // those are subnormal -- x - M is rounded by at most 2^-18 wherever its exponential is not 0 -- and so has what lies below
+    // thresholds from 0.06 on.  The threshold can be an element's value: of logits that went through bfloat16 the list ended with
+    // the group in a few rows of every call ([64,128256]
+    // k = 50 18.7 us, [64,32000] k = 40 15.4, [32,50257] k = 40 17.0; so 14.0, 10.2, 11.4).  Halves: the probabilities of logits closer
     // than 0.01 are often equal, and seldom those of others (from 100 of the smallest half on).  It is one candidate in a hundred more: sampling
     // [32,50257] k = 40 by the inputs 14.0 / 14.0 / 19.3 us, with the threshold as found 13.8 to 22.2.
     // Not in rows so narrow that it is many more: a wave with four times its share of k + 1 blocks keeps to the threshold.
+    constexpr bool kByDifference = SOFTMAX && sizeof(T) == 2;
+    if constexpr (SOFTMAX && !kByDifference) thr = max(thr - 1024u, kKeyNegInf + 1u);
     uint32_t low = thr;
-    if constexpr (SOFTMAX) {
-        constexpr float kBelow = sizeof(T) == 2 ? 1e-2f : 0x1p-16f;
-        low = max(min(thr, order_key(ordered_to_float(thr) - kBelow)), kKeyNegInf + 1u);
-    }
+    if constexpr (kByDifference) low = max(min(thr, order_key(ordered_to_float(thr) - 1e-2f)), kKeyNegInf + 1u);
     if (wave_lists) {
         uint32_t wave_n = 0, own_thr = low;  // wave-uniform
 #pragma unroll
         for (int e = 0; e < GE; e++) wave_n += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= low)));
-        if constexpr (SOFTMAX) {
+        if constexpr (kByDifference) {
             if (wave_n > min(want / (NW / 4) + 4u, kWaveHitCap)) {
                 own_thr = thr;
                 wave_n = 0;
@@ -640,12 +640,11 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         s_base = sh.total;
     }
     bool listed = wave_lists && sh.wave_overflow == 0u;  // every wave listed all of its elements at or above thr (the same in every thread)
-    if constexpr (SOFTMAX) {
+    if constexpr (kByDifference) {
         // The list as far down as all waves went, and so far only where that leaves it within what the ranking of E1 takes at its
         // quickest (past 128 entries 4 us more): what some waves listed below the threshold goes out again otherwise (about 1 us).
-        // us, [32,50257] k = 40, every list to the threshold / below it / so: f16 rows spread by 0.3 21.0 / 13.0 / 13.0, 0.05 22.2 /
-        // 14.9 / 14.8, 0.02 23.0 / 31.0 / 24.5, 0.001 32.4 / 38.5 / 34.2; f32 1e-4 12.5 / 16.6 / 12.7, 2e-5 12.4 / 24.0 / 12.3; k = 100
-        // f16 0.3 15.7 / 22.0 / 16.2; spread by 1 12.4 and 11.4 either way.
+        // us, [32,50257] k = 40, every list to the threshold / below it / so: rows spread by 0.3 21.0 / 13.0 / 13.0, 0.05 22.2 /
+        // 14.9 / 14.8, 0.02 23.0 / 31.0 / 24.5, 0.001 32.4 / 38.5 / 34.2; k = 100 0.3 15.7 / 22.0 / 16.2; spread by 1 12.4 either way.
         const uint32_t above = smem.pick.waves_above, have = sh.count;
         if (listed && above == 0u && have <= (want <= 112u ? 128u : 256u)) {
             thr = low;
