@@ -283,6 +283,30 @@ def test_softmax_nan_of_any_payload(ops, shape, axis):
         assert np.array_equal(np.isnan(best), held) and np.array_equal(best[~held], got[~held].max(-1)), dtype
 
 
+@pytest.mark.parametrize("dtype,shape,axis", [
+    ("f16", (170001, 100), -1), ("f32", (61001, 197), -1), ("f32", (85001, 100), -1),   # pieces off the lines: both ordinary
+    ("f16", (660001, 50), -1), ("f16", (66001, 256), -1), ("f32", (2001, 1000), -1),    # loads alone
+    ("f32", (100001, 256), -1), ("f16", (110001, 500), -1),                             # stores alone
+    ("f32", (1301, 8191), -1), ("f16", (2441, 8192), -1),                               # a row a workgroup
+    ("f32", (32, 512, 1024), 1), ("f32", (8, 80, 13108), 1), ("f32", (8, 100, 11001), 1), ("f32", (8, 21, 163840), 1),
+    ("f32", (8, 100, 42001), 1), ("f16", (8, 21, 262144), 1), ("f16", (8, 100, 84001), 1), ("f16", (8, 100, 50001), 1),
+])
+def test_softmax_ordinary_accesses(ops, dtype, shape, axis):
+    """Tensors of every size and place that takes other accesses than non-temporal ones, whole, against 64 bits, out of place and in
+    place; their largest probability is the tensor's maximum bit for bit.  Bounds: 2 ulp of float, one of half."""
+    gen = torch.Generator(device="cuda").manual_seed(sum(shape))
+    x = torch.empty(shape, dtype=torch.float16 if dtype == "f16" else torch.float32, device="cuda").normal_(0.0, 2.0, generator=gen)
+    got = ops.softmax(x, axis)
+    best = ops.softmax_reduce_max(x, axis)
+    e = torch.exp((x.float() - x.float().amax(axis, keepdim=True)).double())  # (the difference in float, as the softmax is defined)
+    e /= e.sum(axis, keepdim=True)
+    rel, least = (2.0 ** -10, 2.0 ** -24) if dtype == "f16" else (2.0 ** -22, 0.0)
+    assert bool(((got.double() - e).abs() <= rel * e + least).all())
+    assert torch.equal(best, got.amax(axis).reshape(best.shape))
+    ops.softmax(x, axis, out=x)
+    assert torch.equal(x, got)
+
+
 def test_softmax_in_place(ops):
     x = synth.classifier_logits(16, 1000, seed=3)
     xd = dev(x)

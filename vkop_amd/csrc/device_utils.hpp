@@ -59,9 +59,9 @@ template <> __device__ __forceinline__ float round_to_storage<uint16_t>(float v)
 // 16 bytes of a tensor that start on any element: a 128-bit load or store needs no more than the
 // element's own alignment on this chip (rows of odd length start anywhere).  Measured on a stream
 // of 128 MB: starts on 4 or 8 bytes cost nothing (6.3 TB/s read), starts on 2 bytes a fifth (5.1).
-// The stores, and the loads they go with, are non-temporal: what a softmax tensor holds is not
-// used again by the call, and keeping it out of the caches' way takes a copy of 32 MB from 3.0 to
-// 5.8 TB/s, of 1 GB from 5.7 to 6.2 (four vectors a thread).
+// The _stream ones are non-temporal: what a softmax tensor holds is not
+// used again by the call, and keeping it out of the caches' way takes a copy of 1 GB from 5.7 to 6.2 TB/s
+// (four vectors a thread).  Where ordinary ones are better: softmax_caching.
 typedef uint32_t vec16_any __attribute__((ext_vector_type(4), aligned(2)));
 template <typename T> __device__ __forceinline__ uint4 load16_stream(const T *p) {
     const auto v = __builtin_nontemporal_load(reinterpret_cast<const vec16_any *>(p));
@@ -81,6 +81,18 @@ template <typename T> __device__ __forceinline__ void store16_any(T *p, const ui
     vec16_any v;
     v.x = u.x, v.y = u.y, v.z = u.z, v.w = u.w;
     *reinterpret_cast<vec16_any *>(p) = v;
+}
+
+// Which accesses of a softmax kernel to its tensors are ordinary ones (a template parameter: of two branches on a flag the
+// compiler makes one).
+enum Caching : int { kCacheNone = 0, kCacheLoads = 1, kCacheStores = 2, kCacheBoth = kCacheLoads | kCacheStores };
+template <int CACHE, typename T> __device__ __forceinline__ uint4 load16(const T *p) {
+    if constexpr ((CACHE & kCacheLoads) != 0) return load16_any(p);
+    else return load16_stream(p);
+}
+template <int CACHE, typename T> __device__ __forceinline__ void store16(T *p, const uint4 &u) {
+    if constexpr ((CACHE & kCacheStores) != 0) store16_any(p, u);
+    else store16_stream(p, u);
 }
 
 // Larger of three floats, quiet NaN dropped (fmaxf on loaded values costs one more instruction an operand:

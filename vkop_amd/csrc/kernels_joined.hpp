@@ -82,7 +82,7 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *in, T *out,
     const T *rowp = in + row0;
     uint64_t *rrecs = recs + static_cast<size_t>(row) * G * kJoinedWords;
     Chunk<T, NT, V> ch;
-    ch.template load<false>(rowp, own, n);
+    ch.template load<kCacheNone>(rowp, own, n);
     const ChunkStat mine = chunk_stats(ch, own, n, sh);
     if (tid < static_cast<uint32_t>(kWave)) {
         if (tid == 0) publish_chunk(rrecs + own * kJoinedWords, mine, tag);
@@ -115,7 +115,7 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *in, T *out,
     if (sh_missing != 0ull) {
         for (uint64_t left = sh_missing; left != 0ull; left &= left - 1ull) {
             const uint32_t c = static_cast<uint32_t>(__builtin_ctzll(left));
-            ch.template load<false>(rowp, c, n);
+            ch.template load<kCacheNone>(rowp, c, n);
             ChunkStat st = chunk_stats(ch, c, n, sh);
             if (tid < static_cast<uint32_t>(kWave)) {
                 // (in place the chunk's workgroup may have started and written over it by now: then its record came first)
@@ -133,7 +133,7 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *in, T *out,
         }
         uint32_t again = own;
         asm volatile("" : "+s"(again));  // (places again: the first load's, kept till here, are 16 registers)
-        ch.template load<false>(rowp, again, n);
+        ch.template load<kCacheNone>(rowp, again, n);
         __syncthreads();
     }
     // This workgroup has read what it needs of the row's records.  (Whose answer is not waited for here: at an address the

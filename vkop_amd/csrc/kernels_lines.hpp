@@ -118,17 +118,15 @@ template <int P, int L> __device__ __forceinline__ uint32_t owned_line(uint32_t 
 // K = ceil(n / (P * W)): every element but a lane's last exists.
 // Launch: blockDim = teams * W waves, a team of W waves per 64 / P vectors; LDS for W > 1:
 // 64 / P * L * (W * teams) doubles.
-// cached: ordinary stores.  A piece of a row that begins or ends inside a cache line shares that line with another wave's;
-// stored past the caches each part goes to memory by itself ([8,100,83886] f32 235 us, ordinary 120; [8,128,65537] f16 169 /
-// 85).  On whole lines, and on tensors that the caches hold anyway, non-temporal ones stay ahead ([8,21,262144] 66 / 71;
-// [8,32,16385] f32 12.4 / 14.1).
+// CACHE: softmax_caching (stored past the caches, the parts of a cache line go to memory one by one: [8,100,83886] f32 235 us,
+// with ordinary stores 120; [8,128,65537] f16 169 / 85).
 // WIDE: a lane adds its terms in double.  Halves in one wave a line add up to eight of them in float (TermSum), which
 // [8,21,262144] is worth 2 %; longer lines, more of them in all, do not.
 // (the largest probability of halves is held to 64 registers, which K = 8 exceeds by one: two workgroups of 16 waves a CU
 // instead of one, [8,1000,8000] 47 against 61 us)
-template <typename T, int K, int P, bool MAX_ONLY, bool WIDE>
+template <typename T, int K, int P, bool MAX_ONLY, bool WIDE, int CACHE>
 __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 2 && MAX_ONLY ? 8 : 4))) void softmax_lines_reg_kernel(const T *in, T *out, LineGeom g, uint32_t W,
-                                                                                int nan_where, float nan_value, bool cached) {
+                                                                                int nan_where, float nan_value) {
     constexpr int L = Vec128<T>::N;
     constexpr uint32_t LPW = kWave / P;  // vectors (of L lines) a wave
     extern __shared__ double lines_lds[];
@@ -150,7 +148,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
 #pragma unroll
     for (int i = 0; i < K; i++) {
         const uint32_t j = static_cast<uint32_t>(i) * parts + part;
-        q[i].v = load16_stream(in + base + static_cast<size_t>(i < K - 1 || last_ok ? j : n - 1u) * g.inner);
+        q[i].v = load16<CACHE>(in + base + static_cast<size_t>(i < K - 1 || last_ok ? j : n - 1u) * g.inner);
     }
     constexpr int C = L / kLineSharers<P>, EXTRA = P / kLineSharers<P>;  // lines a lane owns, lanes that own the same
     const uint32_t own0 = owned_line<P, L>(lane), extra = (lane / LPW) % EXTRA;
@@ -298,8 +296,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
             r.set(c, p[c]);
         }
         if (live && (i < K - 1 || last_ok)) {
-            if (skip == 0 && !cached) store16_stream(out + at, r.v);
-            else if (skip == 0) store16_any(out + at, r.v);
+            if (skip == 0) store16<CACHE>(out + at, r.v);
             else {
                 // (its own lines alone: the others are another wave's, which may have stored them, in place, already)
 #pragma unroll

@@ -59,11 +59,12 @@ struct ChunkStat {
 // moved back to end with the row: the elements it shares with the vector before are loaded twice,
 // left out of the sum once, and stored twice with the same bits (the launch makes every slot but a
 // lane's last a full vector: (V - 1) * G * VEC < n).
-// What bounds it is the memory system, once the arithmetic is out of its way: loads and stores are
-// non-temporal, a thread keeps few vectors, and a wave takes its rows and ends -- a loop over rows
+// What bounds it is the memory system, once the arithmetic is out of its way: large tensors' loads and stores are
+// non-temporal (CACHE: softmax_caching), a thread keeps few vectors, and a wave takes its rows and ends -- a loop over rows
 // with the next one's loads in flight, the form before, copies at 4.8 to 5.7 TB/s where waves that
 // end copy at 6.2 to 6.6.  [524288,1024] f16 422 -> 343 us (6.3 TB/s), f32 827 -> 728; [302592,197]
-// f16 83 -> 48 us (element by element before), f32 133 -> 102; [65536,64] f32 13.7 -> 7.2 us.
+// f16 83 -> 48 us (element by element before), f32 133 -> 102 -> 84; [65536,64] f32 13.7 -> 7.2 us; with ordinary accesses
+// [165000,50] f32 19.7 -> 12.6, [300000,100] f32 64 -> 43.
 template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
 }
@@ -120,7 +121,7 @@ __device__ __forceinline__ double reciprocal_of_sum(double s) {
 // What a lane of a row does with its V vectors, in the group kernel and in the row kernel: `stride`
 // vectors lie between two of them, `at` is the first one's number in the row.  Only the last may
 // reach the row's end.
-template <typename T, int V> struct RowPiece {
+template <typename T, int V, int CACHE> struct RowPiece {
     static constexpr int VEC = Vec128<T>::N;
     Vec128<T> q[V];
     float e[V][VEC];
@@ -131,7 +132,7 @@ template <typename T, int V> struct RowPiece {
         for (int i = 0; i < V; i++) {
             const uint32_t e0 = (static_cast<uint32_t>(i) * stride + at) * VEC;
             first[i] = i == V - 1 ? min(e0, n - VEC) : e0;
-            q[i].v = load16_stream(rowp + first[i]);
+            q[i].v = load16<CACHE>(rowp + first[i]);
         }
         const uint32_t e_last = (static_cast<uint32_t>(V - 1) * stride + at) * VEC;
         dup = e_last > n - VEC ? min(e_last - (n - VEC), static_cast<uint32_t>(VEC)) : 0u;
@@ -189,7 +190,7 @@ template <typename T, int V> struct RowPiece {
                 for (int c = 0; c < VEC; c++)
                     if (e[i][c] != e[i][c]) r.set(c, nan_value);
             }
-            if (live && (i < V - 1 || dup < static_cast<uint32_t>(VEC))) store16_stream(orow + first[i], r.v);
+            if (live && (i < V - 1 || dup < static_cast<uint32_t>(VEC))) store16<CACHE>(orow + first[i], r.v);
         }
     }
 };
@@ -200,18 +201,18 @@ template <typename T> __device__ __forceinline__ void store_largest(T *out, size
 }
 
 constexpr int kSoftmaxGroupThreads = 256;
-template <typename T, int G, int V, bool MAX_ONLY>
+template <typename T, int G, int V, bool MAX_ONLY, int CACHE>
 __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(const T *in, T *out, uint32_t rows, uint32_t n,
                                                                             int nan_where, float nan_value) {
     const uint32_t row = blockIdx.x * (kSoftmaxGroupThreads / G) + threadIdx.x / G;
     const bool live = row < rows;
     const size_t row0 = static_cast<size_t>(live ? row : rows - 1u) * n;  // (lanes past the last row shadow it and store nothing)
-    RowPiece<T, V> p;
+    RowPiece<T, V, CACHE> p;
     p.load(in + row0, n, threadIdx.x % G, G);
     const float m = group_max<G>(p.largest());
     // (halves: the shorter the row, the fewer terms are added in float -- n up to 64: 1, 128: 2, 256: 4, else 8)
     constexpr int SUM = G == 8 ? (V == 1 ? 1 : V == 2 ? 2 : 4) : G == 16 && V <= 2 ? 4 : 8;
-    const double rinv = reciprocal_of_sum(group_sum<G>(p.template terms<SUM < RowPiece<T, V>::VEC ? SUM : RowPiece<T, V>::VEC>(m)));
+    const double rinv = reciprocal_of_sum(group_sum<G>(p.template terms<SUM < Vec128<T>::N ? SUM : Vec128<T>::N>(m)));
     if constexpr (MAX_ONLY) {
         if (live && threadIdx.x % G == 0) store_largest(out, row, m, rinv);
     } else {
@@ -225,14 +226,14 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(con
 // half of it idle.  One read, one write, two barriers.  [9872,8296] f32 241 -> 114 us, f16 88 -> 61;
 // [2000,20001] f32 225 -> 60 us, f16 133 -> 39 (element by element before); [256,8192] f32 8.4 -> 5.5.
 constexpr int kSoftmaxRowWavesMax = 16;
-template <typename T, int V, bool MAX_ONLY>
+template <typename T, int V, bool MAX_ONLY, int CACHE>
 __global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel(const T *in, T *out, uint32_t n, int nan_where,
                                                                                 float nan_value) {
     __shared__ float fscratch[kSoftmaxRowWavesMax];
     __shared__ double dscratch[kSoftmaxRowWavesMax];
     const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave, waves = blockDim.x / kWave;
     const size_t row0 = static_cast<size_t>(blockIdx.x) * n;
-    RowPiece<T, V> p;
+    RowPiece<T, V, CACHE> p;
     p.load(in + row0, n, tid, blockDim.x);
     float m = group_max<kWave>(p.largest());
     if (waves > 1) {
@@ -241,7 +242,7 @@ __global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel
         const uint32_t w = lane & (kSoftmaxRowWavesMax - 1);
         m = group_max<kSoftmaxRowWavesMax>(w < waves ? fscratch[w] : -INFINITY);
     }
-    double s = group_sum<kWave>(p.template terms<RowPiece<T, V>::VEC>(m));
+    double s = group_sum<kWave>(p.template terms<Vec128<T>::N>(m));
     if (waves > 1) {
         if (lane == 0) dscratch[wave] = s;
         __syncthreads();
@@ -303,14 +304,12 @@ template <typename T, int NT, int V> struct Chunk {
     static constexpr uint32_t VEC = Vec128<T>::N;
     Vec128<T> q[V];
     static __device__ __forceinline__ uint32_t first(uint32_t chunk) { return (chunk * (V * NT) + threadIdx.x) * VEC; }
-    // KEPT: ordinary loads, for what is read again; else non-temporal ones
-    template <bool KEPT> __device__ __forceinline__ void load(const T *rowp, uint32_t chunk, uint32_t n) {
+    template <int CACHE> __device__ __forceinline__ void load(const T *rowp, uint32_t chunk, uint32_t n) {
         const uint32_t e_first = first(chunk);
 #pragma unroll
         for (int i = 0; i < V; i++) {
             const uint32_t at = min(e_first + static_cast<uint32_t>(i) * (NT * VEC), n - VEC) * static_cast<uint32_t>(sizeof(T));  // (bytes: below 2^27)
-            const T *p = reinterpret_cast<const T *>(reinterpret_cast<const char *>(rowp) + at);
-            q[i].v = KEPT ? load16_any(p) : load16_stream(p);
+            q[i].v = load16<CACHE>(reinterpret_cast<const T *>(reinterpret_cast<const char *>(rowp) + at));
         }
     }
 };
@@ -415,7 +414,7 @@ __global__ __launch_bounds__(NT) void softmax_stats_kernel(const T *__restrict__
     __shared__ ChunkScratch<NT> sh;
     const uint32_t row = blockIdx.x / G, chunk = blockIdx.x - row * G;
     Chunk<T, NT, V> ch;
-    ch.template load<true>(in + static_cast<size_t>(row) * n, chunk, n);
+    ch.template load<kCacheLoads>(in + static_cast<size_t>(row) * n, chunk, n);
     const ChunkStat st = chunk_stats(ch, chunk, n, sh);
     if (threadIdx.x == 0) stats[blockIdx.x] = st;
 }

@@ -14,17 +14,17 @@ template <typename T> bool launch_softmax_lines(const LinesLaunch &a) {
     const size_t lds = a.w > 1 ? static_cast<size_t>(teams) * a.w * per_team * L * sizeof(double) : 0;
     const T *in = static_cast<const T *>(a.in);
     T *out = static_cast<T *>(a.out);
-    // Ordinary stores where rows lie off the cache lines, in a tensor of 28 MB and more -- 40 MB where a wave's piece of a row is
-    // a kilobyte, or rows start on 16 bytes and the pieces are not the shortest (P = 8 in one wave).  At 33.5 MB f32, us
-    // non-temporal / ordinary: [8,80,13107] 24.5 / 18.4, [8,80,13108] 23.1 / 18.6, but [8,200,5240] 16.5 / 18.0 and
-    // [8,16,65537] 16.2 / 17.4; at half of that size [8,64,8193] 12.7 / 14.7.
-    const size_t row_bytes = static_cast<size_t>(a.g.inner) * sizeof(T);
-    const uintptr_t places = reinterpret_cast<uintptr_t>(out) | row_bytes;
-    const bool late = a.p == 1 || (places % 16 == 0 && !(a.p == 8 && a.w == 1));
-    const bool cached = places % 128 != 0 && a.bytes >= (size_t{late ? 40u : 28u} << 20);
+#define VKOP_LINES_CACHED(K, P, WIDE, CACHE) \
+    softmax_lines_reg_kernel<T, K, P, false, WIDE, CACHE><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, a.nan_where, a.nan_value)
 #define VKOP_LINES_LAUNCH(K, P, WIDE)                                                                                                      \
-    if (a.max_only) softmax_lines_reg_kernel<T, K, P, true, WIDE><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, 0, 0.f, false);          \
-    else softmax_lines_reg_kernel<T, K, P, false, WIDE><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, a.nan_where, a.nan_value, cached)
+    if (a.max_only && a.caching == kCacheNone)                                                                                             \
+        softmax_lines_reg_kernel<T, K, P, true, WIDE, kCacheNone><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, 0, 0.f);           \
+    else if (a.max_only)                                                                                                                   \
+        softmax_lines_reg_kernel<T, K, P, true, WIDE, kCacheLoads><<<blocks, threads, lds, a.stream>>>(in, out, a.g, a.w, 0, 0.f);          \
+    else if (a.caching == kCacheLoads) VKOP_LINES_CACHED(K, P, WIDE, kCacheLoads);                                                          \
+    else if (a.caching == kCacheStores) VKOP_LINES_CACHED(K, P, WIDE, kCacheStores);                                                        \
+    else if (a.caching == kCacheBoth) VKOP_LINES_CACHED(K, P, WIDE, kCacheBoth);                                                            \
+    else VKOP_LINES_CACHED(K, P, WIDE, kCacheNone)
 #define VKOP_LINES(K, P)                                                                                                                   \
     if (a.k == K && a.p == P) {                                                                                                            \
         if (sizeof(T) == 4 || a.w > 1) VKOP_LINES_LAUNCH(K, P, true);                                                                      \
@@ -47,6 +47,7 @@ template <typename T> bool launch_softmax_lines(const LinesLaunch &a) {
 #undef VKOP_LINES_5_8
 #undef VKOP_LINES
 #undef VKOP_LINES_LAUNCH
+#undef VKOP_LINES_CACHED
     return false;
 }
 

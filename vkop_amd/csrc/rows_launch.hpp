@@ -108,7 +108,7 @@ struct LinesLaunch {
     LineGeom g;
     uint32_t k, p, w;  // elements of a line a lane, lane groups of a wave a line, waves a line
     bool max_only;
-    size_t bytes;  // of the whole tensor
+    int caching;  // Caching
     int nan_where;
     float nan_value;
     hipStream_t stream;

@@ -389,12 +389,64 @@ SoftmaxPlan plan_softmax(const View &v, int dtype) {
     return p;
 }
 
+// Which accesses of the kernels that hold a row (group, row) or a line (lines) in registers are ordinary ones.  Non-temporal ones
+// keep a stream out of the caches: the better way for a tensor that those cannot serve.
+// * The chip's last cache (256 MB) holds an input of up to 90 MB until it is read again, or since it was written, beside two more
+//   like it (ordinary loads); the L2s (32 MB in all) those of up to 10 MB.  Between the two floats' whole lines lose a little by it.
+// * Two outputs of up to half of it wait there for their reader instead of for memory (ordinary stores).  Smaller ones have to leave
+//   the L2s at the kernel's end all the same, which a stream has done by then.
+// * A piece of a row that begins or ends inside a 128-byte line shares that line with another wave's, and past the caches each of the
+//   two fetches and stores it by itself: pieces of at most 256 bytes of rows, and lines whose rows lie off the 128 bytes, want both.
+// us a call, none / loads / stores / both (three inputs and two outputs in turn):
+//   rows of whole lines: f32 n = 256  8 MB 4.6 / 4.0 / 4.6 / 4.6, 16 MB 8.1 / 8.4 / 11.2 / 10.6, 50 MB 17.0 / 15.7 / 17.3 / 15.0,
+//   120 MB 39.6 / 41.1 / 38.2 / 43.4, 250 MB 82 / 86 / 87 / 90; f16 n = 8192  50 MB 17.6 / 16.0 / 18.1 / 16.0
+//   off the lines: f32 n = 197 (pieces of 256 bytes)  50 MB 22.4 / 19.3 / 20.0 / 17.0, 400 MB 173 / 166 / 150 / 140, f16 n = 197  64 MB
+//   26.2 / 22.0 / 24.4 / 21.7, 250 MB 99 / 93 / 98 / 91; of 512 bytes f16 n = 500  180 MB 63 / 62 / 65 / 63; a lane's only
+//   vector, where a wave's rows are one piece, f16 n = 50  180 MB 73 / 72 / 75 / 74
+//   lines: f32 [8,21,n] of 50 MB 21.5 / 18.0 / 20.8 / 20.4, of 180 MB 68 / 70 / 71 / 75; off the 128 bytes f32 [8,100,n] of 50 MB
+//   40 / 36 / 27 / 21, 180 MB 145 / 135 / 97 / 87, f16 [8,80,n] of 120 MB 93 / 82 / 55 / 56, 250 MB 190 / 163 / 131 / 105
+// (The one-launch kernel of long rows, whose tensor is in registers before any of it is written, is as fast or faster without:
+// f32 [64,128256] 15.7 / 16.4 / 18.0 / 17.7.)
+template <typename T> int softmax_caching(const View &v, const SoftmaxPlan &p, const T *in, const T *out, bool max_only) {
+    constexpr size_t kMega = 1000000, kHalfLastCache = size_t{128} << 20;
+    const size_t bytes = v.elems * sizeof(T), row_bytes = static_cast<size_t>(v.g.inner == 1 ? v.g.n : v.g.inner) * sizeof(T);
+    const uintptr_t places = reinterpret_cast<uintptr_t>(in) | (max_only ? 0u : reinterpret_cast<uintptr_t>(out)) | row_bytes;
+    const bool lines = p.kind == SoftmaxPlan::kLinesRegs, group = p.kind == SoftmaxPlan::kGroup, off128 = places % 128 != 0;
+    if (!lines && !group && p.kind != SoftmaxPlan::kRow) return vkop::kCacheNone;
+    const bool in_last = bytes >= (lines ? 30 : 24) * kMega && bytes <= 90 * kMega;
+    if (max_only) return in_last ? vkop::kCacheLoads : vkop::kCacheNone;
+    const bool in_l2s = bytes <= 10 * kMega || (bytes < 24 * kMega && !lines && (sizeof(T) == 2 || off128));
+    const int loads = in_last || (in_l2s && !(p.kind == SoftmaxPlan::kRow)) ? vkop::kCacheLoads : vkop::kCacheNone;
+    if (lines && off128) {
+        // (a wave's piece of a row of a kilobyte, or pieces that start on 16 bytes, have fewer lines in part: from 40 MB on, the
+        // others from 28.  At 33.5 MB f32, none / stores: [8,80,13107] 24.5 / 18.4, [8,80,13108] 23.1 / 18.6, but [8,200,5240]
+        // 16.5 / 18.0 and [8,16,65537] 16.2 / 17.4)
+        const bool on16 = places % 16 == 0, late = p.lines_p == 1 || (on16 && !(p.lines_p == 8 && p.lines_w == 1));
+        if (bytes < (late ? 40u : 28u) * kMega) return loads;
+        if (bytes <= 80 * kMega) return on16 ? vkop::kCacheLoads : vkop::kCacheBoth;
+        return bytes > kHalfLastCache ? vkop::kCacheBoth : vkop::kCacheStores;
+    }
+    if (group && off128 && p.shape.v > 1 && p.shape.nt <= 16 && bytes >= 24 * kMega) return vkop::kCacheBoth;
+    if (loads != vkop::kCacheNone) return loads;
+    const bool one_piece = group && off128 && p.shape.v == 1;
+    return (lines || (group && !one_piece)) && bytes > 90 * kMega && bytes <= kHalfLastCache ? vkop::kCacheStores : vkop::kCacheNone;
+}
+// f(std::integral_constant<int, CACHE>) for a run-time `caching`
+template <typename F> void with_caching(int caching, F &&f) {
+    switch (caching) {
+    case vkop::kCacheLoads: return f(std::integral_constant<int, vkop::kCacheLoads>{});
+    case vkop::kCacheStores: return f(std::integral_constant<int, vkop::kCacheStores>{});
+    case vkop::kCacheBoth: return f(std::integral_constant<int, vkop::kCacheBoth>{});
+    default: return f(std::integral_constant<int, vkop::kCacheNone>{});
+    }
+}
+
 template <typename T>
 int launch_lines(const T *in, T *out, const View &v, const SoftmaxPlan &p, bool max_only, int nan_where, float nan_value,
                  hipStream_t st) {
     return in_slices(v.g.outer, lines_threads(v, 16 / sizeof(T), p.lines_p, p.lines_w), [&](uint64_t first, uint32_t outer) {
         vkop::LinesLaunch a{in + first * v.g.n * v.g.inner, out + first * (max_only ? 1u : v.g.n) * v.g.inner, v.g, p.lines_k, p.lines_p,
-                            p.lines_w, max_only, v.elems * sizeof(T), nan_where, nan_value, st};
+                            p.lines_w, max_only, softmax_caching(v, p, in, out, max_only), nan_where, nan_value, st};
         a.g.outer = outer;
         if (!vkop::launch_softmax_lines<T>(a))
             return fail(VKOP_HIP_ERR_UNSUPPORTED, "no softmax_lines_reg_kernel for %u elements x %u", a.k, a.p);
@@ -444,6 +496,7 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
                  size_t ws_bytes, hipStream_t st) {
     const uint32_t lines = v.g.outer;
     const uint64_t out_row = MAX_ONLY ? 1u : v.g.n;
+    const int caching = softmax_caching(v, p, in, out, MAX_ONLY);
     const auto kind = MAX_ONLY && v.g.n <= vkop::kSoftmaxThreadMaxN ? SoftmaxPlan::kThread : p.kind;
     switch (kind) {
     case SoftmaxPlan::kThread: {
@@ -460,7 +513,11 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
             const uint32_t rows = static_cast<uint32_t>(std::min<uint64_t>(lines - row0, static_cast<uint64_t>(blocks) * per_block));
 #define VKOP_GROUP(G, V)                                                                                                       \
     if (p.shape.nt == G && p.shape.v == V) {                                                                                   \
-        vkop::softmax_group_kernel<T, G, V, MAX_ONLY><<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(from, to, rows, v.g.n, nan_where, nan_value); \
+        with_caching(caching, [&](auto cache) {                                                                                \
+            constexpr int CACHE = MAX_ONLY ? cache & vkop::kCacheLoads : cache;                                                \
+            vkop::softmax_group_kernel<T, G, V, MAX_ONLY, CACHE>                                                               \
+                <<<blocks, vkop::kSoftmaxGroupThreads, 0, st>>>(from, to, rows, v.g.n, nan_where, nan_value);                  \
+        });                                                                                                                    \
         return launched("softmax_group_kernel");                                                                               \
     }
 #define VKOP_GROUPS(G) VKOP_GROUP(G, 1) VKOP_GROUP(G, 2) VKOP_GROUP(G, 3) if constexpr (sizeof(T) == 4) { VKOP_GROUP(G, 4) }
@@ -476,7 +533,10 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
             T *to = out + row0 * out_row;
 #define VKOP_ROW(V)                                                                                     \
     if (p.shape.v == V) {                                                                               \
-        vkop::softmax_row_kernel<T, V, MAX_ONLY><<<rows, p.shape.nt, 0, st>>>(from, to, v.g.n, nan_where, nan_value); \
+        with_caching(caching, [&](auto cache) {                                                         \
+            constexpr int CACHE = MAX_ONLY || cache == vkop::kCacheBoth ? cache & vkop::kCacheLoads : cache; \
+            vkop::softmax_row_kernel<T, V, MAX_ONLY, CACHE><<<rows, p.shape.nt, 0, st>>>(from, to, v.g.n, nan_where, nan_value); \
+        });                                                                                             \
         return launched("softmax_row_kernel");                                                          \
     }
             VKOP_ROW(1) VKOP_ROW(2) VKOP_ROW(3) VKOP_ROW(4)
