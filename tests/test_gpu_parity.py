@@ -283,6 +283,35 @@ def test_softmax_nan_of_any_payload(ops, shape, axis):
         assert np.array_equal(np.isnan(best), held) and np.array_equal(best[~held], got[~held].max(-1)), dtype
 
 
+@pytest.mark.parametrize("shape,axis", [
+    ((40, 17), -1), ((40, 64), -1), ((40, 65), -1), ((40, 191), -1), ((40, 197), -1), ((40, 511), -1), ((1030, 1023), -1), ((1030, 1535), -1),
+    ((40, 8191), -1), ((40, 1537), -1), ((40, 20001), -1), ((3, 200001), -1), ((8, 33, 65537), 1), ((2, 700, 1001), 1), ((33, 1000, 64), 1), ((2, 5, 40001), 1),
+])
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+def test_softmax_lines_without_a_finite_maximum(ops, dtype, shape, axis):
+    """NaN or +inf at the first, the last and another element of a line, nothing but -inf, and -inf beside numbers, the lowest finite
+    value among them: by every kernel's own maximum, with the tensor's last vectors moved back or not."""
+    t = torch.float16 if dtype == "f16" else torch.float32
+    x = torch.empty(shape, dtype=t, device="cuda").normal_(0.0, 2.0, generator=torch.Generator(device="cuda").manual_seed(sum(shape)))
+    lines = x.movedim(axis, -1).reshape(-1, shape[axis])  # (a copy where the axis is not the last)
+    inf, low, n = float("inf"), torch.finfo(t).min, shape[axis]
+    kinds = [lambda v: v[:1].fill_(float("nan")), lambda v: v[-1:].fill_(float("nan")), lambda v: v[n // 2:n // 2 + 1].fill_(float("nan")),
+             lambda v: v[:1].fill_(inf), lambda v: v[-1:].fill_(inf), lambda v: v.fill_(-inf), lambda v: v[1:].fill_(-inf),
+             lambda v: (v.fill_(-inf), v[-2:].fill_(low)), lambda v: v[:n - 3].fill_(-inf), lambda v: v.fill_(low)]
+    for i in range(min(len(lines), 3 * len(kinds))):
+        kinds[i % len(kinds)](lines[-1 - i])
+    x = lines.reshape(x.movedim(axis, -1).shape).movedim(-1, axis).contiguous()
+    d = x.float() - x.float().amax(axis, keepdim=True)  # (NaN in such a line; -inf - -inf too)
+    e = torch.exp(d.double())
+    e /= e.sum(axis, keepdim=True)
+    got = ops.softmax(x, axis)
+    assert torch.equal(got.isnan(), e.isnan())
+    rel, least = (2.0 ** -10, 2.0 ** -24) if dtype == "f16" else (2.0 ** -22, 2.0 ** -149)
+    assert bool((((got.double() - e).abs() <= rel * e + least) | e.isnan()).all())
+    best = ops.softmax_reduce_max(x, axis)
+    assert torch.equal(best.nan_to_num(7.0), got.amax(axis).reshape(best.shape).nan_to_num(7.0))
+
+
 @pytest.mark.parametrize("dtype,shape,axis", [
     ("f16", (170001, 100), -1), ("f32", (61001, 197), -1), ("f32", (85001, 100), -1),   # pieces off the lines: both ordinary
     ("f16", (660001, 50), -1), ("f16", (66001, 256), -1), ("f32", (2001, 1000), -1),    # loads alone

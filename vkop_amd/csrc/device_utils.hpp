@@ -116,10 +116,36 @@ __device__ __forceinline__ uint32_t max_half2(uint32_t a, uint32_t b) {
     return r;
 }
 
+// The larger halves of three pairs and the larger of three floats, NaN wherever one of them is NaN.
+__device__ __forceinline__ uint32_t maximum_half2(uint32_t a, uint32_t b, uint32_t c) {
+    uint32_t r;
+    asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float maximum(float a, float b, float c) {
+    float r;
+    asm("v_maximum3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 __device__ __forceinline__ uint32_t min_half2(uint32_t a, uint32_t b) {
     uint32_t r;
     asm("v_pk_min_f16 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
+}
+
+// A half of a word, widened, minus m: one instruction and one rounding, as the conversion and the difference have.
+__device__ __forceinline__ float half_minus(uint32_t w, bool high, float m) {
+    float d;
+    if (high) asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d) : "v"(w), "v"(m));
+    else asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(d) : "v"(w), "v"(m));
+    return d;
+}
+// (a s, b t), each rounded to float and then to a half.
+__device__ __forceinline__ uint32_t half2_of_products(float a, float s, float b, float t) {
+    uint32_t w;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\tv_fma_mixhi_f16 %0, %3, %4, 0" : "=&v"(w) : "v"(a), "v"(s), "v"(b), "v"(t));
+    return w;
 }
 
 // x * scale rounded to float on its own: never contracted into a fused multiply-add
@@ -293,18 +319,18 @@ template <bool NAN_TOO = true> __device__ __forceinline__ float exp_accurate(flo
 __device__ __forceinline__ float softmax_term(float x, float m) { return exp_accurate(x - m); }
 
 // exp(d) in single precision throughout, good to about two units in the last place of a float: the
-// hardware exponential of a = fl(d log2 e), and what that rounding and the low part of log2 e left
-// out as a first-order factor (2^(a + l) = 2^a (1 + l ln 2), |l| < 1e-6).  For results that are
-// stored in half precision: 2^-22 relative before a rounding to 11 bits moves one result in two
+// hardware exponential of a = fl(d log2 e), and what d is more than a ln 2 as a first-order factor
+// (exp(d) = 2^a e^r, r = d - a ln 2, |r| < 2^-18: the first product-and-sum is exact but for its last rounding).  For results that are
+// stored in half precision: 2^-22.8 relative (every 29th float from 0 to -87; 2^-25.3 in the mean square) before a rounding to 11 bits moves one result in two
 // thousand by one unit of a half, and costs a third of exp_accurate.  Results below 2^-126 are 0.
 template <bool NAN_TOO = true> __device__ __forceinline__ float exp_half_grade(float d) {
-    constexpr float kHi = 1.44269502162933349609375f;  // float(log2 e)
-    constexpr float kLo = 1.925963033500011e-8f;       // log2 e - kHi
+    constexpr float kLog2E = 1.44269502162933349609375f;
+    constexpr float kLn2Hi = 0.693147182464599609375f, kLn2Lo = -1.904654323148236017e-9f;  // ln 2 in two floats
     d = at_least_minus_104<NAN_TOO>(d);  // (there the hardware exponential is 0, and what follows is finite)
-    const float a = d * kHi;
-    const float l = fmaf(d, kLo, fmaf(d, kHi, -a));
+    const float a = d * kLog2E;
+    const float r = fmaf(-a, kLn2Lo, fmaf(-a, kLn2Hi, d));
     const float e = __builtin_amdgcn_exp2f(a);
-    return fmaf(e, l * 0.693147180559945309f, e);
+    return fmaf(e, r, e);
 }
 
 // The term as the element type asks for it: float tensors get the correctly rounded exponential,
@@ -313,13 +339,6 @@ template <bool NAN_TOO = true> __device__ __forceinline__ float exp_half_grade(f
 template <typename T> __device__ __forceinline__ float softmax_term_as(float x, float m) {
     if constexpr (sizeof(T) == 2) return exp_half_grade(x - m);
     else return exp_accurate(x - m);
-}
-
-// The same for kernels whose row's sum holds every term already, NaN included: whatever at a NaN element, since 1 / sum is NaN
-// with it.
-template <typename T> __device__ __forceinline__ float softmax_term_of_row(float x, float m) {
-    if constexpr (sizeof(T) == 2) return exp_half_grade<false>(x - m);
-    else return exp_accurate<false>(x - m);
 }
 
 // What a thread adds its own few terms up in, and how a term becomes a probability, in the same

@@ -148,22 +148,17 @@ __global__ __launch_bounds__(NT) void softmax_joined_kernel(const T *in, T *out,
 #pragma unroll
     for (int i = 0; i < V; i++) {
         const uint32_t e0 = e_first + static_cast<uint32_t>(i) * (NT * VEC);
-        float p[VEC];
-        Vec128<T> r;
-        r.v = make_uint4(0, 0, 0, 0);
+        float e[VEC];
 #pragma unroll
-        for (int c = 0; c < static_cast<int>(VEC); c++) {
-            p[c] = over_sum(softmax_term_of_row<T>(ch.q[i].get(c), m));
-            if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
-            r.set(c, p[c]);
-        }
+        for (int c = 0; c < static_cast<int>(VEC); c++) e[c] = term_of_row(ch.q[i], c, m);
+        const Vec128<T> r = probabilities<T>(e, [&](int) { return over_sum; }, nan_where, nan_value);
         if (e0 <= n - VEC) {
             store16_stream(orow + e0, r.v);
         } else if (e0 < n) {
             const uint32_t dup = e0 - (n - VEC);
 #pragma unroll
             for (int c = 1; c < static_cast<int>(VEC); c++)
-                if (static_cast<uint32_t>(c) >= dup) store_elem(orow, n - VEC + static_cast<uint32_t>(c), p[c]);
+                if (static_cast<uint32_t>(c) >= dup) store_elem(orow, n - VEC + static_cast<uint32_t>(c), r.get(c));
         }
     }
     // the last workgroup to have read what it needs of the row's records clears them

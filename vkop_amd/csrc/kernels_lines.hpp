@@ -156,13 +156,12 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
     if constexpr (sizeof(T) == 2) {
         uint32_t pk[4] = {q[0].v.x, q[0].v.y, q[0].v.z, q[0].v.w};
 #pragma unroll
-        for (int i = 0; i < K; i++) {  // (q[0] again: max_half2 drops NaN only against a number)
-            pk[0] = max_half2(pk[0], q[i].v.x), pk[1] = max_half2(pk[1], q[i].v.y);
-            pk[2] = max_half2(pk[2], q[i].v.z), pk[3] = max_half2(pk[3], q[i].v.w);
+        for (int i = 1; i < K; i += 2) {
+            const Vec128<T> &a = q[i], &b = q[i + 1 < K ? i + 1 : i];
+            pk[0] = maximum_half2(pk[0], a.v.x, b.v.x), pk[1] = maximum_half2(pk[1], a.v.y, b.v.y);
+            pk[2] = maximum_half2(pk[2], a.v.z, b.v.z), pk[3] = maximum_half2(pk[3], a.v.w, b.v.w);
         }
-#pragma unroll
-        for (int w = 0; w < 4; w++) pk[w] = max_half2(pk[w], 0xFC00FC00u);
-        share_out<P>(pk, [](uint32_t a, uint32_t b) { return max_half2(a, b); });
+        share_out<P>(pk, [](uint32_t a, uint32_t b) { return maximum_half2(a, b, b); });
 #pragma unroll
         for (int w = 0; w < C / 2; w++) {
             m[2 * w] = __half2float(__ushort_as_half(static_cast<uint16_t>(pk[w] & 0xFFFFu)));
@@ -172,17 +171,16 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         uint32_t mu[L];
 #pragma unroll
         for (int c = 0; c < L; c++) {
-            m[c] = -INFINITY;
+            m[c] = K == 1 ? maximum(q[0].get(c), q[0].get(c), q[0].get(c)) : q[0].get(c);
 #pragma unroll
-            for (int i = 0; i + 1 < K; i += 2) m[c] = max3(m[c], q[i].get(c), q[i + 1].get(c));  // (drops NaN)
-            if constexpr (K % 2 != 0) m[c] = max3(m[c], m[c], q[K - 1].get(c));
+            for (int i = 1; i < K; i += 2) m[c] = maximum(m[c], q[i].get(c), q[i + 1 < K ? i + 1 : i].get(c));
             mu[c] = __float_as_uint(m[c]);
         }
-        share_out<P>(mu, [](uint32_t a, uint32_t b) { return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b))); });
+        share_out<P>(mu, [](uint32_t a, uint32_t b) { return __float_as_uint(maximum(__uint_as_float(a), __uint_as_float(b), __uint_as_float(b))); });
 #pragma unroll
         for (int c = 0; c < C; c++) m[c] = __uint_as_float(mu[c]);
     }
-    auto larger = [](float a, float b) { return fmaxf(a, b); };
+    auto larger = [](float a, float b) { return maximum(a, b, b); };  // (NaN where a line holds one)
     if (W > 1) {
         // a wave's maxima go to LDS, and the lanes that own the same lines read their share of the waves
         float *fl = reinterpret_cast<float *>(lines_lds) + team * (W * LPW * L);
@@ -193,7 +191,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         __syncthreads();
         for (uint32_t w = extra; w < W; w += EXTRA) {
 #pragma unroll
-            for (int c = 0; c < C; c++) m[c] = fmaxf(m[c], fl[(w * L + own0 + c) * LPW + slot]);
+            for (int c = 0; c < C; c++) m[c] = larger(m[c], fl[(w * L + own0 + c) * LPW + slot]);
         }
 #pragma unroll
         for (int c = 0; c < C; c++) m[c] = join_rest<P>(m[c], larger);
@@ -213,7 +211,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         asm volatile("" : "+v"(q[i].v.x), "+v"(q[i].v.y), "+v"(q[i].v.z), "+v"(q[i].v.w));
 #pragma unroll
         for (int c = 0; c < L; c++) {
-            e[i][c] = softmax_term_as<T>(q[i].get(c), m[c]);
+            e[i][c] = term_of_row(q[i], c, m[c]);
             acc[c] += i < K - 1 || last_ok ? e[i][c] : 0.f;
         }
     }
@@ -247,7 +245,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
             float p[C];
 #pragma unroll
             for (int c = 0; c < C; c++) {
-                p[c] = scale_term<T>(softmax_term_as<T>(own_m[c], own_m[c]), reciprocal_of_sum(s[c]));
+                p[c] = scale_term<T>(softmax_term_as<T>(own_m[c], own_m[c]), row_reciprocal(s[c], own_m[c]));
                 if constexpr (C == L) r.set(c, p[c]);
             }
             if (C == L && skip == 0) store16_stream(out + at, r.v);
@@ -263,7 +261,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
     if constexpr (sizeof(T) == 2) {
         float high[L];
 #pragma unroll
-        for (int c = 0; c < C; c++) high[c] = Quotient<T>(reciprocal_of_sum(s[c])).high;
+        for (int c = 0; c < C; c++) high[c] = Quotient<T>(row_reciprocal(s[c], own_m[c])).high;
         hand_out<P>(high);
 #pragma unroll
         for (int c = 0; c < L; c++) over_sum[c].high = high[c];
@@ -272,7 +270,7 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
         float low[L], high[L];
 #pragma unroll
         for (int c = 0; c < C; c++) {
-            const double r = reciprocal_of_sum(s[c]);
+            const double r = row_reciprocal(s[c], own_m[c]);
             low[c] = __int_as_float(__double2loint(r)), high[c] = __int_as_float(__double2hiint(r));
         }
         hand_out<P>(low);
@@ -284,24 +282,16 @@ __global__ __launch_bounds__(kLinesWavesMax *kWave) __attribute__((amdgpu_waves_
     asm volatile("" : "+v"(at));  // (places again: sixteen of them kept from the loads are 32 registers)
 #pragma unroll
     for (int i = 0; i < K; i++, at += static_cast<size_t>(parts) * g.inner) {
-        float p[L];
-        Vec128<T> r;
-        r.v = make_uint4(0, 0, 0, 0);
 #pragma unroll
         for (int c = 0; c < L; c++) asm volatile("" : "+v"(e[i][c]));
-#pragma unroll
-        for (int c = 0; c < L; c++) {
-            p[c] = over_sum[c](e[i][c]);
-            if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
-            r.set(c, p[c]);
-        }
+        const Vec128<T> r = probabilities<T>(e[i], [&](int c) { return over_sum[c]; }, nan_where, nan_value);
         if (live && (i < K - 1 || last_ok)) {
             if (skip == 0) store16<CACHE>(out + at, r.v);
             else {
                 // (its own lines alone: the others are another wave's, which may have stored them, in place, already)
 #pragma unroll
                 for (int c = 1; c < L; c++)
-                    if (static_cast<uint32_t>(c) >= skip) store_elem(out, at + c, p[c]);
+                    if (static_cast<uint32_t>(c) >= skip) store_elem(out, at + c, r.get(c));
             }
         }
     }

@@ -60,30 +60,38 @@ struct ChunkStat {
 // left out of the sum once, and stored twice with the same bits (the launch makes every slot but a
 // lane's last a full vector: (V - 1) * G * VEC < n).
 // What bounds it is the memory system, once the arithmetic is out of its way: large tensors' loads and stores are
-// non-temporal (CACHE: softmax_caching), a thread keeps few vectors, and a wave takes its rows and ends -- a loop over rows
+// non-temporal (CACHE: softmax_caching), halves' terms have the fewest instructions (below: half_minus, half2_of_products), NaN shows
+// in the row's maximum instead of in every term, a thread keeps few vectors, and a wave takes its rows and ends -- a loop over rows
 // with the next one's loads in flight, the form before, copies at 4.8 to 5.7 TB/s where waves that
 // end copy at 6.2 to 6.6.  [524288,1024] f16 422 -> 343 us (6.3 TB/s), f32 827 -> 728; [302592,197]
 // f16 83 -> 48 us (element by element before), f32 133 -> 102 -> 84; [65536,64] f32 13.7 -> 7.2 us; with ordinary accesses
-// [165000,50] f32 19.7 -> 12.6, [300000,100] f32 64 -> 43.
+// [165000,50] f32 19.7 -> 12.6, [300000,100] f32 64 -> 43.  By the terms f16 [304568,197] 49.9 -> 44.9, [83756,197] 15.6 -> 13.5,
+// [2441,8192] 14.2 -> 13.0, [8,1000,8000] axis 1 73 -> 68, f32 [64,128256] 16.2 -> 15.4.
 template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
 }
-template <int G> __device__ __forceinline__ float group_max(float v) {
+template <int G, typename F> __device__ __forceinline__ uint32_t group_join(uint32_t v, F op) {
     static_assert(G >= 8 && G <= kWave, "lanes a row");
-    auto step = [](float a, auto tag) { return fmaxf(a, __uint_as_float(dpp_u32<decltype(tag)::value>(__float_as_uint(a)))); };
-    v = step(v, std::integral_constant<int, 0xB1>{});   // lane ^ 1
-    v = step(v, std::integral_constant<int, 0x4E>{});   // lane ^ 2
-    v = step(v, std::integral_constant<int, 0x141>{});  // the other four of eight
-    if constexpr (G >= 16) v = step(v, std::integral_constant<int, 0x140>{});  // the other eight of sixteen
+    v = op(v, dpp_u32<0xB1>(v));   // lane ^ 1
+    v = op(v, dpp_u32<0x4E>(v));   // lane ^ 2
+    v = op(v, dpp_u32<0x141>(v));  // the other four of eight
+    if constexpr (G >= 16) v = op(v, dpp_u32<0x140>(v));  // the other eight of sixteen
     if constexpr (G >= 32) {
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        v = op(r[0], r[1]);
     }
     if constexpr (G >= 64) {
-        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-        v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        v = op(r[0], r[1]);
     }
     return v;
+}
+template <int G> __device__ __forceinline__ float group_max(float v) {
+    return __uint_as_float(group_join<G>(__float_as_uint(v), [](uint32_t a, uint32_t b) { return __float_as_uint(fmaxf(__uint_as_float(a), __uint_as_float(b))); }));
+}
+// (NaN where a lane has NaN)
+template <int G> __device__ __forceinline__ float group_maximum(float v) {
+    return __uint_as_float(group_join<G>(__float_as_uint(v), [](uint32_t a, uint32_t b) { return __float_as_uint(maximum(__uint_as_float(a), __uint_as_float(b), __uint_as_float(b))); }));
 }
 template <int G> __device__ __forceinline__ double group_sum(double v) {
     auto join = [](uint32_t lo, uint32_t hi) { return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo)); };
@@ -118,6 +126,36 @@ __device__ __forceinline__ double reciprocal_of_sum(double s) {
     y = fma(fma(-s, y, 1.0), y, y);
     return fma(fma(-s, y, 1.0), y, y);
 }
+// 1 / s where the row's maximum m is a number; NaN, which every probability then is, where an element is NaN or the maximum infinite.
+__device__ __forceinline__ double row_reciprocal(double s, float m) {
+    return reciprocal_of_sum(m > -INFINITY && m < INFINITY ? s : __longlong_as_double(0x7FF8000000000000ll));
+}
+// The term of element c of a vector, softmax_term_as without its step for NaN: where the row's maximum or sum makes NaN of all.
+__device__ __forceinline__ float term_of_row(const Vec128<float> &q, int c, float m) { return exp_accurate<false>(q.get(c) - m); }
+__device__ __forceinline__ float term_of_row(const Vec128<uint16_t> &q, int c, float m) {
+    return exp_half_grade<false>(half_minus(c < 2 ? q.v.x : c < 4 ? q.v.y : c < 6 ? q.v.z : q.v.w, c & 1, m));
+}
+// A vector of probabilities as they are stored, the term of element c over the sum that over(c) stands for.
+template <typename T, typename F>
+__device__ __forceinline__ Vec128<T> probabilities(const float (&e)[Vec128<T>::N], F &&over, int nan_where, float nan_value) {
+    Vec128<T> r;
+    if constexpr (sizeof(T) == 2) {
+        auto pair = [&](int c) { return half2_of_products(e[c], over(c).high, e[c + 1], over(c + 1).high); };
+        r.v = make_uint4(pair(0), pair(2), pair(4), pair(6));
+    } else {
+        r.v = make_uint4(0, 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < Vec128<T>::N; c++) r.set(c, over(c)(e[c]));
+    }
+    if (nan_where) {  // (the same in every thread)
+#pragma unroll
+        for (int c = 0; c < Vec128<T>::N; c++) {
+            const float p = r.get(c);
+            if (p != p) r.set(c, nan_value);
+        }
+    }
+    return r;
+}
 // What a lane of a row does with its V vectors, in the group kernel and in the row kernel: `stride`
 // vectors lie between two of them, `at` is the first one's number in the row.  Only the last may
 // reach the row's end.
@@ -137,38 +175,56 @@ template <typename T, int V, int CACHE> struct RowPiece {
         const uint32_t e_last = (static_cast<uint32_t>(V - 1) * stride + at) * VEC;
         dup = e_last > n - VEC ? min(e_last - (n - VEC), static_cast<uint32_t>(VEC)) : 0u;
     }
-    __device__ __forceinline__ float largest() const {  // (drops NaN)
-        float m = -INFINITY;
+    // The largest of the G lanes' elements, NaN where one of them is NaN.
+    template <int G> __device__ __forceinline__ float largest() const {
         if constexpr (sizeof(T) == 2) {
-            uint32_t pk = 0xFC00FC00u;
+            uint32_t pk = maximum_half2(q[0].v.x, q[0].v.y, q[0].v.z);
 #pragma unroll
-            for (int i = 0; i < V; i++)
-                pk = max_half2(max_half2(pk, max_half2(q[i].v.x, q[i].v.y)), max_half2(q[i].v.z, q[i].v.w));
-            m = fmaxf(__half2float(__ushort_as_half(static_cast<uint16_t>(pk & 0xFFFFu))),
-                      __half2float(__ushort_as_half(static_cast<uint16_t>(pk >> 16))));
+            for (int i = 1; i < V; i++) pk = maximum_half2(maximum_half2(pk, q[i - 1].v.w, q[i].v.x), q[i].v.y, q[i].v.z);
+            pk = maximum_half2(pk, q[V - 1].v.w, q[V - 1].v.w);
+            pk = group_join<G>(pk, [](uint32_t a, uint32_t b) { return maximum_half2(a, b, b); });
+            const float other = __half2float(__ushort_as_half(static_cast<uint16_t>(pk >> 16)));
+            return maximum(__half2float(__ushort_as_half(static_cast<uint16_t>(pk & 0xFFFFu))), other, other);
         } else {
+            float m = maximum(q[0].get(0), q[0].get(1), q[0].get(2));
 #pragma unroll
-            for (int i = 0; i < V; i++)
-                m = max3(max3(m, q[i].get(0), q[i].get(1)), q[i].get(2), q[i].get(3));
+            for (int i = 1; i < V; i++) m = maximum(maximum(m, q[i - 1].get(3), q[i].get(0)), q[i].get(1), q[i].get(2));
+            m = maximum(m, q[V - 1].get(3), q[V - 1].get(3));
+            return group_maximum<G>(m);
         }
-        return m;
     }
-    // the terms, and their sum over this lane's elements: halves' terms added in float SUM at a time (TermSum)
-    template <int SUM> __device__ __forceinline__ double terms(float m) {
+    // The terms, and their sum over this lane's elements: halves' terms added in float SUM at a time (TermSum).  (Numbers, whatever
+    // the elements: a row with NaN, or whose maximum is not finite, shows in m -- row_reciprocal.)  n: the row's length.
+    template <int SUM> __device__ __forceinline__ double terms(float m, uint32_t n) {
         static_assert(VEC % SUM == 0, "a vector's terms in equal parts");
         double acc = 0.0;
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            TermSum<T> part = 0;
 #pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                e[i][c] = softmax_term_as<T>(q[i].get(c), m);
-                const float counted = i < V - 1 || static_cast<uint32_t>(c) >= dup ? e[i][c] : 0.f;
-                if constexpr (sizeof(T) == 4) {
-                    acc += static_cast<double>(counted);
-                } else {
-                    part = c % SUM == 0 ? counted : part + counted;
-                    if (c % SUM == SUM - 1) acc += static_cast<double>(part);
+            for (int c = 0; c < VEC; c++) e[i][c] = term_of_row(q[i], c, m);
+            if constexpr (sizeof(T) == 4) {
+#pragma unroll
+                for (int c = 0; c < VEC; c++) acc += static_cast<double>(i < V - 1 || static_cast<uint32_t>(c) >= dup ? e[i][c] : 0.f);
+            } else {
+                // The last vector repeats none of its elements (dup = 0), all of them, or, in one lane of a row, as many as
+                // n says: the same number in every row, so that lane's sum has weights that are the same in every lane
+                // (by a condition an element 16 instructions, which issue in 4.4 cycles, not 8 in 2.4).
+                const uint32_t some = (0u - n) % VEC;
+                auto weight = [&](int c) {  // (a scalar register's)
+                    return __int_as_float(__builtin_amdgcn_readfirstlane(static_cast<uint32_t>(c) >= some ? 0x3F800000 : 0));
+                };
+#pragma unroll
+                for (int c0 = 0; c0 < VEC; c0 += SUM) {
+                    float part = e[i][c0];
+#pragma unroll
+                    for (int c = c0 + 1; c < c0 + SUM; c++) part += e[i][c];
+                    if (i == V - 1) {
+                        float rest = e[i][c0] * weight(c0);
+#pragma unroll
+                        for (int c = c0 + 1; c < c0 + SUM; c++) rest = fmaf(e[i][c], weight(c), rest);
+                        part = dup == 0u ? part : dup < static_cast<uint32_t>(VEC) ? rest : 0.f;
+                    }
+                    acc += static_cast<double>(part);
                 }
             }
         }
@@ -178,18 +234,7 @@ template <typename T, int V, int CACHE> struct RowPiece {
         const Quotient<T> over_sum(rinv);
 #pragma unroll
         for (int i = 0; i < V; i++) {
-            Vec128<T> r;
-            r.v = make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                e[i][c] = over_sum(e[i][c]);
-                r.set(c, e[i][c]);
-            }
-            if (nan_where) {  // (the same in every thread)
-#pragma unroll
-                for (int c = 0; c < VEC; c++)
-                    if (e[i][c] != e[i][c]) r.set(c, nan_value);
-            }
+            const Vec128<T> r = probabilities<T>(e[i], [&](int) { return over_sum; }, nan_where, nan_value);
             if (live && (i < V - 1 || dup < static_cast<uint32_t>(VEC))) store16<CACHE>(orow + first[i], r.v);
         }
     }
@@ -209,10 +254,10 @@ __global__ __launch_bounds__(kSoftmaxGroupThreads) void softmax_group_kernel(con
     const size_t row0 = static_cast<size_t>(live ? row : rows - 1u) * n;  // (lanes past the last row shadow it and store nothing)
     RowPiece<T, V, CACHE> p;
     p.load(in + row0, n, threadIdx.x % G, G);
-    const float m = group_max<G>(p.largest());
+    const float m = p.template largest<G>();
     // (halves: the shorter the row, the fewer terms are added in float -- n up to 64: 1, 128: 2, 256: 4, else 8)
     constexpr int SUM = G == 8 ? (V == 1 ? 1 : V == 2 ? 2 : 4) : G == 16 && V <= 2 ? 4 : 8;
-    const double rinv = reciprocal_of_sum(group_sum<G>(p.template terms<SUM < Vec128<T>::N ? SUM : Vec128<T>::N>(m)));
+    const double rinv = row_reciprocal(group_sum<G>(p.template terms<SUM < Vec128<T>::N ? SUM : Vec128<T>::N>(m, n)), m);
     if constexpr (MAX_ONLY) {
         if (live && threadIdx.x % G == 0) store_largest(out, row, m, rinv);
     } else {
@@ -235,14 +280,14 @@ __global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel
     const size_t row0 = static_cast<size_t>(blockIdx.x) * n;
     RowPiece<T, V, CACHE> p;
     p.load(in + row0, n, tid, blockDim.x);
-    float m = group_max<kWave>(p.largest());
+    float m = p.template largest<kWave>();
     if (waves > 1) {
         if (lane == 0) fscratch[wave] = m;
         __syncthreads();
         const uint32_t w = lane & (kSoftmaxRowWavesMax - 1);
-        m = group_max<kSoftmaxRowWavesMax>(w < waves ? fscratch[w] : -INFINITY);
+        m = group_maximum<kSoftmaxRowWavesMax>(w < waves ? fscratch[w] : -INFINITY);
     }
-    double s = group_sum<kWave>(p.template terms<Vec128<T>::N>(m));
+    double s = group_sum<kWave>(p.template terms<Vec128<T>::N>(m, n));
     if (waves > 1) {
         if (lane == 0) dscratch[wave] = s;
         __syncthreads();
@@ -250,9 +295,9 @@ __global__ __launch_bounds__(kSoftmaxRowWavesMax *kWave) void softmax_row_kernel
         s = group_sum<kSoftmaxRowWavesMax>(w < waves ? dscratch[w] : 0.0);
     }
     if constexpr (MAX_ONLY) {
-        if (tid == 0) store_largest(out, blockIdx.x, m, reciprocal_of_sum(s));
+        if (tid == 0) store_largest(out, blockIdx.x, m, row_reciprocal(s, m));
     } else {
-        p.store(out + row0, reciprocal_of_sum(s), true, nan_where, nan_value);
+        p.store(out + row0, row_reciprocal(s, m), true, nan_where, nan_value);
     }
 }
 
@@ -485,15 +530,10 @@ __global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(con
 #pragma unroll
     for (int i = 0; i < V; i++) {
         const uint32_t e0 = e_first + static_cast<uint32_t>(i) * NT * VEC;
-        float p[VEC];
-        Vec128<T> r;
-        r.v = make_uint4(0, 0, 0, 0);
+        float e[VEC];
 #pragma unroll
-        for (int c = 0; c < static_cast<int>(VEC); c++) {
-            p[c] = over_sum(softmax_term_of_row<T>(q[i].get(c), m));
-            if (nan_where && p[c] != p[c]) p[c] = nan_value;  // (nan_where: the same in every thread)
-            r.set(c, p[c]);
-        }
+        for (int c = 0; c < static_cast<int>(VEC); c++) e[c] = term_of_row(q[i], c, m);
+        const Vec128<T> r = probabilities<T>(e, [&](int) { return over_sum; }, nan_where, nan_value);
         if (e0 <= n - VEC) {
             store16_stream(orow + e0, r.v);
         } else if (e0 < n) {
@@ -502,7 +542,7 @@ __global__ __launch_bounds__(kSoftmaxScaleThreads) void softmax_scale_kernel(con
             const uint32_t dup = e0 - (n - VEC);
 #pragma unroll
             for (int c = 1; c < static_cast<int>(VEC); c++)
-                if (static_cast<uint32_t>(c) >= dup) store_elem(orow, n - VEC + static_cast<uint32_t>(c), p[c]);
+                if (static_cast<uint32_t>(c) >= dup) store_elem(orow, n - VEC + static_cast<uint32_t>(c), r.get(c));
         }
     }
 }
