@@ -456,6 +456,26 @@ def test_sampling_half_rows_whose_probabilities_tie(ops, n, k):
         assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])
 
 
+@pytest.mark.parametrize("k", [4, 40, 120])
+def test_half_rows_whose_cut_is_a_few_of_the_smallest_half(ops, k):
+    """Rows whose k-th probability is 1 to 60 of the smallest half, so that its group spans a logit or a sixtieth of one, far below
+    the first k: the list goes on as far as the group can, or the row is looked at again."""
+    rng = np.random.default_rng(k)
+    rows, n = 48, 50257
+    x = rng.standard_normal((rows, n)).astype(np.float32) * np.float32(1.25)
+    cut = np.sort(x, axis=-1)[:, -k]
+    units = np.exp(np.linspace(np.log(0.8), np.log(60.0), rows))
+    x[np.arange(rows), rng.integers(0, n, rows)] = cut + np.log(2.0 ** 24 / units).astype(np.float32)
+    x = x.astype(np.float16)
+    v, ix = (host(t) for t in ops.softmax_topk(dev(x), k))
+    ov, oix = oracle.softmax_topk(x, k)
+    # (sums agree to 2^-22: a probability that close to a boundary between two halves may fall on either side of it)
+    same = (v.view(np.uint16) == ov.view(np.uint16)).all(axis=-1)
+    assert half_ulp_diff(v, ov).max() <= 1 and same.sum() >= rows - 2 and np.array_equal(ix[same], oix[same])
+    equal = v[:, 1:] == v[:, :-1]
+    assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])
+
+
 @pytest.mark.parametrize("k", [3, 20, 40, 90])
 def test_half_rows_with_a_tie_at_the_cut_where_the_list_may_end(ops, k):
     """k + 5 elements above the rest, t + 1 neighbouring ones of them around the k-th place a last place of their logits apart, whose

@@ -269,6 +269,7 @@ struct PickShared {
     uint32_t stage_e[kPickThreads / kWave][kWave];  // ... and the index of their first element
     uint32_t trial_cnt[kPickThreads / kWave][kPickThreads / kWave];  // [wave][trial]: the wave's thread maxima that reach another wave's bound
     uint32_t waves_above;  // waves whose list does not go on below the threshold
+    uint32_t wave_top[kPickThreads / kWave];  // the largest key of each wave's blocks
 };
 union PickSharedUnion {
     PickShared pick;
@@ -429,7 +430,25 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     // sorted row -- make the smallest of the waves' bounds far too low).
     // bits: how many leading bits of the answer are worked out when one wave does it (32:
     // the exact (k+1)-th largest, the key of an element).
-    auto threshold_of_thread_maxima = [&](uint32_t mine_max, bool by_quota, int bits = 20) -> uint32_t {
+    // row_top: with_top_tag true, the largest key of all the threads as well; a wave's steps to it go between those of its descent,
+    // which wait for each other (one after the other 0.2 us a call).
+    uint32_t row_top = 0;
+    auto max_step = [](uint32_t v, int step) __attribute__((always_inline)) -> uint32_t {  // after six the last lane has the wave's largest
+        auto of = [&](auto ctrl, auto rows) {
+            return max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), decltype(ctrl)::value, decltype(rows)::value, 0xF, false)));
+        };
+        using std::integral_constant;
+        return step == 0   ? of(integral_constant<int, 0xB1>{}, integral_constant<int, 0xF>{})
+               : step == 1 ? of(integral_constant<int, 0x4E>{}, integral_constant<int, 0xF>{})
+               : step == 2 ? of(integral_constant<int, 0x141>{}, integral_constant<int, 0xF>{})
+               : step == 3 ? of(integral_constant<int, 0x140>{}, integral_constant<int, 0xF>{})
+               : step == 4 ? of(integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{})   // row_bcast:15
+               : step == 5 ? of(integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{})   // row_bcast:31
+                           : v;
+    };
+    auto threshold_of_thread_maxima = [&](uint32_t mine_max, bool by_quota, int bits, auto with_top_tag) -> uint32_t {
+        constexpr bool WITH_TOP = decltype(with_top_tag)::value;
+        uint32_t top = mine_max;
         const uint32_t quota = (want + NW - 1) / NW;
         uint32_t mine_q = 0;
         if (by_quota && quota <= 32u) {
@@ -439,11 +458,18 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                 const uint32_t c1 = static_cast<uint32_t>(__popcll(__ballot(mine_max >= t1)));
                 const uint32_t c2 = static_cast<uint32_t>(__popcll(__ballot(mine_max >= t2)));
                 const uint32_t c3 = static_cast<uint32_t>(__popcll(__ballot(mine_max >= t3)));
+                if constexpr (WITH_TOP) top = max_step(top, (30 - bit) / 2);
                 mine_q = c3 >= quota ? t3 : c2 >= quota ? t2 : c1 >= quota ? t1 : mine_q;
             }
+        } else if constexpr (WITH_TOP) {
+#pragma unroll
+            for (int step = 0; step < 6; step++) top = max_step(top, step);
         }
         sh.lane_key[tid] = mine_max;
         if (lane == 0) sh.wave_thr[wave] = mine_q;
+        if constexpr (WITH_TOP) {
+            if (lane == kWave - 1) smem.pick.wave_top[wave] = top;
+        }
         __syncthreads();
         uint32_t bound[NW];
         uint32_t t = 0xFFFFFFFFu;
@@ -451,6 +477,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         for (int w = 0; w < NW; w++) {
             bound[w] = sh.wave_thr[w];
             t = min(t, bound[w]);
+            if constexpr (WITH_TOP) row_top = max(row_top, smem.pick.wave_top[w]);
         }
         if (by_quota && t > 1u) {
             // The smallest of the waves' bounds is reached by k+1 thread maxima but is lower than it need be
@@ -483,7 +510,8 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         }
         return t;
     };
-    uint32_t thr = threshold_of_thread_maxima(lmk, true);
+    constexpr bool kByDifference = SOFTMAX && sizeof(T) == 2;
+    uint32_t thr = threshold_of_thread_maxima(lmk, true, 20, std::integral_constant<bool, kByDifference>{});
     BPS(10);
     // -inf never becomes a candidate: a row with k+1 larger elements does not need it,
     // and finish_row fills any other row's last places from the row itself
@@ -515,11 +543,20 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     // k = 50 18.7 us, [64,32000] k = 40 15.4, [32,50257] k = 40 17.0; so 14.0, 10.2, 11.4).  Halves: the probabilities of logits closer
     // than 0.01 are often equal, and seldom those of others (from 100 of the smallest half on).  It is one candidate in a hundred more: sampling
     // [32,50257] k = 40 by the inputs 14.0 / 14.0 / 19.3 us, with the threshold as found 13.8 to 22.2.
+    // Where the row's maximum stands so far above the threshold that the probability there is less than 100 of the smallest half (at
+    // most exp(t - max) of 2^-24: the sum is at least 1), one of that probability reaches as far as one such unit is of it, and so
+    // does the list, down to one and a half units: [32,50257] k = 40, a row in two hundred of which had a group of 60 beyond the
+    // first 40, 17.1 -> 14.3 us, [256,50257] k = 50 26.7 -> 21.6; calls without one pay 0.1 us for the maximum.
     // Not in rows so narrow that it is many more: a wave with four times its share of k + 1 blocks keeps to the threshold.
-    constexpr bool kByDifference = SOFTMAX && sizeof(T) == 2;
     if constexpr (SOFTMAX && !kByDifference) thr = max(thr - 1024u, kKeyNegInf + 1u);
     uint32_t low = thr;
-    if constexpr (kByDifference) low = max(min(thr, order_key(ordered_to_float(thr) - 1e-2f)), kKeyNegInf + 1u);
+    float reach = 1e-2f;
+    if constexpr (kByDifference) {
+        const float t = ordered_to_float(thr);
+        const float unit = __builtin_amdgcn_exp2f(fmaf(ordered_to_float(row_top) - t, 1.44269504f, -24.f));
+        if (unit > reach && unit < 0.7f) reach = unit;
+        low = max(min(thr, order_key(t - reach)), kKeyNegInf + 1u);
+    }
     if (wave_lists) {
         uint32_t wave_n = 0, own_thr = low;  // wave-uniform
 #pragma unroll
@@ -646,7 +683,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         // us, [32,50257] k = 40, every list to the threshold / below it / so: rows spread by 0.3 21.0 / 13.0 / 13.0, 0.05 22.2 /
         // 14.9 / 14.8, 0.02 23.0 / 31.0 / 24.5, 0.001 32.4 / 38.5 / 34.2; k = 100 0.3 15.7 / 22.0 / 16.2; spread by 1 12.4 either way.
         const uint32_t above = smem.pick.waves_above, have = sh.count;
-        if (listed && above == 0u && have <= (want <= 112u ? 128u : 256u)) {
+        if (listed && above == 0u && have <= (want <= 112u && reach < 0.05f ? 128u : 256u)) {
             thr = low;
         } else if (listed && above != static_cast<uint32_t>(NW) && low < thr) {
             listed = have <= static_cast<uint32_t>(kFastCap);
@@ -1006,7 +1043,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         dry_max = 0;
         gather(thr, 1ull << 32, std::true_type{});
         level_max = dry_max;
-        const uint32_t tight = threshold_of_thread_maxima(dry_max, false);  // (the barrier at the end of gather lies between this and the last use of its LDS)
+        const uint32_t tight = threshold_of_thread_maxima(dry_max, false, 20, std::false_type{});  // (the barrier at the end of gather lies between this and the last use of its LDS)
         if (tid == 0) sh.count = 0;
         __syncthreads();
         thr = max(thr, tight);
@@ -1068,7 +1105,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
         // (thr so far is a value rounded down; this needs the key of an element: the exact
         // (k+1)-th largest of the thread maxima it came from)
         __syncthreads();
-        thr = max(thr, threshold_of_thread_maxima(level_max, false, 32));
+        thr = max(thr, threshold_of_thread_maxima(level_max, false, 32, std::false_type{}));
     }
     if ((many_groups || C2 > static_cast<uint32_t>(kFastCap)) && thr < 0xFFFFFFFFu) {
         __syncthreads();
