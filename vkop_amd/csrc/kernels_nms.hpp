@@ -20,10 +20,12 @@
 //      candidates, held in registers, against the block's survivors and clears
 //      their bits in the active mask.  Two barriers per block of 64 instead of
 //      one per selection;
-//   4. the selected box indices go to the pair's segment of the workspace.
-// nms_pack_kernel then writes the (batch, class, box) records of all pairs one
-// after the other, in order of batch and class: the result does not depend on
-// scheduling (the reference appends through a global atomic counter).
+//   4. the (batch, class, box) records of all pairs are written one after the other, in order of
+//      batch and class: the result does not depend on scheduling (the reference appends through a
+//      global atomic counter).  Of pairs that the chip holds at once every workgroup publishes its
+//      number of records, waits for those of the pairs before it and writes its own (place_records);
+//      of more, the selected box indices go to the pair's segment of the workspace and
+//      nms_pack_kernel writes them all.
 #pragma once
 
 #include "device_utils.hpp"
@@ -39,6 +41,10 @@ constexpr int kNmsThreadsNarrow = 256;  // twice as many as the chip holds wide 
 // [32,20,8400] 33.3 / 34.7.  From 513 pairs on narrow ones gain where candidates are
 // few, but where all of 2048 are they lose more: [8,80,2048] 285 / 424)
 constexpr int kNmsNarrowMinPairs = 1024;
+// One launch where the chip holds all workgroups at once (six narrow ones a CU, two wide: waves_per_eu of nms_kernel).  Of more, those
+// that wait for the pairs before them keep the rest from starting: us, two launches / one, [8,91,1917] f32 11.7 / 13.4, [20,90,3000]
+// 14.1 / 16.5; held at once [16,80,8400] 18.7 / 17.4, [1,80,8400] 9.8 / 8.3, [2,80,1000] 9.8 / 7.3.
+constexpr uint32_t kNmsHeldNarrow = 1536, kNmsHeldWide = 512;
 constexpr int kNmsMaxCandidates = 2048;  // per (batch, class); the reference's shader holds 1024
 constexpr int kNmsRankSortMax = 512;     // up to here a counting sort beats the bitonic network's barriers
 
@@ -96,7 +102,146 @@ __device__ __forceinline__ bool nms_overlap(const float4 &a, const float4 &b, fl
     return (uni > 0.f ? __fdiv_rn(inter, uni) : 0.f) > threshold;
 }
 
-// counts[pair] = boxes selected; counts[pairs + pair] = 1 if more than
+// ---- a pair's records, by the workgroup that selected them ---------------------------------------
+// What a workgroup publishes: under a tag of 40 bits, its number of records (at most 2048), whether boxes were left out, and whether
+// it has given up waiting.  The tag comes from the launch and from a word in memory that every call moves on, so that neither the
+// workspace's former contents nor a recording's replay before has it: nothing has to be cleared.
+struct NmsJoined {
+    uint64_t *words;  // a word a pair, kNmsCopies times, then the word of the call and the tag of the call a workgroup last gave up in
+    int32_t *out, *out_count;
+    uint32_t capacity, polls;
+    uint64_t launch;
+};
+// Copies of the words, each read by every eighth workgroup: a thousand that read the same few lines again and again wait for each
+// other ([16,80,8400] f32 18.5 us with one copy, 17.0 with 8, 17.1 with 32).
+constexpr uint32_t kNmsCopies = 8;
+__host__ __device__ constexpr uint32_t nms_copy_stride(uint32_t pairs) { return (pairs + 31u) / 32u * 32u; }
+constexpr size_t nms_words(uint32_t pairs) { return static_cast<size_t>(kNmsCopies) * nms_copy_stride(pairs) + 2; }
+constexpr int kNmsCallWord = 0, kNmsLateWord = 1;  // (behind the copies)
+constexpr uint32_t kNmsCount = 0xFFFFu, kNmsOver = 1u << 16, kNmsGaveUp = 1u << 17;
+__device__ __forceinline__ uint64_t nms_tag(uint64_t launch, uint64_t call) {  // (1 .. 2^40 - 1)
+    return ((call * 0x9E3779B97F4A7C15ull + launch * 0xC2B2AE3D27D4EB4Full) >> 24) | 1ull;
+}
+__device__ __forceinline__ void nms_put_record(int32_t *out, uint32_t capacity, uint32_t at, int32_t batch, int32_t cls, int32_t box) {
+    if (at >= capacity) return;
+    out[static_cast<size_t>(at) * 3 + 0] = batch;
+    out[static_cast<size_t>(at) * 3 + 1] = cls;
+    out[static_cast<size_t>(at) * 3 + 2] = box;
+}
+// The end of a call, one thread: the number of all records, the overflow flag, the (-1, -1, -1) behind the last record, and the word
+// of the next call (every workgroup has published by now, with this one's).
+__device__ __forceinline__ void nms_put_total(const NmsJoined &j, uint64_t *extra, uint64_t call, uint32_t total, bool over) {
+    j.out_count[0] = static_cast<int32_t>(total);
+    j.out_count[1] = over ? 1 : 0;
+    nms_put_record(j.out, j.capacity, total, -1, -1, -1);
+    publish(extra + kNmsCallWord, call + 1u);
+}
+// The records of workgroups that gave up, as far as all the pairs before them have arrived: a wave.  (Two that find the same ones
+// write the same.)
+__device__ __forceinline__ void nms_place_late(const NmsJoined &j, uint64_t *extra, uint64_t call, uint64_t tag, const int32_t *selected,
+                                               uint32_t pairs, uint32_t C, uint32_t max_sel) {
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    uint32_t total = 0, over = 0;
+    for (uint32_t base = 0; base < pairs; base += kWave) {
+        const uint32_t q = base + lane;
+        const uint64_t word = q < pairs ? fetch(j.words + q) : tag << 24;
+        const uint64_t absent = __ballot((word >> 24) != tag);
+        const uint32_t w = static_cast<uint32_t>(word), have = absent != 0ull ? static_cast<uint32_t>(__builtin_ctzll(absent)) : static_cast<uint32_t>(kWave);
+        const uint32_t incl = wave_inclusive_sum_u32(w & kNmsCount);
+        over |= w & kNmsOver;
+        for (uint64_t left = __ballot(lane < have && (w & kNmsGaveUp) != 0u); left != 0ull; left &= left - 1ull) {
+            const int l = static_cast<int>(__builtin_ctzll(left));
+            const uint32_t m = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(w), l)) & kNmsCount;
+            const uint32_t first = total + static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), l)) - m;
+            const uint32_t of = base + static_cast<uint32_t>(l);
+            for (uint32_t r = lane; r < m; r += kWave) {
+                const int32_t box = __hip_atomic_load(selected + static_cast<size_t>(of) * max_sel + r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                nms_put_record(j.out, j.capacity, first + r, static_cast<int32_t>(of / C), static_cast<int32_t>(of % C), box);
+            }
+        }
+        if (have != static_cast<uint32_t>(kWave)) return;
+        total += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), kWave - 1));
+    }
+    const bool any_over = __ballot(over != 0u) != 0ull;
+    if (lane == 0) nms_put_total(j, extra, call, total, any_over);
+}
+// All threads call, behind a barrier after the last write to picks (LDS: the n selected boxes in order).  The wait needs no
+// particular number of workgroups on the chip to end: after `polls` looks a workgroup leaves its boxes in its segment, says so, and
+// looks once more; one that has published then looks whether any has.  Each does so after its own word is in memory, so that
+// at least one of the two finds the other, and the records are placed.  (A counter of the workgroups that are done, on whose
+// last one the rest could be left, costs their turns at one address: 1280 of them 10 us.)
+template <int NT>
+__device__ __forceinline__ void place_records(const NmsJoined &j, uint64_t call, const uint32_t *picks, uint32_t n, bool over, int32_t *selected,
+                                              uint32_t pair, uint32_t pairs, uint32_t C, uint32_t max_sel, uint32_t *scratch) {
+    constexpr int NW = NT / kWave, U = NT >= 1024 ? 2 : 6;
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform_u32(tid) / kWave;
+    const uint64_t tag = nms_tag(j.launch, call), own = (tag << 24) | (over ? kNmsOver : 0u) | n;
+    const uint32_t stride = nms_copy_stride(pairs);
+    uint64_t *extra = j.words + kNmsCopies * stride;
+    if (tid < kNmsCopies) publish(j.words + tid * stride + pair, own);
+    const uint64_t *words = j.words + pair % kNmsCopies * stride;
+    uint32_t before = 0, flags = over ? kNmsOver : 0u;
+    for (uint32_t base = 0; base < pair; base += U * NT) {
+        uint64_t w[U];
+        auto at = [&](int u) { return base + static_cast<uint32_t>(u) * NT + tid; };
+#pragma unroll
+        for (int u = 0; u < U; u++) w[u] = at(u) < pair ? fetch(words + at(u)) : tag << 24;
+        for (uint32_t poll = 0;; poll++) {
+            bool absent = false;
+#pragma unroll
+            for (int u = 0; u < U; u++) absent = absent || (w[u] >> 24) != tag;
+            if (!absent) break;
+            if (poll >= j.polls) {
+                flags |= kNmsGaveUp;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+#pragma unroll
+            for (int u = 0; u < U; u++)
+                if ((w[u] >> 24) != tag) w[u] = fetch(words + at(u));
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            before += static_cast<uint32_t>(w[u]) & kNmsCount;
+            flags |= static_cast<uint32_t>(w[u]) & kNmsOver;
+        }
+    }
+    before = wave_sum(before);
+    flags = (__ballot((flags & kNmsOver) != 0u) != 0ull ? kNmsOver : 0u) | (__ballot((flags & kNmsGaveUp) != 0u) != 0ull ? kNmsGaveUp : 0u);
+    drain_stores();  // (this workgroup's word: its loads have come back behind it)
+    if (lane == 0) {
+        scratch[wave] = before;
+        scratch[NW + wave] = flags;
+    }
+    __syncthreads();
+    before = flags = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        before += scratch[w];
+        flags |= scratch[NW + w];
+    }
+    if ((flags & kNmsGaveUp) != 0u) {  // (the same in every thread)
+        for (uint32_t r = tid; r < n; r += NT)
+            __hip_atomic_store(selected + static_cast<size_t>(pair) * max_sel + r, static_cast<int32_t>(picks[r]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        drain_stores();
+        __syncthreads();
+        if (wave != 0) return;
+        if (lane == 0) {
+            publish(j.words + pair, own | kNmsGaveUp);
+            publish(extra + kNmsLateWord, tag);
+        }
+        drain_stores();
+        nms_place_late(j, extra, call, tag, selected, pairs, C, max_sel);
+        return;
+    }
+    const uint64_t late = wave == 0 ? fetch(extra + kNmsLateWord) : 0ull;
+    const int32_t batch = static_cast<int32_t>(pair / C), cls = static_cast<int32_t>(pair % C);
+    for (uint32_t r = tid; r < n; r += NT) nms_put_record(j.out, j.capacity, before + r, batch, cls, static_cast<int32_t>(picks[r]));
+    if (pair == pairs - 1 && tid == 0) nms_put_total(j, extra, call, before + n, (flags & kNmsOver) != 0u);
+    if (wave == 0 && late == tag) nms_place_late(j, extra, call, tag, selected, pairs, C, max_sel);
+}
+
+// Without JOINED: counts[pair] = boxes selected; counts[pairs + pair] = 1 if more than
 // kNmsMaxCandidates boxes passed the score threshold (the later ones were left out).
 // selected: [pairs][max_sel] box indices.  Launch: B * C workgroups of NT threads:
 // 1024 when there are few pairs (one pair's work spread wide), 256 when there are
@@ -108,15 +253,16 @@ __device__ __forceinline__ bool nms_overlap(const float4 &a, const float4 &b, fl
 // boxes 1.3, the block's overlaps 1.5, its kept set 0.4 (a second block, one pair in twenty, 1.6).  A chain this
 // short is bound by instruction fetch as much as by anything: a launch finds none of its code in the CUs' caches,
 // and forms of these steps that run fewer instructions out of more code were slower, step by step.  us a call with the
-// pack kernel, 0.25 / 0.45, 51 kept a pair: [16,80,8400] f32 26.1 -> 18.3, f16 24.1 -> 15.5; [16,91,8399] f32
-// 27.0 -> 18.4; [1,80,8400] f32 11.6 -> 10.8; [8,91,1917] f32 15.2 -> 11.6; [16,20,8400], 400 candidates, 26.1 -> 24.1;
+// records, 0.25 / 0.45, 51 kept a pair: [16,80,8400] f32 26.1 -> 18.5 -> 17.2 (by place_records), f16 24.1 -> 16.5 -> 15.7; [16,91,8399]
+// f32 27.0 -> 18.7 -> 17.1; [1,80,8400] f32 11.6 -> 9.9 -> 8.3; [8,91,1917] f32 15.2 -> 11.6; [16,20,8400], 400 candidates, 26.1 -> 24.7 -> 23.2;
 // [8,80,400] all candidates 33.4 -> 29.3; more than 2048 of 8400 ([4,4,8400], the list made twice) 64.2 -> 64.6.
+// JOINED: the records too (joined); else nms_pack_kernel follows.
 // WHOLE: N is a multiple of four, and no load needs the step for a row's end (it costs a row that has one 0.4 us).
-template <typename T, int NT, bool WHOLE>
+template <typename T, int NT, bool WHOLE, bool JOINED>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ? 8 : 6))) void nms_kernel(
     const T *__restrict__ boxes, const T *__restrict__ scores, int32_t *__restrict__ selected, uint32_t *__restrict__ counts,
     uint32_t pairs, uint32_t C, uint32_t N, int center_point_box, uint32_t max_out, float iou_threshold, float score_threshold,
-    uint32_t max_sel) {
+    uint32_t max_sel, NmsJoined joined) {
     static_assert(NT % kWave == 0 && kNmsMaxCandidates % NT == 0 && (kNmsRankSortMax % NT == 0 || NT % kNmsRankSortMax == 0), "workgroup size");
     constexpr int NW = NT / kWave;
     constexpr int PER = kNmsMaxCandidates / NT;      // sorted candidates per thread
@@ -128,8 +274,12 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
     __shared__ unsigned long long block_cols[kWave];
     __shared__ unsigned long long block_keep, block_gone;
     __shared__ uint32_t wave_n[2][NW], listed;
+    // the selected boxes, where nothing else of a step lies any more: the list before its sort, or sorted candidates at or below the block's
+    typedef uint32_t __attribute__((may_alias)) Pick;
+    Pick *const picks = reinterpret_cast<Pick *>(comp);
     const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform_u32(tid) / kWave;  // (scalar)
     const uint32_t pair = blockIdx.x, batch = pair / C;
+    const uint64_t call = JOINED ? fetch(joined.words + kNmsCopies * nms_copy_stride(pairs) + kNmsCallWord) : 0ull;  // (under the scores' loads)
     const T *srow = scores + static_cast<size_t>(pair) * N;
     const T *brow = boxes + static_cast<size_t>(batch) * N * 4;
     if (tid < static_cast<uint32_t>(kNmsMaxCandidates / 64)) active[tid] = ~0ull;  // positions at or after K are masked where read
@@ -301,10 +451,19 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
         if (lane == 0) block_keep = keep;
         if ((keep >> lane) & 1u) {
             const uint32_t slot = chosen + lanes_below(keep);
-            if (slot < max_sel)
-                selected[static_cast<size_t>(pair) * max_sel + slot] = static_cast<int32_t>(composite_index(sorted[base + lane]));
+            const uint32_t box = composite_index(sorted[base + lane]);
+            if (JOINED) picks[slot] = box;
+            else if (slot < max_sel) selected[static_cast<size_t>(pair) * max_sel + slot] = static_cast<int32_t>(box);
         }
         return keep;
+    };
+    auto finish = [&](bool over) __attribute__((always_inline)) {
+        if constexpr (JOINED) {
+            place_records<NT>(joined, call, picks, min(chosen, max_sel), over, selected, pair, pairs, C, max_sel, &wave_n[0][0]);
+        } else if (tid == 0) {
+            counts[pair] = min(chosen, max_sel);
+            counts[pairs + pair] = over ? 1u : 0u;
+        }
     };
     auto uniform_keep = [&]() -> uint64_t {
         const unsigned long long kept = block_keep;
@@ -406,10 +565,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
             __syncthreads();
             chosen += static_cast<uint32_t>(__popcll(uniform_keep()));
         }
-        if (tid == 0) {
-            counts[pair] = min(chosen, max_sel);
-            counts[pairs + pair] = 0;
-        }
+        finish(false);
         return;
     }
 
@@ -468,10 +624,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
         }
         // (no barrier here: the next block writes the other box buffer, and its barriers order the rest)
     }
-    if (tid == 0) {
-        counts[pair] = min(chosen, max_sel);
-        counts[pairs + pair] = found > static_cast<uint32_t>(kNmsMaxCandidates) ? 1u : 0u;
-    }
+    finish(found > static_cast<uint32_t>(kNmsMaxCandidates));
 }
 
 // The records of all pairs one after the other.  out: [capacity][3]; out_count[0] =

@@ -137,11 +137,14 @@ std::atomic<int> g_rows_stages{3};
 inline int measured_stages() { return g_rows_stages.load(); }
 std::atomic<uint32_t> g_joined_polls{100};
 inline uint32_t joined_polls() { return g_joined_polls.load(); }
+inline uint32_t nms_polls() { return g_joined_polls.load() * 40u; }
 #else
 inline int measured_stages() { return 3; }
 // How often a workgroup of softmax_joined_kernel looks for its row's other chunks before it reads what it misses: a look takes
 // about a microsecond, the wait for a row whose workgroups run a few of them.
 constexpr uint32_t joined_polls() { return 100; }
+// The same of nms_kernel, whose pairs take from 6 to 700 us.
+constexpr uint32_t nms_polls() { return 4000; }
 #endif
 // (what tells the records of a call of softmax_joined_kernel from whatever the workspace held before)
 std::atomic<uint32_t> g_joined_calls{0};
@@ -1338,10 +1341,17 @@ size_t nms_workspace(int B, int C, int N, int max_per_class) {
     const size_t pairs = static_cast<size_t>(B) * C;
     return kTicketBytes + align_up(2 * pairs * sizeof(uint32_t)) + align_up(pairs * nms_max_sel(N, max_per_class) * sizeof(int32_t));
 }
+// With the words of the one launch (in a workspace of the size above, without them, a call takes the two).
+size_t nms_joined_workspace(int B, int C, int N, int max_per_class) {
+    const uint64_t pairs = static_cast<uint64_t>(B) * C;
+    const size_t two = nms_workspace(B, C, N, max_per_class);
+    return pairs > vkop::kNmsHeldNarrow ? two : two + align_up(vkop::nms_words(static_cast<uint32_t>(pairs)) * sizeof(uint64_t));
+}
 
 template <typename T>
 int nms_impl(const T *boxes, const T *scores, int32_t *out, int out_capacity, int32_t *out_count, int B, int C, int N,
-             int center_point_box, int max_per_class, float iou_threshold, float score_threshold, void *ws, hipStream_t st) {
+             int center_point_box, int max_per_class, float iou_threshold, float score_threshold, void *ws, size_t ws_bytes,
+             hipStream_t st) {
     const uint32_t pairs = static_cast<uint32_t>(B) * static_cast<uint32_t>(C);
     auto *base = static_cast<unsigned char *>(ws) + kTicketBytes;
     auto *counts = reinterpret_cast<uint32_t *>(base);
@@ -1350,16 +1360,31 @@ int nms_impl(const T *boxes, const T *scores, int32_t *out, int out_capacity, in
     const uint32_t per = max_per_class > 0 ? static_cast<uint32_t>(max_per_class) : 0u;
     const int knob = g_nms_threads;  // 0: by the number of pairs
     const bool narrow = knob > 0 ? knob == vkop::kNmsThreadsNarrow : pairs >= static_cast<uint32_t>(vkop::kNmsNarrowMinPairs);
-#define VKOP_NMS_LAUNCH(NT, WHOLE)                                                                                         \
-    vkop::nms_kernel<T, NT, WHOLE><<<pairs, NT, 0, st>>>(boxes, scores, selected, counts, pairs, static_cast<uint32_t>(C), \
-                                                         static_cast<uint32_t>(N), center_point_box, per, iou_threshold,  \
-                                                         score_threshold, max_sel)
-    if (narrow && N % 4 == 0) VKOP_NMS_LAUNCH(vkop::kNmsThreadsNarrow, true);
-    else if (narrow) VKOP_NMS_LAUNCH(vkop::kNmsThreadsNarrow, false);
-    else if (N % 4 == 0) VKOP_NMS_LAUNCH(vkop::kNmsThreadsWide, true);
-    else VKOP_NMS_LAUNCH(vkop::kNmsThreadsWide, false);
+    const bool one_launch = pairs <= (narrow ? vkop::kNmsHeldNarrow : vkop::kNmsHeldWide) && ws_bytes >= nms_joined_workspace(B, C, N, max_per_class) &&
+                            reinterpret_cast<uintptr_t>(ws) % sizeof(uint64_t) == 0;
+    auto *words = reinterpret_cast<uint64_t *>(static_cast<unsigned char *>(ws) + nms_workspace(B, C, N, max_per_class));
+    const vkop::NmsJoined joined{one_launch ? words : nullptr, out, out_count, static_cast<uint32_t>(out_capacity), nms_polls(),
+                                 one_launch ? g_joined_calls.fetch_add(1, std::memory_order_relaxed) : 0u};
+#define VKOP_NMS_LAUNCH(NT, WHOLE, JOINED)                                                                                 \
+    vkop::nms_kernel<T, NT, WHOLE, JOINED><<<pairs, NT, 0, st>>>(boxes, scores, selected, counts, pairs,                   \
+                                                                 static_cast<uint32_t>(C), static_cast<uint32_t>(N),       \
+                                                                 center_point_box, per, iou_threshold, score_threshold,    \
+                                                                 max_sel, joined)
+#define VKOP_NMS_FORM(NT, WHOLE)                            \
+    if (one_launch) VKOP_NMS_LAUNCH(NT, WHOLE, true);       \
+    else VKOP_NMS_LAUNCH(NT, WHOLE, false)
+    if (narrow && N % 4 == 0) {
+        VKOP_NMS_FORM(vkop::kNmsThreadsNarrow, true);
+    } else if (narrow) {
+        VKOP_NMS_FORM(vkop::kNmsThreadsNarrow, false);
+    } else if (N % 4 == 0) {
+        VKOP_NMS_FORM(vkop::kNmsThreadsWide, true);
+    } else {
+        VKOP_NMS_FORM(vkop::kNmsThreadsWide, false);
+    }
+#undef VKOP_NMS_FORM
 #undef VKOP_NMS_LAUNCH
-    if (int rc = launched("nms_kernel")) return rc;
+    if (int rc = launched("nms_kernel"); rc != VKOP_HIP_OK || one_launch) return rc;
     const uint32_t packers = (pairs + vkop::kNmsPackPairs - 1) / vkop::kNmsPackPairs;
     vkop::nms_pack_kernel<<<packers, 256, 0, st>>>(selected, counts, out, out_count, pairs, static_cast<uint32_t>(C), max_sel,
                                                    static_cast<uint32_t>(out_capacity));
@@ -1865,7 +1890,7 @@ int vkop_hip_softmax_reduce_max(const void *in, void *out, int dtype, const int 
 
 size_t vkop_hip_nms_workspace_bytes(int B, int C, int N, int max_output_boxes_per_class) {
     if (B < 0 || C < 0 || N < 0) return 0;
-    return nms_workspace(B, C, N, max_output_boxes_per_class);
+    return nms_joined_workspace(B, C, N, max_output_boxes_per_class);
 }
 
 int vkop_hip_nms(const void *boxes, const void *scores, int32_t *out, int out_capacity, int32_t *out_count, int dtype, int B,
@@ -1890,10 +1915,10 @@ int vkop_hip_nms(const void *boxes, const void *scores, int32_t *out, int out_ca
     if (dtype == VKOP_HIP_F32)
         return nms_impl(static_cast<const float *>(boxes), static_cast<const float *>(scores), out, out_capacity, out_count,
                         B, C, N, center_point_box, max_output_boxes_per_class, iou_threshold, score_threshold, workspace,
-                        as_stream(stream));
+                        workspace_bytes, as_stream(stream));
     return nms_impl(static_cast<const uint16_t *>(boxes), static_cast<const uint16_t *>(scores), out, out_capacity, out_count,
                     B, C, N, center_point_box, max_output_boxes_per_class, iou_threshold, score_threshold, workspace,
-                    as_stream(stream));
+                    workspace_bytes, as_stream(stream));
 }
 
 }  // extern "C"
