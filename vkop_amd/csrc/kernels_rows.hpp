@@ -279,6 +279,7 @@ template <int NT> struct ChunkShared {  // chunk phase
     uint4 stage_v[NT];     // per wave: up to 64 vectors holding an element at or above the threshold ...
     uint32_t stage_e[NT];  // ... and the index of their first element
     uint32_t wave_thr[16];
+    uint32_t reached[2][NT / kWave];  // lane maxima that reach each wave's value, two rounds in turn
     uint32_t refine[42];  // element counts per bit of the exact threshold search; [32], [33]: smallest key at or above a bound / elements
                           // above that key, and the same in [34] ... [39] for the next two distinct values up
     uint32_t thr, total, over;
@@ -1653,12 +1654,33 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
                 for (int w = 0; w < NW; w++) kv[w] = cs.lane_key[w * kWave + lane];
                 const int d = 31 - __clz(static_cast<int>(lo ^ hi));  // highest bit in which they differ
                 t = hi & ~((2u << d) - 1u);                            // their common prefix
-                for (int bit = d; bit > 15; bit--) {
-                    const uint32_t trial = t | (1u << bit);
+                auto count = [&](uint32_t trial) -> uint32_t {
                     uint32_t cnt = 0;
 #pragma unroll
                     for (int w = 0; w < NW; w++) cnt += static_cast<uint32_t>(__popcll(__ballot(kv[w] >= trial)));
-                    if (cnt >= want) t = trial;
+                    return cnt;
+                };
+                if constexpr (NW >= 8) {
+                    // Many waves: four bits (eight waves: three) a round, each wave a value of them.  (Every wave every bit, 16
+                    // ballots each and four waves a SIMD, was this kernel's longest step: [16,8400] f32 k = 300 9.9 -> 8.7 us, [256,6000] k = 200 by a tenth.)
+                    constexpr int B = NW >= 16 ? 4 : 3;
+                    for (int top = d, round = 0; top > 15; top -= B, round ^= 1) {
+                        const int low = max(top - B + 1, 16);
+                        const uint32_t values = 2u << (top - low);
+                        if (wave != 0 && wave < values) {
+                            const uint32_t cnt = count(t | (wave << low));
+                            if (lane == 0) cs.reached[round][wave] = cnt;
+                        }
+                        __syncthreads();
+                        // (fewer reach a larger value: the last that k+1 do; none: as it was)
+                        const uint64_t ok = __ballot(lane != 0u && lane < values && lane < static_cast<uint32_t>(NW) && cs.reached[round][lane & (NW - 1u)] >= want);
+                        if (ok != 0ull) t |= (63u - static_cast<uint32_t>(__clzll(static_cast<long long>(ok)))) << low;
+                    }
+                } else {
+                    for (int bit = d; bit > 15; bit--) {
+                        const uint32_t trial = t | (1u << bit);
+                        if (count(trial) >= want) t = trial;
+                    }
                 }
             }
             thr_block = t;
