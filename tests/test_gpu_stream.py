@@ -839,3 +839,19 @@ def test_rows_of_few_values_whose_keys_end_in_ones(ops, rows, n, k, dtype):
     ev, eix = oracle.softmax_topk(x, k)
     assert np.array_equal(ix, eix)
     assert (half_ulp_diff(v, ev) if dtype == np.float16 else ulp_diff(v, ev)).max() <= (1 if dtype == np.float16 else 2)
+
+
+@pytest.mark.parametrize("n,k", [(50257, 40), (128256, 50), (262144, 600)])
+def test_nan_of_any_payload_among_the_block_maxima_and_minima(ops, n, k):
+    """Quiet and signalling NaN, alone, side by side and a block of nothing else: first in a plain top-k, last in the other direction."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((4, n)).astype(np.float32)
+    b = x.view(np.uint32)
+    b[0, rng.choice(n, 3, replace=False)] = 0x7F800001
+    b[1, 64 * 9:64 * 11] = 0xFF800123
+    b[2, rng.choice(n, k + 5, replace=False)] = 0x7FC00001
+    b[3, [0, n - 1]] = (0x7F800001, 0xFFFFFFFF)
+    xd = torch.from_numpy(x.view(np.int32)).cuda().view(torch.float32)
+    for largest in (True, False):
+        _, ix = (host(t) for t in ops.topk(xd, k, largest=largest))
+        assert np.array_equal(ix, oracle.topk(x, k, largest=largest)[1]), largest

@@ -116,7 +116,7 @@ __device__ __forceinline__ uint32_t max_half2(uint32_t a, uint32_t b) {
     return r;
 }
 
-// The larger halves of three pairs and the larger of three floats, NaN wherever one of them is NaN.
+// The larger halves of three pairs, the larger and the smaller of three floats, NaN wherever one of them is NaN.
 __device__ __forceinline__ uint32_t maximum_half2(uint32_t a, uint32_t b, uint32_t c) {
     uint32_t r;
     asm("v_pk_maximum3_f16 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
@@ -125,6 +125,12 @@ __device__ __forceinline__ uint32_t maximum_half2(uint32_t a, uint32_t b, uint32
 __device__ __forceinline__ float maximum(float a, float b, float c) {
     float r;
     asm("v_maximum3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+__device__ __forceinline__ float minimum(float a, float b, float c) {
+    float r;
+    asm("v_minimum3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
     return r;
 }
 

@@ -58,8 +58,8 @@ struct ScanWorkspace {
     uint64_t *recs2;   // [rows][G][kScanWaves]: the value whose copies the wave counted apart (float bits, high half)
                        // and how many it found (low half; 0: none): its sum leaves them out
     uint32_t blocks;   // blocks per row: ceil(n / (16 * vector width))
-    uint32_t *bmin;    // null, or (WITH_MIN) [rows][blocks]: order key of the block's minimum (NaN dropped; the key
-                       // of -inf for a block that reaches past the row's end or holds -inf)
+    uint32_t *bmin;    // null, or (WITH_MIN) [rows][blocks]: order key of the block's minimum (the key of -inf for a
+                       // block that reaches past the row's end or holds -inf or NaN)
     uint32_t *zero;    // null, or [rows][zero_words] words the scan kernel clears for the kernels behind it
     uint32_t zero_words;  // (at most 256)
 };
@@ -134,17 +134,20 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
         static_for<0, V>([&](auto i_tag) {
             constexpr int i = decltype(i_tag)::value;
             if constexpr (!FULL && !ALIGNED) settle_vec(q[i], e_first + static_cast<uint32_t>(i) * NT * VEC, n);
+            // Three values an instruction (fmaxf and fminf take two, and another to make each loaded value a quiet NaN first: eight
+            // of 38 instructions a vector).  Softmax: NaN dropped.  Plain top-k, where NaN ranks first, and the minima: kept.
             float xv[VEC];
-            float vm = -INFINITY;
 #pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                xv[c] = elem(i_tag, c);
-                vm = fmaxf(vm, xv[c]);  // (drops NaN)
-            }
+            for (int c = 0; c < VEC; c++) xv[c] = elem(i_tag, c);
+            constexpr bool kKeepNan = !SOFTMAX && !kReversed<T>;
+            auto larger = [](float a, float b, float c) { return kKeepNan ? maximum(a, b, c) : max3(a, b, c); };
+            float vm = larger(xv[0], xv[1], xv[2]);
+#pragma unroll
+            for (int c = 3; c < VEC; c += 2) vm = larger(vm, xv[c], xv[c + 1 < VEC ? c + 1 : c]);
             if constexpr (WITH_MIN) {
-                float vn = INFINITY;
+                float vn = minimum(xv[0], xv[1], xv[2]);  // (an element past the chunk's end counts as -inf)
 #pragma unroll
-                for (int c = 0; c < VEC; c++) vn = fminf(vn, xv[c]);  // (an element past the chunk's end counts as -inf)
+                for (int c = 3; c < VEC; c += 2) vn = minimum(vn, xv[c], xv[c + 1 < VEC ? c + 1 : c]);
                 vmin_lds[wave][i][lane ^ ((i & 3) << 2)] = vn;
             }
             if constexpr (SOFTMAX) {
@@ -166,12 +169,6 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
                 // the sum so far exists HERE, under the loads still in flight (or the
                 // compiler moves all of it behind the last load)
                 asm volatile("" : "+v"(acc));
-            } else if constexpr (!kReversed<T>) {
-                // NaN ranks first in a plain top-k: the vector's maximum is then NaN
-                bool has_nan = false;
-#pragma unroll
-                for (int c = 0; c < VEC; c += 2) has_nan = has_nan || __builtin_isunordered(xv[c], xv[c + 1]);
-                vm = has_nan ? __uint_as_float(0x7FC00000u) : vm;
             }
             vm_lds[wave][i][lane ^ ((i & 3) << 2)] = vm;
         });
@@ -179,21 +176,23 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
         // (block (vector i, lanes 16 r .. 16 r + 15) is the wave's block 4 i + r, and its 16
         // lane values lie side by side; the wave's blocks are read by the wave that wrote them)
         __builtin_amdgcn_wave_barrier();
+        constexpr bool kKeepNan = !SOFTMAX && !kReversed<T>;
+        auto larger = [](float a, float b, float c) { return kKeepNan ? maximum(a, b, c) : max3(a, b, c); };
         float bm = -INFINITY;
-        bool b_nan = false;
         if (lane < static_cast<uint32_t>(WB)) {
             const float4 *src = reinterpret_cast<const float4 *>(&vm_lds[wave][0][0] + lane * kBlockLanes);
 #pragma unroll
             for (int j = 0; j < kBlockLanes / 4; j++) {
                 const float4 v4 = src[j ^ ((lane >> 2) & 3)];  // (the block of vector lane / 4: its words are in the order 0..3 ^ that vector's number mod 4)
-                bm = fmaxf(fmaxf(bm, fmaxf(v4.x, v4.y)), fmaxf(v4.z, v4.w));
-                if constexpr (!SOFTMAX && !kReversed<T>) b_nan = b_nan || __builtin_isunordered(v4.x, v4.y) || __builtin_isunordered(v4.z, v4.w);
+                bm = j == 0 ? larger(v4.x, v4.y, v4.z) : larger(larger(bm, v4.x, v4.y), v4.z, v4.w);
+                if (j == 0) bm = larger(bm, v4.w, v4.w);
             }
+            if (SOFTMAX && bm != bm) bm = -INFINITY;  // (nothing but NaN)
             // the wave's block L = vector L / 4, lane row L % 4 starts at element
             // c0 + ((L / 4) * NT + wave * 64 + (L % 4) * 16) * VEC of the row
             const uint32_t e_block = c0 + ((lane / 4u) * NT + wave * kWave + (lane % 4u) * kBlockLanes) * VEC;
             if (FULL || e_block < c1) {
-                const uint32_t key = b_nan ? 0xFFFFFFFFu : order_key(bm);
+                const uint32_t key = order_key(bm);  // (all ones for NaN)
                 ws.bmax[static_cast<size_t>(row) * ws.blocks + e_block / (kBlockLanes * VEC)] = key;
                 if constexpr (WITH_MIN) {
                     const float4 *srcn = reinterpret_cast<const float4 *>(&vmin_lds[wave][0][0] + lane * kBlockLanes);
@@ -201,9 +200,9 @@ __device__ __forceinline__ void scan_chunk(const T *__restrict__ in, uint32_t n,
 #pragma unroll
                     for (int j = 0; j < kBlockLanes / 4; j++) {
                         const float4 v4 = srcn[j ^ ((lane >> 2) & 3)];
-                        bn = fminf(fminf(bn, fminf(v4.x, v4.y)), fminf(v4.z, v4.w));
+                        bn = minimum(minimum(bn, v4.x, v4.y), v4.z, v4.w);
                     }
-                    ws.bmin[static_cast<size_t>(row) * ws.blocks + e_block / (kBlockLanes * VEC)] = order_key(bn);
+                    ws.bmin[static_cast<size_t>(row) * ws.blocks + e_block / (kBlockLanes * VEC)] = bn == bn ? order_key(bn) : kKeyNegInf;  // (a NaN among them: nothing is known of the rest)
                 }
             }
         }
