@@ -841,6 +841,35 @@ def test_rows_of_few_values_whose_keys_end_in_ones(ops, rows, n, k, dtype):
     assert (half_ulp_diff(v, ev) if dtype == np.float16 else ulp_diff(v, ev)).max() <= (1 if dtype == np.float16 else 2)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("n,k", [(33000, 5), (128256, 50), (131073, 40), (300001, 60), (1000003, 200)])
+def test_rows_whose_cut_is_a_value_of_many_blocks(ops, dtype, n, k):
+    """One value in every sixth block or so, with none, some and k elements above it, in the row's first and last element and in
+    neighbours: more blocks reach it than are read again, and its first members come from the blocks in index order."""
+    rng = np.random.default_rng(n + k)
+    x = np.minimum(rng.standard_normal((5, n)).astype(np.float32), np.float32(3.0))
+    for r in range(5):
+        x[r, rng.choice(n, max(n // 400, 8 * (k + 1)), replace=False)] = 5.0
+        if r:
+            x[r, rng.choice(n, (k // 2, k - 1, k, 1)[r - 1], replace=False)] = 5.0 + rng.random((k // 2, k - 1, k, 1)[r - 1]).astype(np.float32)
+    x[:, -1] = 5.0
+    x[1, :3] = 5.0
+    x[3, 7] = -0.0
+    x = np.ascontiguousarray(x.astype(dtype))
+    for largest in (True, False):
+        y = x if largest else -x
+        v, ix = (host(t) for t in ops.topk(dev(y), k, largest=largest))
+        ov, oix = oracle.topk(y, k, largest=largest)
+        assert np.array_equal(ix, oix) and np.array_equal(v.view(np.uint8), ov.view(np.uint8)), largest
+    v, ix = (host(t) for t in ops.softmax_topk(dev(x), k))
+    ov, oix = oracle.softmax_topk(x, k)
+    if dtype == np.float32:   # (the values are within 2 ulp; which logit is the larger one, and so the order, does not depend on them)
+        assert ulp_diff(v, ov).max() <= 2 and np.array_equal(ix, oix)
+    else:                     # (sums agree to 2^-22: a probability on a boundary between two halves moves the row's order with it)
+        same = (v == ov).all(axis=-1)
+        assert half_ulp_diff(v, ov).max() <= 1 and same.sum() >= 3 and np.array_equal(ix[same], oix[same])
+
+
 @pytest.mark.parametrize("n,k", [(50257, 40), (128256, 50), (262144, 600)])
 def test_nan_of_any_payload_among_the_block_maxima_and_minima(ops, n, k):
     """Quiet and signalling NaN, alone, side by side and a block of nothing else: first in a plain top-k, last in the other direction."""

@@ -999,26 +999,50 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
     hit_cap = min(static_cast<uint32_t>(kPickHitCap), 3u * want + 64u);
     if (blocks > want + want / 4u) hit_cap = min(hit_cap, blocks - 1u);
     bool many_groups = have_list ? false : gather(thr, 1ull << 32, std::false_type{});
+    bool at_top = false;  // thr is the row's largest key, and k+1 blocks reach it
     if (many_groups) {
         // More than kPickHitCap blocks reach thr: the threads' shares of the block maxima are
         // not alike (rows sorted in runs as long as the stride between a thread's blocks put
         // every run's top block into the same few threads, and the (k+1)-th largest THREAD
         // maximum is then far below the (k+1)-th largest block maximum).  That one exactly,
-        // by a descent over all the keys, a barrier a bit: a dozen microseconds, on such rows.
+        // by a descent over all the keys, a barrier for two bits: some microseconds, on such rows.
+        // The row's largest key first: where k+1 blocks reach it -- a row of few values -- it is the answer.
         uint32_t exact_thr = 0;
-        for (int bit = 31; bit >= 0; bit--) {
-            const uint32_t trial = exact_thr | (1u << bit);
-            uint32_t c = 0;  // wave-uniform
+        const uint32_t wave_top = wave_max_u32(lmk);
+        if (lane == 0) sh.wave_thr[wave] = wave_top;
+        __syncthreads();
+        uint32_t top = sh.wave_thr[0];
 #pragma unroll
-            for (int e = 0; e < GE; e++) c += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= trial)));
-            uint32_t *wc = sh.scan_counts + (round & 1u) * NW;
+        for (int w = 1; w < NW; w++) top = max(top, sh.wave_thr[w]);
+        // (every thread gets the number of blocks that reach each of three values; a barrier inside)
+        auto reach3 = [&](uint32_t t1, uint32_t t2, uint32_t t3, uint32_t(&total)[3]) __attribute__((always_inline)) {
+            uint32_t c1 = 0, c2 = 0, c3 = 0;  // wave-uniform
+#pragma unroll
+            for (int e = 0; e < GE; e++) {
+                c1 += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= t1)));
+                c2 += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= t2)));
+                c3 += static_cast<uint32_t>(__popcll(__ballot(gk[e] >= t3)));
+            }
+            uint32_t *wc = sh.lane_key + (round & 1u) * (3 * NW);
             round++;
-            if (lane == 0) wc[wave] = c;
+            if (lane < 3u) wc[lane * NW + wave] = lane == 0u ? c1 : lane == 1u ? c2 : c3;
             __syncthreads();
-            uint32_t total = 0;
 #pragma unroll
-            for (int w = 0; w < NW; w++) total += wc[w];
-            if (total >= want) exact_thr = trial;
+            for (int i = 0; i < 3; i++) {
+                total[i] = 0;
+#pragma unroll
+                for (int w = 0; w < NW; w++) total[i] += wc[i * NW + w];
+            }
+        };
+        uint32_t total[3];
+        reach3(top, top, top, total);
+        at_top = total[0] >= want;
+        if (at_top) exact_thr = top;
+#pragma unroll 1
+        for (int bit = at_top ? -2 : 30; bit >= 0; bit -= 2) {
+            const uint32_t t1 = exact_thr | (1u << bit), t2 = exact_thr | (2u << bit), t3 = exact_thr | (3u << bit);
+            reach3(t1, t2, t3, total);
+            exact_thr = total[2] >= want ? t3 : total[1] >= want ? t2 : total[0] >= want ? t1 : exact_thr;
         }
         if (exact_thr > thr) {
             thr = exact_thr;
@@ -1094,17 +1118,91 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
             many_groups = true;
         }
     }
+    // emit(pos, j) for the first `need` elements with key `at`, in index order; fewer than k+1 elements lie above it.  They are in
+    // the first k+1 blocks, in index order, whose maximum reaches it: of those at most as many as there are elements above it hold
+    // none.  All threads call; returns how many were found (at least `need` unless the row has fewer).  (By reading the
+    // row from its start, as many rounds as the value is rare: [64,128256] k = 50 of 513 values 41 -> 20 us.)
+    auto first_equal = [&](uint32_t at, uint32_t need, auto emit) __attribute__((always_inline)) -> uint32_t {
+        uint32_t *offset = sh.lane_key;  // [block round][wave]
+        static_assert(GE * NW <= NT, "a word for each");
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < GE; e++) {
+            const uint32_t c = static_cast<uint32_t>(__popcll(__ballot(gk[e] >= at)));
+            if (lane == 0) offset[e * NW + wave] = c;
+        }
+        __syncthreads();
+        if (wave == 0) {
+            constexpr int PER = (GE * NW + kWave - 1) / kWave;
+            uint32_t c[PER], sum = 0;
+#pragma unroll
+            for (int i = 0; i < PER; i++) {
+                const uint32_t at_word = lane * PER + static_cast<uint32_t>(i);
+                c[i] = at_word < static_cast<uint32_t>(GE * NW) ? offset[at_word] : 0u;
+                sum += c[i];
+            }
+            uint32_t before = wave_inclusive_sum_u32(sum) - sum;
+            if (lane == kWave - 1) sh.wave_thr[0] = before + sum;
+#pragma unroll
+            for (int i = 0; i < PER; i++) {
+                const uint32_t at_word = lane * PER + static_cast<uint32_t>(i);
+                if (at_word < static_cast<uint32_t>(GE * NW)) offset[at_word] = before;
+                before += c[i];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < GE; e++) {
+            const bool pass = gk[e] >= at;
+            const uint64_t mask = __ballot(pass);
+            const uint32_t pos = offset[e * NW + wave] + lanes_below(mask);
+            if (pass && pos < static_cast<uint32_t>(kPickHitCap)) hits[pos] = static_cast<uint32_t>(e) * NT + tid;
+        }
+        __syncthreads();
+        const uint32_t items = min(sh.wave_thr[0], static_cast<uint32_t>(kPickHitCap)) * kBlockLanes;
+        uint32_t found = 0;  // the same in every thread
+#pragma unroll 1
+        for (uint32_t j0 = 0, turn = 0; j0 < items && found < need; j0 += NT, turn++) {
+            const uint32_t j = j0 + tid;
+            const uint32_t e0 = hits[j < items ? j / kBlockLanes : 0u] * BE + (j % kBlockLanes) * VEC;
+            const uint32_t end = j < items ? n : 0u;
+            Vec128<T> r;
+            r.v = make_uint4(0, 0, 0, 0);
+            if constexpr (ALIGNED) r.load(rowp + (e0 < end ? e0 : 0u));
+            else {
+                load_vec_any<false>(r, rowp, e0, n);
+                settle_vec(r, e0, n);
+            }
+            uint32_t members = 0;
+#pragma unroll
+            for (int c = 0; c < VEC; c++)
+                members |= e0 + static_cast<uint32_t>(c) < end && order_key(times_scale(r.get(c))) == at ? 1u << c : 0u;
+            const uint32_t mine_n = static_cast<uint32_t>(__popc(members)), incl = wave_inclusive_sum_u32(mine_n);
+            uint32_t *wc = sh.scan_counts + (turn & 1u) * NW;
+            if (lane == kWave - 1) wc[wave] = incl;
+            __syncthreads();
+            uint32_t pos = found + incl - mine_n;
+#pragma unroll
+            for (int w = 0; w < NW; w++) {
+                const uint32_t c = wc[w];
+                pos += static_cast<uint32_t>(w) < wave ? c : 0u;
+                found += c;
+            }
+            for (uint32_t left = members; left != 0u; left &= left - 1u, pos++)
+                if (pos < need) emit(pos, e0 + static_cast<uint32_t>(__builtin_ctz(left)));
+        }
+        return found;
+    };
     // Still too many: equal values en masse AT the threshold (rows of few distinct
     // values, constant rows).  k+1 elements reach thr, so the row's k+1 largest are the
     // elements above it -- fewer than k+1, or thr + 1 is the threshold to use -- and then
-    // the first elements equal to it, in index order: those are found by reading the row
-    // from its start, where a value this frequent turns up at once.
+    // the first elements equal to it, in index order.
     bool first_equals_only = false;  // the candidates hold only some of the elements equal to thr
     if ((many_groups || C2 > static_cast<uint32_t>(kFastCap)) && !thr_is_exact) {
         // (thr so far is a value rounded down; this needs the key of an element: the exact
         // (k+1)-th largest of the thread maxima it came from)
         __syncthreads();
-        thr = max(thr, threshold_of_thread_maxima(level_max, false, 32, std::false_type{}));
+        if (!at_top) thr = max(thr, threshold_of_thread_maxima(level_max, false, 32, std::false_type{}));
     }
     if ((many_groups || C2 > static_cast<uint32_t>(kFastCap)) && thr < 0xFFFFFFFFu) {
         __syncthreads();
@@ -1120,8 +1218,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
                 many_groups = false;
             } else {
                 const uint32_t need = want - above, at = thr;
-                const uint32_t found = first_members_by_scan<T, NT>(sh.scan_counts, rowp, n, need, at, at, scale,
-                                                                    [&](uint32_t pos, uint32_t j) { sh.cand[above + pos] = composite(at, j); });
+                const uint32_t found = first_equal(at, need, [&](uint32_t pos, uint32_t j) { sh.cand[above + pos] = composite(at, j); });
                 __syncthreads();
                 if (found >= need) {
                     if (tid == 0) sh.count = want;
