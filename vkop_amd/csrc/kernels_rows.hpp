@@ -1582,19 +1582,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
 #pragma unroll
         for (int i = 0; i < V; i++) {
             const uint32_t e0 = e_first + static_cast<uint32_t>(i) * NT * VEC;
+            // Plain top-k: three values an instruction and a key a vector, by a maximum that is NaN where the vector holds one
+            // (fmaxf of loaded values takes two instructions a value, a key six: [256,8400] f16 k = 80 9.3 -> 8.4 us,
+            // [64,24000] f32 10.6 -> 9.4). With a softmax the chain of three-operand maxima stood in the way of the
+            // exponentials beside it ([100,32000] f16 15.7 -> 17.4): there it stays a value at a time.
             float xv[VEC];
             float vm = -INFINITY;
             uint32_t vk = 0u;
 #pragma unroll
-            for (int c = 0; c < VEC; c++) {
-                xv[c] = in_range(ALIGNED ? e0 : e0 + c) ? getq(q[i], c) : -INFINITY;
-                vm = fmaxf(vm, xv[c]);
-                if constexpr (!SOFTMAX) vk = max(vk, in_range(ALIGNED ? e0 : e0 + c) ? order_key(xv[c]) : 0u);
+            for (int c = 0; c < VEC; c++) xv[c] = in_range(ALIGNED ? e0 : e0 + c) ? getq(q[i], c) : -INFINITY;
+            if constexpr (SOFTMAX) {
+#pragma unroll
+                for (int c = 0; c < VEC; c++) vm = fmaxf(vm, xv[c]);
+                lmax = fmaxf(lmax, vm);
+            } else {
+                vm = maximum(xv[0], xv[1], xv[2]);
+#pragma unroll
+                for (int c = 3; c < VEC; c += 2) vm = maximum(vm, xv[c], xv[c + 1 < VEC ? c + 1 : c]);
+                vk = in_range(e0) ? order_key(vm) : 0u;
+                lmax = max3(lmax, vm, vm);
+                lkey = max(lkey, vk);
             }
             vmax[i] = vm;
             vkey[i] = vk;
-            lmax = fmaxf(lmax, vm);
-            lkey = max(lkey, vk);
             if constexpr (SOFTMAX) {
                 if (i == 0 && !LOCAL) {
                     // reference of the wave's partial sum: the maximum of its first
