@@ -884,3 +884,24 @@ def test_nan_of_any_payload_among_the_block_maxima_and_minima(ops, n, k):
     for largest in (True, False):
         _, ix = (host(t) for t in ops.topk(xd, k, largest=largest))
         assert np.array_equal(ix, oracle.topk(x, k, largest=largest)[1]), largest
+
+
+@pytest.mark.parametrize("n,k", [(700, 20), (2999, 100), (8192, 40), (8191, 300), (16384, 10), (30000, 120)])
+def test_tie_at_the_cut_of_a_row_in_one_workgroup(ops, n, k):
+    """Half probabilities of 2 to 6000 of the smallest half at the k-th place: the tied group ends within the list of
+    candidates (its lower end is then read off the list) or goes on below it (it is looked for, and the row read again)."""
+    rng = np.random.default_rng(n + k)
+    rows = 40
+    x = rng.standard_normal((rows, n)).astype(np.float32) * np.float32(1.25)
+    cut = np.sort(x, axis=-1)[:, -k]
+    units = np.exp(np.linspace(np.log(2.0), np.log(6000.0), rows))
+    x[np.arange(rows), rng.integers(0, n, rows)] = cut + np.log(2.0 ** 24 / units).astype(np.float32)
+    x = x.astype(np.float16)
+    v, ix = (host(t) for t in ops.softmax_topk(dev(x), k))
+    ov, oix = oracle.softmax_topk(x, k)
+    # Sums agree to 2^-22, so a probability that close to a boundary between two halves, 2^-11 apart, may fall on either
+    # side of it: at most one in 2^10 of the values, a unit each.
+    same = (v.view(np.uint16) == ov.view(np.uint16)).all(axis=-1)
+    assert half_ulp_diff(v, ov).max() <= 1 and same.sum() >= rows - max(4, 2 * v.size >> 10) and np.array_equal(ix[same], oix[same])
+    equal = v[:, 1:] == v[:, :-1]
+    assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])

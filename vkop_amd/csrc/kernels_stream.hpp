@@ -1252,7 +1252,7 @@ __device__ __forceinline__ void pick_row(PickSharedUnion &smem, float *fscratch,
             return true;
         };
         BPS(12);
-        finish_row<T, NT, SOFTMAX>(sh, C2, partial, M, s_base, rowp, ov, oi, n, kk, want, wave_of, add_missing, scale,
+        finish_row<T, NT, SOFTMAX>(sh, C2, partial, M, s_base, rowp, ov, oi, n, kk, want, wave_of, add_missing, thr, scale,
                                    counts != nullptr ? counts + row : nullptr, top_p);
         BPS(13);
 #ifdef VKOP_STAMPS
