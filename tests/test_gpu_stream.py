@@ -905,3 +905,25 @@ def test_tie_at_the_cut_of_a_row_in_one_workgroup(ops, n, k):
     assert half_ulp_diff(v, ov).max() <= 1 and same.sum() >= rows - max(4, 2 * v.size >> 10) and np.array_equal(ix[same], oix[same])
     equal = v[:, 1:] == v[:, :-1]
     assert np.all(ix[:, 1:][equal] > ix[:, :-1][equal])
+
+
+@pytest.mark.parametrize("n", [8193, 12288, 16384, 16385, 32767])
+@pytest.mark.parametrize("k", [1, 33, 64])
+def test_a_small_k_of_rows_that_one_workgroup_holds(ops, n, k):
+    """Past the rows that 256 threads hold: one workgroup a row, or the scan, against the chunk kernels and the select
+    (rows.path = 1), bit for bit in plain top-k, whatever the order, the NaN and the equal values of the row."""
+    from vkop_amd import capi
+    rng = np.random.default_rng(n + k)
+    for dtype in (np.float32, np.float16):
+        for kind in ("llm", "levels", "sorted", "runs", "masked90", "nan_and_inf", "constant"):
+            x = dev(np.ascontiguousarray(_rows(kind, 5, n, rng).astype(dtype)))
+            for largest in (True, False):
+                got = []
+                for path in (0, 1):
+                    capi.tune("rows.path", path)
+                    got.append([host(t) for t in ops.topk(x, k, largest=largest)])
+                capi.tune("rows.path", 0)
+                (v, ix), (w, jx) = got
+                assert np.array_equal(ix, jx) and v.tobytes() == w.tobytes(), (kind, largest)
+        _compare_paths(ops, n, k, dtype, 5, ["llm", "levels", "masked90", "nan_and_inf", "coarse_levels"],
+                       capi.measure_path(capi.F32 if dtype == np.float32 else capi.F16, (5, n), -1, k))

@@ -671,10 +671,12 @@ constexpr int kWaveRowMaxK = 32;  // largest k served by the one-wave-per-row la
 constexpr int kTwoAndHalfListsMaxK = 408;  // largest k with rows_cap(k) <= kLocalCap
 constexpr int kWideRowMinK = 64;  // above it a row that fits one workgroup is given to one (of enough threads)
 
-// (for_size: what a call could use whatever rows.path says at that time.  full_list: also a k whose places the list of a
-// one-workgroup row holds less than 2.5 times, 409 to 511: usual rows list 1.2 to 1.4 times the places, and a second listing at most
+enum RowsKind { kPlainRows, kFusedRows, kScaledRows };  // top-k, softmax and top-k, the sampling form of that
+
+// (for_size: what a call could use whatever rows.path says at that time.  kind: which call it is for.
+// full_list: also a k whose places the list of a one-workgroup row holds less than 2.5 times, 409 to 511: usual rows list 1.2 to 1.4 times the places, and a second listing at most
 // 2 k + 1 elements, 1023 of the list's 1024.)
-RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false, bool full_list = false) {
+RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false, bool full_list = false, RowsKind kind = kFusedRows) {
     RowsCfg c;
     if (v.g.inner != 1 || k > vkop::kFastMaxK || v.g.n == 0 || v.g.outer == 0) return c;
     const uint32_t vec = dtype == VKOP_HIP_F32 ? 4u : 8u;
@@ -739,6 +741,19 @@ RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false, 
         const uint32_t blocks = (n + vkop::kBlockLanes * vec - 1) / (vkop::kBlockLanes * vec);
         if (pick < 0 && wide >= 0 && !forced_nt && g_rows_path.load() != 1 &&
             4ull * blocks < (rows <= 16 ? 8ull : 7ull) * (static_cast<uint64_t>(k) + 1u))
+            pick = wide;
+        // The rows that 512 threads hold (to 16384 elements), and in plain top-k of halves with k > 32 those that 1024
+        // hold, whatever the blocks: one launch that reads a row once and keeps it, for the scan's two.  us a call, scan
+        // and pick / one workgroup a row: top-k [64,16384] f16 k = 64 14.6 / 7.6, k = 5 9.0 / 6.5, [256,8400] f32 k = 40
+        // 11.2 / 7.4, [3000,12000] f16 k = 20 78 / 69, of 513 values 85 / 76, [64,24000] f16 k = 64 12.0 / 9.1; fused
+        // [256,16384] f16 k = 64 20.5 / 13.2, [16,12000] f32 k = 20 10.2 / 9.3.  Beyond 16384 elements the scan stays
+        // ahead where it spreads the work over more CUs: fused ([16,28000] f32 k = 20 10.0 / 12.0, all exponentials of a
+        // row on one), and in rows of few values ([64,24000] k = 5 f32 10.0 / 13.8, f16 10.6 / 13.1; k = 40 f16 13.7 /
+        // 13.1, f32 10.6 / 12.9); and so it does in the scaled form of a few float rows that start off 16 bytes
+        // ([2,12001] k = 20 10.6 / 11.0, [200,12001] 12.8 / 11.7, [1500,12001] 153 / 66).
+        if (pick < 0 && wide >= 0 && !forced_nt && !for_size && g_rows_path.load() != 1 && g_rows_fused.load() == 0 &&
+            (shapes[wide][0] <= 512 ? kind != kScaledRows || rows > 64 || vec == 8u || n % vec == 0u
+                                    : kind == kPlainRows && vec == 8u && k > kWaveRowMaxK))
             pick = wide;
         const bool one_workgroup = pick >= 0;
         for (int i = 0; i < 6 && !one_workgroup; i++) {
@@ -814,7 +829,7 @@ struct ScanCfg {
 // blocks per wanted place (below), or with more blocks than the kernel behind the scan takes
 // in, are left to the other kernels.
 // (for_size: what a call could use whatever the tuning knobs say at that time)
-ScanCfg choose_scan_cfg(const View &v, int k, int dtype, bool for_size = false) {
+ScanCfg choose_scan_cfg(const View &v, int k, int dtype, bool for_size = false, RowsKind kind = kFusedRows) {
     ScanCfg c;
     if (v.g.inner != 1 || k > vkop::kMaxK || v.g.n == 0 || v.g.outer == 0) return c;
     const uint32_t vec = dtype == VKOP_HIP_F32 ? 4u : 8u;
@@ -852,10 +867,10 @@ ScanCfg choose_scan_cfg(const View &v, int k, int dtype, bool for_size = false) 
     }
     if (4ull * blocks < quarters * places) return c;
     if (k <= vkop::kFastMaxK && !for_size) {
-        // a row that ONE workgroup of the chunk kernel holds (up to 8192 elements for k <= 64, up to
-        // 32768 beyond): one launch instead of two, measured 1.4 to 1.6 times faster on spread-out
+        // a row that ONE workgroup of the chunk kernel holds (up to 16384 elements, for a larger k up to
+        // 32768): one launch instead of two, measured 1.1 to 1.9 times faster on spread-out
         // rows ([1024,4096] k = 16: 9.0 against 14.5 us; [64,32768] k = 200: 12.5 against 20.3 us)
-        const RowsCfg one = choose_rows_cfg(v, k, dtype);
+        const RowsCfg one = choose_rows_cfg(v, k, dtype, false, false, kind);
         if (one.ok && one.g == 1 && one.nt >= 256) return c;
     }
     if (!big && (blocks + vkop::kPickThreads - 1) / vkop::kPickThreads > 32u) return c;
@@ -1169,10 +1184,10 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
     // [64,128256] k = 50 61 -> 12.9, [8,262144] k = 1024 46.8 -> 21.2, [1024,4096] k = 64 29.7 -> 10.2.
     // (2^22 rows and more: a grid of a thousand threads a row is more than HIP takes, the select's is not.)
     const bool routed = largest || (g_rows_path.load() != 1 && v.g.outer < (1u << 22));
-    ScanCfg sc = routed ? choose_scan_cfg(v, k, dtype) : ScanCfg{};
+    ScanCfg sc = routed ? choose_scan_cfg(v, k, dtype, false, kPlainRows) : ScanCfg{};
     // (without an order, the rows of the large-k kernels keep the select and the listing it has always given)
     if (!largest && !sorted && sc.g2 != 0) sc = ScanCfg{};
-    RowsCfg c = (routed && !sc.ok) ? choose_rows_cfg(v, k, dtype) : RowsCfg{};
+    RowsCfg c = (routed && !sc.ok) ? choose_rows_cfg(v, k, dtype, false, false, kPlainRows) : RowsCfg{};
     if (!largest && (c.g != 1 || c.nt < 256 || c.cap > static_cast<uint32_t>(vkop::kLocalCap))) c = RowsCfg{};
     if (c.ok && g_rows_path.load() != 1 && select_is_faster(v, k, c, 16 / sizeof(T), largest != 0)) c = RowsCfg{};
     if (routed && !sc.ok && !c.ok && k > kTwoAndHalfListsMaxK && v.g.outer <= 256 && g_rows_path.load() != 1) {
@@ -1180,7 +1195,7 @@ int topk_impl(const T *in, T *values, int32_t *indices, const View &v, int k, in
         // whatever workspace is given, as the kernels below that need none.  us a call, those below / this, f32: [16,16000] k = 500
         // 30.9 / 13.2, of levels 49 / 19, sorted 28.7 / 25.3; [256,8400] k = 420 25.6 / 12.5, smallest first 25.8 / 12.4; [8,5000]
         // k = 450 18.9 / 11.1; f16 [16,16000] k = 500 44.4 / 13.3; but [300,5000] f32 25.3 / 33.9, [300,9000] f16 42.1 / 44.1.
-        const RowsCfg full = choose_rows_cfg(v, k, dtype, false, true);
+        const RowsCfg full = choose_rows_cfg(v, k, dtype, false, true, kPlainRows);
         if (full.ok && full.g == 1 && !select_is_faster(v, k, full, 16 / sizeof(T), largest != 0)) {
             const RowsLayout none;
             if (largest) return launch_rows<T, false>(in, values, indices, v, k, full, nullptr, none, st);
@@ -1662,7 +1677,7 @@ int vkop_hip_softmax_topk_sampling(const void *in, void *out_values, int32_t *ou
     if ((reinterpret_cast<uintptr_t>(workspace) & (kAlign - 1)) != 0)
         return fail(VKOP_HIP_ERR_WORKSPACE, "workspace must be %zu-byte aligned", kAlign);
     const hipStream_t st = as_stream(stream);
-    const ScanCfg sc = choose_scan_cfg(v, k, dtype);
+    const ScanCfg sc = choose_scan_cfg(v, k, dtype, false, kScaledRows);
     auto run = [&](auto tag) -> int {
         using T = decltype(tag);
         const T *x = static_cast<const T *>(in);
@@ -1676,7 +1691,7 @@ int vkop_hip_softmax_topk_sampling(const void *in, void *out_values, int32_t *ou
             return launch_tiny<T, true>(x, values, out_indices, v, k, tiny, st, false, true, scale, out_counts, top_p);
         // a row that one workgroup holds: its kernel in the scaled form
         if (!sc.ok) {
-            const RowsCfg rc = choose_rows_cfg(v, k, dtype);
+            const RowsCfg rc = choose_rows_cfg(v, k, dtype, false, false, kScaledRows);
             if (rc.ok && rc.g == 1 && rows_cap(k) <= static_cast<uint32_t>(vkop::kLocalCap) && g_rows_fused.load() == 0) {
                 const RowsLayout lr = rows_layout(v, rc);
                 return launch_rows<T, true>(x, values, out_indices, v, k, rc, workspace, lr, st, true, scale, out_counts, top_p);
