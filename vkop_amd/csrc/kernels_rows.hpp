@@ -1704,6 +1704,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
                 hi = max(hi, cs.wave_thr[w]);
             }
             uint32_t t = lo;
+            // (1024 threads full of halves that start on any element, with a softmax, are at the end of their registers: there the
+            // rounds below took [5,23197] k = 81 from 19.1 to 19.9 us; the scaled form from 22.3 to 20.8)
+            constexpr bool kBitByBit = SOFTMAX && !SAMPLING && !ALIGNED && sizeof(T) == 2 && NT >= 1024 && V >= 4;
             if (lo != hi) {
                 uint32_t kv[NW];
 #pragma unroll
@@ -1716,7 +1719,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(T) ==
                     for (int w = 0; w < NW; w++) cnt += static_cast<uint32_t>(__popcll(__ballot(kv[w] >= trial)));
                     return cnt;
                 };
-                if constexpr (NW >= 8) {
+                if constexpr (NW >= 8 && !kBitByBit) {
                     // Many waves: four bits (eight waves: three) a round, each wave a value of them.  (Every wave every bit, 16
                     // ballots each and four waves a SIMD, was this kernel's longest step: [16,8400] f32 k = 300 9.9 -> 8.7 us, [256,6000] k = 200 by a tenth.)
                     constexpr int B = NW >= 16 ? 4 : 3;
