@@ -91,8 +91,7 @@ def test_one_launch_and_two_whatever_the_wait(lib, B, C, N, dtype):
 
 
 def test_a_recording_replayed(lib):
-    """A recording's launch is the same in every replay; the call's word in the workspace is not.  Other inputs each time, eager calls
-    on the same workspace between."""
+    """Other inputs in every replay, eager calls on the same workspace between."""
     from vkop_amd import capi
     lib.vkop_hip_measure_polls(100)
     B, C, N = 8, 40, 900
@@ -124,3 +123,47 @@ def test_a_recording_replayed(lib):
         total = int(two.count[0])
         for rec, n in ((got, count), (one.out, one.count)):
             assert torch.equal(n, two.count) and torch.equal(rec[:total], two.out[:total]), seed
+
+
+@pytest.mark.parametrize("B,C", [(2, 80), (8, 20)])
+def test_a_recording_whose_workspace_serves_another_operator(B, C):
+    """Every replay has its arguments from the recording, and the same top-k before it in the same workspace, whose lists, keys and
+    counters lie where a call's own words do; the end of that workspace is put back, too, to what it was before the replay.  (Fewer
+    candidates than places: the pairs' numbers differ from replay to replay.)"""
+    from vkop_amd import capi
+    capi.init(0)
+    N, per_class, n, k = 700, 300, 33600, 300
+    boxes, scores = make(B, C, N, torch.float32, 1)
+    rows = torch.randn((1, n), generator=torch.Generator(device="cuda").manual_seed(2), device="cuda")
+    values, indices = torch.empty((1, k), device="cuda"), torch.empty((1, k), dtype=torch.int32, device="cuda")
+    room = B * C * per_class
+    out, count = torch.zeros((room, 3), dtype=torch.int32, device="cuda"), torch.zeros(2, dtype=torch.int32, device="cuda")
+    nms_bytes = capi.nms_workspace_bytes(B, C, N, per_class)
+    need = max(nms_bytes, capi.topk_workspace_bytes(capi.F32, (1, n), -1, k))
+    memory = torch.zeros(need + 256, dtype=torch.uint8, device="cuda")
+    at = memory.data_ptr() + (-memory.data_ptr()) % 256
+    end = memory[at - memory.data_ptr():][nms_bytes - 256:nms_bytes]
+
+    def calls(stream):
+        capi.topk(rows.data_ptr(), values.data_ptr(), indices.data_ptr(), capi.F32, (1, n), -1, k, 1, 1, at, need, stream)
+        capi.nms(boxes.data_ptr(), scores.data_ptr(), out.data_ptr(), room, count.data_ptr(), capi.F32, B, C, N, 0, per_class, 0.45, 0.8,
+                 at, need, stream)
+
+    stream = torch.cuda.Stream()
+    calls(stream.cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        calls(stream.cuda_stream)
+    for seed in range(3, 9):
+        b, s = make(B, C, N, torch.float32, seed)
+        boxes.copy_(b)
+        scores.copy_(s)
+        before = end.clone()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = oracle.nms(b.cpu().numpy(), s.cpu().numpy(), 0.45, 0.8, per_class, max_candidates=2048)
+        assert count.tolist() == [len(want), 0], seed
+        assert np.array_equal(out[:len(want)].cpu().numpy(), want), seed
+        if seed % 2:
+            end.copy_(before)

@@ -24,8 +24,8 @@
 //      batch and class: the result does not depend on scheduling (the reference appends through a
 //      global atomic counter).  Of pairs that the chip holds at once every workgroup publishes its
 //      number of records, waits for those of the pairs before it and writes its own (place_records);
-//      of more, the selected box indices go to the pair's segment of the workspace and
-//      nms_pack_kernel writes them all.
+//      of more, and in a recording, the selected box indices go to the pair's segment of the
+//      workspace and nms_pack_kernel writes them all.
 #pragma once
 
 #include "device_utils.hpp"
@@ -103,49 +103,44 @@ __device__ __forceinline__ bool nms_overlap(const float4 &a, const float4 &b, fl
 }
 
 // ---- a pair's records, by the workgroup that selected them ---------------------------------------
-// What a workgroup publishes: under a tag of 40 bits, its number of records (at most 2048), whether boxes were left out, and whether
-// it has given up waiting.  The tag comes from the launch and from a word in memory that every call moves on, so that neither the
-// workspace's former contents nor a recording's replay before has it: nothing has to be cleared.
+// What a workgroup publishes: under the call's tag of 40 bits, its number of records (at most 2048), whether boxes were left out, and
+// whether it has given up waiting.  No other call has the tag, so nothing has to be cleared, whatever operator the workspace served
+// before.  (It is an argument of the launch.  In a recording, whose every replay has the same arguments, the words of the replay
+// before would pass for this one's: a recorded call takes the two launches.  A word of the workspace that every replay moves
+// on does not tell them apart: it is scratch to the other operators.)
 struct NmsJoined {
-    uint64_t *words;  // a word a pair, kNmsCopies times, then the word of the call and the tag of the call a workgroup last gave up in
+    uint64_t *words;  // a word a pair, kNmsCopies times, then the tag of the call that a workgroup last gave up in
     int32_t *out, *out_count;
     uint32_t capacity, polls;
-    uint64_t launch;
+    uint64_t tag;  // 1 .. 2^40 - 1
 };
 // Copies of the words, each read by every eighth workgroup: a thousand that read the same few lines again and again wait for each
 // other ([16,80,8400] f32 18.5 us with one copy, 17.0 with 8, 17.1 with 32).
 constexpr uint32_t kNmsCopies = 8;
 __host__ __device__ constexpr uint32_t nms_copy_stride(uint32_t pairs) { return (pairs + 31u) / 32u * 32u; }
-constexpr size_t nms_words(uint32_t pairs) { return static_cast<size_t>(kNmsCopies) * nms_copy_stride(pairs) + 2; }
-constexpr int kNmsCallWord = 0, kNmsLateWord = 1;  // (behind the copies)
+constexpr size_t nms_words(uint32_t pairs) { return static_cast<size_t>(kNmsCopies) * nms_copy_stride(pairs) + 1; }
 constexpr uint32_t kNmsCount = 0xFFFFu, kNmsOver = 1u << 16, kNmsGaveUp = 1u << 17;
-__device__ __forceinline__ uint64_t nms_tag(uint64_t launch, uint64_t call) {  // (1 .. 2^40 - 1)
-    return ((call * 0x9E3779B97F4A7C15ull + launch * 0xC2B2AE3D27D4EB4Full) >> 24) | 1ull;
-}
 __device__ __forceinline__ void nms_put_record(int32_t *out, uint32_t capacity, uint32_t at, int32_t batch, int32_t cls, int32_t box) {
     if (at >= capacity) return;
     out[static_cast<size_t>(at) * 3 + 0] = batch;
     out[static_cast<size_t>(at) * 3 + 1] = cls;
     out[static_cast<size_t>(at) * 3 + 2] = box;
 }
-// The end of a call, one thread: the number of all records, the overflow flag, the (-1, -1, -1) behind the last record, and the word
-// of the next call (every workgroup has published by now, with this one's).
-__device__ __forceinline__ void nms_put_total(const NmsJoined &j, uint64_t *extra, uint64_t call, uint32_t total, bool over) {
+// The end of a call, one thread: the number of all records, the overflow flag, and the (-1, -1, -1) behind the last record.
+__device__ __forceinline__ void nms_put_total(const NmsJoined &j, uint32_t total, bool over) {
     j.out_count[0] = static_cast<int32_t>(total);
     j.out_count[1] = over ? 1 : 0;
     nms_put_record(j.out, j.capacity, total, -1, -1, -1);
-    publish(extra + kNmsCallWord, call + 1u);
 }
 // The records of workgroups that gave up, as far as all the pairs before them have arrived: a wave.  (Two that find the same ones
 // write the same.)
-__device__ __forceinline__ void nms_place_late(const NmsJoined &j, uint64_t *extra, uint64_t call, uint64_t tag, const int32_t *selected,
-                                               uint32_t pairs, uint32_t C, uint32_t max_sel) {
+__device__ __forceinline__ void nms_place_late(const NmsJoined &j, const int32_t *selected, uint32_t pairs, uint32_t C, uint32_t max_sel) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
     uint32_t total = 0, over = 0;
     for (uint32_t base = 0; base < pairs; base += kWave) {
         const uint32_t q = base + lane;
-        const uint64_t word = q < pairs ? fetch(j.words + q) : tag << 24;
-        const uint64_t absent = __ballot((word >> 24) != tag);
+        const uint64_t word = q < pairs ? fetch(j.words + q) : j.tag << 24;
+        const uint64_t absent = __ballot((word >> 24) != j.tag);
         const uint32_t w = static_cast<uint32_t>(word), have = absent != 0ull ? static_cast<uint32_t>(__builtin_ctzll(absent)) : static_cast<uint32_t>(kWave);
         const uint32_t incl = wave_inclusive_sum_u32(w & kNmsCount);
         over |= w & kNmsOver;
@@ -163,7 +158,7 @@ __device__ __forceinline__ void nms_place_late(const NmsJoined &j, uint64_t *ext
         total += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(incl), kWave - 1));
     }
     const bool any_over = __ballot(over != 0u) != 0ull;
-    if (lane == 0) nms_put_total(j, extra, call, total, any_over);
+    if (lane == 0) nms_put_total(j, total, any_over);
 }
 // All threads call, behind a barrier after the last write to picks (LDS: the n selected boxes in order).  The wait needs no
 // particular number of workgroups on the chip to end: after `polls` looks a workgroup leaves its boxes in its segment, says so, and
@@ -171,13 +166,13 @@ __device__ __forceinline__ void nms_place_late(const NmsJoined &j, uint64_t *ext
 // at least one of the two finds the other, and the records are placed.  (A counter of the workgroups that are done, on whose
 // last one the rest could be left, costs their turns at one address: 1280 of them 10 us.)
 template <int NT>
-__device__ __forceinline__ void place_records(const NmsJoined &j, uint64_t call, const uint32_t *picks, uint32_t n, bool over, int32_t *selected,
+__device__ __forceinline__ void place_records(const NmsJoined &j, const uint32_t *picks, uint32_t n, bool over, int32_t *selected,
                                               uint32_t pair, uint32_t pairs, uint32_t C, uint32_t max_sel, uint32_t *scratch) {
     constexpr int NW = NT / kWave, U = NT >= 1024 ? 2 : 6;
     const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform_u32(tid) / kWave;
-    const uint64_t tag = nms_tag(j.launch, call), own = (tag << 24) | (over ? kNmsOver : 0u) | n;
+    const uint64_t tag = j.tag, own = (tag << 24) | (over ? kNmsOver : 0u) | n;
     const uint32_t stride = nms_copy_stride(pairs);
-    uint64_t *extra = j.words + kNmsCopies * stride;
+    uint64_t *late_word = j.words + kNmsCopies * stride;
     if (tid < kNmsCopies) publish(j.words + tid * stride + pair, own);
     const uint64_t *words = j.words + pair % kNmsCopies * stride;
     uint32_t before = 0, flags = over ? kNmsOver : 0u;
@@ -228,17 +223,17 @@ __device__ __forceinline__ void place_records(const NmsJoined &j, uint64_t call,
         if (wave != 0) return;
         if (lane == 0) {
             publish(j.words + pair, own | kNmsGaveUp);
-            publish(extra + kNmsLateWord, tag);
+            publish(late_word, tag);
         }
         drain_stores();
-        nms_place_late(j, extra, call, tag, selected, pairs, C, max_sel);
+        nms_place_late(j, selected, pairs, C, max_sel);
         return;
     }
-    const uint64_t late = wave == 0 ? fetch(extra + kNmsLateWord) : 0ull;
+    const uint64_t late = wave == 0 ? fetch(late_word) : 0ull;
     const int32_t batch = static_cast<int32_t>(pair / C), cls = static_cast<int32_t>(pair % C);
     for (uint32_t r = tid; r < n; r += NT) nms_put_record(j.out, j.capacity, before + r, batch, cls, static_cast<int32_t>(picks[r]));
-    if (pair == pairs - 1 && tid == 0) nms_put_total(j, extra, call, before + n, (flags & kNmsOver) != 0u);
-    if (wave == 0 && late == tag) nms_place_late(j, extra, call, tag, selected, pairs, C, max_sel);
+    if (pair == pairs - 1 && tid == 0) nms_put_total(j, before + n, (flags & kNmsOver) != 0u);
+    if (wave == 0 && late == tag) nms_place_late(j, selected, pairs, C, max_sel);
 }
 
 // Without JOINED: counts[pair] = boxes selected; counts[pairs + pair] = 1 if more than
@@ -279,7 +274,6 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
     Pick *const picks = reinterpret_cast<Pick *>(comp);
     const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform_u32(tid) / kWave;  // (scalar)
     const uint32_t pair = blockIdx.x, batch = pair / C;
-    const uint64_t call = JOINED ? fetch(joined.words + kNmsCopies * nms_copy_stride(pairs) + kNmsCallWord) : 0ull;  // (under the scores' loads)
     const T *srow = scores + static_cast<size_t>(pair) * N;
     const T *brow = boxes + static_cast<size_t>(batch) * N * 4;
     if (tid < static_cast<uint32_t>(kNmsMaxCandidates / 64)) active[tid] = ~0ull;  // positions at or after K are masked where read
@@ -459,7 +453,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT >= 1024 ?
     };
     auto finish = [&](bool over) __attribute__((always_inline)) {
         if constexpr (JOINED) {
-            place_records<NT>(joined, call, picks, min(chosen, max_sel), over, selected, pair, pairs, C, max_sel, &wave_n[0][0]);
+            place_records<NT>(joined, picks, min(chosen, max_sel), over, selected, pair, pairs, C, max_sel, &wave_n[0][0]);
         } else if (tid == 0) {
             counts[pair] = min(chosen, max_sel);
             counts[pairs + pair] = over ? 1u : 0u;

@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -1356,11 +1357,26 @@ size_t nms_workspace(int B, int C, int N, int max_per_class) {
     const size_t pairs = static_cast<size_t>(B) * C;
     return kTicketBytes + align_up(2 * pairs * sizeof(uint32_t)) + align_up(pairs * nms_max_sel(N, max_per_class) * sizeof(int32_t));
 }
-// With the words of the one launch (in a workspace of the size above, without them, a call takes the two).
+// With the words of the one launch (in a workspace of the size above, without them, a call takes the two, as a recorded one does).
 size_t nms_joined_workspace(int B, int C, int N, int max_per_class) {
     const uint64_t pairs = static_cast<uint64_t>(B) * C;
     const size_t two = nms_workspace(B, C, N, max_per_class);
     return pairs > vkop::kNmsHeldNarrow ? two : two + align_up(vkop::nms_words(static_cast<uint32_t>(pairs)) * sizeof(uint64_t));
+}
+
+// A tag of the one launch: not 0, and no two of 2^38 calls have the same.  Another process that has had the workspace, or another build of
+// the library in this one, starts somewhere else.
+uint64_t nms_call_tag() {
+    static std::atomic<uint64_t> calls{(static_cast<uint64_t>(std::chrono::system_clock::now().time_since_epoch().count()) ^
+                                        reinterpret_cast<uintptr_t>(&g_nms_threads)) * 0xD6E8FEB86659FD93ull};
+    return ((calls.fetch_add(1, std::memory_order_relaxed) * 0x9E3779B97F4A7C15ull) >> 24) | 1ull;  // (the golden ratio's multiples lie apart)
+}
+// Whether calls on the stream are being recorded, or the runtime does not say.
+bool recorded(hipStream_t st) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
 }
 
 template <typename T>
@@ -1376,10 +1392,10 @@ int nms_impl(const T *boxes, const T *scores, int32_t *out, int out_capacity, in
     const int knob = g_nms_threads;  // 0: by the number of pairs
     const bool narrow = knob > 0 ? knob == vkop::kNmsThreadsNarrow : pairs >= static_cast<uint32_t>(vkop::kNmsNarrowMinPairs);
     const bool one_launch = pairs <= (narrow ? vkop::kNmsHeldNarrow : vkop::kNmsHeldWide) && ws_bytes >= nms_joined_workspace(B, C, N, max_per_class) &&
-                            reinterpret_cast<uintptr_t>(ws) % sizeof(uint64_t) == 0;
+                            reinterpret_cast<uintptr_t>(ws) % sizeof(uint64_t) == 0 && !recorded(st);
     auto *words = reinterpret_cast<uint64_t *>(static_cast<unsigned char *>(ws) + nms_workspace(B, C, N, max_per_class));
     const vkop::NmsJoined joined{one_launch ? words : nullptr, out, out_count, static_cast<uint32_t>(out_capacity), nms_polls(),
-                                 one_launch ? g_joined_calls.fetch_add(1, std::memory_order_relaxed) : 0u};
+                                 one_launch ? nms_call_tag() : 0u};
 #define VKOP_NMS_LAUNCH(NT, WHOLE, JOINED)                                                                                 \
     vkop::nms_kernel<T, NT, WHOLE, JOINED><<<pairs, NT, 0, st>>>(boxes, scores, selected, counts, pairs,                   \
                                                                  static_cast<uint32_t>(C), static_cast<uint32_t>(N),       \
