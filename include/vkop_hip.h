@@ -262,7 +262,9 @@ int vkop_hip_tune(const char *name, int value);
  * are 0 when the radix select or the general one-workgroup-per-line kernels would
  * run.  The plain top-k takes the same shape, except on rows that one workgroup
  * of this kernel holds but an exact select ranks sooner (many short rows for a large
- * k), where it runs that, and for k from 409 to 511 on up to 256 rows that one
+ * k), where it runs that, on rows that one workgroup of this kernel could hold and
+ * that have few elements a place (half precision up to 32768 elements, and more than 256
+ * rows), where it runs this kernel and the fused call the scan + pick pair, and for k from 409 to 511 on up to 256 rows that one
  * workgroup holds, where it runs this kernel and the fused call the general ones.
  * The sampling call takes the same threads and chunks, on rows that 512 or 1024
  * threads hold with more loads a thread (8, half precision 4).  Any out pointer may

@@ -149,6 +149,16 @@ def test_route_planner_without_a_gpu(lib):
     assert 64 * 1024 < need <= 4 << 20
 
 
+def test_rows_of_one_workgroup_up_to_a_row_a_cu(lib):
+    """Rows that 512 threads hold go to one workgroup each while there are no more of them than CUs, and to the scan beyond."""
+    for dt in (capi.F32, capi.F16):
+        for n in (8193, 8400, 10001, 12000, 16383, 16384):
+            for k in (1, 5, 20, 32):
+                for rows in (1, 17, 255, 256, 257, 300, 1023, 1024, 5000):
+                    assert capi.measure_path(dt, (rows, n), -1, k) == (1 if rows <= 256 else 2), (dt, rows, n, k)
+    assert capi.measure_path(capi.F32, (256, 16385), -1, 20) == 2
+
+
 def test_rows_plan_tells_the_loads_that_run(lib):
     """Rows that a wide workgroup holds are launched with as few vectors a thread as hold the row, unless the shape is forced."""
     F32, F16 = capi.F32, capi.F16

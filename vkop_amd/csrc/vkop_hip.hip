@@ -744,18 +744,29 @@ RowsCfg choose_rows_cfg(const View &v, int k, int dtype, bool for_size = false, 
             4ull * blocks < (rows <= 16 ? 8ull : 7ull) * (static_cast<uint64_t>(k) + 1u))
             pick = wide;
         // The rows that 512 threads hold (to 16384 elements), and in plain top-k of halves with k > 32 those that 1024
-        // hold, whatever the blocks: one launch that reads a row once and keeps it, for the scan's two.  us a call, scan
+        // hold, on up to a row a CU: one launch that reads a row once and keeps it, for the scan's two.  us a call, scan
         // and pick / one workgroup a row: top-k [64,16384] f16 k = 64 14.6 / 7.6, k = 5 9.0 / 6.5, [256,8400] f32 k = 40
-        // 11.2 / 7.4, [3000,12000] f16 k = 20 78 / 69, of 513 values 85 / 76, [64,24000] f16 k = 64 12.0 / 9.1; fused
-        // [256,16384] f16 k = 64 20.5 / 13.2, [16,12000] f32 k = 20 10.2 / 9.3.  Beyond 16384 elements the scan stays
+        // 11.2 / 7.4, [64,24000] f16 k = 64 12.0 / 9.1; fused [256,16384] f16 k = 64 20.5 / 13.2, [16,12000] f32 k = 20
+        // 10.2 / 9.3.  Beyond 16384 elements the scan stays
         // ahead where it spreads the work over more CUs: fused ([16,28000] f32 k = 20 10.0 / 12.0, all exponentials of a
         // row on one), and in rows of few values ([64,24000] k = 5 f32 10.0 / 13.8, f16 10.6 / 13.1; k = 40 f16 13.7 /
-        // 13.1, f32 10.6 / 12.9); and so it does in the scaled form of a few float rows that start off 16 bytes
-        // ([2,12001] k = 20 10.6 / 11.0, [200,12001] 12.8 / 11.7, [1500,12001] 153 / 66).
-        if (pick < 0 && wide >= 0 && !forced_nt && !for_size && g_rows_path.load() != 1 && g_rows_fused.load() == 0 &&
-            (shapes[wide][0] <= 512 ? kind != kScaledRows || rows > 64 || vec == 8u || n % vec == 0u
-                                    : kind == kPlainRows && vec == 8u && k > kWaveRowMaxK))
-            pick = wide;
+        // 13.1, f32 10.6 / 12.9); and so it does in the scaled form of a few float rows whose length takes them off 16 bytes
+        // ([2,12001] k = 20 10.6 / 11.0, [200,12001] 12.8 / 11.7; rows of a whole number of vectors in a tensor that starts off
+        // them are as fast either way or faster so, [64,16384] k = 50 12.3 / 10.2).
+        // With more rows than CUs the workgroups take turns, and the scan is ahead again: fused f32 k = 5 [256,12000] 12.4 /
+        // 10.0, [257,12000] 13.4 / 16.8, k = 20 [768,16384] 20.7 / 30.0, [3000,16384] 68 / 113, f16 k = 5 [3000,12000] 71 / 97;
+        // scaled f32 k = 40 of 513 values [300,12000] 16.8 / 28.8; top-k k = 5 f32 [300,12000] 11.6 / 13.6, f16 [1000,10001]
+        // 21.3 / 27.0, smallest first f32 k = 20 [1500,10001] 33 / 78.  Not in plain top-k of few blocks a place, which the
+        // scan's threshold hardly tells apart: f16 [300,10001] k = 40 17.6 / 13.9, [300,16384] k = 64 17.7 / 13.5, f32
+        // [768,8400] k = 64 28.3 / 23.3; at 2.7 a place f16 k = 40 [300,14003] 13.9 / 14.2, of 513 values 19.9 / 16.1, [1000,14003]
+        // 25.5 / 28.4.
+        if (pick < 0 && wide >= 0 && !forced_nt && !for_size && g_rows_path.load() != 1 && g_rows_fused.load() == 0) {
+            const bool narrow = shapes[wide][0] <= 512, half = vec == 8u, plain = kind == kPlainRows;
+            const bool few_blocks = plain && 4ull * blocks < (half && rows <= 768 ? 11ull : 9ull) * (static_cast<uint64_t>(k) + 1u);
+            const bool one = narrow ? kind != kScaledRows || rows > 64 || half || n % vec == 0u : plain && half && k > kWaveRowMaxK;
+            if (one && rows > 256 && !few_blocks) return c;
+            if (one) pick = wide;
+        }
         const bool one_workgroup = pick >= 0;
         for (int i = 0; i < 6 && !one_workgroup; i++) {
             const uint32_t span = static_cast<uint32_t>(shapes[i][0]) * shapes[i][1] * vec;
@@ -1153,7 +1164,7 @@ int launch_rows(const T *in, T *values, int32_t *indices, const View &v, int k, 
 //  * about as many vectors as places, or fewer, whose maxima bound nothing, in rows that the list does not hold whole: [8,1500] f16
 //    k = 196 29 / 19, [1500,1500] 167 / 28;
 //  * smallest first up to two vectors a place, where the select ran before and its time does not depend on the data, and by the
-//    thousand of rows just past what 256 threads hold: [3300,8196] k = 23 f16 189 / 124, f32 132 / 121, [3300,10094] f16 191 / 161;
+//    thousand of rows just past what 256 threads hold, where they have too few blocks for the scan (choose_rows_cfg): [3300,8196] k = 23 f16 189 / 124, f32 132 / 121, [3300,10094] f16 191 / 161;
 //  * 256 threads, short rows by the thousand, which the select reads again from the cache: [6000,400] f32 k = 44 40 / 30, k = 104
 //    52 / 36, [30000,800] f16 k = 104 275 / 207; but [300,400] f32 k = 104 9.3 / 10.8, [1500,800] f16 k = 75 18 / 20;
 //  * 512 and 1024 threads, more rows than CUs (a workgroup each at a time) of few elements for so many threads, a line for each of the

@@ -36,7 +36,8 @@ int vkop_hip_measure_tags(unsigned first, unsigned count, unsigned *tags);
 
 /* Which kernels a fused call (largest first) on this tensor would run -- and a plain
  * top-k, which leaves route 1 for an exact select where that is faster (select_is_faster,
- * vkop_hip.hip) -- with the current tuning settings: 4 = rows_tiny_kernel (one wave per row), 2 =
+ * vkop_hip.hip) and takes it on some rows of few blocks a place that the fused call leaves
+ * to route 2 (choose_rows_cfg) -- with the current tuning settings: 4 = rows_tiny_kernel (one wave per row), 2 =
  * rows_scan_kernel + rows_pick_kernel, 3 = rows_scan_kernel + bigpick_gather_kernel +
  * bigpick_rank_kernel, 1 = rows_chunk_kernel (+ rows_merge_kernel when a row is
  * split), 0 = other kernels, -1 = bad arguments. */
