@@ -124,6 +124,10 @@ WALK_KINDS = ["half_half", "three_allowed", "nan_and_inf", "huge", "masked90", "
               "flat_with_peaks"]
 
 
+# a row of halves has half as many blocks as one of floats: too few for the pick kernel, or few enough for the large-k pair
+OTHER_TYPE_ONLY = {(50257, 300, "float16"), (40000, 255, "float16"), (50257, 200, "float32")}
+
+
 def _compare_paths(ops, n, k, dtype, rows, kinds, path):
     """The library's choice of kernels (which has to be `path`) against the kernels
     rows.path = 1 selects, and both against the oracle."""
@@ -131,8 +135,9 @@ def _compare_paths(ops, n, k, dtype, rows, kinds, path):
     rng = np.random.default_rng(n * 31 + k)
     dt = capi.F32 if dtype == np.float32 else capi.F16
     capi.tune("rows.path", 0)
-    if capi.measure_path(dt, (rows, n), -1, k) != path:
+    if (n, k, np.dtype(dtype).name) in OTHER_TYPE_ONLY:
         pytest.skip("not a shape these kernels take in this element type")
+    assert capi.measure_path(dt, (rows, n), -1, k) == path, (rows, n, k)
     for kind in kinds:
         x = np.ascontiguousarray(_rows(kind, rows, n, rng).astype(dtype))
         xd = dev(x)
@@ -182,8 +187,8 @@ def _compare_paths(ops, n, k, dtype, rows, kinds, path):
                                  (262144, 64), (100003, 33), (500000, 100), (300000, 511), (50257, 300)])
 def test_scan_pick_pair_equals_chunk_merge_and_oracle(ops, n, k, dtype):
     """(From k = 256 on the pair is the library's choice on more than 16 rows only, there also
-    with fewer than two blocks per wanted place.)"""
-    _compare_paths(ops, n, k, dtype, 20 if k >= 256 else 6, KINDS, 2)
+    with fewer than two blocks per wanted place; of rows that one workgroup holds on more than 256.)"""
+    _compare_paths(ops, n, k, dtype, 20 if k >= 256 else 260 if n <= 16384 else 6, KINDS, 2)
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
@@ -927,3 +932,54 @@ def test_a_small_k_of_rows_that_one_workgroup_holds(ops, n, k):
                 assert np.array_equal(ix, jx) and v.tobytes() == w.tobytes(), (kind, largest)
         _compare_paths(ops, n, k, dtype, 5, ["llm", "levels", "masked90", "nan_and_inf", "coarse_levels"],
                        capi.measure_path(capi.F32 if dtype == np.float32 else capi.F16, (5, n), -1, k))
+
+
+@pytest.mark.parametrize("rows,n,k,off,kernels", [(3, 12001, 20, 0, 2), (64, 8401, 5, 0, 2), (1, 16383, 40, 1, 2), (3, 12000, 20, 0, 1), (3, 12000, 20, 1, 1),
+                                                  (65, 12001, 20, 0, 1), (257, 12001, 20, 0, 2), (257, 16384, 64, 2, 2), (16, 8193, 64, 0, 1)])
+def test_sampling_of_float_rows_that_one_workgroup_or_the_scan_takes(ops, rows, n, k, off, kernels):
+    """The scaled form on rows of 8193 to 16384 floats: up to 64 whose length takes them off 16 bytes, and more than 256, the scan and
+    the pick kernel, others one workgroup a row (16 of 8193 and k = 64 have too few blocks for the scan); a tensor's start does not
+    count.  With the first kernel alone (a library that can leave one out) the results are written by one-workgroup rows only."""
+    import ctypes
+    from vkop_amd import capi
+    rng = np.random.default_rng(n + k)
+    x = np.concatenate([_rows(kind, rows, n, rng) for kind in ("llm", "bf16")])[::2] if rows > 1 else _rows("llm", 1, n, rng)
+    big = torch.empty(rows * n + 4, device="cuda")
+    xd = big[off:off + rows * n].view(rows, n)
+    xd.copy_(dev(x))
+    v, ix, c = (host(t) for t in ops.softmax_topk_sampling(xd, k, 1.25, 0.9))
+    ov, oix, _ = oracle.softmax_topk_sampling(x, k, 1.25, 0.9)
+    assert ulp_diff(v, ov).max() <= 2 and np.array_equal(c, oracle.topp_count(v, 0.9))
+    xs = x * np.float32(1.25)
+    op = oracle.softmax(xs)
+    for r in range(rows):
+        check_fused_invariants(xs[r], v[r], ix[r])
+        if well_separated_cut(op[r], xs[r], k):
+            assert np.array_equal(ix[r], oix[r]), r
+    part = ctypes.CDLL(capi.BENCH_LIB_PATH)
+    part.vkop_hip_softmax_topk_sampling.argtypes = capi.lib()._signatures["vkop_hip_softmax_topk_sampling"][1]
+    values, indices, counts = torch.full((rows, k), -7.0, device="cuda"), *(torch.full((m,), -7, dtype=torch.int32, device="cuda") for m in (rows * k, rows))
+    ws, size = ops.Workspace().get(capi.softmax_topk_workspace_bytes(capi.F32, (rows, n), -1, k))
+    try:
+        assert part.vkop_hip_measure_stages(1) == 0
+        assert part.vkop_hip_softmax_topk_sampling(xd.data_ptr(), values.data_ptr(), indices.data_ptr(), counts.data_ptr(), capi.F32,
+                                                   (ctypes.c_int * 2)(rows, n), 2, -1, k, 1.25, 0.9, ws, size,
+                                                   torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+    finally:
+        part.vkop_hip_measure_stages(3)
+    assert bool((values == -7.0).all()) == (kernels == 2) and (kernels == 2 or np.array_equal(host(values), v))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16], ids=["f32", "f16"])
+@pytest.mark.parametrize("rows,n,k", [(257, 10001, 40), (300, 8400, 64), (257, 9361, 64), (257, 16640, 64), (260, 24000, 40), (1024, 8193, 5)])
+def test_plain_topk_on_more_rows_than_cus(ops, rows, n, k, dtype):
+    """One workgroup a row where the row has few blocks a place, the scan otherwise: the oracle's values and indices either way."""
+    rng = np.random.default_rng(rows + n)
+    bits = np.uint16 if dtype == np.float16 else np.uint32
+    for kind in ("bf16", "levels", "runs") if rows < 1000 else ("bf16",):
+        x = np.ascontiguousarray(_rows(kind, rows, n, rng).astype(dtype))
+        for largest in (True, False):
+            t, tj = ops.topk(dev(x), k, largest=largest)
+            et, ej = oracle.topk(x, k, largest=largest)
+            assert np.array_equal(host(tj), ej) and np.array_equal(host(t).view(bits), et.view(bits)), (kind, largest)
