@@ -538,7 +538,7 @@ int softmax_rows(const T *in, T *out, const View &v, const SoftmaxPlan &p, int n
 #define VKOP_ROW(V)                                                                                     \
     if (p.shape.v == V) {                                                                               \
         with_caching(caching, [&](auto cache) {                                                         \
-            constexpr int CACHE = MAX_ONLY || cache == vkop::kCacheBoth ? cache & vkop::kCacheLoads : cache; \
+            constexpr int CACHE = cache & vkop::kCacheLoads; /* (no more: softmax_caching) */            \
             vkop::softmax_row_kernel<T, V, MAX_ONLY, CACHE><<<rows, p.shape.nt, 0, st>>>(from, to, v.g.n, nan_where, nan_value); \
         });                                                                                             \
         return launched("softmax_row_kernel");                                                          \
