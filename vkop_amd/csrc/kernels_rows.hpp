@@ -145,12 +145,6 @@ __device__ __forceinline__ float wave_max_f32_uniform(float v) {
 
 constexpr uint32_t kKeyNegInf = 0x007FFFFFu;  // order key of -inf, the smallest key of a real element
 
-// Float threshold equivalent to an order-key threshold: x passes iff
-// !(x < thr_f).  Keys at or below the key of -inf mean "everything passes".
-__device__ __forceinline__ float key_threshold_to_float(uint32_t thr) {
-    return thr <= kKeyNegInf ? -INFINITY : ordered_to_float(thr);
-}
-
 // One wave finds a lower bound of the `want`-th largest of NW * 64 keys held in
 // LDS (key 0 = no element): bitwise descent over the top `bits` bits, counting
 // with ballots; the untouched low bits stay zero, which only lowers the bound.
