@@ -65,8 +65,8 @@ struct ChunkStat {
 // with the next one's loads in flight, the form before, copies at 4.8 to 5.7 TB/s where waves that
 // end copy at 6.2 to 6.6.  [524288,1024] f16 422 -> 343 us (6.3 TB/s), f32 827 -> 728; [302592,197]
 // f16 83 -> 48 us (element by element before), f32 133 -> 102 -> 84; [65536,64] f32 13.7 -> 7.2 us; with ordinary accesses
-// [165000,50] f32 19.7 -> 12.6, [300000,100] f32 64 -> 43.  By the terms f16 [304568,197] 49.9 -> 44.9, [83756,197] 15.6 -> 13.5,
-// [2441,8192] 14.2 -> 13.0, [8,1000,8000] axis 1 73 -> 68, f32 [64,128256] 16.2 -> 15.4.
+// [165000,50] f32 19.7 -> 12.6, [300000,100] f32 64 -> 43.  By the terms f16 [304568,197] 48.4 -> 43.8, [83756,197] 14.9 -> 12.9,
+// [2441,8192] 14.1 -> 13.1, [8,1000,8000] axis 1 73 -> 68, f32 [64,128256] 15.7 -> 15.2.
 template <int CTRL> __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
 }

@@ -409,6 +409,12 @@ SoftmaxPlan plan_softmax(const View &v, int dtype) {
 //   vector, where a wave's rows are one piece, f16 n = 50  180 MB 73 / 72 / 75 / 74
 //   lines: f32 [8,21,n] of 50 MB 21.5 / 18.0 / 20.8 / 20.4, of 180 MB 68 / 70 / 71 / 75; off the 128 bytes f32 [8,100,n] of 50 MB
 //   40 / 36 / 27 / 21, 180 MB 145 / 135 / 97 / 87, f16 [8,80,n] of 120 MB 93 / 82 / 55 / 56, 250 MB 190 / 163 / 131 / 105
+// How much of it is the residency of those five buffers, all non-temporal / so: the shared lines' part hardly (f32 [300000,100] 64.6 /
+// 46.4, of buffers that each wait for a gigabyte of others 65.5 / 46.5, [482233,197] 166 / 132 and 166 / 132, f16 [8,80,93750] axis 1
+// 144 / 68 and 145 / 77, [302592,197] 46.8 / 43.7 and 47.1 / 43.9), the whole lines' all: f32 [60000,256] 25.9 / 19.4, of buffers that come from
+// memory 26.1 / 27.9, behind a kernel that writes the input 40.1 / 39.7 with it, between that and one that reads the output, a
+// buffer each, 61.4 / 60.2; [2400,8192] 31.8 / 25.3, 32.7 / 33.4, 50.2 / 49.9, 75.6 / 76.3; with stores [120000,256] 44.0 / 39.1, 47.0 / 45.2, 75.2 / 89.2
+// (what waits is written back under the next kernel's reads), 122.8 / 118.8; lines [8,21,180224] 50.2 / 42.3, 50.5 / 50.0, 82.9 / 85.4, 123 / 126.
 // (The one-launch kernel of long rows, whose tensor is in registers before any of it is written, is as fast or faster without:
 // f32 [64,128256] 15.7 / 16.4 / 18.0 / 17.7.)
 template <typename T> int softmax_caching(const View &v, const SoftmaxPlan &p, const T *in, const T *out, bool max_only) {
@@ -1375,12 +1381,13 @@ size_t nms_joined_workspace(int B, int C, int N, int max_per_class) {
     return pairs > vkop::kNmsHeldNarrow ? two : two + align_up(vkop::nms_words(static_cast<uint32_t>(pairs)) * sizeof(uint64_t));
 }
 
-// A tag of the one launch: not 0, and no two of 2^38 calls have the same.  Another process that has had the workspace, or another build of
+// A tag of the one launch: not 0, and no two of 2^37 calls in a row have the same (N of the golden ratio's multiples lie 2^64 / (sqrt(5) N)
+// apart at least, and a tag tells 2^25 apart).  Another process that has had the workspace, or another build of
 // the library in this one, starts somewhere else.
 uint64_t nms_call_tag() {
     static std::atomic<uint64_t> calls{(static_cast<uint64_t>(std::chrono::system_clock::now().time_since_epoch().count()) ^
                                         reinterpret_cast<uintptr_t>(&g_nms_threads)) * 0xD6E8FEB86659FD93ull};
-    return ((calls.fetch_add(1, std::memory_order_relaxed) * 0x9E3779B97F4A7C15ull) >> 24) | 1ull;  // (the golden ratio's multiples lie apart)
+    return ((calls.fetch_add(1, std::memory_order_relaxed) * 0x9E3779B97F4A7C15ull) >> 24) | 1ull;
 }
 // Whether calls on the stream are being recorded, or the runtime does not say.
 bool recorded(hipStream_t st) {
